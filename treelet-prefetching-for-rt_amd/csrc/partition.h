@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 #include "rtx.h"
 
 namespace rtxk {
@@ -19,16 +21,14 @@ struct Partition {
   uint64_t* list_offsets = nullptr;  // [n+1]
   uint64_t* list_nodes = nullptr;    // [n_list] node offsets
   // Treelet-contiguous images for LDS staging: image t holds the bytes of
-  // the nodes treelet t owns, in list order; stage_slot[s] is the 64-byte
-  // position of node slot s inside its owner's image.
+  // the nodes treelet t owns, in list order.
   uint8_t* images = nullptr;
   uint64_t* image_offset = nullptr;  // [n]
   uint32_t* image_bytes = nullptr;   // [n]
-  uint32_t* stage_slot = nullptr;    // [arena_bytes/64]
   uint32_t* image_slots = nullptr;   // [images_total/64] node slot at each 64-byte unit (instance tail: none)
   uint64_t images_total = 0;
-  uint32_t max_image_bytes = 0;
   rtx_treelet_summary summary{};
+  std::vector<void*> owned;  // the allocations behind the arrays above
   // treelet layout (remapBVHToTreeletLayout), built on request
   uint64_t* layout_remap = nullptr;    // [arena_bytes/64] layout offset of each node, ~0 for none
   int32_t* layout_metadata = nullptr;  // [n * budget/64] entry places relative to the root's, -1 past a list

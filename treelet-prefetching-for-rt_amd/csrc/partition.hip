@@ -10,13 +10,17 @@
 //  * When the next breadth-first entry does not fit, every entry still queued
 //    becomes a pending root (:1132-1211).
 //  * A treelet depends only on its root, so all pending roots of one round
-//    are formed in parallel, one wave each, and a root reached twice (a BLAS
-//    shared by several instances) is formed once; the reference forms it
-//    again with an identical result.
-//  * The wave walks the breadth-first queue in chunks of 64 entries: an
+//    are formed in parallel, by eight lanes or a wave each, and a root reached
+//    twice (a BLAS shared by several instances) is formed once; the reference
+//    forms it again with an identical result.
+//  * The lanes walk the breadth-first queue in chunks of 8 or 64 entries: an
 //    inclusive scan of the entry sizes finds how many fit, the accepted
 //    entries append their children in order (exclusive scan of child counts),
-//    which is exactly the sequential pop-front / push-back order.
+//    which is exactly the sequential pop-front / push-back order whatever the
+//    chunk.
+//  * Forming the treelets visits every reachable node and checks what the
+//    structural walk (run_validate) checks; the walk itself runs only on a
+//    failure, to report the error it finds first.
 //  * Node lists keep first occurrences (:1310-1336); roots are numbered in
 //    ascending offset order (:1332); a node belongs to the largest root offset
 //    whose list holds it, which is what iterating the ordered root map and
@@ -50,191 +54,475 @@ __device__ __forceinline__ T wave_incl_scan(T v, uint32_t lane) {
   return v;
 }
 
+// [off, off + len) lies in the arena (no overflow for any offset)
+__device__ __forceinline__ bool in_arena(uint64_t off, uint64_t len, uint64_t bytes) {
+  return off <= bytes && bytes - off >= len;
+}
+
+// Running totals of a partition: list entries (also the next free place of the
+// raw lists), treelet bytes, error bits, whether some node is in two lists or
+// twice in one, and the largest treelet.
+struct FormTotals {
+  unsigned long long listed, bytes;
+  uint32_t error, shared, max_bytes, max_nodes;
+};
+
+// Rounds launched between two host synchronisations: round j of a batch reads
+// its frontier's size from cnt[j], which round j - 1 counted up, so the host
+// waits once per batch (a 1M-triangle scene takes four rounds at 8 KiB).
+constexpr uint32_t kRoundBatch = 4;
+
 struct FormParams {
   const uint8_t* A;
   uint64_t bytes;
   uint64_t tlas;
   uint32_t budget;
-  uint32_t first_round;
-  const uint64_t* frontier_in;
-  uint32_t n_in;
-  uint64_t* frontier_out;
-  uint32_t* n_out;
+  uint32_t first;  // the frontier is the TLAS header (one treelet)
+  uint32_t round;  // within the batch
+  uint32_t n0;     // frontier entries of the batch's first round
+  uint32_t base0;  // treelets of all earlier batches
+  uint32_t* cnt;   // [kRoundBatch + 1] frontier entries of round j (j > 0)
+  uint32_t* nbig;  // [kRoundBatch] entries of round j left to form_large
+  const uint64_t* in;
+  uint64_t* out;
+  uint32_t* big;  // their frontier indices
   uint32_t* root_flag;
   uint32_t* owner_root1;
+  uint8_t* kind;
   uint32_t* raw_list;
   uint64_t raw_cap;
-  unsigned long long* raw_count;
-  uint4* desc;
-  uint32_t* desc_count;
-  uint64_t* scratch;
-  uint32_t qcap;
-  uint32_t lcap;
-  uint32_t* work;
-  uint32_t* error;
+  uint4* desc;  // per treelet: root slot, place and length of its raw list, bytes
+  FormTotals* tot;
+  // form_large's queues when they do not fit in LDS, queue_bytes per workgroup
+  uint8_t* scratch;
+  uint64_t queue_bytes;
+  uint32_t qcap, lcap;
 };
 
-__global__ __launch_bounds__(256) void form_treelets(FormParams p) {
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t wave = blockIdx.x * 4 + (threadIdx.x >> 6);
-  uint64_t* Q = p.scratch + (uint64_t)wave * (p.qcap + (p.lcap + 1) / 2);
-  uint32_t* L = reinterpret_cast<uint32_t*>(Q + p.qcap);
-  const uint8_t* A = p.A;
-  while (true) {
-    uint32_t idx = 0;
-    if (lane == 0) idx = atomicAdd(p.work, 1u);
-    idx = __shfl(idx, 0, 64);
-    if (idx >= p.n_in) break;
-    uint32_t err = 0;
-    uint32_t head = 0, tail = 1, nl = 0;
-    int64_t remaining = p.budget;
-    uint64_t acc_bytes = 0;
-    uint32_t root_slot;
-    if (p.first_round) {
-      root_slot = (uint32_t)(p.tlas >> 6);
-      const uint64_t rootoff = *reinterpret_cast<const uint64_t*>(A + p.tlas);
-      const uint64_t top = p.tlas + rootoff;
-      if ((top & 63) || top + 64 > p.bytes) err |= kErrRange;
-      if (lane == 0) {
-        L[0] = root_slot;
-        Q[0] = qentry((uint32_t)(top >> 6), kTopInternal);
-      }
-      nl = 1;
-      remaining -= 64;
-      acc_bytes = 64;
-    } else {
-      const uint64_t e = p.frontier_in[idx];
-      root_slot = q_slot(e);
-      if (lane == 0) Q[0] = e;
-    }
-    __threadfence();
-    bool first_chunk = true;
-    while (err == 0) {
-      const uint32_t chunk = min(64u, tail - head);
-      uint64_t e = 0;
-      uint32_t sz = 0;
-      if (lane < chunk) {
-        e = Q[head + lane];
-        sz = q_kind(e) == kTopLeaf ? 192u : 64u;
-      }
-      const uint32_t incl = wave_incl_scan<uint32_t>(sz, lane);
-      const bool acc = lane < chunk && (int64_t)incl <= remaining;
-      const uint64_t accmask = __ballot(acc);
-      const uint32_t count = (uint32_t)__popcll(accmask);
-      if (count == 0) {
-        if (first_chunk) err |= kErrBudget;
-        break;
-      }
-      // children and list additions of accepted entries
-      uint32_t ladd = 0, nch = 0;
-      uint64_t ch[6];
-      uint32_t extra_slot = 0;
-      if (acc) {
-        const uint32_t slot = q_slot(e), kind = q_kind(e);
-        const uint64_t off = (uint64_t)slot << 6;
-        ladd = 1;
-        if (kind == kTopInternal || kind == kBotInternal) {
-          if (off + 64 > p.bytes) {
-            err |= kErrRange;
-          } else {
-            const uint8_t* nd = A + off;
-            const int32_t co = *reinterpret_cast<const int32_t*>(nd + 12);
-            uint64_t c = off + (uint64_t)((int64_t)co * 64);
+__device__ __forceinline__ uint32_t frontier_count(const FormParams& p) { return p.round ? p.cnt[p.round] : p.n0; }
+// index of the round's first treelet
+__device__ __forceinline__ uint32_t treelet_base(const FormParams& p) {
+  uint32_t b = p.base0;
+  for (uint32_t j = 0; j < p.round; ++j) b += j ? p.cnt[j] : p.n0;
+  return b;
+}
+
+__device__ __forceinline__ uint8_t slot_kind(uint32_t qkind) {
+  return qkind == kTopLeaf ? kSlotInstance : qkind == kBotLeaf ? kSlotPrim : kSlotInternal;
+}
+
+// Child offset and the six size/type bytes (22..27) of the internal node at off.
+struct NodeKids {
+  uint64_t first;
+  uint32_t lo, hi;  // info bytes of children 0-3, 4-5
+  __device__ __forceinline__ uint32_t info(int i) const { return ((i < 4 ? lo >> (8 * i) : hi >> (8 * (i - 4)))) & 0x3fu; }
+};
+__device__ __forceinline__ NodeKids load_kids(const uint8_t* A, uint64_t off) {
+  const uint4 a = *reinterpret_cast<const uint4*>(A + off);
+  const uint4 b = *reinterpret_cast<const uint4*>(A + off + 16);
+  NodeKids k;
+  k.first = off + (uint64_t)((int64_t)(int32_t)a.w * 64);
+  k.lo = __builtin_amdgcn_alignbyte(b.z, b.y, 2);
+  k.hi = b.z >> 16;
+  return k;
+}
+
+// The structural walk's checks of one internal node's children; counts them.
+__device__ __forceinline__ uint32_t check_kids(const NodeKids& n, uint32_t kind, uint64_t bytes, uint32_t& count) {
+  uint32_t err = 0;
+  uint64_t c = n.first;
+  count = 0;
 #pragma unroll
-            for (int i = 0; i < 6; ++i) {
-              const uint32_t info = nd[22 + i] & 0x3fu;
-              const uint32_t size = info & 3u, type = info >> 2;
-              if (size > 0) {
-                if ((c & 63) || c + 64 > p.bytes) err |= kErrRange;
-                uint32_t k;
-                if (kind == kTopInternal) {
-                  if (type != 0 && type != 1) err |= kErrType;
-                  k = type != 0 ? kTopLeaf : kTopInternal;
-                } else {
-                  k = type != 0 ? kBotLeaf : kBotInternal;
-                }
-                ch[nch++] = qentry((uint32_t)(c >> 6), k);
-              }
-              c += (uint64_t)size * 64;
-            }
-          }
-        } else if (kind == kTopLeaf) {
-          if (off + 128 > p.bytes) {
-            err |= kErrRange;
-          } else {
-            const uint64_t bvh = *reinterpret_cast<const uint64_t*>(A + off + 64);
-            const uint64_t h = off + bvh;
-            if ((h & 63) || h + 64 > p.bytes) {
-              err |= kErrRange;
-            } else {
-              const uint64_t r = h + *reinterpret_cast<const uint64_t*>(A + h);
-              if ((r & 63) || r + 64 > p.bytes) err |= kErrRange;
-              extra_slot = (uint32_t)(h >> 6);
-              ladd = 2;
-              ch[nch++] = qentry((uint32_t)(r >> 6), kBotInternal);
-            }
-          }
-        } else {
-          if (off + 64 > p.bytes) err |= kErrRange;
+  for (int i = 0; i < 6; ++i) {
+    const uint32_t info = n.info(i), size = info & 3u, type = info >> 2;
+    if (size == 0) continue;
+    count++;
+    if (!in_arena(c, (uint64_t)size * 64, bytes)) err |= kErrRange;
+    if (kind == kTopInternal ? (type > 1u || (type == 1u && size != 2u)) : type == 1u) err |= kErrType;
+    c += (uint64_t)size * 64;
+  }
+  return err;
+}
+
+template <typename F>
+__device__ __forceinline__ void each_kid(const NodeKids& n, uint32_t kind, F&& f) {
+  uint32_t slot = (uint32_t)(n.first >> 6);
+#pragma unroll
+  for (int i = 0; i < 6; ++i) {
+    const uint32_t info = n.info(i), size = info & 3u;
+    if (size == 0) continue;
+    f(slot, kind + (info >> 2 ? 1u : 0u));  // the leaf kind follows the internal one
+    slot += size;
+  }
+}
+static_assert(kTopLeaf == kTopInternal + 1 && kBotLeaf == kBotInternal + 1, "each_kid");
+
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// ---- small treelets: eight lanes each, 32 per workgroup ----------------------
+// Most treelets are small (5.5 nodes on average on the 1M-triangle scene at 8
+// KiB: what a BLAS's first treelet leaves over), so a wave per treelet idles
+// 58 of its 64 lanes, and the time was its chain of queue writes, device-scope
+// fences and four atomics on shared counters.  Here eight treelets share a
+// wave, their queues stay in LDS, and a workgroup's 32 treelets reserve their
+// list, frontier and statistics with one atomic each.  A treelet with an
+// instance leaf, or whose queue outgrows kSmallQueue, is left to form_large.
+// On the 1M-triangle scene at 8 KiB (253,071 treelets) forming them took 12.3
+// ms with a wave each and takes 0.44 ms; bound now by the dependent reads of a
+// treelet (entry, node, its leaves' flags) and the shared counters.
+// Frontiers of fewer than kSmallMin entries go to form_large at once: they are
+// the scene's few large treelets (TLAS, BLAS roots), which 64 lanes walk
+// faster, and a wave each does not fill the chip.  The whole build at 1,024 /
+// 2,048 / 16,384: 16 instances of 1,024 triangles 242 / 244 / 386 us (8 KiB),
+// 256 instances 500 / 464 / 788, and at 1 KiB 603 / 616 / 748.
+constexpr uint32_t kSmallLanes = 8;
+constexpr uint32_t kSmallGroups = 256 / kSmallLanes;
+constexpr uint32_t kSmallQueue = 128;
+constexpr uint32_t kSmallStride = kSmallQueue + kSmallLanes;  // the groups of a wave start in different banks
+constexpr uint32_t kSmallMin = 2048;
+
+__global__ __launch_bounds__(256) void form_small(FormParams p) {
+  const uint32_t n_in = frontier_count(p);
+  if (p.first || n_in < kSmallMin) return;
+  __shared__ uint32_t qs[kSmallGroups * kSmallStride];
+  __shared__ uint8_t qk[kSmallGroups * kSmallStride];
+  __shared__ uint32_t g_list[kSmallGroups], g_pend[kSmallGroups], g_big[kSmallGroups];
+  __shared__ unsigned long long list_base;
+  const uint32_t lane = threadIdx.x & 63u, j = threadIdx.x & (kSmallLanes - 1), g = threadIdx.x / kSmallLanes;
+  const uint32_t gsh = lane & ~(kSmallLanes - 1);  // the group's first lane in its wave
+  uint32_t* Q = qs + g * kSmallStride;
+  uint8_t* K = qk + g * kSmallStride;
+  const uint32_t base = treelet_base(p);
+  const uint32_t room = p.budget / 64;
+  uint32_t sum_nodes = 0, max_nodes = 0;  // of the workgroup's treelets (thread 0)
+  auto group_any = [&](bool v) -> bool { return ((__ballot(v) >> gsh) & 0xffull) != 0; };
+  for (uint32_t b = blockIdx.x; b * kSmallGroups < n_in; b += gridDim.x) {
+    const uint32_t idx = b * kSmallGroups + g;
+    uint32_t head = 0, tail = 0, err = 0, root_slot = 0;
+    bool large = false;
+    if (idx < n_in) {
+      const uint64_t e = p.in[idx];
+      root_slot = q_slot(e);
+      large = q_kind(e) == kTopLeaf;
+      if (j == 0) {
+        Q[0] = q_slot(e);
+        K[0] = (uint8_t)q_kind(e);
+      }
+      tail = 1;
+    }
+    wave_fence();
+    // every entry is 64 bytes here: the budget is a node count
+    bool more = tail != 0 && !large;
+    while (more) {
+      const uint32_t chunk = min(kSmallLanes, tail - head), take = min(chunk, room - head);
+      if (take == 0) break;
+      uint32_t kind = kBotLeaf, slot = 0, count = 0, bad = 0;
+      NodeKids kids{0, 0, 0};
+      if (j < take) {
+        slot = Q[head + j];
+        kind = K[head + j];
+        if (kind == kTopInternal || kind == kBotInternal) {
+          kids = load_kids(p.A, (uint64_t)slot << 6);
+          bad = check_kids(kids, kind, p.bytes, count);
         }
       }
-      if (__ballot(err != 0)) {
-        for (int o = 32; o > 0; o >>= 1) err |= __shfl_xor(err, o, 64);
+      if (group_any(kind == kTopLeaf)) {
+        large = true;
         break;
       }
-      const uint32_t lincl = wave_incl_scan<uint32_t>(ladd, lane);
-      const uint32_t cincl = wave_incl_scan<uint32_t>(nch, lane);
-      const uint32_t ltot = __shfl(lincl, 63, 64);
-      const uint32_t ctot = __shfl(cincl, 63, 64);
-      if (nl + ltot > p.lcap || tail + ctot > p.qcap) {
-        err |= kErrQueue;
+      if (group_any(bad != 0)) {
+        err |= bad;
         break;
       }
-      if (acc) {
-        uint32_t lp = nl + lincl - ladd;
-        L[lp] = q_slot(e);
-        if (ladd == 2) L[lp + 1] = extra_slot;
-        uint32_t cp = tail + cincl - nch;
-        for (uint32_t k = 0; k < nch; ++k) Q[cp + k] = ch[k];
+      uint32_t incl = count;
+#pragma unroll
+      for (uint32_t d = 1; d < kSmallLanes; d <<= 1) {
+        const uint32_t y = __shfl_up(incl, d, kSmallLanes);
+        if (j >= d) incl += y;
       }
-      __threadfence();
-      const uint32_t used = __shfl(incl, (int)count - 1, 64);
-      remaining -= used;
-      acc_bytes += used;
-      head += count;
-      tail += ctot;
-      nl += ltot;
-      first_chunk = false;
-      if (count < chunk || head == tail) break;
+      const uint32_t total = __shfl(incl, kSmallLanes - 1, kSmallLanes);
+      if (tail + total > kSmallQueue) {
+        large = true;
+        break;
+      }
+      uint32_t at = tail + incl - count;
+      if (count)
+        each_kid(kids, kind, [&](uint32_t s, uint32_t k) {
+          Q[at] = s;
+          K[at] = (uint8_t)k;
+          at++;
+        });
+      wave_fence();
+      head += take;
+      tail += total;
+      more = take == chunk && head < tail;
     }
-    if (err) {
-      if (lane == 0) atomicOr(p.error, err);
-      continue;
+    if (err) atomicOr(&p.tot->error, err);
+    const bool done = idx < n_in && !large && !group_any(err != 0);
+    // entries still queued become roots, each once: the new ones move to the front
+    uint32_t pend = 0;
+    if (done)
+      for (uint32_t k0 = head; k0 < tail; k0 += kSmallLanes) {
+        const uint32_t k = k0 + j;
+        uint32_t s = 0, kd = 0;
+        bool fresh = false;
+        if (k < tail) {
+          s = Q[k];
+          kd = K[k];
+          fresh = atomicCAS(&p.root_flag[s], 0u, 1u) == 0u;
+        }
+        const uint32_t m = (uint32_t)(__ballot(fresh) >> gsh) & 0xffu;
+        wave_fence();
+        if (fresh) {
+          const uint32_t at = head + pend + (uint32_t)__popc(m & ((1u << j) - 1u));
+          Q[at] = s;
+          K[at] = (uint8_t)kd;
+        }
+        wave_fence();
+        pend += (uint32_t)__popc(m);
+      }
+    if (j == 0) {
+      g_list[g] = done ? head : 0u;
+      g_pend[g] = pend;
+      g_big[g] = large ? 1u : 0u;
     }
-    // publish the node list, owner candidates, descriptor and pending roots
-    unsigned long long pos = 0;
-    if (lane == 0) pos = atomicAdd(p.raw_count, (unsigned long long)nl);
-    pos = __shfl(pos, 0, 64);
-    if (pos + nl > p.raw_cap) {
-      if (lane == 0) atomicOr(p.error, kErrQueue);
-      continue;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+      // the first wave reserves the workgroup's places (exclusive prefixes per group)
+      const bool in = lane < kSmallGroups;
+      const uint32_t nl = in ? g_list[lane] : 0u, np = in ? g_pend[lane] : 0u, nb = in ? g_big[lane] : 0u;
+      const uint32_t li = wave_incl_scan<uint32_t>(nl, lane), pi = wave_incl_scan<uint32_t>(np, lane),
+                     bi = wave_incl_scan<uint32_t>(nb, lane);
+      const uint32_t lt = __shfl(li, 63, 64), pt = __shfl(pi, 63, 64), bt = __shfl(bi, 63, 64);
+      uint32_t mx = nl;
+      for (int o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor(mx, o, 64));
+      uint32_t po = 0, bo = 0;
+      if (lane == 0) {
+        list_base = lt ? atomicAdd(&p.tot->listed, (unsigned long long)lt) : 0ull;
+        sum_nodes += lt;
+        max_nodes = max(max_nodes, mx);
+        if (pt) po = atomicAdd(&p.cnt[p.round + 1], pt);
+        if (bt) bo = atomicAdd(&p.nbig[p.round], bt);
+      }
+      po = __shfl(po, 0, 64);
+      bo = __shfl(bo, 0, 64);
+      if (in) {
+        g_list[lane] = li - nl;
+        g_pend[lane] = po + pi - np;
+        g_big[lane] = bo + bi - nb;
+      }
     }
-    for (uint32_t k = lane; k < nl; k += 64) {
-      const uint32_t s = L[k];
-      p.raw_list[pos + k] = s;
-      atomicMax(&p.owner_root1[s], root_slot + 1);
+    __syncthreads();
+    if (large && j == 0) p.big[g_big[g]] = idx;
+    if (done) {
+      const unsigned long long pos = list_base + g_list[g];
+      if (pos + head > p.raw_cap) {
+        if (j == 0) atomicOr(&p.tot->error, kErrQueue);
+      } else {
+        // Q[0, head) was overwritten by nothing: the roots moved to head and on
+        bool twice = false;
+        for (uint32_t k = j; k < head; k += kSmallLanes) {
+          const uint32_t s = Q[k];
+          p.raw_list[pos + k] = s;
+          p.kind[s] = slot_kind(K[k]);
+          twice |= atomicMax(&p.owner_root1[s], root_slot + 1) != 0u;
+        }
+        if (twice) atomicOr(&p.tot->shared, 1u);
+        if (j == 0) p.desc[base + idx] = make_uint4(root_slot, (uint32_t)pos, head, head * 64u);
+        for (uint32_t k = j; k < pend; k += kSmallLanes)
+          p.out[g_pend[g] + k] = qentry(Q[head + k], K[head + k]);
+      }
     }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0 && sum_nodes) {
+    atomicAdd(&p.tot->bytes, (unsigned long long)sum_nodes * 64ull);
+    atomicMax(&p.tot->max_nodes, max_nodes);
+    atomicMax(&p.tot->max_bytes, max_nodes * 64u);
+  }
+}
+
+// ---- large treelets: one wave each ---------------------------------------------
+// The breadth-first queue and the list are in LDS when qcap entries fit (5
+// bytes each; budgets up to 64 KiB), else in global memory.
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
+typedef __attribute__((address_space(3))) uint8_t lds_u8;
+typedef __attribute__((address_space(1))) uint32_t glb_u32;
+typedef __attribute__((address_space(1))) uint8_t glb_u8;
+
+template <bool LDS, typename W, typename B>
+__device__ __forceinline__ void form_one(const FormParams& p, uint32_t idx, uint32_t base, W* Q, W* L, B* K) {
+  const uint32_t lane = threadIdx.x;
+  auto fence = [&]() {
+    if constexpr (!LDS) __threadfence_block();
+    wave_fence();
+  };
+  uint32_t err = 0, head = 0, tail = 1, nl = 0;
+  int64_t remaining = p.budget;
+  uint32_t root_slot;
+  if (p.first) {
+    root_slot = (uint32_t)(p.tlas >> 6);
+    const uint64_t top = p.tlas + *reinterpret_cast<const uint64_t*>(p.A + p.tlas);
+    if ((top & 63) || !in_arena(top, 64, p.bytes)) err |= kErrRange;
     if (lane == 0) {
-      const uint32_t d = atomicAdd(p.desc_count, 1u);
-      p.desc[d] = make_uint4(root_slot, (uint32_t)pos, nl, (uint32_t)acc_bytes);
+      L[0] = root_slot;
+      Q[0] = (uint32_t)(top >> 6);
+      K[0] = (uint8_t)kTopInternal;
+      p.kind[root_slot] = kSlotHeader;
     }
-    for (uint32_t k = head + lane; k < tail; k += 64) {
-      const uint64_t e = Q[k];
-      if (atomicCAS(&p.root_flag[q_slot(e)], 0u, 1u) == 0u) {
-        const uint32_t o = atomicAdd(p.n_out, 1u);
-        p.frontier_out[o] = e;
+    nl = 1;
+    remaining -= 64;
+  } else {
+    const uint64_t e = p.in[idx];
+    root_slot = q_slot(e);
+    if (lane == 0) {
+      Q[0] = q_slot(e);
+      K[0] = (uint8_t)q_kind(e);
+    }
+  }
+  fence();
+  bool first_chunk = true;
+  while (err == 0) {
+    const uint32_t chunk = min(64u, tail - head);
+    uint32_t slot = 0, kind = kBotLeaf, sz = 0;
+    if (lane < chunk) {
+      slot = Q[head + lane];
+      kind = K[head + lane];
+      sz = kind == kTopLeaf ? 192u : 64u;
+    }
+    const uint32_t incl = wave_incl_scan<uint32_t>(sz, lane);
+    const bool acc = lane < chunk && (int64_t)incl <= remaining;
+    const uint32_t count = (uint32_t)__popcll(__ballot(acc));
+    if (count == 0) {
+      if (first_chunk) err |= kErrBudget;
+      break;
+    }
+    // children and list additions of accepted entries
+    uint32_t ladd = 0, nch = 0, header = 0, blas_root = 0;
+    NodeKids kids{0, 0, 0};
+    if (acc) {
+      const uint64_t off = (uint64_t)slot << 6;
+      ladd = 1;
+      p.kind[slot] = slot_kind(kind);
+      if (kind == kTopInternal || kind == kBotInternal) {
+        kids = load_kids(p.A, off);
+        err |= check_kids(kids, kind, p.bytes, nch);
+      } else if (kind == kTopLeaf) {
+        const uint64_t h = off + *reinterpret_cast<const uint64_t*>(p.A + off + 64);
+        if ((h & 63) || !in_arena(h, 64, p.bytes)) {
+          err |= kErrRange;
+        } else {
+          const uint64_t r = h + *reinterpret_cast<const uint64_t*>(p.A + h);
+          if ((r & 63) || !in_arena(r, 64, p.bytes)) err |= kErrRange;
+          header = (uint32_t)(h >> 6);
+          blas_root = (uint32_t)(r >> 6);
+          ladd = 2;
+          nch = 1;
+        }
       }
     }
+    if (__ballot(err != 0)) {
+      for (int o = 32; o > 0; o >>= 1) err |= __shfl_xor(err, o, 64);
+      break;
+    }
+    const uint32_t lincl = wave_incl_scan<uint32_t>(ladd, lane);
+    const uint32_t cincl = wave_incl_scan<uint32_t>(nch, lane);
+    const uint32_t ltot = __shfl(lincl, 63, 64);
+    const uint32_t ctot = __shfl(cincl, 63, 64);
+    if (nl + ltot > p.lcap || tail + ctot > p.qcap) {
+      err |= kErrQueue;
+      break;
+    }
+    if (acc) {
+      const uint32_t lp = nl + lincl - ladd;
+      uint32_t cp = tail + cincl - nch;
+      L[lp] = slot;
+      if (kind == kTopLeaf) {
+        p.kind[header] = kSlotHeader;
+        L[lp + 1] = header;
+        Q[cp] = blas_root;
+        K[cp] = (uint8_t)kBotInternal;
+      } else if (nch) {
+        each_kid(kids, kind, [&](uint32_t s, uint32_t k) {
+          Q[cp] = s;
+          K[cp] = (uint8_t)k;
+          cp++;
+        });
+      }
+    }
+    fence();
+    remaining -= __shfl(incl, (int)count - 1, 64);
+    head += count;
+    tail += ctot;
+    nl += ltot;
+    first_chunk = false;
+    if (count < chunk || head == tail) break;
+  }
+  if (err) {
+    if (lane == 0) atomicOr(&p.tot->error, err);
+    return;
+  }
+  // publish the node list, owner candidates, descriptor and pending roots
+  const uint32_t used = p.budget - (uint32_t)remaining;
+  unsigned long long pos = 0;
+  if (lane == 0) {
+    pos = atomicAdd(&p.tot->listed, (unsigned long long)nl);
+    atomicAdd(&p.tot->bytes, (unsigned long long)used);
+    atomicMax(&p.tot->max_bytes, used);
+    atomicMax(&p.tot->max_nodes, nl);
+  }
+  pos = __shfl(pos, 0, 64);
+  if (pos + nl > p.raw_cap) {
+    if (lane == 0) atomicOr(&p.tot->error, kErrQueue);
+    return;
+  }
+  bool twice = false;
+  for (uint32_t k = lane; k < nl; k += 64) {
+    const uint32_t s = L[k];
+    p.raw_list[pos + k] = s;
+    twice |= atomicMax(&p.owner_root1[s], root_slot + 1) != 0u;
+  }
+  if (twice) atomicOr(&p.tot->shared, 1u);
+  if (lane == 0) p.desc[base + idx] = make_uint4(root_slot, (uint32_t)pos, nl, used);
+  for (uint32_t k0 = head; k0 < tail; k0 += 64) {
+    const uint32_t k = k0 + lane;
+    uint32_t s = 0;
+    bool fresh = false;
+    if (k < tail) {
+      s = Q[k];
+      fresh = atomicCAS(&p.root_flag[s], 0u, 1u) == 0u;
+    }
+    const uint64_t m = __ballot(fresh);
+    uint32_t o = 0;
+    if (m) {
+      if (lane == 0) o = atomicAdd(&p.cnt[p.round + 1], (uint32_t)__popcll(m));
+      o = __shfl(o, 0, 64);
+    }
+    if (fresh) p.out[o + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = qentry(s, K[k]);
+  }
+}
+
+template <bool LDS>
+__global__ __launch_bounds__(64) void form_large(FormParams p) {
+  extern __shared__ uint32_t smem[];
+  const uint32_t n_in = frontier_count(p);
+  const bool all = p.first || n_in < kSmallMin;
+  const uint32_t n = all ? n_in : p.nbig[p.round];
+  if (blockIdx.x >= n) return;
+  const uint32_t base = treelet_base(p);
+  for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+    const uint32_t idx = all ? i : p.big[i];
+    if constexpr (LDS) {
+      form_one<true>(p, idx, base, (lds_u32*)smem, (lds_u32*)smem + p.qcap, (lds_u8*)((lds_u32*)smem + p.qcap + p.lcap));
+    } else {
+      glb_u32* q = (glb_u32*)(p.scratch + (uint64_t)blockIdx.x * p.queue_bytes);
+      form_one<false>(p, idx, base, q, q + p.qcap, (glb_u8*)(q + p.qcap + p.lcap));
+    }
+    wave_fence();
   }
 }
 
@@ -312,7 +600,6 @@ hipError_t exclusive_scan(In in, uint64_t n, uint64_t* out, uint64_t* sums, uint
   return hipGetLastError();
 }
 
-// ---- finalisation --------------------------------------------------------
 __global__ void owner_and_roots(uint64_t slots, const uint32_t* root_flag, const uint64_t* rank,
                                 const uint32_t* owner_root1, uint32_t* owner, uint64_t* roots) {
   for (uint64_t s = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; s < slots; s += (uint64_t)gridDim.x * blockDim.x) {
@@ -322,10 +609,86 @@ __global__ void owner_and_roots(uint64_t slots, const uint32_t* root_flag, const
   }
 }
 
+// ---- finalisation of a tree: every node is in exactly one list ------------------
+// A treelet's list is its nodes, its image the same nodes packed, and its bytes
+// (64 per node, 192 per instance leaf with its BLAS header) the image's size.
+__global__ __launch_bounds__(256) void rank_treelets(const uint4* desc, uint32_t n, const uint64_t* rank,
+                                                     uint64_t* roots, uint32_t* list_len, uint32_t* image_bytes,
+                                                     uint32_t* desc_of_rank) {
+  const uint32_t d = blockIdx.x * 256 + threadIdx.x;
+  if (d >= n) return;
+  const uint4 ds = desc[d];
+  const uint32_t r = (uint32_t)rank[ds.x];
+  roots[r] = (uint64_t)ds.x << 6;
+  list_len[r] = ds.z;
+  image_bytes[r] = ds.w;
+  desc_of_rank[r] = d;
+}
+
+// Eight lanes per treelet (5.5 nodes on average): list, owners and image in one
+// pass over its nodes.  Bound by HBM: a node is read and written once more
+// (64 B each way) beside 20 B of list, owner and unit words.  Four lanes copy
+// one node, so the eight nodes of a step are four 16-byte loads per lane, all
+// in flight together: 94 us for the 1.47M nodes of the 1M-triangle scene, where
+// a wave per treelet and a kernel per array took 290 us.
+__global__ __launch_bounds__(256) void emit_treelets(const uint4* desc, uint32_t n, const uint32_t* raw,
+                                                     const uint32_t* desc_of_rank, const uint8_t* kind,
+                                                     const uint64_t* list_offsets, const uint64_t* image_offset,
+                                                     const uint8_t* A, uint64_t* list_nodes, uint32_t* owner,
+                                                     uint8_t* images, uint32_t* image_slots) {
+  const uint32_t j = threadIdx.x & 7u;
+  for (uint32_t r = blockIdx.x * 32 + threadIdx.x / 8; r < n; r += gridDim.x * 32) {
+    const uint4 ds = desc[desc_of_rank[r]];
+    const uint64_t lo = list_offsets[r];
+    uint64_t unit = image_offset[r] / 64;
+    for (uint32_t k0 = 0; k0 < ds.z; k0 += 8) {
+      const uint32_t k = k0 + j;
+      const bool in = k < ds.z;
+      uint32_t s = 0, units = 0;
+      if (in) {
+        s = raw[ds.y + k];
+        units = kind[s] == kSlotInstance ? 2u : 1u;
+      }
+      uint32_t incl = units;
+#pragma unroll
+      for (uint32_t d = 1; d < 8; d <<= 1) {
+        const uint32_t y = __shfl_up(incl, d, 8);
+        if (j >= d) incl += y;
+      }
+      const uint64_t at = unit + incl - units;
+      if (in) {
+        list_nodes[lo + k] = (uint64_t)s << 6;
+        owner[s] = r;
+        image_slots[at] = s;
+        if (units == 2u) image_slots[at + 1] = 0xffffffffu;
+      }
+      uint4 v[4];
+#pragma unroll
+      for (uint32_t q = 0; q < 4; ++q) {
+        const uint32_t from = 2 * q + (j >> 2);
+        const uint32_t src = __shfl(s, (int)from, 8);
+        // entries past the list read slot 0 and are not stored
+        v[q] = *reinterpret_cast<const uint4*>(A + ((uint64_t)src << 6) + (j & 3u) * 16);
+      }
+#pragma unroll
+      for (uint32_t q = 0; q < 4; ++q) {
+        const uint32_t from = 2 * q + (j >> 2);
+        const uint32_t src = __shfl(s, (int)from, 8), un = __shfl(units, (int)from, 8);
+        const uint64_t place = (unit + __shfl(incl, (int)from, 8) - un) * 64 + (j & 3u) * 16;
+        if (un) *reinterpret_cast<uint4*>(images + place) = v[q];
+        if (un == 2u)
+          *reinterpret_cast<uint4*>(images + place + 64) =
+              *reinterpret_cast<const uint4*>(A + ((uint64_t)src << 6) + 64 + (j & 3u) * 16);
+      }
+      unit += __shfl(incl, 7, 8);
+    }
+  }
+}
+
+// ---- finalisation where nodes are shared ------------------------------------------
 // One wave per descriptor: de-duplicated length (first occurrence kept).
 __global__ __launch_bounds__(256) void dedupe_count(const uint4* desc, uint32_t n_desc, const uint32_t* raw,
-                                                    const uint64_t* rank, uint32_t* dlen, uint32_t* desc_of_rank,
-                                                    uint32_t check_dupes) {
+                                                    const uint64_t* rank, uint32_t* dlen, uint32_t* desc_of_rank) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = blockIdx.x * 4 + (threadIdx.x >> 6);
   for (uint32_t d = wave; d < n_desc; d += gridDim.x * 4) {
@@ -334,14 +697,12 @@ __global__ __launch_bounds__(256) void dedupe_count(const uint4* desc, uint32_t 
     uint32_t kept = 0;
     for (uint32_t j = lane; j < ds.z; j += 64) {
       bool keep = true;
-      if (check_dupes) {
-        const uint32_t v = l[j];
-        for (uint32_t k = 0; k < j; ++k)
-          if (l[k] == v) {
-            keep = false;
-            break;
-          }
-      }
+      const uint32_t v = l[j];
+      for (uint32_t k = 0; k < j; ++k)
+        if (l[k] == v) {
+          keep = false;
+          break;
+        }
       kept += keep ? 1u : 0u;
     }
     for (int o = 32; o > 0; o >>= 1) kept += __shfl_xor(kept, o, 64);
@@ -355,7 +716,7 @@ __global__ __launch_bounds__(256) void dedupe_count(const uint4* desc, uint32_t 
 
 __global__ __launch_bounds__(256) void dedupe_copy(const uint4* desc, uint32_t n, const uint32_t* raw,
                                                    const uint32_t* desc_of_rank, const uint64_t* list_offsets,
-                                                   uint64_t* list_nodes, uint32_t check_dupes) {
+                                                   uint64_t* list_nodes) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = blockIdx.x * 4 + (threadIdx.x >> 6);
   for (uint32_t r = wave; r < n; r += gridDim.x * 4) {
@@ -368,12 +729,11 @@ __global__ __launch_bounds__(256) void dedupe_copy(const uint4* desc, uint32_t n
       uint32_t v = 0;
       if (keep) {
         v = l[j];
-        if (check_dupes)
-          for (uint32_t k = 0; k < j; ++k)
-            if (l[k] == v) {
-              keep = false;
-              break;
-            }
+        for (uint32_t k = 0; k < j; ++k)
+          if (l[k] == v) {
+            keep = false;
+            break;
+          }
       }
       const uint64_t m = __ballot(keep);
       if (keep) {
@@ -442,7 +802,7 @@ __global__ void validate_level(ValParams p) {
       // lower x/y/z at bytes 28/40/52 + k, upper at 34/46/58 + k
       if (nd[28 + k] > nd[34 + k] || nd[40 + k] > nd[46 + k] || nd[52 + k] > nd[58 + k]) atomicOr(p.unordered, 1u);
       const uint64_t len = (uint64_t)size * 64;
-      if ((c & 63) || c + len > p.bytes) {
+      if ((c & 63) || !in_arena(c, len, p.bytes)) {
         atomicOr(p.error, kErrRange);
         return;
       }
@@ -455,12 +815,12 @@ __global__ void validate_level(ValParams p) {
           return;
         }
         const uint64_t h = c + *reinterpret_cast<const uint64_t*>(p.A + c + 64);
-        if ((h & 63) || h + 64 > p.bytes) {
+        if ((h & 63) || !in_arena(h, 64, p.bytes)) {
           atomicOr(p.error, kErrRange);
           return;
         }
         const uint64_t r = h + *reinterpret_cast<const uint64_t*>(p.A + h);
-        if ((r & 63) || r + 64 > p.bytes) {
+        if ((r & 63) || !in_arena(r, 64, p.bytes)) {
           atomicOr(p.error, kErrRange);
           return;
         }
@@ -564,6 +924,24 @@ struct Scratch {
   }
 };
 
+// Offsets of several 256-byte aligned arrays in one allocation.
+struct Layout {
+  size_t size = 0;
+  size_t add(size_t bytes) {
+    const size_t at = size;
+    size += (bytes + 255) & ~(size_t)255;
+    return at;
+  }
+};
+
+// Device memory that lives as long as the partition.
+template <typename T>
+rtx_status own_alloc(Partition& p, T** q, size_t count) {
+  rtx_status st = dmalloc(q, count);
+  if (st == RTX_OK) p.owned.push_back(*q);
+  return st;
+}
+
 rtx_status map_err(uint32_t bits) {
   if (bits & kErrRange) return RTX_ERR_OFFSET_OUT_OF_ARENA;
   if (bits & kErrType) return RTX_ERR_BAD_NODE_TYPE;
@@ -606,7 +984,7 @@ rtx_status run_validate(const uint8_t* A, uint64_t bytes, uint64_t tlas, hipStre
   CK(hipMemcpyAsync(hdr, A + tlas, 8, hipMemcpyDeviceToHost, s));
   CK(hipStreamSynchronize(s));
   const uint64_t root = tlas + hdr[0];
-  if ((root & 63) || root + 64 > bytes) return RTX_ERR_OFFSET_OUT_OF_ARENA;
+  if ((root & 63) || root > bytes || bytes - root < 64) return RTX_ERR_OFFSET_OUT_OF_ARENA;
   const uint32_t one = 1;
   const uint8_t khdr = kSlotHeader, kint = kSlotInternal;
   CK(hipMemcpyAsync(refs + tlas / 64, &one, 4, hipMemcpyHostToDevice, s));
@@ -764,38 +1142,43 @@ __global__ void first_bits_kernel(const uint8_t* A, uint64_t bytes, const uint8_
   }
 }
 
-rtx_status build_images(const uint8_t* A, uint64_t bytes, hipStream_t s, const uint8_t* kind, Partition& p) {
+hipError_t launch_first_bits(const uint8_t* A, uint64_t bytes, hipStream_t s, const uint8_t* kind, Partition& p) {
   const uint64_t slots = bytes / 64;
   hipLaunchKernelGGL(first_bits_kernel, dim3((uint32_t)std::min<uint64_t>(8192, (slots + 255) / 256)), dim3(256), 0, s, A,
                      bytes, kind, p.owner, p.first_treelet, slots, reinterpret_cast<uint8_t*>(p.owner + slots));
-  CK(hipGetLastError());
-  CS(dmalloc(&p.stage_slot, slots));
-  CS(dmalloc(&p.image_bytes, p.n));
-  CS(dmalloc(&p.image_offset, (size_t)p.n + 1));
-  CK(hipMemsetAsync(p.stage_slot, 0xff, slots * 4, s));
+  return hipGetLastError();
+}
+
+// Images of a partition whose lists and owners are in place (shared nodes, or
+// installed by the caller).
+rtx_status build_images(const uint8_t* A, uint64_t bytes, hipStream_t s, const uint8_t* kind, Partition& p) {
+  const uint64_t slots = bytes / 64;
+  CK(launch_first_bits(A, bytes, s, kind, p));
+  Scratch sc;
+  uint32_t* stage_slot;  // the 64-byte position of a node inside its owner's image
+  uint64_t* sums;
+  CS(sc.alloc(&stage_slot, slots));
+  CS(sc.alloc(&sums, p.n / kTile + 2));
+  CS(own_alloc(p, &p.image_bytes, p.n));
+  CS(own_alloc(p, &p.image_offset, (size_t)p.n + 1));
+  CK(hipMemsetAsync(stage_slot, 0xff, slots * 4, s));
   const uint32_t g = std::min<uint32_t>(4096, (p.n + 3) / 4);
   hipLaunchKernelGGL(image_layout, dim3(g), dim3(256), 0, s, p.n, p.list_offsets, p.list_nodes, p.owner, kind,
-                     p.stage_slot, p.image_bytes);
+                     stage_slot, p.image_bytes);
   CK(hipGetLastError());
-  Scratch sc;
-  uint64_t* sums;
-  CS(sc.alloc(&sums, p.n / kTile + 2));
   CK(exclusive_scan(U32In{p.image_bytes}, p.n, p.image_offset, sums, p.image_offset + p.n, s));
   uint64_t total = 0;
   CK(hipMemcpyAsync(&total, p.image_offset + p.n, 8, hipMemcpyDeviceToHost, s));
-  std::vector<uint32_t> ib(p.n);
-  CK(hipMemcpyAsync(ib.data(), p.image_bytes, (size_t)p.n * 4, hipMemcpyDeviceToHost, s));
   CK(hipStreamSynchronize(s));
   p.images_total = total;
-  p.max_image_bytes = 0;
-  for (uint32_t v : ib) p.max_image_bytes = std::max(p.max_image_bytes, v);
-  CS(dmalloc(&p.images, total));
-  CS(dmalloc(&p.image_slots, total / 64));
+  CS(own_alloc(p, &p.images, total));
+  CS(own_alloc(p, &p.image_slots, total / 64));
   // units no node claims stay "none", so staging never inserts them
   if (total) CK(hipMemsetAsync(p.image_slots, 0xff, total / 64 * 4, s));
   hipLaunchKernelGGL(image_copy, dim3(g), dim3(256), 0, s, p.n, p.list_offsets, p.list_nodes, p.owner, kind,
-                     p.stage_slot, p.image_offset, A, p.images, p.image_slots);
+                     stage_slot, p.image_offset, A, p.images, p.image_slots);
   CK(hipGetLastError());
+  CK(hipStreamSynchronize(s));  // stage_slot is freed on return
   return RTX_OK;
 }
 
@@ -866,15 +1249,7 @@ __global__ __launch_bounds__(256) void layout_metadata_kernel(uint32_t n, uint32
 void partition_free(Partition& p) {
   hipFree(p.layout_remap);
   hipFree(p.layout_metadata);
-  hipFree(p.owner);
-  hipFree(p.roots);
-  hipFree(p.list_offsets);
-  hipFree(p.list_nodes);
-  hipFree(p.images);
-  hipFree(p.image_offset);
-  hipFree(p.image_bytes);
-  hipFree(p.stage_slot);
-  hipFree(p.image_slots);
+  for (void* q : p.owned) hipFree(q);
   p = Partition{};
 }
 
@@ -964,135 +1339,177 @@ rtx_status partition_validate(const uint8_t* A, uint64_t bytes, uint64_t tlas, h
   return ck.cyclic ? RTX_ERR_CYCLE : RTX_OK;
 }
 
-rtx_status build_images(const uint8_t* A, uint64_t bytes, hipStream_t s, const uint8_t* kind, Partition& p);
-
 rtx_status partition_build(const uint8_t* A, uint64_t bytes, uint64_t tlas, uint32_t budget, hipStream_t s,
                            Partition& out) {
   partition_free(out);
   const uint64_t slots = bytes / 64;
-  Scratch sc;
-  uint8_t* kind;
-  CS(sc.alloc(&kind, slots));
-  uint32_t shared = 0;
-  CS(run_validate(A, bytes, tlas, s, sc, kind, &shared, nullptr));
-
-  uint32_t *root_flag, *owner_root1, *ctr;  // ctr: [0] n_out [1] error [2] desc_count [3] work
-  uint64_t *fa, *fb;
-  unsigned long long* raw_count;
-  CS(sc.alloc(&root_flag, slots));
-  CS(sc.alloc(&owner_root1, slots));
-  CS(sc.alloc(&fa, slots));
-  CS(sc.alloc(&fb, slots));
-  CS(sc.alloc(&ctr, 8));
-  CS(sc.alloc(&raw_count, 1));
-  uint4* desc;
-  CS(sc.alloc(&desc, slots));
-  uint64_t raw_cap = std::min<uint64_t>(0xffffffffull, 3 * slots + 1024);
-  uint32_t* raw_list;
-  CS(sc.alloc(&raw_list, raw_cap));
-  const uint32_t qcap = 6 * (budget / 64) + 8;
+  const uint32_t qcap = (6 * (budget / 64) + 8 + 3) & ~3u;
   const uint32_t lcap = budget / 64 + 4;
-  const uint64_t per_wave = qcap + (lcap + 1) / 2;
-  uint32_t waves = 1024;
-  while (waves > 64 && per_wave * waves * 8 > (256ull << 20)) waves /= 2;
-  uint64_t* scratch;
-  CS(sc.alloc(&scratch, per_wave * waves));
+  const uint64_t queue_bytes = ((uint64_t)qcap * 5 + (uint64_t)lcap * 4 + 15) & ~15ull;
+  const bool lds = queue_bytes <= 48 * 1024;
+  uint32_t large_grid = 4096;  // form_large workgroups of one wave
+  while (!lds && large_grid > 64 && queue_bytes * large_grid > (256ull << 20)) large_grid /= 2;
+  const uint64_t raw_cap = std::min<uint64_t>(0xffffffffull, 3 * slots + 1024);
 
-  CK(hipMemsetAsync(root_flag, 0, slots * 4, s));
-  CK(hipMemsetAsync(owner_root1, 0, slots * 4, s));
-  CK(hipMemsetAsync(ctr, 0, 32, s));
-  CK(hipMemsetAsync(raw_count, 0, 8, s));
+  // One block of scratch; the words before `zeroed` are cleared together.
+  struct Control {
+    FormTotals tot;
+    uint32_t cnt[kRoundBatch + 1], nbig[kRoundBatch];
+  };
+  Scratch sc;
+  Layout lay;
+  const size_t o_ctl = lay.add(sizeof(Control)), o_flag = lay.add(slots * 4), o_owner1 = lay.add(slots * 4),
+               o_kind = lay.add(slots), zeroed = lay.size, o_fa = lay.add(slots * 8), o_fb = lay.add(slots * 8),
+               o_big = lay.add(slots * 4), o_desc = lay.add(slots * 16), o_raw = lay.add(raw_cap * 4),
+               o_rank = lay.add(slots * 8), o_sums = lay.add((slots / kTile + 2) * 8), o_tot = lay.add(16),
+               o_len = lay.add(slots * 4), o_dor = lay.add(slots * 4),
+               o_queues = lay.add(lds ? 0 : queue_bytes * large_grid);
+  uint8_t* mem;
+  CS(sc.alloc(&mem, lay.size));
+  Control* ctl = reinterpret_cast<Control*>(mem + o_ctl);
+  uint32_t* root_flag = reinterpret_cast<uint32_t*>(mem + o_flag);
+  uint32_t* owner_root1 = reinterpret_cast<uint32_t*>(mem + o_owner1);
+  uint8_t* kind = mem + o_kind;
+  uint64_t* fa = reinterpret_cast<uint64_t*>(mem + o_fa);
+  uint64_t* fb = reinterpret_cast<uint64_t*>(mem + o_fb);
+  uint4* desc = reinterpret_cast<uint4*>(mem + o_desc);
+  uint32_t* raw_list = reinterpret_cast<uint32_t*>(mem + o_raw);
+  uint64_t* rank = reinterpret_cast<uint64_t*>(mem + o_rank);
+  uint64_t* sums = reinterpret_cast<uint64_t*>(mem + o_sums);
+  uint64_t* tot = reinterpret_cast<uint64_t*>(mem + o_tot);
+  uint32_t* list_len = reinterpret_cast<uint32_t*>(mem + o_len);
+  uint32_t* desc_of_rank = reinterpret_cast<uint32_t*>(mem + o_dor);
+
+  CK(hipMemsetAsync(mem, 0, zeroed, s));
   const uint32_t one = 1;
   CK(hipMemcpyAsync(root_flag + tlas / 64, &one, 4, hipMemcpyHostToDevice, s));
-  uint64_t e0 = tlas / 64;
-  CK(hipMemcpyAsync(fa, &e0, 8, hipMemcpyHostToDevice, s));
-  uint32_t n_in = 1;
+  Control h{};
+  uint32_t n_in = 1, n = 0;
   bool first = true;
   while (n_in > 0) {
-    CK(hipMemsetAsync(ctr, 0, 4, s));      // n_out
-    CK(hipMemsetAsync(ctr + 3, 0, 4, s));  // work counter
-    FormParams fp{A, bytes, tlas, budget, first ? 1u : 0u, fa, n_in, fb, ctr, root_flag, owner_root1, raw_list,
-                  raw_cap, raw_count, desc, ctr + 2, scratch, qcap, lcap, ctr + 3, ctr + 1};
-    const uint32_t grid = std::min<uint32_t>(waves / 4, (n_in + 3) / 4);
-    hipLaunchKernelGGL(form_treelets, dim3(std::max(grid, 1u)), dim3(256), 0, s, fp);
-    CK(hipGetLastError());
-    uint32_t c[2];
-    CK(hipMemcpyAsync(c, ctr, 8, hipMemcpyDeviceToHost, s));
+    if (!first) CK(hipMemsetAsync(ctl->cnt, 0, sizeof(Control) - offsetof(Control, cnt), s));
+    for (uint32_t j = 0; j < kRoundBatch; ++j) {
+      FormParams fp{A,  bytes, tlas, budget, first ? 1u : 0u, j, n_in, n, ctl->cnt, ctl->nbig, fa, fb,
+                    reinterpret_cast<uint32_t*>(mem + o_big), root_flag, owner_root1, kind, raw_list, raw_cap, desc,
+                    &ctl->tot, mem + o_queues, queue_bytes, qcap, lcap};
+      if (!first) hipLaunchKernelGGL(form_small, dim3(2048), dim3(256), 0, s, fp);
+      const uint32_t g = first ? 1u : large_grid;
+      if (lds)
+        hipLaunchKernelGGL(form_large<true>, dim3(g), dim3(64), queue_bytes, s, fp);
+      else
+        hipLaunchKernelGGL(form_large<false>, dim3(g), dim3(64), 0, s, fp);
+      CK(hipGetLastError());
+      std::swap(fa, fb);
+      first = false;
+    }
+    CK(hipMemcpyAsync(&h, ctl, sizeof(h), hipMemcpyDeviceToHost, s));
     CK(hipStreamSynchronize(s));
-    if (c[1]) return map_err(c[1]);
-    n_in = c[0];
-    std::swap(fa, fb);
-    first = false;
+    if (h.tot.error) {
+      // a malformed arena reports what its structural walk finds first
+      uint8_t* k2;
+      CS(sc.alloc(&k2, slots));
+      CS(run_validate(A, bytes, tlas, s, sc, k2, nullptr, nullptr));
+      return map_err(h.tot.error);
+    }
+    n += n_in;
+    for (uint32_t j = 1; j < kRoundBatch; ++j) n += h.cnt[j];
+    n_in = h.cnt[kRoundBatch];
   }
-  uint32_t n_desc = 0;
-  CK(hipMemcpyAsync(&n_desc, ctr + 2, 4, hipMemcpyDeviceToHost, s));
 
   // dense numbering of roots in ascending offset order
-  uint64_t *rank, *sums, *tot;
-  CS(sc.alloc(&rank, slots));
-  CS(sc.alloc(&sums, slots / kTile + 2));
-  CS(sc.alloc(&tot, 2));
   CK(exclusive_scan(FlagIn{root_flag}, slots, rank, sums, tot, s));
-  uint64_t n_roots = 0;
-  CK(hipMemcpyAsync(&n_roots, tot, 8, hipMemcpyDeviceToHost, s));
-  CK(hipStreamSynchronize(s));
-  if (n_roots != n_desc || n_roots == 0) return RTX_ERR_HIP;
-  const uint32_t n = (uint32_t)n_roots;
-
   Partition p;
   p.budget = budget;
   p.n = n;
-  CS(dmalloc(&p.owner, slots + (slots + 3) / 4));  // owner words, then the first-treelet bytes
-  CS(dmalloc(&p.roots, n));
-  CS(dmalloc(&p.list_offsets, (size_t)n + 1));
-  hipLaunchKernelGGL(owner_and_roots, dim3(2048), dim3(256), 0, s, slots, root_flag, rank, owner_root1, p.owner,
-                     p.roots);
-  CK(hipGetLastError());
-  uint32_t *dlen, *desc_of_rank;
-  CS(sc.alloc(&dlen, n));
-  CS(sc.alloc(&desc_of_rank, n));
-  const uint32_t g = std::min<uint32_t>(4096, (n + 3) / 4);
-  hipLaunchKernelGGL(dedupe_count, dim3(g), dim3(256), 0, s, desc, n, raw_list, rank, dlen, desc_of_rank, shared);
-  CK(hipGetLastError());
-  CK(exclusive_scan(U32In{dlen}, n, p.list_offsets, sums, p.list_offsets + n, s));
-  uint64_t n_list = 0;
-  CK(hipMemcpyAsync(&n_list, p.list_offsets + n, 8, hipMemcpyDeviceToHost, s));
-  CK(hipStreamSynchronize(s));
-  p.n_list = n_list;
-  CS(dmalloc(&p.list_nodes, n_list));
-  hipLaunchKernelGGL(dedupe_copy, dim3(g), dim3(256), 0, s, desc, n, raw_list, desc_of_rank, p.list_offsets,
-                     p.list_nodes, shared);
-  CK(hipGetLastError());
-
-  // summary
-  std::vector<uint4> hd(n_desc);
-  std::vector<uint32_t> hl(n);
-  CK(hipMemcpyAsync(hd.data(), desc, (size_t)n_desc * sizeof(uint4), hipMemcpyDeviceToHost, s));
-  CK(hipMemcpyAsync(hl.data(), dlen, (size_t)n * 4, hipMemcpyDeviceToHost, s));
-  uint32_t ft = 0;
-  {
-    uint64_t r = 0;
-    CK(hipMemcpyAsync(&r, rank + tlas / 64, 8, hipMemcpyDeviceToHost, s));
-    CK(hipStreamSynchronize(s));
-    ft = (uint32_t)r;
-  }
-  p.first_treelet = ft;
-  rtx_treelet_summary sm{};
-  sm.n_treelets = n;
-  sm.budget_bytes = budget;
-  sm.n_list_entries = n_list;
-  for (const uint4& d : hd) {
-    sm.total_bytes += d.w;
-    sm.max_treelet_bytes = std::max(sm.max_treelet_bytes, d.w);
-  }
-  for (uint32_t v : hl) sm.max_treelet_nodes = std::max(sm.max_treelet_nodes, v);
-  p.summary = sm;
-  rtx_status st = build_images(A, bytes, s, kind, p);
-  if (st != RTX_OK) {
+  const bool shared = h.tot.shared != 0;
+  auto give_back = [&](rtx_status st) {
     partition_free(p);
     return st;
+  };
+#define CKP(expr)                                                \
+  do {                                                           \
+    if ((expr) != hipSuccess) {                                  \
+      (void)hipGetLastError();                                   \
+      return give_back(RTX_ERR_HIP);                             \
+    }                                                            \
+  } while (0)
+#define CSP(expr)                                   \
+  do {                                              \
+    rtx_status _s = (expr);                         \
+    if (_s != RTX_OK) return give_back(_s);         \
+  } while (0)
+  p.summary.n_treelets = n;
+  p.summary.budget_bytes = budget;
+  p.summary.total_bytes = h.tot.bytes;
+  p.summary.max_treelet_bytes = h.tot.max_bytes;
+  p.summary.max_treelet_nodes = h.tot.max_nodes;
+  uint64_t n_roots = 0, first_rank = 0;
+  if (!shared) {
+    // a tree: list and image sizes are known, and one pass writes both
+    p.n_list = h.tot.listed;
+    p.images_total = h.tot.bytes;
+    Layout pl;
+    const size_t q_owner = pl.add((slots + (slots + 3) / 4) * 4), q_roots = pl.add((uint64_t)n * 8),
+                 q_lo = pl.add(((uint64_t)n + 1) * 8), q_ln = pl.add(p.n_list * 8), q_img = pl.add(p.images_total),
+                 q_io = pl.add(((uint64_t)n + 1) * 8), q_ib = pl.add((uint64_t)n * 4),
+                 q_is = pl.add(p.images_total / 64 * 4);
+    uint8_t* pm;
+    CSP(own_alloc(p, &pm, pl.size));
+    p.owner = reinterpret_cast<uint32_t*>(pm + q_owner);  // owner words, then the first-treelet bytes
+    p.roots = reinterpret_cast<uint64_t*>(pm + q_roots);
+    p.list_offsets = reinterpret_cast<uint64_t*>(pm + q_lo);
+    p.list_nodes = reinterpret_cast<uint64_t*>(pm + q_ln);
+    p.images = pm + q_img;
+    p.image_offset = reinterpret_cast<uint64_t*>(pm + q_io);
+    p.image_bytes = reinterpret_cast<uint32_t*>(pm + q_ib);
+    p.image_slots = reinterpret_cast<uint32_t*>(pm + q_is);
+    CKP(hipMemsetAsync(p.owner, 0xff, slots * 4, s));
+    hipLaunchKernelGGL(rank_treelets, dim3((n + 255) / 256), dim3(256), 0, s, desc, n, rank, p.roots, list_len,
+                       p.image_bytes, desc_of_rank);
+    CKP(hipGetLastError());
+    CKP(exclusive_scan(U32In{list_len}, n, p.list_offsets, sums, p.list_offsets + n, s));
+    CKP(exclusive_scan(U32In{p.image_bytes}, n, p.image_offset, sums, p.image_offset + n, s));
+    hipLaunchKernelGGL(emit_treelets, dim3(std::min<uint32_t>(8192, (n + 31) / 32)), dim3(256), 0, s, desc, n, raw_list,
+                       desc_of_rank, kind, p.list_offsets, p.image_offset, A, p.list_nodes, p.owner, p.images,
+                       p.image_slots);
+    CKP(hipGetLastError());
+  } else {
+    CSP(own_alloc(p, &p.owner, slots + (slots + 3) / 4));
+    CSP(own_alloc(p, &p.roots, n));
+    CSP(own_alloc(p, &p.list_offsets, (size_t)n + 1));
+    hipLaunchKernelGGL(owner_and_roots, dim3(2048), dim3(256), 0, s, slots, root_flag, rank, owner_root1, p.owner,
+                       p.roots);
+    CKP(hipGetLastError());
+    const uint32_t g = std::min<uint32_t>(4096, (n + 3) / 4);
+    hipLaunchKernelGGL(dedupe_count, dim3(g), dim3(256), 0, s, desc, n, raw_list, rank, list_len, desc_of_rank);
+    CKP(hipGetLastError());
+    CKP(exclusive_scan(U32In{list_len}, n, p.list_offsets, sums, p.list_offsets + n, s));
+    uint64_t n_list = 0;
+    std::vector<uint32_t> hl(n);
+    CKP(hipMemcpyAsync(&n_list, p.list_offsets + n, 8, hipMemcpyDeviceToHost, s));
+    CKP(hipMemcpyAsync(hl.data(), list_len, (size_t)n * 4, hipMemcpyDeviceToHost, s));
+    CKP(hipStreamSynchronize(s));
+    p.n_list = n_list;
+    p.summary.max_treelet_nodes = *std::max_element(hl.begin(), hl.end());
+    CSP(own_alloc(p, &p.list_nodes, n_list));
+    hipLaunchKernelGGL(dedupe_copy, dim3(g), dim3(256), 0, s, desc, n, raw_list, desc_of_rank, p.list_offsets,
+                       p.list_nodes);
+    CKP(hipGetLastError());
   }
-  CK(hipStreamSynchronize(s));
+  p.summary.n_list_entries = p.n_list;
+  CKP(hipMemcpyAsync(&n_roots, tot, 8, hipMemcpyDeviceToHost, s));
+  CKP(hipMemcpyAsync(&first_rank, rank + tlas / 64, 8, hipMemcpyDeviceToHost, s));
+  CKP(hipStreamSynchronize(s));
+  if (n_roots != n || n_roots == 0) return give_back(RTX_ERR_HIP);
+  p.first_treelet = (uint32_t)first_rank;
+  if (shared) {
+    CSP(build_images(A, bytes, s, kind, p));
+  } else {
+    CKP(launch_first_bits(A, bytes, s, kind, p));
+    CKP(hipStreamSynchronize(s));
+  }
+#undef CKP
+#undef CSP
   p.valid = true;
   out = p;
   return RTX_OK;
@@ -1148,10 +1565,10 @@ rtx_status partition_install(const uint8_t* A, uint64_t bytes, uint64_t tlas, ui
   p.n = n;
   p.n_list = n_list;
   p.first_treelet = ft;
-  CS(dmalloc(&p.owner, slots + (slots + 3) / 4));  // owner words, then the first-treelet bytes
-  CS(dmalloc(&p.roots, n));
-  CS(dmalloc(&p.list_offsets, (size_t)n + 1));
-  CS(dmalloc(&p.list_nodes, n_list));
+  CS(own_alloc(p, &p.owner, slots + (slots + 3) / 4));  // owner words, then the first-treelet bytes
+  CS(own_alloc(p, &p.roots, n));
+  CS(own_alloc(p, &p.list_offsets, (size_t)n + 1));
+  CS(own_alloc(p, &p.list_nodes, n_list));
   CK(hipMemcpyAsync(p.owner, owner, slots * 4, hipMemcpyHostToDevice, s));
   CK(hipMemcpyAsync(p.roots, roots, (size_t)n * 8, hipMemcpyHostToDevice, s));
   CK(hipMemcpyAsync(p.list_offsets, lo, ((size_t)n + 1) * 8, hipMemcpyHostToDevice, s));
