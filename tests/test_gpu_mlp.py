@@ -120,3 +120,32 @@ def test_training_learns_a_treelet_rule(gpu):
         assert last < 0.25 * l0 and acc > 0.9
     finally:
         mlp.close()
+
+
+@pytest.mark.parametrize("T,C,n", [(30, 3, 5), (30, 17, 16), (50, 257, 65), (40, 1000, 4097), (20, 300, 2100)])
+def test_predict_at_tile_edges(gpu, T, C, n):
+    """Fewer than four classes, class counts around the MFMA tile and the LDS
+    stage, row counts around the row tiles and the 4,096-row batches.  Both
+    sides round operands to BF16; a sum of another order may flip one rounding
+    of an activation (2^-8 relative), which moves a logit of this size by at
+    most about 1e-3, so classes closer than 5e-3 may swap and probabilities
+    agree to 5e-3."""
+    rng = np.random.default_rng(C + n)
+    mlp = gpu.mlp(T, C, seed=C)
+    try:
+        s = _samples(rng, T, C, n)
+        top, prob = mlp.predict(s)
+        P = mo.unpack(mlp.params(), T, C)
+        *_, L = mo.forward(P, s, bf16=True)
+        k = min(4, C)
+        order = np.argsort(-L, axis=1, kind="stable")
+        Ls = np.take_along_axis(L, order, axis=1)[:, :k + 1]
+        clear = np.all(-np.diff(Ls, axis=1) > 5e-3, axis=1)
+        assert clear.mean() > 0.5
+        assert np.array_equal(top[clear, :k], order[clear, :k].astype(np.uint32))
+        p = np.exp(L - L.max(axis=1, keepdims=True))
+        p = np.take_along_axis(p / p.sum(axis=1, keepdims=True), order, axis=1)[:, :k]
+        assert np.allclose(prob[clear, :k], p[clear], rtol=5e-3)
+        assert np.all(top[:, k:] == 0xFFFFFFFF) and np.all(prob[:, k:] == 0)
+    finally:
+        mlp.close()

@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <new>
@@ -101,41 +102,142 @@ __global__ void zero_rows(float* C, int M, int N, int ldc) {
     C[(k / N) * ldc + k % N] = 0.f;
 }
 
-// ---- elementwise and reductions ---------------------------------------------------
-__global__ void build_input(const rtx_mlp_sample* s, int n, const float* E, int none, float* X) {
-  const int i = blockIdx.x;
-  if (i >= n) return;
-  rtx_mlp_sample sm = s[i];
-  // out-of-range treelets read the "none" row
-  if (sm.cur > (uint32_t)none) sm.cur = none;
-  for (int h = 0; h < 4; ++h)
-    if (sm.hist[h] != RTX_NO_TREELET && sm.hist[h] > (uint32_t)none) sm.hist[h] = RTX_NO_TREELET;
-  float* x = X + (size_t)i * kInPad;
-  for (int c = threadIdx.x; c < kInPad; c += blockDim.x) {
-    float v = 0.f;
-    if (c < 32) {
-      v = E[(size_t)sm.cur * kEmb + c];
-    } else if (c < 40) {
-      v = (uint32_t)(c - 32) == sm.octant ? 1.f : 0.f;
-    } else if (c == 40) {
-      v = sm.depth;
-    } else if (c < kIn) {
-      const int h = (c - 41) / 32, e = (c - 41) % 32;
-      const uint32_t t = sm.hist[h];
-      v = E[(size_t)(t == RTX_NO_TREELET ? (uint32_t)none : t) * kEmb + e];
+// ---- trunk: x -> h1 -> h2 -> q in one kernel ------------------------------------
+// Weights as MFMA operands: fragment (column tile ct, 32-deep step ks) of a
+// K x N matrix holds, for lane l, the eight k values 32 ks + 8 (l / 16) + t of
+// column 16 ct + l % 16, rounded to BF16, at [(ct * KS + ks) * 64 + l].
+constexpr int kFrag1 = 0;                                       // W1: 192 x 128
+constexpr int kFrag2 = kFrag1 + (kHid / 16) * (kInPad / 32);    // W2: 128 x 128
+constexpr int kFrag3 = kFrag2 + (kHid / 16) * (kHid / 32);      // W3: 128 x 32
+constexpr int kFragEnd = kFrag3 + (kEmb / 16) * (kHid / 32);
+struct Weights {
+  const float *W1, *b1, *W2, *b2, *W3, *b3;
+};
+
+__global__ __launch_bounds__(256) void pack_weights(Weights w, uint4* frags) {
+  const int f = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (f >= kFragEnd) return;
+  const float* W;
+  int cols, ks_n, at;
+  if (f < kFrag2) {
+    W = w.W1, cols = kHid, ks_n = kInPad / 32, at = f - kFrag1;
+  } else if (f < kFrag3) {
+    W = w.W2, cols = kHid, ks_n = kHid / 32, at = f - kFrag2;
+  } else {
+    W = w.W3, cols = kEmb, ks_n = kHid / 32, at = f - kFrag3;
+  }
+  const int col = (at / ks_n) * 16 + (lane & 15), k0 = (at % ks_n) * 32 + (lane >> 4) * 8;
+  bf16x8 v;
+#pragma unroll
+  for (int t = 0; t < 8; ++t) v[t] = (__bf16)W[(size_t)(k0 + t) * cols + col];
+  frags[(size_t)f * 64 + lane] = __builtin_bit_cast(uint4, v);
+}
+
+// One layer of 16 rows held in LDS as BF16 (`stride` values a row): the 16x16
+// tile of columns 16 ct.. of the product.  `chunked` sums 64-deep partial
+// products instead of one chain over K.
+template <int KS>
+__device__ __forceinline__ f32x4 layer_tile(const __bf16* rows, int stride, const uint4* __restrict__ frags, int ct,
+                                            int lane, bool chunked) {
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f}, sum = {0.f, 0.f, 0.f, 0.f};
+  uint4 b[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) b[ks] = frags[(size_t)(ct * KS + ks) * 64 + lane];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const bf16x8 a = *reinterpret_cast<const bf16x8*>(rows + (lane & 15) * stride + ks * 32 + (lane >> 4) * 8);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, b[ks]), acc, 0, 0, 0);
+    if (chunked && (ks & 1)) {
+      for (int i = 0; i < 4; ++i) sum[i] += acc[i];
+      acc = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    x[c] = v;
+  }
+  return chunked ? sum : acc;
+}
+
+// 16 samples per workgroup, each wave two of a layer's eight column tiles; the
+// activations pass from layer to layer through LDS in the BF16 the next product
+// takes.  A layer is a few MFMAs behind one round of weight loads from L2, so
+// the kernel is latency-bound and small workgroups spread it over the chip:
+// 1,024 samples took 75 us in seven launches (gather, three products with
+// zeroing, three bias passes) and take 12.  TRAIN also stores what the backward
+// pass reads (FP32).  Rows from chunk_from on accumulate the first two layers in
+// 64-deep partial products, and the third always does: the order of the K-split
+// products of batches that small, kept so that results stay what they were.
+constexpr int kRowTile = 16;
+constexpr int kXStride = kInPad + 8, kHStride = kHid + 8;  // LDS rows start in different banks
+
+template <bool TRAIN>
+__global__ __launch_bounds__(256) void trunk_forward(const rtx_mlp_sample* __restrict__ samples, int n,
+                                                     const float* __restrict__ E, int none, Weights w,
+                                                     const uint4* __restrict__ frags, int chunk_from, float* X,
+                                                     float* H1, float* H2, float* Q) {
+  __shared__ __attribute__((aligned(16))) __bf16 xs[kRowTile * kXStride], h1s[kRowTile * kHStride],
+      h2s[kRowTile * kHStride];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, g = lane >> 4;
+  const int r0 = blockIdx.x * kRowTile;
+  const bool chunked = r0 >= chunk_from;
+  {
+    // 16 threads per sample, 12 columns each
+    const int row = threadIdx.x >> 4, c0 = (threadIdx.x & 15) * 12;
+    const int i = r0 + row;
+    rtx_mlp_sample sm{};
+    if (i < n) sm = samples[i];
+    // out-of-range treelets read the "none" row
+    if (sm.cur > (uint32_t)none) sm.cur = none;
+#pragma unroll
+    for (int k = 0; k < 12; ++k) {
+      const int c = c0 + k;
+      float v = 0.f;
+      if (c < 32) {
+        v = E[(size_t)sm.cur * kEmb + c];
+      } else if (c < 40) {
+        v = (uint32_t)(c - 32) == sm.octant ? 1.f : 0.f;
+      } else if (c == 40) {
+        v = sm.depth;
+      } else if (c < kIn) {
+        const int h = (c - 41) / 32, e = (c - 41) % 32;
+        const uint32_t t = h == 0 ? sm.hist[0] : h == 1 ? sm.hist[1] : h == 2 ? sm.hist[2] : sm.hist[3];
+        v = E[(size_t)(t > (uint32_t)none ? (uint32_t)none : t) * kEmb + e];
+      }
+      if (i >= n) v = 0.f;
+      xs[row * kXStride + c] = (__bf16)v;
+      if (TRAIN && i < n) X[(size_t)i * kInPad + c] = v;
+    }
+  }
+  __syncthreads();
+  for (int q = 0; q < 2; ++q) {
+    const int col = (2 * wave + q) * 16 + c16;
+    const f32x4 z = layer_tile<kInPad / 32>(xs, kXStride, frags + kFrag1 * 64, 2 * wave + q, lane, chunked);
+    const float bias = w.b1[col];
+    for (int i = 0; i < 4; ++i) {
+      const float v = z[i] + bias, h = v > 0.f ? v : 0.f;
+      h1s[(4 * g + i) * kHStride + col] = (__bf16)h;
+      if (TRAIN && r0 + 4 * g + i < n) H1[(size_t)(r0 + 4 * g + i) * kHid + col] = h;
+    }
+  }
+  __syncthreads();
+  for (int q = 0; q < 2; ++q) {
+    const int col = (2 * wave + q) * 16 + c16;
+    const f32x4 z = layer_tile<kHid / 32>(h1s, kHStride, frags + kFrag2 * 64, 2 * wave + q, lane, chunked);
+    const float bias = w.b2[col];
+    for (int i = 0; i < 4; ++i) {
+      const float v = z[i] + bias, h = v > 0.f ? v : 0.f;
+      h2s[(4 * g + i) * kHStride + col] = (__bf16)h;
+      if (TRAIN && r0 + 4 * g + i < n) H2[(size_t)(r0 + 4 * g + i) * kHid + col] = h;
+    }
+  }
+  __syncthreads();
+  if (wave < kEmb / 16) {
+    const int col = wave * 16 + c16;
+    const f32x4 z = layer_tile<kHid / 32>(h2s, kHStride, frags + kFrag3 * 64, wave, lane, true);
+    const float bias = w.b3[col];
+    for (int i = 0; i < 4; ++i)
+      if (r0 + 4 * g + i < n) Q[(size_t)(r0 + 4 * g + i) * kEmb + col] = z[i] + bias;
   }
 }
 
-__global__ void bias_act(float* Z, int n, int cols, const float* bias, int relu) {
-  const size_t total = (size_t)n * cols;
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < total; k += (size_t)gridDim.x * blockDim.x) {
-    float v = Z[k] + bias[k % cols];
-    Z[k] = relu ? (v > 0.f ? v : 0.f) : v;
-  }
-}
-
+// ---- elementwise and reductions ---------------------------------------------------
 __global__ void relu_mask(float* dH, const float* H, size_t total) {
   for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < total; k += (size_t)gridDim.x * blockDim.x)
     if (!(H[k] > 0.f)) dH[k] = 0.f;
@@ -216,75 +318,6 @@ __global__ void adam_step(float* p, const float* g, float* m, float* v, size_t c
     m[k] = mk;
     v[k] = vk;
     p[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + eps);
-  }
-}
-
-// Top-4 classes of each row of L (+ bias) and their softmax probabilities,
-// one wave per row.
-__global__ __launch_bounds__(64) void top4(const float* L, int n, int C, const float* cbias, uint32_t* out,
-                                           float* prob) {
-  const int r = blockIdx.x;
-  if (r >= n) return;
-  const int lane = threadIdx.x;
-  const float* row = L + (size_t)r * C;
-  float bv[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-  int bi[4] = {-1, -1, -1, -1};
-  for (int c = lane; c < C; c += 64) {
-    const float v = row[c] + cbias[c];
-    if (v > bv[3]) {
-      int k = 3;
-      while (k > 0 && v > bv[k - 1]) {
-        bv[k] = bv[k - 1];
-        bi[k] = bi[k - 1];
-        --k;
-      }
-      bv[k] = v;
-      bi[k] = c;
-    }
-  }
-  // merge the 64 lane lists: 4 rounds of a wave argmax (ties to the lower class)
-  float topv[4];
-  int topi[4];
-  for (int round = 0; round < 4; ++round) {
-    float v = bv[0];
-    int idx = bi[0];
-    int src = lane;
-    for (int o = 32; o > 0; o >>= 1) {
-      const float v2 = __shfl_xor(v, o, 64);
-      const int i2 = __shfl_xor(idx, o, 64);
-      const int s2 = __shfl_xor(src, o, 64);
-      const bool take = i2 >= 0 && (idx < 0 || v2 > v || (v2 == v && i2 < idx));
-      if (take) {
-        v = v2;
-        idx = i2;
-        src = s2;
-      }
-    }
-    topv[round] = v;
-    topi[round] = idx;
-    if (lane == src && idx >= 0) {
-      for (int k = 0; k < 3; ++k) {
-        bv[k] = bv[k + 1];
-        bi[k] = bi[k + 1];
-      }
-      bv[3] = -INFINITY;
-      bi[3] = -1;
-    }
-  }
-  const float mx = topv[0];
-  float se = 0.f;
-  for (int c = lane; c < C; c += 64) se += expf(row[c] + cbias[c] - mx);
-  for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o, 64);
-  if (lane < 4) {
-    float v = topv[0];
-    int idx = topi[0];
-    for (int k = 1; k < 4; ++k)
-      if (lane == k) {
-        v = topv[k];
-        idx = topi[k];
-      }
-    out[(size_t)r * 4 + lane] = idx < 0 ? RTX_NO_TREELET : (uint32_t)idx;
-    if (prob) prob[(size_t)r * 4 + lane] = idx < 0 ? 0.f : expf(v - mx) / se;
   }
 }
 
@@ -431,6 +464,139 @@ __global__ __launch_bounds__(256) void ce_finish(const float* pm, const float* p
   if (lane == 0) part[w] = acc;
   __syncthreads();
   if (threadIdx.x == 0) atomicAdd(loss, part[0] + part[1] + part[2] + part[3]);
+}
+
+// ---- prediction: top-4 classes and probabilities ------------------------------------
+// The best four of a set of logits, best first, ties to the lower class (-1:
+// none), with the set's maximum and exp-sum relative to it.
+struct Top4 {
+  float v[4];
+  int c[4];
+  float m, s;
+};
+static_assert(sizeof(Top4) == 40, "partial results are stored as Top4");
+
+__device__ __forceinline__ void top4_insert(Top4& t, float x, int c) {
+  // x > t.v[3]; classes come in ascending order, so an equal value stays behind
+  const bool b0 = x > t.v[0], b1 = x > t.v[1], b2 = x > t.v[2];
+  t.v[3] = b2 ? t.v[2] : x;
+  t.c[3] = b2 ? t.c[2] : c;
+  t.v[2] = b2 ? (b1 ? t.v[1] : x) : t.v[2];
+  t.c[2] = b2 ? (b1 ? t.c[1] : c) : t.c[2];
+  t.v[1] = b1 ? (b0 ? t.v[0] : x) : t.v[1];
+  t.c[1] = b1 ? (b0 ? t.c[0] : c) : t.c[1];
+  t.v[0] = b0 ? x : t.v[0];
+  t.c[0] = b0 ? c : t.c[0];
+}
+
+__device__ __forceinline__ bool top4_before(float v, int c, float v2, int c2) {
+  return c >= 0 && (c2 < 0 || v > v2 || (v == v2 && c < c2));
+}
+
+// t <- the four best of both, and the exp-sum of the union
+__device__ __forceinline__ void top4_merge(Top4& t, const Top4& o) {
+  // Both are sorted, so the four best of the union are the better of t[k] and
+  // o[3 - k] for each k; two exchange steps order them.
+  float v[4];
+  int c[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const bool keep = top4_before(t.v[k], t.c[k], o.v[3 - k], o.c[3 - k]);
+    v[k] = keep ? t.v[k] : o.v[3 - k];
+    c[k] = keep ? t.c[k] : o.c[3 - k];
+  }
+  auto order = [&](int a, int b) {
+    if (top4_before(v[b], c[b], v[a], c[a])) {
+      const float tv = v[a];
+      const int tc = c[a];
+      v[a] = v[b];
+      c[a] = c[b];
+      v[b] = tv;
+      c[b] = tc;
+    }
+  };
+  order(0, 2);
+  order(1, 3);
+  order(0, 1);
+  order(2, 3);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    t.v[k] = v[k];
+    t.c[k] = c[k];
+  }
+  lse_merge(t.m, t.s, o.m, o.s);
+}
+
+// One block: 64 rows (a wave per 16) against the classes [y * cper, y * cper +
+// cper), staged in LDS kCeCls at a time.  The MFMA's rows are classes and its
+// columns the wave's samples, so a lane keeps one sample's best four over a
+// quarter of the classes, in registers, and the logits are never stored: 20,011
+// samples x 16,384 classes wrote and read 1.3 GB of them twice (3.4 ms in five
+// products and five scans) and take 0.3 ms here.  Bound by the exponential and
+// the compare of each logit (VALU).
+__global__ __launch_bounds__(256) void logits_top4(const float* __restrict__ Q, int n, const float* __restrict__ O,
+                                                   const float* __restrict__ cb, int C, int cper, Top4* part) {
+  __shared__ uint4 Os[kCeCls * 4];
+  __shared__ __attribute__((aligned(16))) float cbs[kCeCls];
+  const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
+  const int row = blockIdx.x * 64 + (threadIdx.x >> 6) * 16 + c16;
+  const bf16x8 b = ld_row8(Q, n, row, 8 * g);
+  Top4 t;
+  for (int k = 0; k < 4; ++k) {
+    t.v[k] = -INFINITY;
+    t.c[k] = -1;
+  }
+  t.m = -INFINITY;
+  t.s = 0.f;
+  const int cbeg = blockIdx.y * cper, cend = min(C, cbeg + cper);
+  for (int cc = cbeg; cc < cend; cc += kCeCls) {
+    const int nc = min(kCeCls, cend - cc);
+    __syncthreads();  // the previous stage is read
+    stage_rows(Os, O, cc, nc);
+    // a class past the end has a logit of -inf
+    for (int i = threadIdx.x; i < kCeCls; i += blockDim.x) cbs[i] = i < nc ? cb[cc + i] : -INFINITY;
+    __syncthreads();
+    for (int ct = 0; ct < nc; ct += 16) {
+      const bf16x8 a = lds_row8(Os, ct + c16, g, ct + c16 < nc);
+      const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      const float4 bias = *reinterpret_cast<const float4*>(cbs + ct + 4 * g);
+      const float x[4] = {acc[0] + bias.x, acc[1] + bias.y, acc[2] + bias.z, acc[3] + bias.w};
+      const float mx = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
+      if (mx > t.v[3]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (x[i] > t.v[3]) top4_insert(t, x[i], cc + ct + 4 * g + i);
+        if (mx > t.m) {
+          t.s *= expf(t.m - mx);
+          t.m = mx;
+        }
+      }
+      if (t.m > -INFINITY) t.s += (expf(x[0] - t.m) + expf(x[1] - t.m)) + (expf(x[2] - t.m) + expf(x[3] - t.m));
+    }
+  }
+  // the four lane groups hold quarters of the same rows' classes
+  for (int o = 16; o < 64; o <<= 1) {
+    Top4 u;
+    for (int k = 0; k < 4; ++k) {
+      u.v[k] = __shfl_xor(t.v[k], o, 64);
+      u.c[k] = __shfl_xor(t.c[k], o, 64);
+    }
+    u.m = __shfl_xor(t.m, o, 64);
+    u.s = __shfl_xor(t.s, o, 64);
+    top4_merge(t, u);
+  }
+  if (g == 0 && row < n) part[(size_t)blockIdx.y * n + row] = t;
+}
+
+// One thread per row: its class splits merged, then classes and probabilities.
+__global__ __launch_bounds__(64) void top4_finish(const Top4* part, int n, int splits, uint32_t* out, float* prob) {
+  const int r = blockIdx.x * 64 + threadIdx.x;
+  if (r >= n) return;
+  Top4 t = part[r];
+  for (int k = 1; k < splits; ++k) top4_merge(t, part[(size_t)k * n + r]);
+  for (int k = 0; k < 4; ++k) out[(size_t)r * 4 + k] = t.c[k] < 0 ? RTX_NO_TREELET : (uint32_t)t.c[k];
+  if (prob)
+    for (int k = 0; k < 4; ++k) prob[(size_t)r * 4 + k] = t.c[k] < 0 ? 0.f : expf(t.v[k] - t.m) / t.s;
 }
 
 // dL of one logit: (softmax - onehot) / n.
@@ -604,10 +770,15 @@ struct rtx_mlp {
   uint32_t steps = 0;
   // activations of one batch
   uint32_t cap = 0;
-  float *X = nullptr, *H1 = nullptr, *H2 = nullptr, *Q = nullptr, *L = nullptr;
+  float *X = nullptr, *H1 = nullptr, *H2 = nullptr, *Q = nullptr;
   float *dQ = nullptr, *dH2 = nullptr, *dH1 = nullptr, *dX = nullptr, *loss = nullptr;
   // fused output layer: per-row chunk maxima and exp-sums, target logits, log-sum-exp
   float *pm = nullptr, *ps = nullptr, *tl = nullptr, *lse = nullptr;
+  // the trunk's weights as MFMA operands (packed before each forward pass)
+  uint4* frags = nullptr;
+  // prediction: queries and per-split results of one chunk of rows
+  float* pred_q = nullptr;
+  Top4* pred_part = nullptr;
 };
 
 namespace {
@@ -615,7 +786,7 @@ namespace {
 int ce_chunks(const rtx_mlp* m) { return (int)((m->C + kCeChunk - 1) / kCeChunk); }
 
 void mlp_free_acts(rtx_mlp* m) {
-  float** bufs[] = {&m->X, &m->H1, &m->H2, &m->Q, &m->L, &m->dQ, &m->dH2, &m->dH1, &m->dX,
+  float** bufs[] = {&m->X, &m->H1, &m->H2, &m->Q, &m->dQ, &m->dH2, &m->dH1, &m->dX,
                     &m->pm, &m->ps, &m->tl, &m->lse};
   for (float** b : bufs) {
     if (*b) (void)hipFree(*b);
@@ -628,13 +799,12 @@ rtx_status mlp_ensure(rtx_mlp* m, uint32_t b) {
   if (b <= m->cap) return RTX_OK;
   mlp_free_acts(m);
   const size_t nch = (size_t)ce_chunks(m);
-  const size_t sizes[] = {(size_t)b * kInPad, (size_t)b * kHid, (size_t)b * kHid, (size_t)b * kEmb,
-                          (size_t)b * m->C,   (size_t)b * kEmb, (size_t)b * kHid, (size_t)b * kHid,
-                          (size_t)b * kInPad, (size_t)b * nch,  (size_t)b * nch,  (size_t)b,
-                          (size_t)b};
-  float** bufs[] = {&m->X, &m->H1, &m->H2, &m->Q, &m->L, &m->dQ, &m->dH2, &m->dH1, &m->dX,
+  const size_t sizes[] = {(size_t)b * kInPad, (size_t)b * kHid,   (size_t)b * kHid, (size_t)b * kEmb,
+                          (size_t)b * kEmb,   (size_t)b * kHid,   (size_t)b * kHid, (size_t)b * kInPad,
+                          (size_t)b * nch,    (size_t)b * nch,    (size_t)b,        (size_t)b};
+  float** bufs[] = {&m->X, &m->H1, &m->H2, &m->Q, &m->dQ, &m->dH2, &m->dH1, &m->dX,
                     &m->pm, &m->ps, &m->tl, &m->lse};
-  for (int k = 0; k < 13; ++k)
+  for (int k = 0; k < 12; ++k)
     if (hipMalloc(bufs[k], sizes[k] * sizeof(float)) != hipSuccess) {
       (void)hipGetLastError();
       mlp_free_acts(m);
@@ -652,28 +822,36 @@ rtx_status mlp_ensure(rtx_mlp* m, uint32_t b) {
     }                               \
   } while (0)
 
-// Forward over n samples; logits stay in m->L (without the output bias) unless
-// `logits` is false (the fused output layer computes them itself).
-rtx_status mlp_forward(rtx_mlp* m, const rtx_mlp_sample* s, uint32_t n, bool logits = true) {
-  hipStream_t st = m->stream;
-  float* P = m->P;
-  hipLaunchKernelGGL(build_input, dim3(n), dim3(64), 0, st, s, (int)n, P + m->oE, (int)m->T, m->X);
-  MK(hipGetLastError());
-  MK(gemm<false, false>(st, n, kHid, kInPad, m->X, kInPad, P + m->oW1, kHid, m->H1, kHid, 0));
-  hipLaunchKernelGGL(bias_act, dim3(256), dim3(256), 0, st, m->H1, (int)n, kHid, P + m->ob1, 1);
-  MK(gemm<false, false>(st, n, kHid, kHid, m->H1, kHid, P + m->oW2, kHid, m->H2, kHid, 0));
-  hipLaunchKernelGGL(bias_act, dim3(256), dim3(256), 0, st, m->H2, (int)n, kHid, P + m->ob2, 1);
-  MK(gemm<false, false>(st, n, kEmb, kHid, m->H2, kHid, P + m->oW3, kEmb, m->Q, kEmb, 0));
-  hipLaunchKernelGGL(bias_act, dim3(64), dim3(256), 0, st, m->Q, (int)n, kEmb, P + m->ob3, 0);
-  // logits = Q . O^T  (O is [C x 32])
-  if (logits) MK(gemm<false, true>(st, n, m->C, kEmb, m->Q, kEmb, P + m->oO, kEmb, m->L, m->C, 0));
+Weights weights_of(const rtx_mlp* m) {
+  return Weights{m->P + m->oW1, m->P + m->ob1, m->P + m->oW2, m->P + m->ob2, m->P + m->oW3, m->P + m->ob3};
+}
+
+hipError_t pack(rtx_mlp* m) {
+  hipLaunchKernelGGL(pack_weights, dim3((kFragEnd + 3) / 4), dim3(256), 0, m->stream, weights_of(m), m->frags);
+  return hipGetLastError();
+}
+
+// Prediction: rows per pass, (row, class split) results it keeps (at most
+// 10 MB), and the workgroups it aims at (eight per CU).
+constexpr uint32_t kPredRows = 65536, kPredParts = 4 * kPredRows, kPredBlocks = 2048;
+
+// Batches of at most this many rows accumulate in 64-deep partial products.
+constexpr uint32_t kChunkedRows = 1984;
+
+// Forward over one training batch, up to the queries (the fused output layer
+// computes the logits itself).
+rtx_status mlp_forward(rtx_mlp* m, const rtx_mlp_sample* s, uint32_t n) {
+  MK(pack(m));
+  hipLaunchKernelGGL(trunk_forward<true>, dim3((n + kRowTile - 1) / kRowTile), dim3(256), 0, m->stream, s, (int)n,
+                     m->P + m->oE, (int)m->T, weights_of(m), m->frags, n <= kChunkedRows ? 0 : INT_MAX, m->X, m->H1,
+                     m->H2, m->Q);
   MK(hipGetLastError());
   return RTX_OK;
 }
 
 // Forward + backward of one batch; gradients are added into m->G.
 rtx_status mlp_fwd_bwd(rtx_mlp* m, const rtx_mlp_sample* s, uint32_t n, float inv_n) {
-  rtx_status stt = mlp_forward(m, s, n, false);
+  rtx_status stt = mlp_forward(m, s, n);
   if (stt != RTX_OK) return stt;
   hipStream_t st = m->stream;
   float *P = m->P, *G = m->G;
@@ -766,7 +944,7 @@ rtx_status rtx_mlp_create(rtx_ctx* c, uint32_t n_treelets, uint32_t n_classes, u
   (void)hipSetDevice(m->device);
   if (hipMalloc(&m->P, o * 4) != hipSuccess || hipMalloc(&m->G, o * 4) != hipSuccess ||
       hipMalloc(&m->M1, o * 4) != hipSuccess || hipMalloc(&m->V1, o * 4) != hipSuccess ||
-      hipMalloc(&m->loss, 4) != hipSuccess) {
+      hipMalloc(&m->loss, 4) != hipSuccess || hipMalloc(&m->frags, kFragEnd * 1024) != hipSuccess) {
     (void)hipGetLastError();
     rtx_mlp_destroy(m);
     return RTX_ERR_OUT_OF_MEMORY;
@@ -799,6 +977,9 @@ rtx_status rtx_mlp_destroy(rtx_mlp* m) {
   float* bufs[] = {m->P, m->G, m->M1, m->V1, m->loss};
   for (float* b : bufs)
     if (b) (void)hipFree(b);
+  if (m->frags) (void)hipFree(m->frags);
+  if (m->pred_q) (void)hipFree(m->pred_q);
+  if (m->pred_part) (void)hipFree(m->pred_part);
   delete m;
   return RTX_OK;
 }
@@ -872,14 +1053,33 @@ rtx_status rtx_mlp_predict(rtx_mlp* m, const rtx_mlp_sample* samples, uint32_t n
                            float* probs_dev) {
   if (!m || !samples || !top4_dev || n == 0) return RTX_ERR_INVALID_ARGUMENT;
   MK(hipSetDevice(m->device));
-  const uint32_t chunk = 4096;
-  rtx_status st = mlp_ensure(m, std::min(n, chunk));
-  if (st != RTX_OK) return st;
-  for (uint32_t b0 = 0; b0 < n; b0 += chunk) {
-    const uint32_t b = std::min(chunk, n - b0);
-    st = mlp_forward(m, samples + b0, b);
-    if (st != RTX_OK) return st;
-    hipLaunchKernelGGL(top4, dim3(b), dim3(64), 0, m->stream, m->L, (int)b, (int)m->C, m->P + m->oc,
+  if (!m->pred_q) {
+    if (hipMalloc(&m->pred_q, (size_t)kPredRows * kEmb * 4) != hipSuccess ||
+        hipMalloc(&m->pred_part, (size_t)kPredParts * sizeof(Top4)) != hipSuccess) {
+      (void)hipGetLastError();
+      return RTX_ERR_OUT_OF_MEMORY;
+    }
+  }
+  // the last rows past a multiple of 4,096 are a batch of their own
+  const uint32_t last = n % 4096;
+  const uint32_t chunk_from = last && last <= kChunkedRows ? n - last : n;
+  MK(pack(m));
+  for (uint32_t b0 = 0; b0 < n; b0 += kPredRows) {
+    const uint32_t b = std::min(kPredRows, n - b0);
+    // class splits: enough workgroups for the chip, of whole LDS stages
+    const uint32_t row_blocks = (b + 63) / 64;
+    uint32_t splits = std::max(1u, std::min((kPredBlocks + row_blocks - 1) / row_blocks, (m->C + kCeCls - 1) / kCeCls));
+    splits = std::min(splits, std::max(1u, kPredParts / b));
+    const uint32_t stages = ((m->C + kCeCls - 1) / kCeCls + splits - 1) / splits;
+    const int cper = (int)(stages * kCeCls);
+    splits = (m->C + cper - 1) / cper;
+    hipLaunchKernelGGL(trunk_forward<false>, dim3((b + kRowTile - 1) / kRowTile), dim3(256), 0, m->stream,
+                       samples + b0, (int)b, m->P + m->oE, (int)m->T, weights_of(m), m->frags,
+                       chunk_from <= b0 ? 0 : (int)std::min(chunk_from - b0, b), (float*)nullptr, (float*)nullptr,
+                       (float*)nullptr, m->pred_q);
+    hipLaunchKernelGGL(logits_top4, dim3(row_blocks, splits), dim3(256), 0, m->stream, m->pred_q, (int)b,
+                       m->P + m->oO, m->P + m->oc, (int)m->C, cper, m->pred_part);
+    hipLaunchKernelGGL(top4_finish, dim3((b + 63) / 64), dim3(64), 0, m->stream, m->pred_part, (int)b, (int)splits,
                        top4_dev + (size_t)b0 * 4, probs_dev ? probs_dev + (size_t)b0 * 4 : nullptr);
     MK(hipGetLastError());
   }
