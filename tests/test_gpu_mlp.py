@@ -149,3 +149,41 @@ def test_predict_at_tile_edges(gpu, T, C, n):
         assert np.all(top[:, k:] == 0xFFFFFFFF) and np.all(prob[:, k:] == 0)
     finally:
         mlp.close()
+
+
+@pytest.mark.parametrize("T,C,n,batch", [(40, 33, 70, 33), (500, 300, 260, 129), (7, 1000, 40, 40)])
+def test_training_matches_oracle_steps(gpu, T, C, n, batch):
+    """Whole Adam epochs (row and class counts off the 16- and 32-wide tiles, a short
+    last batch, embedding rows no sample names) against the oracle's gradients and a
+    plain Adam.  A step moves a weight by at most lr, and BF16 flips change a gradient
+    by about 1%, so after k steps weights agree to 0.1 * k * lr in the mean; a
+    gradient near zero may change sign, which bounds a single weight by 2 * k * lr.
+    Rows without samples stay as they were, bit for bit."""
+    rng = np.random.default_rng(T + C)
+    lr, epochs = 1e-3, 2
+    mlp = gpu.mlp(T, C, seed=T)
+    try:
+        s = _samples(rng, T // 2, C, n)  # the upper half of the rows is never named
+        vec = mlp.params()
+        start = vec.copy()
+        mlp.train(s, epochs=epochs, batch=batch, lr=lr)
+        got, grads = mlp.params(), mlp.grads()
+        m, v, k = np.zeros(len(vec)), np.zeros(len(vec)), 0
+        p = vec.astype(np.float64)
+        for _ in range(epochs):
+            for b in range(0, n, batch):
+                k += 1
+                _, G = mo.loss_and_grad(mo.unpack(p.astype(np.float32), T, C), s[b:b + batch], bf16=True)
+                g = mo.pack(G, T, C).astype(np.float64)
+                m = 0.9 * m + 0.1 * g
+                v = 0.999 * v + 0.001 * g * g
+                p -= lr * (m / (1 - 0.9 ** k)) / (np.sqrt(v / (1 - 0.999 ** k)) + 1e-8)
+        d = np.abs(got - p)
+        moved = np.abs(p - start) > 0
+        assert d.max() <= 2 * k * lr and d[moved].mean() <= 0.1 * k * lr
+        rows = mo.unpack(got, T, C)["E"], mo.unpack(start, T, C)["E"]
+        assert np.array_equal(rows[0][T // 2:T], rows[1][T // 2:T])
+        # the last batch's gradients stay readable
+        assert np.linalg.norm(grads - g) <= 0.1 * np.linalg.norm(g)
+    finally:
+        mlp.close()

@@ -103,34 +103,73 @@ __global__ void zero_rows(float* C, int M, int N, int ldc) {
 }
 
 // ---- trunk: x -> h1 -> h2 -> q in one kernel ------------------------------------
-// Weights as MFMA operands: fragment (column tile ct, 32-deep step ks) of a
+// Matrices as MFMA operands: fragment (column tile ct, 32-deep step ks) of a
 // K x N matrix holds, for lane l, the eight k values 32 ks + 8 (l / 16) + t of
-// column 16 ct + l % 16, rounded to BF16, at [(ct * KS + ks) * 64 + l].
-constexpr int kFrag1 = 0;                                       // W1: 192 x 128
-constexpr int kFrag2 = kFrag1 + (kHid / 16) * (kInPad / 32);    // W2: 128 x 128
-constexpr int kFrag3 = kFrag2 + (kHid / 16) * (kHid / 32);      // W3: 128 x 32
-constexpr int kFragEnd = kFrag3 + (kEmb / 16) * (kHid / 32);
+// column 16 ct + l % 16, rounded to BF16, at [(ct * KS + ks) * 64 + l].  The
+// forward pass takes W1, W2, W3, the backward pass their transposes.
+constexpr int kFrag1 = 0;                                        // W1: 192 x 128
+constexpr int kFrag2 = kFrag1 + (kHid / 16) * (kInPad / 32);     // W2: 128 x 128
+constexpr int kFrag3 = kFrag2 + (kHid / 16) * (kHid / 32);       // W3: 128 x 32
+constexpr int kFragForward = kFrag3 + (kEmb / 16) * (kHid / 32);
+constexpr int kFragT3 = kFragForward;                            // W3^T: 32 x 128
+constexpr int kFragT2 = kFragT3 + (kHid / 16) * (kEmb / 32);     // W2^T: 128 x 128
+constexpr int kFragT1 = kFragT2 + (kHid / 16) * (kHid / 32);     // W1^T: 128 x 192
+constexpr int kFragEnd = kFragT1 + (kInPad / 16) * (kHid / 32);
 struct Weights {
   const float *W1, *b1, *W2, *b2, *W3, *b3;
 };
 
-__global__ __launch_bounds__(256) void pack_weights(Weights w, uint4* frags) {
-  const int f = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (f >= kFragEnd) return;
-  const float* W;
-  int cols, ks_n, at;
-  if (f < kFrag2) {
-    W = w.W1, cols = kHid, ks_n = kInPad / 32, at = f - kFrag1;
-  } else if (f < kFrag3) {
-    W = w.W2, cols = kHid, ks_n = kHid / 32, at = f - kFrag2;
-  } else {
-    W = w.W3, cols = kEmb, ks_n = kHid / 32, at = f - kFrag3;
-  }
-  const int col = (at / ks_n) * 16 + (lane & 15), k0 = (at % ks_n) * 32 + (lane >> 4) * 8;
+// The tile row paired with k-slot 8g + j of an MFMA that takes a result tile as
+// its operand (see the fused output layer).
+__device__ __forceinline__ int kslot_row(int g, int j) { return j < 4 ? 4 * g + j : 16 + 4 * g + j - 4; }
+
+// One wave per fragment: `count` of the trunk's, then (training) the output
+// layer's: for each 16 classes the rows' fragment (lane: class c16, elements
+// 8g..8g+7), for each 32 classes and half e of the embedding the columns'
+// fragment (lane: element 16e + c16 of the classes kslot_row(g, j)).  Classes
+// past C are zero rows with a bias of -inf, so the passes over them test no
+// bounds.
+__global__ __launch_bounds__(256) void pack_operands(Weights w, int count, uint4* frags, const float* O,
+                                                     const float* cb, int C, int c_tiles, uint4* oa, uint4* ot,
+                                                     float* cbp) {
+  const int f = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, c16 = lane & 15, g = lane >> 4;
   bf16x8 v;
+  if (f < count) {
+    const float* W;
+    int cols, ks_n, at;
+    bool tr = false;
+    if (f < kFrag2) {
+      W = w.W1, cols = kHid, ks_n = kInPad / 32, at = f - kFrag1;
+    } else if (f < kFrag3) {
+      W = w.W2, cols = kHid, ks_n = kHid / 32, at = f - kFrag2;
+    } else if (f < kFragT3) {
+      W = w.W3, cols = kEmb, ks_n = kHid / 32, at = f - kFrag3;
+    } else if (f < kFragT2) {
+      W = w.W3, cols = kEmb, ks_n = kEmb / 32, at = f - kFragT3, tr = true;
+    } else if (f < kFragT1) {
+      W = w.W2, cols = kHid, ks_n = kHid / 32, at = f - kFragT2, tr = true;
+    } else {
+      W = w.W1, cols = kHid, ks_n = kHid / 32, at = f - kFragT1, tr = true;
+    }
+    const int col = (at / ks_n) * 16 + c16, k0 = (at % ks_n) * 32 + g * 8;
 #pragma unroll
-  for (int t = 0; t < 8; ++t) v[t] = (__bf16)W[(size_t)(k0 + t) * cols + col];
-  frags[(size_t)f * 64 + lane] = __builtin_bit_cast(uint4, v);
+    for (int t = 0; t < 8; ++t) v[t] = (__bf16)(tr ? W[(size_t)col * cols + k0 + t] : W[(size_t)(k0 + t) * cols + col]);
+    frags[(size_t)f * 64 + lane] = __builtin_bit_cast(uint4, v);
+  } else if (f - count < c_tiles) {
+    const int ct = f - count, cls = ct * 16 + c16;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) v[t] = (__bf16)(cls < C ? O[(size_t)cls * kEmb + 8 * g + t] : 0.f);
+    oa[(size_t)ct * 64 + lane] = __builtin_bit_cast(uint4, v);
+    if (lane < 16) cbp[cls] = cls < C ? cb[cls] : -INFINITY;
+  } else if (f - count < 2 * c_tiles) {
+    const int q = f - count - c_tiles, c0 = (q >> 1) * 32, e = q & 1;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int cls = c0 + kslot_row(g, j);
+      v[j] = (__bf16)(cls < C ? O[(size_t)cls * kEmb + 16 * e + c16] : 0.f);
+    }
+    ot[(size_t)q * 64 + lane] = __builtin_bit_cast(uint4, v);
+  }
 }
 
 // One layer of 16 rows held in LDS as BF16 (`stride` values a row): the 16x16
@@ -165,15 +204,15 @@ __device__ __forceinline__ f32x4 layer_tile(const __bf16* rows, int stride, cons
 // 64-deep partial products, and the third always does: the order of the K-split
 // products of batches that small, kept so that results stay what they were.
 constexpr int kRowTile = 16;
-constexpr int kXStride = kInPad + 8, kHStride = kHid + 8;  // LDS rows start in different banks
+constexpr int kXStride = kInPad + 8, kHStride = kHid + 8, kQStride = kEmb + 8;  // LDS rows start in different banks
 
 template <bool TRAIN>
 __global__ __launch_bounds__(256) void trunk_forward(const rtx_mlp_sample* __restrict__ samples, int n,
                                                      const float* __restrict__ E, int none, Weights w,
                                                      const uint4* __restrict__ frags, int chunk_from, float* X,
-                                                     float* H1, float* H2, float* Q) {
+                                                     float* H1, float* H2, float* Q, uint4* qa, uint4* qt) {
   __shared__ __attribute__((aligned(16))) __bf16 xs[kRowTile * kXStride], h1s[kRowTile * kHStride],
-      h2s[kRowTile * kHStride];
+      h2s[kRowTile * kHStride], qs[TRAIN ? kRowTile * kQStride : 8];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, g = lane >> 4;
   const int r0 = blockIdx.x * kRowTile;
   const bool chunked = r0 >= chunk_from;
@@ -232,112 +271,240 @@ __global__ __launch_bounds__(256) void trunk_forward(const rtx_mlp_sample* __res
     const int col = wave * 16 + c16;
     const f32x4 z = layer_tile<kHid / 32>(h2s, kHStride, frags + kFrag3 * 64, wave, lane, true);
     const float bias = w.b3[col];
-    for (int i = 0; i < 4; ++i)
-      if (r0 + 4 * g + i < n) Q[(size_t)(r0 + 4 * g + i) * kEmb + col] = z[i] + bias;
+    for (int i = 0; i < 4; ++i) {
+      const bool in = r0 + 4 * g + i < n;
+      const float q = z[i] + bias;
+      if (in) Q[(size_t)(r0 + 4 * g + i) * kEmb + col] = q;
+      if (TRAIN) qs[(4 * g + i) * kQStride + col] = (__bf16)(in ? q : 0.f);
+    }
+  }
+  if constexpr (TRAIN) {
+    // the queries as the output layer's operands, both orientations (see
+    // pack_operands; rows past n are zero)
+    __syncthreads();
+    if (wave == 0) {
+      qa[(size_t)blockIdx.x * 64 + lane] = *reinterpret_cast<const uint4*>(qs + c16 * kQStride + 8 * g);
+    } else if (wave < 3) {
+      const int e = wave - 1;
+      __bf16 v[4];
+      for (int j = 0; j < 4; ++j) v[j] = qs[(4 * g + j) * kQStride + 16 * e + c16];
+      uint2* dst = reinterpret_cast<uint2*>(qt + (size_t)((blockIdx.x >> 1) * 2 + e) * 64 + lane) + (blockIdx.x & 1);
+      *dst = *reinterpret_cast<uint2*>(v);
+    }
   }
 }
 
 // ---- elementwise and reductions ---------------------------------------------------
-__global__ void relu_mask(float* dH, const float* H, size_t total) {
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < total; k += (size_t)gridDim.x * blockDim.x)
-    if (!(H[k] > 0.f)) dH[k] = 0.f;
+// One Adam update.  Embedding rows never named by a sample have zero gradients
+// and moments, so their update is exactly zero and only their flag is read:
+// eight lanes per row, then the other parameters.  `clear` leaves the gradients
+// zero for the next batch.  Bound by HBM and the last-level cache: seven or
+// eight 4-byte streams over what has been touched.  7.0M parameters (200,000
+// treelets, a fifth of them named within an epoch of 65,700 samples): 28 us after
+// an 8 us clear -> 16 us.
+__device__ __forceinline__ void adam_one(float& p, float g, float& m, float& v, float lr, float b1, float b2, float eps,
+                                         float c1, float c2) {
+  m = b1 * m + (1.f - b1) * g;
+  v = b2 * v + (1.f - b2) * g * g;
+  p -= lr * (m / c1) / (sqrtf(v / c2) + eps);
 }
 
-// column sums of M[n x cols] added into out; blockIdx.y takes rows
-// [kColsumRows * blockIdx.y, kColsumRows * blockIdx.y + kColsumRows)
-constexpr int kColsumRows = 8;
-__global__ void colsum(const float* M, int n, int cols, float* out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
-  const int r0 = blockIdx.y * kColsumRows, r1 = min(n, r0 + kColsumRows);
-  float s = 0.f;
-  for (int r = r0; r < r1; ++r) s += M[(size_t)r * cols + c];
-  atomicAdd(&out[c], s);
-}
-
-__device__ float block_reduce(float v, float* sm, bool is_max) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  for (int o = 32; o > 0; o >>= 1) {
-    float y = __shfl_xor(v, o, 64);
-    v = is_max ? fmaxf(v, y) : v + y;
-  }
-  if (lane == 0) sm[w] = v;
-  __syncthreads();
-  float r = sm[0];
-  for (int k = 1; k < (int)(blockDim.x >> 6); ++k) r = is_max ? fmaxf(r, sm[k]) : r + sm[k];
-  __syncthreads();
-  return r;
-}
-
-// dE[row of slot h of sample i][e] += dX[i][column of slot h, e] for the five
-// embedding slots (cur, hist 0-3).  One wave takes 64 samples of one (slot,
-// column) pair and adds the values of lanes that name the same row with one
-// atomic: the ancestors in the history are shared by most samples, and
-// per-sample atomics on those rows serialise.  grid.x: 64-sample groups,
-// grid.y: 5 slots x 32 columns.
-__global__ __launch_bounds__(64) void scatter_embed(const float* dX, const rtx_mlp_sample* s, int n, int none,
-                                                   float* dE) {
-  const int lane = threadIdx.x;
-  const int i = blockIdx.x * 64 + lane;
-  const int h = blockIdx.y / kEmb, e = blockIdx.y % kEmb;
-  uint32_t row = 0xffffffffu;
-  float v = 0.f;
-  if (i < n) {
-    const rtx_mlp_sample sm = s[i];
-    uint32_t t;
-    int col;
-    if (h == 0) {
-      t = sm.cur > (uint32_t)none ? (uint32_t)none : sm.cur;  // out-of-range treelets read the "none" row
-      col = e;
+__global__ __launch_bounds__(256) void adam_step(float* p, float* g, float* m, float* v, const uint8_t* touched,
+                                                 size_t rows, size_t count, int clear, float lr, float b1, float b2,
+                                                 float eps, float c1, float c2) {
+  const size_t quads = (count + 3) / 4, row_quads = rows * (kEmb / 4);
+  for (size_t q = blockIdx.x * (size_t)256 + threadIdx.x; q < quads; q += (size_t)gridDim.x * 256) {
+    if (q < row_quads && !touched[q / (kEmb / 4)]) continue;
+    if (q * 4 + 4 <= count) {
+      float4 P = reinterpret_cast<float4*>(p)[q], M = reinterpret_cast<float4*>(m)[q], V = reinterpret_cast<float4*>(v)[q];
+      const float4 G = reinterpret_cast<float4*>(g)[q];
+      adam_one(P.x, G.x, M.x, V.x, lr, b1, b2, eps, c1, c2);
+      adam_one(P.y, G.y, M.y, V.y, lr, b1, b2, eps, c1, c2);
+      adam_one(P.z, G.z, M.z, V.z, lr, b1, b2, eps, c1, c2);
+      adam_one(P.w, G.w, M.w, V.w, lr, b1, b2, eps, c1, c2);
+      reinterpret_cast<float4*>(p)[q] = P;
+      reinterpret_cast<float4*>(m)[q] = M;
+      reinterpret_cast<float4*>(v)[q] = V;
+      if (clear) reinterpret_cast<float4*>(g)[q] = make_float4(0.f, 0.f, 0.f, 0.f);
     } else {
-      t = sm.hist[h - 1];
-      if (t == RTX_NO_TREELET || t > (uint32_t)none) t = (uint32_t)none;
-      col = 41 + (h - 1) * kEmb + e;
+      for (size_t k = q * 4; k < count; ++k) {
+        adam_one(p[k], g[k], m[k], v[k], lr, b1, b2, eps, c1, c2);
+        if (clear) g[k] = 0.f;
+      }
     }
-    row = t;
-    v = dX[(size_t)i * kInPad + col];
-  }
-  uint64_t left = __ballot(i < n);
-  while (left) {
-    const int lead = __ffsll((long long)left) - 1;
-    const uint32_t key = __shfl(row, lead, 64);
-    const bool mine = (left >> lane) & 1ull && row == key;
-    float x = mine ? v : 0.f;
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-    if (lane == lead) atomicAdd(&dE[(size_t)key * kEmb + e], x);
-    left &= ~__ballot(mine);
   }
 }
 
-__global__ void adam_step(float* p, const float* g, float* m, float* v, size_t count, float lr, float b1, float b2,
-                          float eps, float c1, float c2) {
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < count; k += (size_t)gridDim.x * blockDim.x) {
-    const float gk = g[k];
-    const float mk = b1 * m[k] + (1.f - b1) * gk;
-    const float vk = b2 * v[k] + (1.f - b2) * gk * gk;
-    m[k] = mk;
-    v[k] = vk;
-    p[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + eps);
+// ---- trunk backward ---------------------------------------------------------------
+// dq -> dh2 -> dh1 -> dx for 16 samples per workgroup, as trunk_forward goes
+// forward: dh2 and dh1 are stored for the weight gradients, the bias gradients
+// are column sums, and dx goes straight into the embedding rows it came from.
+// Samples of a workgroup that name the same row add up in LDS first: the
+// ancestors in the history are shared by most samples, and one atomic per
+// sample on those rows would serialise.  1,024 samples: 96 us in eleven launches
+// (products with zeroing, masks, column sums, a scatter over 160 passes) -> 12.
+struct Gradients {
+  float *E, *b1, *b2, *b3;
+};
+
+__global__ __launch_bounds__(256) void trunk_backward(const rtx_mlp_sample* __restrict__ samples, int n, int none,
+                                                      const uint4* __restrict__ frags, const float* __restrict__ dQ,
+                                                      const float* __restrict__ H1, const float* __restrict__ H2,
+                                                      float* dH1, float* dH2, Gradients G, uint8_t* touched) {
+  __shared__ __attribute__((aligned(16))) __bf16 qs[kRowTile * kQStride], h2s[kRowTile * kHStride],
+      h1s[kRowTile * kHStride];
+  __shared__ float xs[kRowTile * (kInPad + 4)];
+  __shared__ uint32_t rows[5][kRowTile], same[5][kRowTile];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, g = lane >> 4;
+  const int r0 = blockIdx.x * kRowTile;
+  if (threadIdx.x < 5 * kRowTile) {
+    const int h = threadIdx.x / kRowTile, i = threadIdx.x % kRowTile;
+    uint32_t t = 0xffffffffu;
+    if (r0 + i < n) {
+      const rtx_mlp_sample& sm = samples[r0 + i];
+      t = h == 0 ? sm.cur : sm.hist[h - 1];
+      if (t > (uint32_t)none) t = (uint32_t)none;  // as the forward pass reads it
+    }
+    rows[h][i] = t;
   }
+  {
+    // two rows per wave and pass
+    float sum = 0.f;
+    const int col = threadIdx.x % kEmb;
+    for (int row = threadIdx.x / kEmb; row < kRowTile; row += 8) {
+      const float v = r0 + row < n ? dQ[(size_t)(r0 + row) * kEmb + col] : 0.f;
+      qs[row * kQStride + col] = (__bf16)v;
+      sum += v;
+    }
+    xs[threadIdx.x] = sum;
+  }
+  __syncthreads();
+  if (threadIdx.x < kEmb) {
+    float sum = 0.f;
+    for (int k = 0; k < 8; ++k) sum += xs[k * kEmb + threadIdx.x];
+    atomicAdd(&G.b3[threadIdx.x], sum);
+  } else if (threadIdx.x >= 64 && threadIdx.x < 64 + 5 * kRowTile) {
+    // the samples that name this one's row, none when an earlier one does
+    const int h = (threadIdx.x - 64) / kRowTile, i = (threadIdx.x - 64) % kRowTile;
+    const uint32_t t = rows[h][i];
+    uint32_t m = 0;
+    for (int k = 0; k < kRowTile; ++k) m |= rows[h][k] == t ? 1u << k : 0u;
+    same[h][i] = t == 0xffffffffu || (m & ((1u << i) - 1u)) ? 0u : m;
+  }
+  // masks a layer's tile where its activation was clipped, stores it, adds its column sums
+  auto finish = [&](f32x4 z, int col, const float* H, float* dH, __bf16* lds, float* gb) {
+    float sum = 0.f;
+    for (int i = 0; i < 4; ++i) {
+      const int r = r0 + 4 * g + i;
+      float v = 0.f;
+      if (r < n) {
+        v = H[(size_t)r * kHid + col] > 0.f ? z[i] : 0.f;
+        dH[(size_t)r * kHid + col] = v;
+      }
+      lds[(4 * g + i) * kHStride + col] = (__bf16)v;
+      sum += v;
+    }
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    if (g == 0) atomicAdd(&gb[col], sum);
+  };
+  for (int q = 0; q < 2; ++q) {
+    const int ct = 2 * wave + q;
+    finish(layer_tile<kEmb / 32>(qs, kQStride, frags + kFragT3 * 64, ct, lane, false), ct * 16 + c16, H2, dH2, h2s, G.b2);
+  }
+  __syncthreads();
+  for (int q = 0; q < 2; ++q) {
+    const int ct = 2 * wave + q;
+    finish(layer_tile<kHid / 32>(h2s, kHStride, frags + kFragT2 * 64, ct, lane, false), ct * 16 + c16, H1, dH1, h1s, G.b1);
+  }
+  __syncthreads();
+  for (int q = 0; q < 3; ++q) {
+    const int ct = 3 * wave + q;
+    const f32x4 z = layer_tile<kHid / 32>(h1s, kHStride, frags + kFragT1 * 64, ct, lane, false);
+    for (int i = 0; i < 4; ++i) xs[(4 * g + i) * (kInPad + 4) + ct * 16 + c16] = z[i];
+  }
+  __syncthreads();
+  // 32 threads per (slot, sample): the first sample that names a row adds it for all
+  const int e = threadIdx.x & 31;
+  for (int it = threadIdx.x >> 5; it < 5 * kRowTile; it += 8) {
+    const int h = it / kRowTile, i = it % kRowTile;
+    uint32_t m = same[h][i];
+    if (m == 0) continue;
+    const uint32_t t = rows[h][i];
+    const int col = h == 0 ? e : 41 + (h - 1) * kEmb + e;
+    float sum = 0.f;
+    for (; m; m &= m - 1) sum += xs[(__ffs((int)m) - 1) * (kInPad + 4) + col];
+    atomicAdd(&G.E[(size_t)t * kEmb + e], sum);
+    if (e == 0) touched[t] = 1;
+  }
+}
+
+// The three weight gradients A^T B over the batch's rows in one launch: 32 x 32
+// output tiles (24 of W1, 16 of W2, 4 of W3) by row ranges.  A workgroup's four
+// waves take every fourth 32-row step and add up in LDS, so an output element
+// takes one atomic per row range.  1,024 rows: 28 us in three launches -> 9; at
+// ranges of 256 rows, with two serial steps per wave, 16.
+struct WeightGrad {
+  const float *A, *B;
+  float* C;
+  int lda, ldb;
+};
+
+__global__ __launch_bounds__(256) void weight_grads(WeightGrad w1, WeightGrad w2, WeightGrad w3, int n, int rows_per) {
+  __shared__ float red[3][64 * 17];
+  const int id = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, g = lane >> 4;
+  const WeightGrad w = id < 24 ? w1 : id < 40 ? w2 : w3;
+  const int tile = id < 24 ? id : id < 40 ? id - 24 : (id - 40) * 4;
+  const int m0 = (tile / 4) * 32, n0 = (tile % 4) * 32;
+  const int rend = min(n, (int)(blockIdx.y + 1) * rows_per);
+  f32x4 acc[2][2];
+  for (int i = 0; i < 2; ++i)
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = blockIdx.y * rows_per + wave * 32; k0 < rend; k0 += 128) {
+    bf16x8 a[2], b[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        const int k = k0 + g * 8 + t;
+        a[i][t] = (__bf16)(k < rend ? w.A[(size_t)k * w.lda + m0 + i * 16 + c16] : 0.f);
+        b[i][t] = (__bf16)(k < rend ? w.B[(size_t)k * w.ldb + n0 + i * 16 + c16] : 0.f);
+      }
+    for (int i = 0; i < 2; ++i)
+      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+  }
+  if (wave > 0)
+    for (int q = 0; q < 16; ++q) red[wave - 1][lane * 17 + q] = acc[q >> 3][(q >> 2) & 1][q & 3];
+  __syncthreads();
+  if (wave == 0)
+    for (int q = 0; q < 16; ++q) {
+      const float v = ((acc[q >> 3][(q >> 2) & 1][q & 3] + red[0][lane * 17 + q]) + red[1][lane * 17 + q]) + red[2][lane * 17 + q];
+      atomicAdd(&w.C[(size_t)(m0 + (q >> 3) * 16 + 4 * g + (q & 3)) * w.ldb + n0 + ((q >> 2) & 1) * 16 + c16], v);
+    }
 }
 
 // ---- fused output layer ----------------------------------------------------------
 // The logits L = Q O^T + o (Q: [n x 32] queries, O: [C x 32] class vectors, o the
 // class biases) exist only as 16x16 MFMA tiles in registers.  ce_stats keeps each
 // row's running maximum and exp-sum over a chunk of classes; ce_finish turns the
-// chunks into the row's log-sum-exp and the loss; two gradient passes recompute
-// the tiles to form dL = (softmax - onehot) / n: ce_grad_o per 64 classes and
-// row split (dO = dL^T Q and the bias gradient) and ce_grad_q per 64 rows and
-// class split (dQ = dL O), each summing its splits atomically.  The sum over k inside one MFMA does not depend on which k-slot
-// holds which term, so a dL tile left in the result layout (lane = column, rows
-// 4g..4g+3 of lane group g = lane / 16) feeds the next MFMA as it is: k-slot
-// 8g + j pairs tile row 4g + j (j < 4) of the first 16-row tile with the same
-// k-slot of the other operand, and 4g + j - 4 of the second tile for j >= 4.
-constexpr int kCeChunk = 256;  // classes per ce_stats block
-constexpr int kCeSplit = 32;   // class splits of ce_grad_q
-constexpr int kCeRowSplit = 4; // row splits of ce_grad_o
-constexpr int kCeRows = 512;   // rows per LDS stage of ce_grad_o
-constexpr int kCeCls = 256;    // classes per LDS stage of ce_grad_q
+// chunks into the row's log-sum-exp and the loss; ce_grad recomputes the tiles to
+// form dL = (softmax - onehot) / n, once per 32 classes for dO = dL^T Q and the
+// bias gradient, once per 32 rows for dQ = dL O.  The sum over k inside one MFMA
+// does not depend on which k-slot holds which term, so a dL tile left in the
+// result layout (lane = column, rows 4g..4g+3 of lane group g = lane / 16) feeds
+// the next MFMA as it is: k-slot 8g + j pairs tile row 4g + j (j < 4) of the
+// first 16-row tile with the same k-slot of the other operand, and 4g + j - 4 of
+// the second tile for j >= 4.
+//
+// Every operand comes from a packed fragment (pack_operands, trunk_forward), one
+// 16-byte load per lane from L2, used for two tiles: rows staged through LDS had
+// cost sixteen 2-byte LDS reads per lane and 32 classes for the transposed
+// operand, the FP32 conversions again in each workgroup and two barriers per
+// stage.  1,024 rows x 16,384 classes: statistics 28 -> 12 us, both gradients 54
+// -> 22 us.  Bound by VALU work on each logit, the exponential above all.
+constexpr int kCeChunk = 256;  // classes per ce_stats wave
+constexpr int kCeCls = 256;    // classes per LDS stage of logits_top4
+constexpr int kCeRange = 512;  // classes per ce_grad wave that sums dQ
 
 // Eight FP32 values rounded to BF16 (round to nearest even, as the MFMA operand
 // loads of gemm_bf16), packed into 16 bytes.
@@ -366,12 +533,16 @@ __device__ __forceinline__ bf16x8 lds_row8(const uint4* S, int i, int g, bool va
   return __builtin_bit_cast(bf16x8, valid ? S[4 * i + g] : make_uint4(0, 0, 0, 0));
 }
 
-__device__ __forceinline__ __bf16 lds_elem(const uint4* S, int i, int col) {
-  return reinterpret_cast<const __bf16*>(S)[i * kEmb + col];
+__device__ __forceinline__ bf16x8 frag(const uint4* __restrict__ f, int at, int lane) {
+  return __builtin_bit_cast(bf16x8, f[(size_t)at * 64 + lane]);
 }
 
-// The tile row paired with k-slot 8g + j (see above).
-__device__ __forceinline__ int kslot_row(int g, int j) { return j < 4 ? 4 * g + j : 16 + 4 * g + j - 4; }
+// e^d for the terms of a softmax, d <= 0 up to rounding: one product and the
+// hardware's 2^x.  The product's rounding makes the relative error about
+// 1e-7 |d|, and a term weighs e^d, so a sum relative to its largest term is off by
+// at most 4e-8 per term, as with expf (whose range handling costs a dozen more
+// instructions per logit).
+__device__ __forceinline__ float exp_term(float d) { return __builtin_amdgcn_exp2f(d * 1.44269504088896340736f); }
 
 // (m, s) <- the log-sum-exp pair of the union of two sets: max and exp-sum relative to it.
 __device__ __forceinline__ void lse_merge(float& m, float& s, float m2, float s2) {
@@ -381,89 +552,212 @@ __device__ __forceinline__ void lse_merge(float& m, float& s, float m2, float s2
   m = mx;
 }
 
-// One block: 64 rows (a wave per 16) x kCeChunk classes (staged in LDS).
-// pm/ps[r * nchunk + chunk] get the row's maximum logit and its exp-sum over the
-// chunk; tl[r] the target's logit.
-__global__ __launch_bounds__(256) void ce_stats(const float* __restrict__ Q, int n, const float* __restrict__ O,
-                                                const float* __restrict__ cb, int C,
-                                                const rtx_mlp_sample* __restrict__ s, int nchunk, float* pm,
-                                                float* ps, float* tl) {
-  __shared__ uint4 Os[kCeChunk * 4];
-  __shared__ float cbs[kCeChunk];
+// One wave: 32 rows x kCeChunk classes, the classes as the MFMA's rows, so a lane
+// holds four logits of one sample per tile.  pm/ps[r * nchunk + chunk] get the
+// row's maximum logit and its exp-sum over the chunk.  grid.x: 32-row groups,
+// grid.y: four chunks per workgroup.
+__global__ __launch_bounds__(256) void ce_stats(const uint4* __restrict__ qa, int n, const uint4* __restrict__ oa,
+                                                const float* __restrict__ cbp, int c_tiles, int nchunk, float* pm,
+                                                float* ps) {
   const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
-  const int r0 = blockIdx.x * 64 + (threadIdx.x >> 6) * 16;
-  const int chunk = blockIdx.y;
-  const int c_lo = chunk * kCeChunk, nc = min(kCeChunk, C - c_lo);
-  stage_rows(Os, O, c_lo, nc);
-  for (int c = threadIdx.x; c < nc; c += blockDim.x) cbs[c] = cb[c_lo + c];
-  __syncthreads();
-  const bf16x8 a = ld_row8(Q, n, r0 + c16, 8 * g);
-  float m[4], sm[4];
-  uint32_t t[4];
-  for (int i = 0; i < 4; ++i) {
-    const int r = r0 + 4 * g + i;
-    m[i] = -INFINITY;
-    sm[i] = 0.f;
-    t[i] = r < n ? s[r].target : 0xffffffffu;
-  }
-  for (int ct = 0; ct < nc; ct += 16) {
-    const int cl = ct + c16;
-    const bf16x8 b = lds_row8(Os, cl, g, cl < nc);
-    const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-    if (cl < nc) {
-      const float bias = cbs[cl];
-      for (int i = 0; i < 4; ++i) {
-        const float x = acc[i] + bias;
-        const float mx = fmaxf(m[i], x);
-        sm[i] = sm[i] * expf(m[i] - mx) + expf(x - mx);
-        m[i] = mx;
-        if ((uint32_t)(c_lo + cl) == t[i]) tl[r0 + 4 * g + i] = x;
+  const int chunk = blockIdx.y * 4 + (threadIdx.x >> 6);
+  if (chunk >= nchunk) return;
+  const bf16x8 b[2] = {frag(qa, 2 * blockIdx.x, lane), frag(qa, 2 * blockIdx.x + 1, lane)};
+  float m[2] = {-INFINITY, -INFINITY}, s[2] = {0.f, 0.f};
+  const int t0 = chunk * (kCeChunk / 16), t1 = min(c_tiles, t0 + kCeChunk / 16);
+  for (int ct = t0; ct < t1; ++ct) {
+    const bf16x8 a = frag(oa, ct, lane);
+    const float4 bias = *reinterpret_cast<const float4*>(cbp + ct * 16 + 4 * g);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[k], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      const float x0 = acc[0] + bias.x, x1 = acc[1] + bias.y, x2 = acc[2] + bias.z, x3 = acc[3] + bias.w;
+      const float mx = fmaxf(fmaxf(x0, x1), fmaxf(x2, x3));
+      if (mx > m[k]) {
+        s[k] *= expf(m[k] - mx);
+        m[k] = mx;
       }
+      // a group whose classes are all padding so far keeps its empty sum
+      if (m[k] > -INFINITY) s[k] += (exp_term(x0 - m[k]) + exp_term(x1 - m[k])) + (exp_term(x2 - m[k]) + exp_term(x3 - m[k]));
     }
   }
-  // the 16 lanes of a group hold the same rows
-  for (int o = 1; o < 16; o <<= 1)
-    for (int i = 0; i < 4; ++i) {
-      const float m2 = __shfl_xor(m[i], o, 64), s2 = __shfl_xor(sm[i], o, 64);
-      lse_merge(m[i], sm[i], m2, s2);
+  // the four lane groups hold quarters of the chunk's classes
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    for (int o = 16; o < 64; o <<= 1) {
+      const float m2 = __shfl_xor(m[k], o, 64), s2 = __shfl_xor(s[k], o, 64);
+      lse_merge(m[k], s[k], m2, s2);
     }
-  if (c16 == 0)
-    for (int i = 0; i < 4; ++i) {
-      const int r = r0 + 4 * g + i;
-      if (r < n) {
-        pm[(size_t)r * nchunk + chunk] = m[i];
-        ps[(size_t)r * nchunk + chunk] = sm[i];
-      }
+    const int r = (2 * blockIdx.x + k) * 16 + c16;
+    if (g == 0 && r < n) {
+      pm[(size_t)r * nchunk + chunk] = m[k];
+      ps[(size_t)r * nchunk + chunk] = s[k];
     }
+  }
 }
 
-// Per row: log-sum-exp over the chunks, the loss (one atomic per block of 16
-// rows into *loss), and dQ cleared.  A wave takes 4 rows in turn.
-__global__ __launch_bounds__(256) void ce_finish(const float* pm, const float* ps, int nchunk, const float* tl,
-                                                 const rtx_mlp_sample* s, int n, int C, float inv_n, float* lse,
-                                                 float* loss, float* dQ) {
+// One wave per row: log-sum-exp over the chunks, the target and its logit (the
+// BF16-rounded product in FP32), the loss, and dQ cleared.  Rows past n, up to
+// a multiple of 32, get an infinite log-sum-exp: their dL is zero.
+__global__ __launch_bounds__(256) void ce_finish(const float* pm, const float* ps, int nchunk,
+                                                 const float* __restrict__ Q, const float* __restrict__ O,
+                                                 const float* __restrict__ cb, const rtx_mlp_sample* samples, int n,
+                                                 int C, float inv_n, float* lse, uint32_t* target, float* loss,
+                                                 float* dQ) {
   __shared__ float part[4];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  float acc = 0.f;
-  for (int k = 0; k < 4; ++k) {
-    const int r = blockIdx.x * 16 + w * 4 + k;
-    if (r >= n) break;  // wave-uniform
+  const int r = blockIdx.x * 4 + w;
+  float nll = 0.f;
+  if (r < n) {
     float m = -INFINITY, sm = 0.f;
     for (int c = lane; c < nchunk; c += 64) lse_merge(m, sm, pm[(size_t)r * nchunk + c], ps[(size_t)r * nchunk + c]);
     for (int o = 32; o > 0; o >>= 1) {
       const float m2 = __shfl_xor(m, o, 64), s2 = __shfl_xor(sm, o, 64);
       lse_merge(m, sm, m2, s2);
     }
-    if (lane < kEmb) dQ[(size_t)r * kEmb + lane] = 0.f;
+    const uint32_t t = samples[r].target;
+    float x = 0.f;
+    if (lane < kEmb) {
+      if (t < (uint32_t)C) x = (float)(__bf16)Q[(size_t)r * kEmb + lane] * (float)(__bf16)O[(size_t)t * kEmb + lane];
+      dQ[(size_t)r * kEmb + lane] = 0.f;
+    }
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
     const float l = m + logf(sm);
+    if (t < (uint32_t)C) nll = (l - (x + cb[t])) * inv_n;
     if (lane == 0) {
       lse[r] = l;
-      if (s[r].target < (uint32_t)C) acc += (l - tl[r]) * inv_n;
+      target[r] = t;
+    }
+  } else if (lane == 0) {
+    lse[r] = INFINITY;
+    target[r] = 0xffffffffu;
+  }
+  if (lane == 0) part[w] = nll;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(loss, (part[0] + part[1]) + (part[2] + part[3]));
+}
+
+// dL of one logit: (softmax - onehot) / n.
+__device__ __forceinline__ float ce_dl(float logit, float bias, float lse, bool hot, float inv_n) {
+  return (exp_term(logit + bias - lse) - (hot ? 1.f : 0.f)) * inv_n;
+}
+
+// Two kinds of workgroup in one launch, so that both fill the chip together.
+// The first ceil(C / 32) sum 32 classes' dO and bias gradient: their four waves
+// take every fourth 32-row step and add up in LDS, so each class is written once.
+// The others sum 32 rows' dQ over four ranges of kCeRange classes, one per wave,
+// added up in LDS and then atomically (dQ cleared by ce_finish).
+struct CeGrad {
+  const uint4 *qa, *qt, *oa, *ot;
+  const float *cbp, *lse;
+  const uint32_t* target;
+  int n, row_steps, C, c_steps, q_blocks;  // q_blocks: workgroups per 32 rows
+  float inv_n;
+  float *gO, *gc, *dQ;
+};
+
+__global__ __launch_bounds__(256) void ce_grad(CeGrad p) {
+  __shared__ float red[3][64 * 17];
+  __shared__ float redc[3][32];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c16 = lane & 15;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 d[2][2] = {{zero, zero}, {zero, zero}};  // [tile of 16 classes / rows][half of the embedding]
+  const bool by_class = blockIdx.x < (uint32_t)p.c_steps;
+  const int at = by_class ? blockIdx.x : (blockIdx.x - p.c_steps) / p.q_blocks;  // 32 classes / 32 rows
+  float dc[2] = {0.f, 0.f};
+  if (by_class) {
+    const bf16x8 b[2] = {frag(p.oa, 2 * at, lane), frag(p.oa, 2 * at + 1, lane)};
+    const float bias[2] = {p.cbp[at * 32 + c16], p.cbp[at * 32 + 16 + c16]};
+    const uint32_t cls[2] = {(uint32_t)(at * 32 + c16), (uint32_t)(at * 32 + 16 + c16)};
+    for (int st = wave; st < p.row_steps; st += 4) {
+      const bf16x8 a[2] = {frag(p.qa, 2 * st, lane), frag(p.qa, 2 * st + 1, lane)};
+      const bf16x8 t0 = frag(p.qt, 2 * st, lane), t1 = frag(p.qt, 2 * st + 1, lane);
+      float4 l[2];
+      uint4 t[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        l[h] = *reinterpret_cast<const float4*>(p.lse + st * 32 + h * 16 + 4 * g);
+        t[h] = *reinterpret_cast<const uint4*>(p.target + st * 32 + h * 16 + 4 * g);
+      }
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        bf16x8 v;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h], b[k], zero, 0, 0, 0);
+          const float x[4] = {ce_dl(acc[0], bias[k], l[h].x, t[h].x == cls[k], p.inv_n),
+                              ce_dl(acc[1], bias[k], l[h].y, t[h].y == cls[k], p.inv_n),
+                              ce_dl(acc[2], bias[k], l[h].z, t[h].z == cls[k], p.inv_n),
+                              ce_dl(acc[3], bias[k], l[h].w, t[h].w == cls[k], p.inv_n)};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            dc[k] += x[i];
+            v[4 * h + i] = (__bf16)x[i];
+          }
+        }
+        // dO tile [16 classes x 16 emb] += dL^T (classes x 32 rows) . Q (32 rows x 16 emb)
+        d[k][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, t0, d[k][0], 0, 0, 0);
+        d[k][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, t1, d[k][1], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      dc[k] += __shfl_xor(dc[k], 16, 64);
+      dc[k] += __shfl_xor(dc[k], 32, 64);
+    }
+    if (wave > 0 && g < 2) redc[wave - 1][g * 16 + c16] = g ? dc[1] : dc[0];
+  } else {
+    const bf16x8 b[2] = {frag(p.qa, 2 * at, lane), frag(p.qa, 2 * at + 1, lane)};  // columns of the transposed logits
+    const float l[2] = {p.lse[at * 32 + c16], p.lse[at * 32 + 16 + c16]};
+    const uint32_t t[2] = {p.target[at * 32 + c16], p.target[at * 32 + 16 + c16]};
+    const int s0 = (((blockIdx.x - p.c_steps) % p.q_blocks) * 4 + wave) * (kCeRange / 32);
+    const int s1 = min(p.c_steps, s0 + kCeRange / 32);
+    for (int st = s0; st < s1; ++st) {
+      const bf16x8 a[2] = {frag(p.oa, 2 * st, lane), frag(p.oa, 2 * st + 1, lane)};
+      const bf16x8 t0 = frag(p.ot, 2 * st, lane), t1 = frag(p.ot, 2 * st + 1, lane);
+      float4 bias[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) bias[h] = *reinterpret_cast<const float4*>(p.cbp + st * 32 + h * 16 + 4 * g);
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        bf16x8 v;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h], b[k], zero, 0, 0, 0);
+          const uint32_t c0 = (uint32_t)(st * 32 + h * 16 + 4 * g);
+          v[4 * h] = (__bf16)ce_dl(acc[0], bias[h].x, l[k], t[k] == c0, p.inv_n);
+          v[4 * h + 1] = (__bf16)ce_dl(acc[1], bias[h].y, l[k], t[k] == c0 + 1, p.inv_n);
+          v[4 * h + 2] = (__bf16)ce_dl(acc[2], bias[h].z, l[k], t[k] == c0 + 2, p.inv_n);
+          v[4 * h + 3] = (__bf16)ce_dl(acc[3], bias[h].w, l[k], t[k] == c0 + 3, p.inv_n);
+        }
+        // dQ^T tile [16 emb x 16 rows] += O^T (emb x 32 classes) . dL^T (32 classes x rows)
+        d[k][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t0, v, d[k][0], 0, 0, 0);
+        d[k][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t1, v, d[k][1], 0, 0, 0);
+      }
     }
   }
-  if (lane == 0) part[w] = acc;
+  if (wave > 0)
+    for (int q = 0; q < 16; ++q) red[wave - 1][lane * 17 + q] = d[q >> 3][(q >> 2) & 1][q & 3];
   __syncthreads();
-  if (threadIdx.x == 0) atomicAdd(loss, part[0] + part[1] + part[2] + part[3]);
+  if (wave > 0) return;
+  for (int q = 0; q < 16; ++q) {
+    const int k = q >> 3, e = (q >> 2) & 1, i = q & 3;
+    const float v = ((d[k][e][i] + red[0][lane * 17 + q]) + red[1][lane * 17 + q]) + red[2][lane * 17 + q];
+    if (by_class) {
+      // result layout: emb column c16 (+16), classes 4g + i
+      const int c = at * 32 + k * 16 + 4 * g + i;
+      if (c < p.C) p.gO[(size_t)c * kEmb + e * 16 + c16] = v;
+    } else {
+      // result layout: row column c16, emb 4g + i (+16)
+      const int r = at * 32 + k * 16 + c16;
+      if (r < p.n) atomicAdd(&p.dQ[(size_t)r * kEmb + e * 16 + 4 * g + i], v);
+    }
+  }
+  if (by_class && g < 2) {
+    const int c = at * 32 + g * 16 + c16;
+    const float v = ((g ? dc[1] : dc[0]) + redc[0][g * 16 + c16]) + (redc[1][g * 16 + c16] + redc[2][g * 16 + c16]);
+    if (c < p.C) p.gc[c] = v;
+  }
 }
 
 // ---- prediction: top-4 classes and probabilities ------------------------------------
@@ -532,8 +826,9 @@ __device__ __forceinline__ void top4_merge(Top4& t, const Top4& o) {
 // columns the wave's samples, so a lane keeps one sample's best four over a
 // quarter of the classes, in registers, and the logits are never stored: 20,011
 // samples x 16,384 classes wrote and read 1.3 GB of them twice (3.4 ms in five
-// products and five scans) and take 0.3 ms here.  Bound by the exponential and
-// the compare of each logit (VALU).
+// products and five scans) and take 0.26 ms here.  Bound by the VALU work on each
+// logit: the insertions of a list's first few hundred classes, then its compare
+// and exponential.
 __global__ __launch_bounds__(256) void logits_top4(const float* __restrict__ Q, int n, const float* __restrict__ O,
                                                    const float* __restrict__ cb, int C, int cper, Top4* part) {
   __shared__ uint4 Os[kCeCls * 4];
@@ -571,7 +866,7 @@ __global__ __launch_bounds__(256) void logits_top4(const float* __restrict__ Q, 
           t.m = mx;
         }
       }
-      if (t.m > -INFINITY) t.s += (expf(x[0] - t.m) + expf(x[1] - t.m)) + (expf(x[2] - t.m) + expf(x[3] - t.m));
+      if (t.m > -INFINITY) t.s += (exp_term(x[0] - t.m) + exp_term(x[1] - t.m)) + (exp_term(x[2] - t.m) + exp_term(x[3] - t.m));
     }
   }
   // the four lane groups hold quarters of the same rows' classes
@@ -597,132 +892,6 @@ __global__ __launch_bounds__(64) void top4_finish(const Top4* part, int n, int s
   for (int k = 0; k < 4; ++k) out[(size_t)r * 4 + k] = t.c[k] < 0 ? RTX_NO_TREELET : (uint32_t)t.c[k];
   if (prob)
     for (int k = 0; k < 4; ++k) prob[(size_t)r * 4 + k] = t.c[k] < 0 ? 0.f : expf(t.v[k] - t.m) / t.s;
-}
-
-// dL of one logit: (softmax - onehot) / n.
-__device__ __forceinline__ float ce_dl(float logit, float bias, float lse, uint32_t target, int cls, float inv_n) {
-  return (expf(logit + bias - lse) - (target == (uint32_t)cls ? 1.f : 0.f)) * inv_n;
-}
-
-// One block: 64 classes (a wave per 16) against the rows [y * rper, y * rper + rper),
-// staged in LDS kCeRows at a time.  gO[c] += sum_r dL[r, c] Q[r], gc[c] += sum_r dL[r, c]
-// (atomically: the row splits of a class add up).
-__global__ __launch_bounds__(256) void ce_grad_o(const float* __restrict__ Q, int n, const float* __restrict__ O,
-                                                 const float* __restrict__ cb, int C,
-                                                 const rtx_mlp_sample* __restrict__ s, const float* __restrict__ lse,
-                                                 float inv_n, int rper, float* gO, float* gc) {
-  __shared__ uint4 Qs[kCeRows * 4];
-  __shared__ float ls[kCeRows];
-  __shared__ uint32_t ts[kCeRows];
-  const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
-  const int c0 = blockIdx.x * 64 + (threadIdx.x >> 6) * 16;
-  const int cls = c0 + c16;
-  const bool valid = cls < C;
-  const bf16x8 b = ld_row8(O, C, cls, 8 * g);
-  const float bias = valid ? cb[cls] : 0.f;
-  f32x4 d0 = {0.f, 0.f, 0.f, 0.f}, d1 = {0.f, 0.f, 0.f, 0.f};
-  float dc = 0.f;
-  const int rbeg = blockIdx.y * rper, rend = min(n, rbeg + rper);
-  for (int rc = rbeg; rc < rend; rc += kCeRows) {
-    const int nr = min(kCeRows, rend - rc);
-    __syncthreads();  // the previous stage is read
-    stage_rows(Qs, Q, rc, nr);
-    for (int i = threadIdx.x; i < nr; i += blockDim.x) {
-      ls[i] = lse[rc + i];
-      ts[i] = s[rc + i].target;
-    }
-    __syncthreads();
-    for (int r0 = 0; r0 < nr; r0 += 32) {
-      bf16x8 a2;
-      for (int tt = 0; tt < 2; ++tt) {
-        const int rt = r0 + 16 * tt;
-        const bf16x8 a = lds_row8(Qs, rt + c16, g, rt + c16 < nr);
-        const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-        for (int i = 0; i < 4; ++i) {
-          const int r = rt + 4 * g + i;
-          const float v = (valid && r < nr) ? ce_dl(acc[i], bias, ls[r], ts[r], cls, inv_n) : 0.f;
-          dc += v;
-          a2[4 * tt + i] = (__bf16)v;
-        }
-      }
-      // dO tile [16 classes x 16 emb] += dL^T (classes x 32 rows) . Q (32 rows x 16 emb)
-      bf16x8 q0, q1;
-      for (int j = 0; j < 8; ++j) {
-        const int r = r0 + kslot_row(g, j);
-        const bool in = r < nr;
-        q0[j] = in ? lds_elem(Qs, r, c16) : (__bf16)0.f;
-        q1[j] = in ? lds_elem(Qs, r, 16 + c16) : (__bf16)0.f;
-      }
-      d0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, q0, d0, 0, 0, 0);
-      d1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, q1, d1, 0, 0, 0);
-    }
-  }
-  dc += __shfl_xor(dc, 16, 64);
-  dc += __shfl_xor(dc, 32, 64);
-  if (g == 0 && valid) atomicAdd(&gc[cls], dc);
-  // result layout: emb column c16 (+16), classes c0 + 4g + i
-  for (int i = 0; i < 4; ++i) {
-    const int c2 = c0 + 4 * g + i;
-    if (c2 < C) {
-      atomicAdd(&gO[(size_t)c2 * kEmb + c16], d0[i]);
-      atomicAdd(&gO[(size_t)c2 * kEmb + 16 + c16], d1[i]);
-    }
-  }
-}
-
-// One block: 64 rows (a wave per 16) against the classes [y * cper, y * cper + cper),
-// staged in LDS kCeCls at a time.  dQ[r] += sum_c dL[r, c] O[c] (dQ cleared by ce_finish).
-__global__ __launch_bounds__(256) void ce_grad_q(const float* __restrict__ Q, int n, const float* __restrict__ O,
-                                                 const float* __restrict__ cb, int C,
-                                                 const rtx_mlp_sample* __restrict__ s, const float* __restrict__ lse,
-                                                 float inv_n, int cper, float* dQ) {
-  __shared__ uint4 Os[kCeCls * 4];
-  __shared__ float cbs[kCeCls];
-  const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
-  const int row = blockIdx.x * 64 + (threadIdx.x >> 6) * 16 + c16;
-  const bool vr = row < n;
-  const bf16x8 b = ld_row8(Q, n, row, 8 * g);  // the row's query: column c16 of the transposed logits
-  const float l = vr ? lse[row] : 0.f;
-  const uint32_t t = vr ? s[row].target : 0xffffffffu;
-  const int cbeg = blockIdx.y * cper, cend = min(C, cbeg + cper);
-  f32x4 q0 = {0.f, 0.f, 0.f, 0.f}, q1 = {0.f, 0.f, 0.f, 0.f};
-  for (int cc = cbeg; cc < cend; cc += kCeCls) {
-    const int nc = min(kCeCls, cend - cc);
-    __syncthreads();  // the previous stage is read
-    stage_rows(Os, O, cc, nc);
-    for (int i = threadIdx.x; i < nc; i += blockDim.x) cbs[i] = cb[cc + i];
-    __syncthreads();
-    for (int cb0 = 0; cb0 < nc; cb0 += 32) {
-      bf16x8 b2;
-      for (int tt = 0; tt < 2; ++tt) {
-        const int ct = cb0 + 16 * tt;
-        // logits^T tile: classes ct + 4g + i (rows of the result) against this lane's row
-        const bf16x8 a = lds_row8(Os, ct + c16, g, ct + c16 < nc);
-        const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-        for (int i = 0; i < 4; ++i) {
-          const int cl = ct + 4 * g + i;
-          const float v = (vr && cl < nc) ? ce_dl(acc[i], cbs[cl], l, t, cc + cl, inv_n) : 0.f;
-          b2[4 * tt + i] = (__bf16)v;
-        }
-      }
-      // dQ^T tile [16 emb x 16 rows] += O^T (emb x 32 classes) . dL^T (32 classes x rows)
-      bf16x8 o0, o1;
-      for (int j = 0; j < 8; ++j) {
-        const int cl = cb0 + kslot_row(g, j);
-        const bool in = cl < nc;
-        o0[j] = in ? lds_elem(Os, cl, c16) : (__bf16)0.f;
-        o1[j] = in ? lds_elem(Os, cl, 16 + c16) : (__bf16)0.f;
-      }
-      q0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o0, b2, q0, 0, 0, 0);
-      q1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o1, b2, q1, 0, 0, 0);
-    }
-  }
-  // result layout: row column c16, emb 4g + i (+16)
-  if (vr)
-    for (int i = 0; i < 4; ++i) {
-      atomicAdd(&dQ[(size_t)row * kEmb + 4 * g + i], q0[i]);
-      atomicAdd(&dQ[(size_t)row * kEmb + 16 + 4 * g + i], q1[i]);
-    }
 }
 
 template <bool TA, bool TB, int BN>
@@ -771,11 +940,16 @@ struct rtx_mlp {
   // activations of one batch
   uint32_t cap = 0;
   float *X = nullptr, *H1 = nullptr, *H2 = nullptr, *Q = nullptr;
-  float *dQ = nullptr, *dH2 = nullptr, *dH1 = nullptr, *dX = nullptr, *loss = nullptr;
-  // fused output layer: per-row chunk maxima and exp-sums, target logits, log-sum-exp
-  float *pm = nullptr, *ps = nullptr, *tl = nullptr, *lse = nullptr;
-  // the trunk's weights as MFMA operands (packed before each forward pass)
-  uint4* frags = nullptr;
+  float *dQ = nullptr, *dH2 = nullptr, *dH1 = nullptr, *loss = nullptr;
+  // fused output layer: per-row chunk maxima and exp-sums, log-sum-exp and
+  // target (rows padded to a multiple of 32), queries as MFMA operands
+  float *pm = nullptr, *ps = nullptr, *lse = nullptr, *target = nullptr, *qa = nullptr, *qt = nullptr;
+  // parameters as MFMA operands, packed before each pass: the trunk's weights,
+  // the class vectors in both orientations and the padded class biases
+  uint4 *frags = nullptr, *oa = nullptr, *ot = nullptr;
+  float* cbp = nullptr;
+  // embedding rows that ever had a gradient (one byte each)
+  uint8_t* touched = nullptr;
   // prediction: queries and per-split results of one chunk of rows
   float* pred_q = nullptr;
   Top4* pred_part = nullptr;
@@ -784,10 +958,11 @@ struct rtx_mlp {
 namespace {
 
 int ce_chunks(const rtx_mlp* m) { return (int)((m->C + kCeChunk - 1) / kCeChunk); }
+int ce_steps(const rtx_mlp* m) { return (int)((m->C + 31) / 32); }  // 32 classes each
 
 void mlp_free_acts(rtx_mlp* m) {
-  float** bufs[] = {&m->X, &m->H1, &m->H2, &m->Q, &m->dQ, &m->dH2, &m->dH1, &m->dX,
-                    &m->pm, &m->ps, &m->tl, &m->lse};
+  float** bufs[] = {&m->X,  &m->H1, &m->H2,  &m->Q,      &m->dQ, &m->dH2, &m->dH1,
+                    &m->pm, &m->ps, &m->lse, &m->target, &m->qa, &m->qt};
   for (float** b : bufs) {
     if (*b) (void)hipFree(*b);
     *b = nullptr;
@@ -795,22 +970,21 @@ void mlp_free_acts(rtx_mlp* m) {
   m->cap = 0;
 }
 
-rtx_status mlp_ensure(rtx_mlp* m, uint32_t b) {
-  if (b <= m->cap) return RTX_OK;
+rtx_status mlp_ensure(rtx_mlp* m, uint32_t rows) {
+  if (rows <= m->cap) return RTX_OK;
   mlp_free_acts(m);
-  const size_t nch = (size_t)ce_chunks(m);
-  const size_t sizes[] = {(size_t)b * kInPad, (size_t)b * kHid,   (size_t)b * kHid, (size_t)b * kEmb,
-                          (size_t)b * kEmb,   (size_t)b * kHid,   (size_t)b * kHid, (size_t)b * kInPad,
-                          (size_t)b * nch,    (size_t)b * nch,    (size_t)b,        (size_t)b};
-  float** bufs[] = {&m->X, &m->H1, &m->H2, &m->Q, &m->dQ, &m->dH2, &m->dH1, &m->dX,
-                    &m->pm, &m->ps, &m->tl, &m->lse};
-  for (int k = 0; k < 12; ++k)
+  const size_t nch = (size_t)ce_chunks(m), b = ((size_t)rows + 31) / 32 * 32;
+  const size_t sizes[] = {b * kInPad, b * kHid, b * kHid, b * kEmb, b * kEmb, b * kHid, b * kHid,
+                          b * nch,    b * nch,  b,        b,        b * 16,   b * 16};
+  float** bufs[] = {&m->X,  &m->H1, &m->H2,  &m->Q,      &m->dQ, &m->dH2, &m->dH1,
+                    &m->pm, &m->ps, &m->lse, &m->target, &m->qa, &m->qt};
+  for (int k = 0; k < 13; ++k)
     if (hipMalloc(bufs[k], sizes[k] * sizeof(float)) != hipSuccess) {
       (void)hipGetLastError();
       mlp_free_acts(m);
       return RTX_ERR_OUT_OF_MEMORY;
     }
-  m->cap = b;
+  m->cap = rows;
   return RTX_OK;
 }
 
@@ -826,8 +1000,11 @@ Weights weights_of(const rtx_mlp* m) {
   return Weights{m->P + m->oW1, m->P + m->ob1, m->P + m->oW2, m->P + m->ob2, m->P + m->oW3, m->P + m->ob3};
 }
 
-hipError_t pack(rtx_mlp* m) {
-  hipLaunchKernelGGL(pack_weights, dim3((kFragEnd + 3) / 4), dim3(256), 0, m->stream, weights_of(m), m->frags);
+// Pack the operands of a forward pass, or of a training step.
+hipError_t pack(rtx_mlp* m, bool train) {
+  const int count = train ? kFragEnd : kFragForward, c_tiles = train ? 2 * ce_steps(m) : 0;
+  hipLaunchKernelGGL(pack_operands, dim3((count + 2 * c_tiles + 3) / 4), dim3(256), 0, m->stream, weights_of(m), count,
+                     m->frags, m->P + m->oO, m->P + m->oc, (int)m->C, c_tiles, m->oa, m->ot, m->cbp);
   return hipGetLastError();
 }
 
@@ -838,66 +1015,45 @@ constexpr uint32_t kPredRows = 65536, kPredParts = 4 * kPredRows, kPredBlocks = 
 // Batches of at most this many rows accumulate in 64-deep partial products.
 constexpr uint32_t kChunkedRows = 1984;
 
-// Forward over one training batch, up to the queries (the fused output layer
-// computes the logits itself).
-rtx_status mlp_forward(rtx_mlp* m, const rtx_mlp_sample* s, uint32_t n) {
-  MK(pack(m));
-  hipLaunchKernelGGL(trunk_forward<true>, dim3((n + kRowTile - 1) / kRowTile), dim3(256), 0, m->stream, s, (int)n,
-                     m->P + m->oE, (int)m->T, weights_of(m), m->frags, n <= kChunkedRows ? 0 : INT_MAX, m->X, m->H1,
-                     m->H2, m->Q);
-  MK(hipGetLastError());
-  return RTX_OK;
-}
-
-// Forward + backward of one batch; gradients are added into m->G.
+// Forward + backward of one batch; gradients are added into m->G, whose output
+// layer is overwritten.
 rtx_status mlp_fwd_bwd(rtx_mlp* m, const rtx_mlp_sample* s, uint32_t n, float inv_n) {
-  rtx_status stt = mlp_forward(m, s, n);
-  if (stt != RTX_OK) return stt;
   hipStream_t st = m->stream;
   float *P = m->P, *G = m->G;
-  // output layer, fused: softmax cross-entropy, dO += dL^T . Q, dc += colsum(dL),
-  // dQ = dL . O, the logits never in memory
-  const int C = (int)m->C, nch = ce_chunks(m);
-  const int row_blocks = (int)((n + 63) / 64);
-  hipLaunchKernelGGL(ce_stats, dim3(row_blocks, nch), dim3(256), 0, st, m->Q, (int)n, P + m->oO, P + m->oc, C, s, nch,
-                     m->pm, m->ps, m->tl);
-  hipLaunchKernelGGL(ce_finish, dim3((n + 15) / 16), dim3(256), 0, st, m->pm, m->ps, nch, m->tl, s, (int)n, C, inv_n,
-                     m->lse, m->loss, m->dQ);
-  const int rsplits = std::max(1, std::min(kCeRowSplit, (int)((n + 31) / 32)));
-  const int rper = (int)((n + rsplits - 1) / rsplits + 31) / 32 * 32;
-  hipLaunchKernelGGL(ce_grad_o, dim3((C + 63) / 64, rsplits), dim3(256), 0, st, m->Q, (int)n, P + m->oO, P + m->oc, C,
-                     s, m->lse, inv_n, rper, G + m->oO, G + m->oc);
-  const int splits = std::max(1, std::min(kCeSplit, (C + 31) / 32));
-  const int cper = ((C + splits - 1) / splits + 31) / 32 * 32;
-  hipLaunchKernelGGL(ce_grad_q, dim3(row_blocks, splits), dim3(256), 0, st, m->Q, (int)n, P + m->oO, P + m->oc, C, s,
-                     m->lse, inv_n, cper, m->dQ);
-  MK(hipGetLastError());
-  // q = h2 W3 + b3
-  MK(gemm<true, false>(st, kHid, kEmb, n, m->H2, kHid, m->dQ, kEmb, G + m->oW3, kEmb, 1));
-  hipLaunchKernelGGL(colsum, dim3(1, (n + kColsumRows - 1) / kColsumRows), dim3(64), 0, st, m->dQ, (int)n, kEmb, G + m->ob3);
-  MK(gemm<false, true>(st, n, kHid, kEmb, m->dQ, kEmb, P + m->oW3, kEmb, m->dH2, kHid, 0));
-  hipLaunchKernelGGL(relu_mask, dim3(256), dim3(256), 0, st, m->dH2, m->H2, (size_t)n * kHid);
-  // h2 = relu(h1 W2 + b2)
-  MK(gemm<true, false>(st, kHid, kHid, n, m->H1, kHid, m->dH2, kHid, G + m->oW2, kHid, 1));
-  hipLaunchKernelGGL(colsum, dim3(1, (n + kColsumRows - 1) / kColsumRows), dim3(128), 0, st, m->dH2, (int)n, kHid, G + m->ob2);
-  MK(gemm<false, true>(st, n, kHid, kHid, m->dH2, kHid, P + m->oW2, kHid, m->dH1, kHid, 0));
-  hipLaunchKernelGGL(relu_mask, dim3(256), dim3(256), 0, st, m->dH1, m->H1, (size_t)n * kHid);
-  // h1 = relu(x W1 + b1)
-  MK(gemm<true, false>(st, kInPad, kHid, n, m->X, kInPad, m->dH1, kHid, G + m->oW1, kHid, 1));
-  hipLaunchKernelGGL(colsum, dim3(1, (n + kColsumRows - 1) / kColsumRows), dim3(128), 0, st, m->dH1, (int)n, kHid, G + m->ob1);
-  MK(gemm<false, true>(st, n, kInPad, kHid, m->dH1, kHid, P + m->oW1, kHid, m->dX, kInPad, 0));
-  hipLaunchKernelGGL(scatter_embed, dim3((n + 63) / 64, 5 * kEmb), dim3(64), 0, st, m->dX, s, (int)n, (int)m->T,
-                     G + m->oE);
+  uint4 *qa = reinterpret_cast<uint4*>(m->qa), *qt = reinterpret_cast<uint4*>(m->qt);
+  uint32_t* target = reinterpret_cast<uint32_t*>(m->target);
+  const int C = (int)m->C, nch = ce_chunks(m), c_steps = ce_steps(m), row_steps = (int)((n + 31) / 32);
+  MK(pack(m, true));
+  // whole 32-row steps: the tiles past n are zero queries
+  hipLaunchKernelGGL(trunk_forward<true>, dim3(2 * row_steps), dim3(256), 0, st, s, (int)n, P + m->oE, (int)m->T,
+                     weights_of(m), m->frags, n <= kChunkedRows ? 0 : INT_MAX, m->X, m->H1, m->H2, m->Q, qa, qt);
+  hipLaunchKernelGGL(ce_stats, dim3(row_steps, (nch + 3) / 4), dim3(256), 0, st, qa, (int)n, m->oa, m->cbp, 2 * c_steps,
+                     nch, m->pm, m->ps);
+  hipLaunchKernelGGL(ce_finish, dim3(row_steps * 8), dim3(256), 0, st, m->pm, m->ps, nch, m->Q, P + m->oO, P + m->oc, s,
+                     (int)n, C, inv_n, m->lse, target, m->loss, m->dQ);
+  const int q_blocks = (c_steps + 4 * (kCeRange / 32) - 1) / (4 * (kCeRange / 32));
+  const CeGrad ce{qa,   qt,        m->oa, m->ot,   m->cbp,   m->lse, target,    (int)n,
+                  row_steps, C,    c_steps, q_blocks, inv_n, G + m->oO, G + m->oc, m->dQ};
+  hipLaunchKernelGGL(ce_grad, dim3(c_steps + row_steps * q_blocks), dim3(256), 0, st, ce);
+  hipLaunchKernelGGL(trunk_backward, dim3((n + kRowTile - 1) / kRowTile), dim3(256), 0, st, s, (int)n, (int)m->T,
+                     m->frags, m->dQ, m->H1, m->H2, m->dH1, m->dH2,
+                     Gradients{G + m->oE, G + m->ob1, G + m->ob2, G + m->ob3}, m->touched);
+  // row ranges of at least 128 rows, at most 16
+  const int ranges = std::max(1, std::min(16, (int)(n / 128)));
+  const int rows_per = ((int)n + ranges - 1) / ranges;
+  hipLaunchKernelGGL(weight_grads, dim3(44, ranges), dim3(256), 0, st,
+                     WeightGrad{m->X, m->dH1, G + m->oW1, kInPad, kHid}, WeightGrad{m->H1, m->dH2, G + m->oW2, kHid, kHid},
+                     WeightGrad{m->H2, m->dQ, G + m->oW3, kHid, kEmb}, (int)n, rows_per);
   MK(hipGetLastError());
   return RTX_OK;
 }
 
-rtx_status mlp_adam(rtx_mlp* m, float lr) {
+rtx_status mlp_adam(rtx_mlp* m, float lr, bool clear) {
   m->steps++;
   const float b1 = 0.9f, b2 = 0.999f;
   const float c1 = 1.f - powf(b1, (float)m->steps), c2 = 1.f - powf(b2, (float)m->steps);
-  hipLaunchKernelGGL(adam_step, dim3(1024), dim3(256), 0, m->stream, m->P, m->G, m->M1, m->V1, m->count, lr, b1, b2,
-                     1e-8f, c1, c2);
+  hipLaunchKernelGGL(adam_step, dim3(2048), dim3(256), 0, m->stream, m->P, m->G, m->M1, m->V1, m->touched,
+                     (size_t)m->T + 1, m->count, clear ? 1 : 0, lr, b1, b2, 1e-8f, c1, c2);
   MK(hipGetLastError());
   return RTX_OK;
 }
@@ -944,7 +1100,11 @@ rtx_status rtx_mlp_create(rtx_ctx* c, uint32_t n_treelets, uint32_t n_classes, u
   (void)hipSetDevice(m->device);
   if (hipMalloc(&m->P, o * 4) != hipSuccess || hipMalloc(&m->G, o * 4) != hipSuccess ||
       hipMalloc(&m->M1, o * 4) != hipSuccess || hipMalloc(&m->V1, o * 4) != hipSuccess ||
-      hipMalloc(&m->loss, 4) != hipSuccess || hipMalloc(&m->frags, kFragEnd * 1024) != hipSuccess) {
+      hipMalloc(&m->loss, 4) != hipSuccess || hipMalloc(&m->frags, kFragEnd * 1024) != hipSuccess ||
+      hipMalloc(&m->oa, (size_t)ce_steps(m) * 2048) != hipSuccess ||
+      hipMalloc(&m->ot, (size_t)ce_steps(m) * 2048) != hipSuccess ||
+      hipMalloc(&m->cbp, (size_t)ce_steps(m) * 128) != hipSuccess ||
+      hipMalloc(&m->touched, (size_t)n_treelets + 1) != hipSuccess) {
     (void)hipGetLastError();
     rtx_mlp_destroy(m);
     return RTX_ERR_OUT_OF_MEMORY;
@@ -961,7 +1121,7 @@ rtx_status rtx_mlp_create(rtx_ctx* c, uint32_t n_treelets, uint32_t n_classes, u
   for (size_t k = m->oO; k < m->oc; ++k) h[k] = uni(sqrtf(3.f / kEmb));
   if (hipMemcpy(m->P, h.data(), o * 4, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemset(m->G, 0, o * 4) != hipSuccess || hipMemset(m->M1, 0, o * 4) != hipSuccess ||
-      hipMemset(m->V1, 0, o * 4) != hipSuccess) {
+      hipMemset(m->V1, 0, o * 4) != hipSuccess || hipMemset(m->touched, 0, (size_t)n_treelets + 1) != hipSuccess) {
     rtx_mlp_destroy(m);
     return RTX_ERR_HIP;
   }
@@ -977,7 +1137,9 @@ rtx_status rtx_mlp_destroy(rtx_mlp* m) {
   float* bufs[] = {m->P, m->G, m->M1, m->V1, m->loss};
   for (float* b : bufs)
     if (b) (void)hipFree(b);
-  if (m->frags) (void)hipFree(m->frags);
+  void* more[] = {m->frags, m->oa, m->ot, m->cbp, m->touched};
+  for (void* b : more)
+    if (b) (void)hipFree(b);
   if (m->pred_q) (void)hipFree(m->pred_q);
   if (m->pred_part) (void)hipFree(m->pred_part);
   delete m;
@@ -1032,12 +1194,13 @@ rtx_status rtx_mlp_train(rtx_mlp* m, const rtx_mlp_sample* samples, uint32_t n, 
   for (uint32_t e = 0; e < epochs; ++e) {
     MK(hipMemsetAsync(m->loss, 0, 4, m->stream));
     uint32_t nb = 0;
+    if (e == 0) MK(hipMemsetAsync(m->G, 0, m->count * 4, m->stream));
     for (uint32_t b0 = 0; b0 < n; b0 += batch) {
       const uint32_t b = std::min(batch, n - b0);
-      MK(hipMemsetAsync(m->G, 0, m->count * 4, m->stream));
       st = mlp_fwd_bwd(m, samples + b0, b, 1.f / (float)b);
       if (st != RTX_OK) return st;
-      st = mlp_adam(m, lr);
+      // the last batch's gradients stay readable
+      st = mlp_adam(m, lr, !(e + 1 == epochs && b0 + b == n));
       if (st != RTX_OK) return st;
       ++nb;
     }
@@ -1063,7 +1226,7 @@ rtx_status rtx_mlp_predict(rtx_mlp* m, const rtx_mlp_sample* samples, uint32_t n
   // the last rows past a multiple of 4,096 are a batch of their own
   const uint32_t last = n % 4096;
   const uint32_t chunk_from = last && last <= kChunkedRows ? n - last : n;
-  MK(pack(m));
+  MK(pack(m, false));
   for (uint32_t b0 = 0; b0 < n; b0 += kPredRows) {
     const uint32_t b = std::min(kPredRows, n - b0);
     // class splits: enough workgroups for the chip, of whole LDS stages
@@ -1076,7 +1239,7 @@ rtx_status rtx_mlp_predict(rtx_mlp* m, const rtx_mlp_sample* samples, uint32_t n
     hipLaunchKernelGGL(trunk_forward<false>, dim3((b + kRowTile - 1) / kRowTile), dim3(256), 0, m->stream,
                        samples + b0, (int)b, m->P + m->oE, (int)m->T, weights_of(m), m->frags,
                        chunk_from <= b0 ? 0 : (int)std::min(chunk_from - b0, b), (float*)nullptr, (float*)nullptr,
-                       (float*)nullptr, m->pred_q);
+                       (float*)nullptr, m->pred_q, (uint4*)nullptr, (uint4*)nullptr);
     hipLaunchKernelGGL(logits_top4, dim3(row_blocks, splits), dim3(256), 0, m->stream, m->pred_q, (int)b,
                        m->P + m->oO, m->P + m->oc, (int)m->C, cper, m->pred_part);
     hipLaunchKernelGGL(top4_finish, dim3((b + 63) / 64), dim3(64), 0, m->stream, m->pred_part, (int)b, (int)splits,
