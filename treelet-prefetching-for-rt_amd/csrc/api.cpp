@@ -29,6 +29,9 @@ static constexpr uint32_t kReportWord = 8;
 // most device memory the per-ray record slabs (8 bytes per record) may take
 static constexpr uint64_t kSlabBytesMax = 16ull << 30;
 
+// most coherence scratch a context keeps (ten million rays)
+static constexpr size_t kCoherenceKept = 256ull << 20;
+
 struct rtx_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -81,6 +84,9 @@ struct rtx_ctx {
   size_t overflow_entries = 0;
   uint32_t* rec_counts = nullptr;  // per-ray record counts of a slab traversal
   size_t rec_count_entries = 0;
+  // rtx_coherence_order's scratch, kept between calls up to kCoherenceKept bytes
+  uint8_t* coherence = nullptr;
+  size_t coherence_bytes = 0;
   // level pass: per-lane tree_level_maps, zeroed when allocated (the pass
   // leaves them zeroed)
   uint8_t* lm_mem = nullptr;
@@ -357,6 +363,7 @@ rtx_status rtx_destroy(rtx_ctx* c) {
   if (c->slabs) hipFree(c->slabs);
   if (c->overflow_list) hipFree(c->overflow_list);
   if (c->rec_counts) hipFree(c->rec_counts);
+  if (c->coherence) hipFree(c->coherence);
   if (c->lm_mem) hipFree(c->lm_mem);
   for (auto& sc : c->scenes) {
     if (sc.arena) hipFree(sc.arena);
@@ -1076,8 +1083,16 @@ rtx_status rtx_coherence_order(rtx_ctx* c, const rtx_ray* rays, uint32_t n, cons
   rtx_coherence_config k = *cfg;
   k.hash = h;
   if (n == 0) return RTX_OK;
-  const hipError_t e = coherence_order(rays, n, k, wmin, wmax, order, hashes, c->stream);
-  if (e == hipErrorOutOfMemory) return RTX_ERR_OUT_OF_MEMORY;
+  rtx_status st = ensure_buffer(c->coherence, c->coherence_bytes, coherence_scratch_bytes(n));
+  if (st != RTX_OK) return st;
+  hipError_t e = coherence_order(rays, n, k, wmin, wmax, order, hashes, c->coherence, c->stream);
+  const hipError_t done = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = done;
+  if (c->coherence_bytes > kCoherenceKept) {
+    (void)hipFree(c->coherence);
+    c->coherence = nullptr;
+    c->coherence_bytes = 0;
+  }
   return e == hipSuccess ? RTX_OK : RTX_ERR_HIP;
 }
 

@@ -150,9 +150,11 @@ hipError_t launch_scan_records(const rtx_hit* hits, const uint32_t* counts, uint
 // accessed bytes (acc must start at 0; records may be null).
 hipError_t launch_trace_stats(const rtx_hit* hits, uint32_t n, const rtx_record* records, uint64_t n_records,
                               unsigned long long* acc, hipStream_t s);
-// The coherence engine's claim order of n rays (coherence.hip).
+// The coherence engine's claim order of n rays (coherence.hip), queued on s.
+// `scratch` holds coherence_scratch_bytes(n) bytes, 4-byte aligned.
+size_t coherence_scratch_bytes(uint32_t n);
 hipError_t coherence_order(const rtx_ray* rays, uint32_t n, const rtx_coherence_config& cfg, const float wmin[3],
-                           const float wmax[3], uint32_t* order, uint32_t* hashes_out, hipStream_t s);
+                           const float wmax[3], uint32_t* order, uint32_t* hashes_out, void* scratch, hipStream_t s);
 // Slab records: each lane holds its last kRecRing entries in LDS and writes
 // them to the slab in aligned groups of four (32 bytes), so slab rows are
 // padded to a multiple of four entries.
