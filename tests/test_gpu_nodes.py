@@ -1,0 +1,71 @@
+"""Node forms that decide which traversal code a scene takes: children with gaps
+between them (pushed one by one instead of as a group), scales above the range of
+the sign-ordered slab test, NaN origins.  Hits and records are exact by contract,
+so they equal the oracle's bit for bit, with one and with eight lanes per ray."""
+import numpy as np
+import pytest
+
+from conftest import assert_hits_equal, assert_records_equal
+
+pytestmark = pytest.mark.gpu
+
+
+def _internal_nodes(arena, tlas):
+    """Offsets of the internal nodes reachable from the TLAS."""
+    u64 = lambda o: int(arena[o:o + 8].view(np.uint64)[0])  # noqa: E731
+    todo, seen = [(tlas + u64(tlas), True)], []
+    while todo:
+        off, top = todo.pop()
+        seen.append(off)
+        c = off + 64 * int(arena[off + 12:off + 16].view(np.int32)[0])
+        for i in range(6):
+            info = int(arena[off + 22 + i])
+            size, kind = info & 3, (info >> 2) & 15
+            if size and kind == 0:
+                todo.append((c, top))
+            elif size and top:
+                h = c + u64(c + 64)
+                todo.append((h + u64(h), False))
+            c += 64 * size
+    return seen
+
+
+def _gaps(arena, nodes, rng):
+    # the last child moves to the last place: a gap before it, the same memory layout
+    n = 0
+    for off in nodes:
+        used = [i for i in range(6) if arena[off + 22 + i] & 3]
+        if len(used) < 6 and rng.random() < 0.7:
+            for base in (22, 28, 34, 40, 46, 52, 58):
+                arena[off + base + 5] = arena[off + base + used[-1]]
+            arena[off + 22 + used[-1]] = 0
+            n += 1
+    assert n > 10
+
+
+def _scales(arena, nodes, rng):
+    for off in rng.choice(nodes, 20):
+        arena[off + 18 + rng.integers(0, 3)] = rng.integers(105, 127)
+
+
+def _nan_origins(arena, nodes, rng):
+    for off in rng.choice(nodes[1:], 5):
+        arena[off:off + 4].view(np.float32)[0] = np.nan
+
+
+@pytest.mark.parametrize("change", [_gaps, _scales, _nan_origins])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_unusual_nodes_match_the_oracle(gpu, oracle, instanced, mode, change):
+    scene, rays = instanced
+    arena = scene.arena.copy()
+    change(arena, _internal_nodes(arena, scene.tlas_offset), np.random.default_rng(4))
+    part = oracle.Partition(arena, scene.tlas_offset, 1024)
+    h_ref, o_ref, r_ref = oracle.trace(arena, scene.tlas_offset, rays, mode=mode, partition=part)
+    gpu.set_scene(arena, scene.tlas_offset)
+    gpu.build_treelets(1024)
+    for stack in (4, 8, 16):
+        h, o, r = gpu.trace(rays, mode=mode, records=True, lds_stack=stack)
+        assert_hits_equal(h, h_ref, f"stack {stack}")
+        assert_records_equal(o, r, o_ref, r_ref, f"stack {stack}")
+    for lanes in (1, 8):
+        assert_hits_equal(gpu.trace(rays, mode=mode, lanes_per_ray=lanes), h_ref, f"{lanes} lanes")

@@ -47,6 +47,7 @@ struct rtx_ctx {
   uint64_t arena_bytes = 0;
   uint64_t tlas = 0;
   bool ordered = false;  // every child box the TLAS reaches has lo <= hi (scene_check)
+  bool regular = false;  // every node's children are packed and of their kind's size (scene_check)
   // every reachable node has one tree level (scene_check); otherwise hits take
   // their max_level from the level pass
   bool levels_consistent = false;
@@ -100,6 +101,7 @@ struct rtx_ctx {
     uint64_t bytes = 0;
     uint64_t tlas = 0;
     bool ordered = false;            // scene_check() of the arena
+    bool regular = false;            // scene_check() of the arena
     bool levels_consistent = false;  // scene_check() of the arena
     Partition part;
     uint64_t part_gen = 0;  // bumped whenever the scene's partition is rebuilt
@@ -166,6 +168,7 @@ void free_scene(rtx_ctx* c) {
   c->arena = nullptr;
   c->arena_bytes = 0;
   c->ordered = false;
+  c->regular = false;
   c->levels_consistent = false;
 }
 
@@ -506,6 +509,7 @@ rtx_status rtx_set_scene(rtx_ctx* c, const void* host, size_t bytes, uint64_t tl
   c->tlas = tlas;
   const SceneCheck ck = scene_check(d, bytes, tlas, c->stream);
   c->ordered = ck.valid && ck.ordered;
+  c->regular = ck.valid && ck.regular;
   c->levels_consistent = ck.valid && ck.level_consistent;
   return RTX_OK;
 }
@@ -525,6 +529,7 @@ rtx_status rtx_set_scene_device(rtx_ctx* c, const void* dev, size_t bytes, uint6
   c->tlas = tlas;
   const SceneCheck ck = scene_check(c->arena, bytes, tlas, c->stream);
   c->ordered = ck.valid && ck.ordered;
+  c->regular = ck.valid && ck.regular;
   c->levels_consistent = ck.valid && ck.level_consistent;
   return RTX_OK;
 }
@@ -701,6 +706,7 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
   // faster than 32 and 1.2 % faster than 48)
   p.refill = opts->refill ? opts->refill : 40;
   p.ordered_boxes = c->ordered ? 1u : 0u;
+  p.regular_nodes = c->regular ? 1u : 0u;
   p.hits = hits;
   p.records = nullptr;
   p.record_capacity = 0;
@@ -983,6 +989,7 @@ rtx_status rtx_trace_static(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const r
   p.n = n;
   p.refill = opts->refill ? opts->refill : 40;
   p.ordered_boxes = c->ordered ? 1u : 0u;
+  p.regular_nodes = c->regular ? 1u : 0u;
   p.hits = hits;
   p.owner = c->part.valid ? c->part.owner : nullptr;
   p.first_treelet = c->part.valid ? c->part.first_treelet : 0;
@@ -1237,9 +1244,11 @@ TraceParams batch_params(rtx_ctx* c, const BatchJob* jobs_dev, uint32_t n_jobs, 
   p.jobs = jobs_dev;
   p.n_jobs = n_jobs;
   // sign-ordered slab tests only when every scene of the context allows them
-  p.ordered_boxes = 1;
-  for (const auto& sc : c->scenes)
+  p.ordered_boxes = p.regular_nodes = 1;
+  for (const auto& sc : c->scenes) {
     if (!sc.ordered) p.ordered_boxes = 0;
+    if (!sc.regular) p.regular_nodes = 0;
+  }
   return p;
 }
 
@@ -1307,6 +1316,7 @@ rtx_status rtx_add_scene(rtx_ctx* c, const void* host, size_t bytes, uint64_t tl
   sc.tlas = tlas;
   const SceneCheck ck = scene_check(sc.arena, bytes, tlas, c->stream);
   sc.ordered = ck.valid && ck.ordered;
+  sc.regular = ck.valid && ck.regular;
   sc.levels_consistent = ck.valid && ck.level_consistent;
   c->scenes.push_back(sc);
   *id = (uint32_t)(c->scenes.size() - 1);

@@ -95,9 +95,13 @@ struct TraceParams {
   // multi-scene batch (batch kernels only): rays are numbered across jobs
   const BatchJob* jobs;
   uint32_t n_jobs;
-  // every child box of the scene(s) has lower bound bytes <= upper ones, so a
-  // finite ray may pick each axis's near and far bound by its direction sign
+  // every child box of the scene(s) has lower bound bytes <= upper ones, and no
+  // node a NaN origin or a scale above 2^103, so a finite ray may pick each
+  // axis's near and far bound by its direction sign
   uint32_t ordered_boxes;
+  // every node of the scene(s) has its children packed from slot 0 on, an
+  // instance leaf in two slots and any other child in one, all in the arena
+  uint32_t regular_nodes;
 };
 
 // Most treelets resident at once in a wave's staging area.

@@ -49,7 +49,9 @@ rtx_status partition_install(const uint8_t* arena, uint64_t bytes, uint64_t tlas
 // compare-select slab tests, and the level pass.
 struct SceneCheck {
   bool valid = false;
-  bool ordered = false;           // every child box the TLAS reaches has lo <= hi bytes on all axes
+  bool regular = false;           // children packed from slot 0 on, instance leaves two slots, others one
+  bool ordered = false;           // every child box the TLAS reaches has lo <= hi bytes on all axes, and no node
+                                  // a NaN origin or a scale above 2^103
   bool level_consistent = false;  // every reachable node has one tree level (every path agrees)
   bool cyclic = false;            // some node reaches itself
 };

@@ -757,7 +757,9 @@ struct ValParams {
   uint8_t* kind;
   uint32_t* shared;
   uint32_t* error;
-  uint32_t* unordered;  // set when a valid child box has a lower bound byte above its upper one
+  uint32_t* irregular;  // set when a node has a gap before a child, or a child of another size than its kind's
+  uint32_t* unordered;  // set when a valid child box has a lower bound byte above its upper one, or its node a
+                        // NaN origin or a scale above 2^103 (the sign-ordered slab test's conditions)
   // tree levels (tree_level_map values): nodes processed in this round are at
   // level round + 1 (the TLAS root at 1), their children and a BLAS root
   // reached through an instance leaf at round + 2; lvl[slot] keeps the first
@@ -795,10 +797,20 @@ __global__ void validate_level(ValParams p) {
     const int32_t co = *reinterpret_cast<const int32_t*>(nd + 12);
     uint64_t c = off + (uint64_t)((int64_t)co * 64);
     const uint32_t child_level = p.round + 2;
+    const float* org = reinterpret_cast<const float*>(nd);
+    const int8_t* ex = reinterpret_cast<const int8_t*>(nd + 18);
+    if (__builtin_isnan(org[0]) || __builtin_isnan(org[1]) || __builtin_isnan(org[2]) || ex[0] > 111 || ex[1] > 111 ||
+        ex[2] > 111)
+      atomicOr(p.unordered, 1u);
+    bool gap = false;
     for (int k = 0; k < 6; ++k) {
       const uint32_t info = nd[22 + k] & 0x3fu;
       const uint32_t size = info & 3u, type = info >> 2;
-      if (size == 0) continue;
+      if (size == 0) {
+        gap = true;
+        continue;
+      }
+      if (gap || size != (kind == kTopInternal && type != 0 ? 2u : 1u)) atomicOr(p.irregular, 1u);
       // lower x/y/z at bytes 28/40/52 + k, upper at 34/46/58 + k
       if (nd[28 + k] > nd[34 + k] || nd[40 + k] > nd[46 + k] || nd[52 + k] > nd[58 + k]) atomicOr(p.unordered, 1u);
       const uint64_t len = (uint64_t)size * 64;
@@ -970,7 +982,7 @@ rtx_status run_validate(const uint8_t* A, uint64_t bytes, uint64_t tlas, hipStre
   const uint64_t slots = bytes / 64;
   uint32_t *refs, *lvl;
   uint64_t *qa, *qb;
-  uint32_t* ctr;  // [0] n_out, [1] error, [2] shared, [3] unordered, [4] inconsistent, [5] nonzero
+  uint32_t* ctr;  // [0] n_out, [1] error, [2] shared, [3] unordered, [4] inconsistent, [5] nonzero, [6] irregular
   CS(sc.alloc(&refs, slots));
   CS(sc.alloc(&lvl, slots));
   CS(sc.alloc(&qa, slots));
@@ -999,7 +1011,7 @@ rtx_status run_validate(const uint8_t* A, uint64_t bytes, uint64_t tlas, hipStre
   uint32_t round = 0;
   while (n_in > 0) {
     CK(hipMemsetAsync(ctr, 0, 4, s));
-    ValParams vp{A, bytes, qa, n_in, qb, ctr, refs, kind, ctr + 2, ctr + 1, ctr + 3, lvl, round++, ctr + 4};
+    ValParams vp{A, bytes, qa, n_in, qb, ctr, refs, kind, ctr + 2, ctr + 1, ctr + 6, ctr + 3, lvl, round++, ctr + 4};
     uint32_t grid = std::min<uint32_t>(4096, (n_in + 255) / 256);
     hipLaunchKernelGGL(validate_level, dim3(grid), dim3(256), 0, s, vp);
     CK(hipGetLastError());
@@ -1012,13 +1024,14 @@ rtx_status run_validate(const uint8_t* A, uint64_t bytes, uint64_t tlas, hipStre
     std::swap(qa, qb);
   }
   // count every referenced slot (leaves and headers included)
-  uint32_t c[5];
-  CK(hipMemcpyAsync(c, ctr, 20, hipMemcpyDeviceToHost, s));
+  uint32_t c[7];
+  CK(hipMemcpyAsync(c, ctr, 28, hipMemcpyDeviceToHost, s));
   CK(hipStreamSynchronize(s));
   if (shared_out) *shared_out = c[2];
   if (unordered_out) *unordered_out = c[3];
   if (check) {
     check->ordered = c[3] == 0;
+    check->regular = c[6] == 0;
     check->level_consistent = c[4] == 0;
     check->cyclic = false;
     // A cycle reaches a node at two levels, so only inconsistent scenes are peeled.

@@ -11,7 +11,7 @@
 //    hit children in slot order; that is the same sequence as pushing all hit
 //    children in slot order with the first internal child pushed last.  Only
 //    one instance is open at a time, so the instance context lives in
-//    registers.
+//    registers.  A node's hit children are pushed as one group (see Groups).
 //  * TREELET (traceRayWithTreelets, :1522-2307): two LIFO lists.  A child goes
 //    to the "current" list while the current treelet is still the one rooted
 //    at the TLAS header and the child's owner is that treelet; after the
@@ -23,8 +23,8 @@
 //    is recomputed from that leaf when it differs from the cached one (same
 //    inputs, same floats).
 //
-// Stacks: a ring of K entries per lane in LDS, spilling the oldest entries to
-// a per-lane region in global memory (exact LIFO order).
+// Stacks: a ring of K entries (plain order: K groups) per lane in LDS, spilling
+// the oldest to a per-lane region in global memory (exact LIFO order).
 //
 // One wave iteration runs three passes, each only for the lanes that need it:
 // instance leaves, triangle leaves, then internal nodes.  A lane that finishes
@@ -122,6 +122,95 @@ __device__ __forceinline__ uint64_t st_pop(Stack& s, lds_u64* lds, glb_u64* g) {
 
 __device__ __forceinline__ bool st_empty(const Stack& s) { return s.cnt == 0 && s.g == 0; }
 
+// ---- plain order: stack of child groups ---------------------------------------
+// A node's hit children left for later are one group: the slot of its first
+// child and a word with the children still to visit (bits 16-21), which children
+// are leaves (10-15), the tree level (2-9) and whether it is a TLAS node (0).
+// The children are visited highest slot first, which is the order of popping
+// them after pushing each in slot order; the first internal child, which is
+// pushed last, goes on as the lane's next entry.  The newest group stays in
+// registers, older ones are a ring of K per lane in LDS whose oldest groups
+// spill to global memory.  `depth` counts the children outstanding, one entry
+// each, and the ray reports a stack overflow at K + spill_cap of them.
+// A group needs a regular node: children packed from slot 0 on, an instance leaf
+// two slots and any other child one.  The scene walk checks that once for all
+// nodes; other scenes push every child as a group of its own.
+// A push of up to six entries, each placed and stored under its own branch, was
+// a third of the vector instructions of an internal node; a group takes 45
+// instead of 155 and at most one LDS store, and the next internal child reaches
+// the next iteration without LDS.  With the slab test on halves below, 1.34M
+// camera and bounce rays on the 1M-triangle scene take 263 -> 228 M vector
+// instructions and 594 -> 558 us; the registers it frees keep five waves.
+struct Groups {
+  uint32_t base, word;  // the newest group; word < kGroupFirst: none left in it
+  // older groups (bits 0-7; position p of them is in LDS unless p < bits 8-15),
+  // depth (16-23, at most 144) and the ray's opaque and terminate flags (24, 25)
+  uint32_t state;
+};
+constexpr uint32_t kGroupDepth = 1u << 16, kGroupDepthMask = 0xff0000u, kGroupOpaque = 1u << 24, kGroupTerminate = 1u << 25;
+constexpr uint32_t kGroupFirst = 1u << 16, kGroupLeaf = 10;
+__device__ __forceinline__ uint32_t group_word(uint32_t flags, uint32_t level, uint32_t leaves, uint32_t mask) {
+  return (flags & kFlTop) | ((level > 255u ? 255u : level) << 2) | (leaves << kGroupLeaf) | (mask << 16);
+}
+
+// the slot of child i of a group and its entry's upper word (flags and level)
+__device__ __forceinline__ uint64_t group_entry(uint32_t base, uint32_t word, uint32_t i) {
+  const uint32_t leaves = __builtin_amdgcn_ubfe(word, kGroupLeaf, i);  // the leaves below child i
+  const uint32_t two = (uint32_t)__builtin_amdgcn_sbfe((int)word, 0, 1) & leaves;
+  const uint32_t leaf = (word >> (kGroupLeaf + i)) & 1u;
+  return (uint64_t)(base + i + (uint32_t)__popc(two)) | ((uint64_t)((word & 0x3fdu) | (leaf << 1)) << 32);
+}
+
+template <int K, uint32_t BS, typename Spill>
+__device__ __forceinline__ void groups_save(Groups& q, lds_u64* lds, Spill&& spill) {
+  if (q.word < kGroupFirst) return;
+  const uint32_t cnt = q.state & 0xffu, out = (q.state >> 8) & 0xffu;
+  if (cnt - out == (uint32_t)K) {
+    spill()[out] = lds[(out & (K - 1)) * BS];
+    q.state += 0x100u;
+  }
+  lds[(cnt & (K - 1)) * BS] = (uint64_t)q.base | ((uint64_t)q.word << 32);
+  q.state++;
+}
+
+// the next entry; false when nothing is left
+template <int K, uint32_t BS, typename Spill>
+__device__ __forceinline__ bool groups_pop(Groups& q, uint64_t& e, lds_u64* lds, Spill&& spill) {
+  if (q.word < kGroupFirst) {
+    const uint32_t cnt = q.state & 0xffu;
+    if (cnt == 0) return false;
+    q.state--;
+    uint64_t v;
+    if (cnt <= ((q.state >> 8) & 0xffu)) {
+      v = spill()[cnt - 1];
+      q.state -= 0x100u;
+    } else {
+      v = lds[((cnt - 1) & (K - 1)) * BS];
+    }
+    q.base = (uint32_t)v;
+    q.word = (uint32_t)(v >> 32);
+  }
+  const uint32_t i = 15u - (uint32_t)__builtin_clz(q.word);
+  e = group_entry(q.base, q.word, i);
+  q.word ^= kGroupFirst << i;
+  q.state -= kGroupDepth;
+  return true;
+}
+
+// Masks of a node's six children from its size/type bytes (22-27), one bit a
+// child: the bytes' flags times 1, 2, 4, ... summed by a four-byte dot product.
+struct KidBytes {
+  uint32_t lo, hi;  // children 0-3, 4-5
+};
+__device__ __forceinline__ uint32_t kid_mask(uint32_t lo, uint32_t hi) {
+  return __builtin_amdgcn_udot4(lo & 0x01010101u, 0x08040201u, __builtin_amdgcn_udot4(hi & 0x0101u, 0x2010u, 0u, false),
+                                false);
+}
+__device__ __forceinline__ uint32_t kids_present(KidBytes k) { return kid_mask(k.lo | (k.lo >> 1), k.hi | (k.hi >> 1)); }
+__device__ __forceinline__ uint32_t kids_leaves(KidBytes k) {
+  return kid_mask(((k.lo & 0x3c3c3c3cu) + 0x7c7c7c7cu) >> 7, ((k.hi & 0x3c3cu) + 0x7c7cu) >> 7);
+}
+
 __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
@@ -208,8 +297,14 @@ void trace_kernel(TraceParams p) {
   lds_u64* ldsB = (lds_u64*)(lds_stack + (NS - 1) * K * BS + tid);
   lds_u64* ring = (lds_u64*)(rec_ring + (REC == kRecSlab ? tid : 0u));
   const uint64_t lane_slot = (uint64_t)blockIdx.x * BS + tid;
-  glb_u64* gA = (glb_u64*)(p.spill + lane_slot * (uint64_t)p.spill_cap * NS);
-  glb_u64* gB = gA + (NS - 1) * (uint64_t)p.spill_cap;
+  // The lane's spill area, formed where it is used (rarely) instead of held in
+  // two registers for the whole launch.
+  auto spill_a = [&]() -> glb_u64* {
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return (glb_u64*)(p.spill + ((uint64_t)blockIdx.x * BS + t) * (uint64_t)p.spill_cap * NS);
+  };
+  auto spill_b = [&]() -> glb_u64* { return spill_a() + (NS - 1) * (uint64_t)p.spill_cap; };
   // Scene of the lane's current ray (a batch kernel switches it per ray).
   const uint8_t* __restrict__ A = p.arena;
   uint64_t bytes = p.arena_bytes;
@@ -225,14 +320,15 @@ void trace_kernel(TraceParams p) {
     __syncthreads();
   }
 
-  Stack sa{0, 0, 0}, sb{0, 0, 0};
+  Stack sa{0, 0, 0}, sb{0, 0, 0};  // treelet order
+  Groups gs{0, 0, 0};              // plain order
   bool active = false, exhausted = false;
   bool pending = false;  // the lane's completed ray still has to write its hit record
   uint32_t err = 0;
 
   F3 ro{}, rd{}, ridir{};
   float rtmin = 0.f, rtmax = 0.f;
-  uint32_t rflags = 0;
+  uint32_t rflags = 0;  // treelet order (plain order keeps them in gs.state)
   float min_thit = 0.f, min_thit_obj = 0.f;
   uint32_t closest_leaf = kNoSlot, closest_inst = kNoSlot;
   ObjRay cur{};
@@ -338,11 +434,23 @@ void trace_kernel(TraceParams p) {
   };
 
   auto push_entry = [&](uint64_t e, bool to_a) {
+    if constexpr (MODE == 0) {
+      // a group of one child
+      if ((gs.state & kGroupDepthMask) >= ((uint32_t)K + p.spill_cap) * kGroupDepth) {
+        err |= kErrStack;
+        return;
+      }
+      groups_save<K, BS>(gs, ldsA, spill_a);
+      gs.base = e_slot(e);
+      gs.word = group_word(e_flags(e), e_level(e), (e_flags(e) >> 1) & 1u, 1u);
+      gs.state += kGroupDepth;
+      return;
+    }
     bool ok;
-    if (MODE == 0 || to_a)
-      ok = st_push<K, BS>(sa, e, ldsA, gA, p.spill_cap);
+    if (to_a)
+      ok = st_push<K, BS>(sa, e, ldsA, spill_a(), p.spill_cap);
     else
-      ok = st_push<K, BS>(sb, e, ldsB, gB, p.spill_cap);
+      ok = st_push<K, BS>(sb, e, ldsB, spill_b(), p.spill_cap);
     if (!ok) err |= kErrStack;
   };
 
@@ -583,14 +691,15 @@ void trace_kernel(TraceParams p) {
 
   // Pop the lane's next entry into `e`; false when its stacks are empty.
   auto pop_next = [&]() -> bool {
-    if (MODE == 0 ? st_empty(sa) : (st_empty(sa) && st_empty(sb))) return false;
-    if (MODE == 0) {
-      e = st_pop<K, BS>(sa, ldsA, gA);
+    if constexpr (MODE == 0) {
+      if (!groups_pop<K, BS>(gs, e, ldsA, spill_a)) return false;
+    } else if (st_empty(sa) && st_empty(sb)) {
+      return false;
     } else if (!st_empty(sa)) {
-      e = st_pop<K, BS>(sa, ldsA, gA);
+      e = st_pop<K, BS>(sa, ldsA, spill_a());
     } else {
       phase2 = true;  // current_treelet_root := host address of the moved node (:1748-1754)
-      e = st_pop<K, BS>(sb, ldsB, gB);
+      e = st_pop<K, BS>(sb, ldsB, spill_b());
     }
     // every processed entry emits at least one record
     if (n_rec > kMaxStepsPerRay) err |= kErrSteps;
@@ -733,6 +842,8 @@ void trace_kernel(TraceParams p) {
           if constexpr (REC == kRecCsr) rec_base = p.record_offsets[r];
           sa = Stack{0, 0, 0};
           sb = Stack{0, 0, 0};
+          gs = Groups{0, 0, ((r2.x & RTX_RAY_FLAG_OPAQUE) ? kGroupOpaque : 0u) |
+                                ((r2.x & RTX_RAY_FLAG_TERMINATE_ON_FIRST_HIT) ? kGroupTerminate : 0u)};
           phase2 = false;
           err = 0;
           // TLAS header record and bounds test (vulkan_ray_tracing.cc:2444-2484)
@@ -961,7 +1072,7 @@ void trace_kernel(TraceParams p) {
             bool accept;
             if (MODE == 0) {
               accept = h && rtmin <= wt && wt <= rtmax;
-              if (accept && (rflags & RTX_RAY_FLAG_OPAQUE) && wt < min_thit) min_thit = th / cur.tmult;
+              if (accept && (gs.state & kGroupOpaque) && wt < min_thit) min_thit = th / cur.tmult;
             } else {
               accept = h && rtmin <= wt && wt <= rtmax && wt < min_thit;
               if (accept) min_thit = th / cur.tmult;
@@ -972,10 +1083,11 @@ void trace_kernel(TraceParams p) {
               closest_inst = cur_inst;
               emit(off, 64, RTX_TX_BVH_QUAD_LEAF_HIT, level);
               n_nodes++;
-              if (MODE == 0 && !(rflags & RTX_RAY_FLAG_OPAQUE)) n_any++;
-              if (rflags & RTX_RAY_FLAG_TERMINATE_ON_FIRST_HIT) {
+              if (MODE == 0 && !(gs.state & kGroupOpaque)) n_any++;
+              if (MODE == 0 ? (gs.state & kGroupTerminate) : (rflags & RTX_RAY_FLAG_TERMINATE_ON_FIRST_HIT)) {
                 sa = Stack{0, 0, 0};
                 sb = Stack{0, 0, 0};
+                gs = Groups{0, 0, gs.state & (kGroupOpaque | kGroupTerminate)};
               }
             } else {
               emit(off, 64, RTX_TX_BVH_QUAD_LEAF, level);
@@ -1022,21 +1134,22 @@ void trace_kernel(TraceParams p) {
             if (top) {
               o = ro;
               idir = ridir;
-              tmin = rtmin;
-              tmax = rtmax;
-              cull = min_thit;
             } else {
               o = cur.o;
               idir = cur.idir;
-              tmin = cur.tmin;
-              tmax = cur.tmax;
-              cull = min_thit * cur.tmult;
             }
+            // the object-space range and cull distance scale with the direction
+            // (x * 1 = x for the TLAS); formed per node, they hold no registers
+            const float tscale = top ? 1.0f : cur.tmult;
+            tmin = rtmin * tscale;
+            tmax = rtmax * tscale;
+            cull = min_thit * tscale;
             const uint64_t first_child = off + (uint64_t)((int64_t)(int32_t)nd.w[3] * 64);
             const F3 sc = child_scales(ex, ey, ez);
+            const KidBytes kids{__builtin_amdgcn_alignbyte(nd.w[6], nd.w[5], 2), nd.w[6] >> 16};
             uint32_t hitmask = 0;
-            // When no lane can produce a NaN (finite ray, non-NaN node origin)
-            // and the arena's child boxes all have lo <= hi, each axis's near
+            // When no lane can produce a NaN (finite ray; the scene walk found
+            // no NaN node origin) and the arena's child boxes all have lo <= hi, each axis's near
             // and far bound is picked by the sign of the inverse direction and
             // the slab test needs only the max of the near and the min of the
             // far distances: for such boxes min(lo', hi') and max(lo', hi')
@@ -1044,25 +1157,37 @@ void trace_kernel(TraceParams p) {
             // v_min/v_max forms differ from the reference's compare-selects
             // only in the sign of a zero, which only enters comparisons.
             // Otherwise the reference's compare-selects run.
-            const bool fast = (top ? ray_ok : cur_ok) && !__builtin_isnan(f_of(nd, 0) + f_of(nd, 1) + f_of(nd, 2)) &&
-                              cull != -__builtin_inff();
+            const bool fast = (top ? ray_ok : cur_ok) && cull != -__builtin_inff();
             auto test_children = [&](auto fast_tag) {
               constexpr bool FAST = decltype(fast_tag)::value;
               if constexpr (FAST) {
-                // near / far bound bytes per axis chosen by the ray's direction sign
-                uint32_t nw[3][2], fw[3][2];
+                // Near / far bounds per axis chosen by the ray's direction sign:
+                // one v_perm takes two children's bytes out of two node words,
+                // each as the low byte of a half, which is q * 2^-24 exactly as
+                // a (denormal) half; v_fma_mix takes halves, so a bound is one
+                // instruction from there, with the single rounding of
+                // child_box.  The scales carry the 2^24 (the scene walk allows
+                // this path for scales up to 2^103).  36 conversions and 24
+                // selects became 18 permutes.
+                uint32_t nq[3][3], fq[3][3];
 #pragma unroll
                 for (int a = 0; a < 3; ++a) {
-                  const int lw = 7 + 3 * a;
                   const float d = a == 0 ? idir.x : a == 1 ? idir.y : idir.z;
-                  const bool neg = d < 0.0f;
-                  const uint32_t l0 = nd.w[lw], l1 = nd.w[lw + 1];
-                  const uint32_t u0 = __builtin_amdgcn_alignbyte(nd.w[lw + 2], nd.w[lw + 1], 2), u1 = nd.w[lw + 2] >> 16;
-                  nw[a][0] = neg ? u0 : l0;
-                  nw[a][1] = neg ? u1 : l1;
-                  fw[a][0] = neg ? l0 : u0;
-                  fw[a][1] = neg ? l1 : u1;
+                  const uint32_t w0 = nd.w[7 + 3 * a], w1 = nd.w[8 + 3 * a], w2 = nd.w[9 + 3 * a];
+                  const uint32_t n0 = d < 0.0f ? 0x0c070c06u : 0x0c010c00u, f0 = n0 ^ 0x00060006u;
+                  const uint32_t n1 = n0 ^ 0x00020002u, f1 = f0 ^ 0x00020002u;
+                  nq[a][0] = __builtin_amdgcn_perm(w1, w0, n0);
+                  nq[a][1] = __builtin_amdgcn_perm(w2, w0, n1);
+                  nq[a][2] = __builtin_amdgcn_perm(w2, w1, n0);
+                  fq[a][0] = __builtin_amdgcn_perm(w1, w0, f0);
+                  fq[a][1] = __builtin_amdgcn_perm(w2, w0, f1);
+                  fq[a][2] = __builtin_amdgcn_perm(w2, w1, f0);
                 }
+                const float sx = sc.x * 0x1p24f, sy = sc.y * 0x1p24f, sz = sc.z * 0x1p24f;
+                auto bound = [](uint32_t pair, int i, float scale, float origin) -> float {
+                  const uint16_t h = (uint16_t)((i & 1) ? pair >> 16 : pair & 0xffffu);
+                  return __builtin_fmaf((float)__builtin_bit_cast(_Float16, h), scale, origin);
+                };
                 const float ox = f_of(nd, 0), oy = f_of(nd, 1), oz = f_of(nd, 2);
                 // The cull test folded into the far bound: for a non-NaN tn
                 // and a cull above -inf, !(tn >= cull) is tn < cull, which is
@@ -1080,21 +1205,17 @@ void trace_kernel(TraceParams p) {
                 // distances, never a NaN, and its result is discarded
 #pragma unroll
                 for (int i = 0; i < 6; ++i) {
-                  const uint32_t info = byte_of(nd, 22 + i) & 0x3fu;
-                  const int wi = i >> 2, sh = 8 * (i & 3);
-                  const float nx = __builtin_fmaf((float)((nw[0][wi] >> sh) & 0xffu), sc.x, ox);
-                  const float ny = __builtin_fmaf((float)((nw[1][wi] >> sh) & 0xffu), sc.y, oy);
-                  const float nz = __builtin_fmaf((float)((nw[2][wi] >> sh) & 0xffu), sc.z, oz);
-                  const float fx = __builtin_fmaf((float)((fw[0][wi] >> sh) & 0xffu), sc.x, ox);
-                  const float fy = __builtin_fmaf((float)((fw[1][wi] >> sh) & 0xffu), sc.y, oy);
-                  const float fz = __builtin_fmaf((float)((fw[2][wi] >> sh) & 0xffu), sc.z, oz);
+                  const float nx = bound(nq[0][i >> 1], i, sx, ox), ny = bound(nq[1][i >> 1], i, sy, oy),
+                              nz = bound(nq[2][i >> 1], i, sz, oz);
+                  const float fx = bound(fq[0][i >> 1], i, sx, ox), fy = bound(fq[1][i >> 1], i, sy, oy),
+                              fz = bound(fq[2][i >> 1], i, sz, oz);
                   const float tn = __builtin_fmaxf(__builtin_fmaxf(__builtin_fmaxf((nx - o.x) * idir.x, (ny - o.y) * idir.y),
                                                                    (nz - o.z) * idir.z), tmin);
                   const float tf = __builtin_fminf(__builtin_fminf(__builtin_fminf((fx - o.x) * idir.x, (fy - o.y) * idir.y),
                                                                    (fz - o.z) * idir.z), tfc);
-                  const bool h = (info & 3u) != 0u && tn <= tf;
-                  hitmask |= h ? 1u << i : 0u;
+                  hitmask |= tn <= tf ? 1u << i : 0u;
                 }
+                hitmask &= kids_present(kids);
               } else {
 #pragma unroll
                 for (int i = 0; i < 6; ++i) {
@@ -1124,54 +1245,35 @@ void trace_kernel(TraceParams p) {
               const uint32_t inst = top ? 0u : e_inst_rel(e);
               const uint32_t base_flags = top ? kFlTop : 0u;
               bool pushed = false;
-              if constexpr (MODE == 0 && !LM && K >= 8) {
-                // Plain order without the level map, for a node whose children
-                // lie in the arena and (under the TLAS) are internal nodes or
-                // instance leaves: the pushes below give the same stack as one
-                // push per child.  The ring's oldest entries are spilled first,
-                // as many as pushing one by one would spill (up to six new
-                // entries never spill each other when K >= 8), then each hit
-                // child is stored at its place: children in slot order, the
-                // first internal one last.
-                const uint32_t iw0 = __builtin_amdgcn_alignbyte(nd.w[6], nd.w[5], 2);  // info bytes of children 0-3
-                const uint32_t iw1 = nd.w[6] >> 16;                                    // children 4-5
-                uint32_t pre[6], tot = 0, leafm = 0;
-#pragma unroll
-                for (int i = 0; i < 6; ++i) {
-                  const uint32_t info = (i < 4 ? iw0 >> (8 * i) : iw1 >> (8 * (i - 4))) & 0x3fu;
-                  pre[i] = tot;
-                  tot += info & 3u;
-                  leafm |= (info >> 2) != 0u ? 1u << i : 0u;
-                }
-                const uint32_t n_push = (uint32_t)__builtin_popcount(hitmask);
-                const uint32_t need = sa.cnt + n_push;
-                const uint32_t sp = need > (uint32_t)K ? need - (uint32_t)K : 0u;
-                const bool ok = first_child < bytes && first_child + (uint64_t)tot * 64 <= bytes &&
-                                !(top && ((iw0 & 0x38383838u) | (iw1 & 0x3838u)) != 0u) && sa.g + sp <= p.spill_cap;
-                if (ok) {
+              if constexpr (MODE == 0 && !LM) {
+                // Plain order in a scene of regular nodes: the hit children are
+                // one group, without the first internal one, which is the
+                // lane's next entry.  No child needs a check here: the scene
+                // walk placed all of them in the arena.
+                if (p.regular_nodes) {
                   pushed = true;
-                  for (uint32_t j = 0; j < sp; ++j) {
-                    gA[sa.g++] = ldsA[sa.bot * BS];
-                    sa.bot = (sa.bot + 1) & (K - 1);
-                    sa.cnt--;
-                  }
-                  const uint32_t im = hitmask & ~leafm;
-                  const uint32_t dbit = im & (0u - im);  // the first internal hit child
-                  const uint32_t pm = hitmask & ~dbit;
-                  const uint32_t first_slot = (uint32_t)(first_child >> 6);
-                  const uint32_t hi = base_flags | ((lvl > 255u ? 255u : lvl) << 2) | ((inst & 0x3fffffu) << 10);
-                  const uint32_t top_pos = sa.bot + sa.cnt;
-#pragma unroll
-                  for (int i = 0; i < 6; ++i) {
-                    if ((hitmask >> i) & 1u) {
-                      // the deferred child takes the last place
-                      const uint32_t r = ((dbit >> i) & 1u) ? n_push - 1u
-                                                             : (uint32_t)__builtin_popcount(pm & ((1u << i) - 1u));
-                      ldsA[((top_pos + r) & (K - 1)) * BS] =
-                          (uint64_t)(first_slot + pre[i]) | ((uint64_t)(hi | (((leafm >> i) & 1u) ? kFlLeaf : 0u)) << 32);
+                  const uint32_t n_push = (uint32_t)__popc(hitmask);
+                  if ((gs.state & kGroupDepthMask) + n_push * kGroupDepth > ((uint32_t)K + p.spill_cap) * kGroupDepth) {
+                    err |= kErrStack;
+                  } else {
+                    const uint32_t leaves = kids_leaves(kids);
+                    const uint32_t word = group_word(base_flags, lvl, leaves, 0u);
+                    const uint32_t first = slot + nd.w[3];
+                    const uint32_t im = hitmask & ~leaves;
+                    const uint32_t rest = hitmask & ~(im & (0u - im));
+                    gs.state += n_push * kGroupDepth;
+                    if (rest) {
+                      groups_save<K, BS>(gs, ldsA, spill_a);
+                      gs.base = first;
+                      gs.word = word | (rest << 16);
+                    }
+                    if (im) {
+                      e = group_entry(first, word, (uint32_t)__builtin_ctz(im));
+                      has_e = true;
+                      gs.state -= kGroupDepth;
+                      if (n_rec > kMaxStepsPerRay) err |= kErrSteps;
                     }
                   }
-                  sa.cnt += n_push;
                 }
               } else if constexpr (MODE == 1 && !LM) {
                 // Treelet order, same conditions: the children go in slot
@@ -1208,8 +1310,8 @@ void trace_kernel(TraceParams p) {
                       st.cnt--;
                     }
                   };
-                  spill_list(sa, ldsA, gA, spA);
-                  spill_list(sb, ldsB, gB, spB);
+                  if (spA) spill_list(sa, ldsA, spill_a(), spA);
+                  if (spB) spill_list(sb, ldsB, spill_b(), spB);
                   // one store per hit child, into the list it goes to
                   const uint32_t topA = sa.bot + sa.cnt, topB = sb.bot + sb.cnt;
 #pragma unroll
@@ -1401,6 +1503,13 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
 
   bool active = false, exhausted = false, pending = false;
   bool phase2 = false;
+  // plain order: the groups of trace_kernel, their older ones (da of them) in LDS
+  Groups gs{0, 0, 0};
+  uint32_t depth = 0;
+  // this lane's child in the byte arrays of a node's words (a zero-extended byte
+  // by one v_perm from two words): lower bounds start a word, upper bounds and the
+  // size/type bytes start in a word's third byte
+  const uint32_t jj = min(j, 5u), sel_lo = 0x0c0c0c00u | jj, sel_hi = 0x0c0c0c00u | (jj + 2u);
   uint32_t da = 0, db = 0, err = 0, local_id = 0;
   F3 ro{}, rd{}, ridir{};
   float rtmin = 0.f, rtmax = 0.f;
@@ -1421,8 +1530,24 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
   // lane 0 of the group writes; the group's later pops read it back in order
   // (the list depths are updated through selects, not a reference to one of
   // them, which would put both in scratch memory)
+  auto save_group = [&]() {
+    if (gs.word < kGroupFirst) return;
+    if (j == 0) sta[da] = (uint64_t)gs.base | ((uint64_t)gs.word << 32);
+    da++;
+  };
   auto push = [&](uint64_t v, bool to_a) {
-    const bool a = MODE == 0 || to_a;
+    if constexpr (MODE == 0) {
+      if (depth >= cap) {
+        err |= kErrStack;
+        return;
+      }
+      save_group();
+      gs.base = e_slot(v);
+      gs.word = group_word(e_flags(v), e_level(v), (e_flags(v) >> 1) & 1u, 1u);
+      depth++;
+      return;
+    }
+    const bool a = to_a;
     const uint32_t d = a ? da : db;
     if (d >= cap) {
       err |= kErrStack;
@@ -1433,8 +1558,22 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
     db = a ? db : d + 1;
   };
   auto pop_next = [&]() -> bool {
+    if constexpr (MODE == 0) {
+      if (gs.word < kGroupFirst) {
+        if (da == 0) return false;
+        const uint64_t v = sta[--da];
+        gs.base = (uint32_t)v;
+        gs.word = (uint32_t)(v >> 32);
+      }
+      const uint32_t i = 15u - (uint32_t)__builtin_clz(gs.word);
+      e = group_entry(gs.base, gs.word, i);
+      gs.word ^= kGroupFirst << i;
+      depth--;
+      if (n_rec > kMaxStepsPerRay) err |= kErrSteps;
+      return true;
+    }
     if (da == 0 && db == 0) return false;
-    const bool a = MODE == 0 || da > 0;
+    const bool a = da > 0;
     // moving to the other list: current_treelet_root := host address of the moved node (:1748-1754)
     if (!a) phase2 = true;
     const uint32_t d = (a ? da : db) - 1;
@@ -1564,6 +1703,8 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
           n_rec = n_nodes = fetch_bytes = n_any = 0;
           max_level = 1;
           da = db = 0;
+          gs = Groups{0, 0, 0};
+          depth = 0;
           phase2 = false;
           err = 0;
           has_e = false;
@@ -1687,7 +1828,11 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
               emit(64, RTX_TX_BVH_QUAD_LEAF_HIT);
               n_nodes++;
               if (MODE == 0 && !(rflags & RTX_RAY_FLAG_OPAQUE)) n_any++;
-              if (rflags & RTX_RAY_FLAG_TERMINATE_ON_FIRST_HIT) da = db = 0;
+              if (rflags & RTX_RAY_FLAG_TERMINATE_ON_FIRST_HIT) {
+                da = db = 0;
+                gs = Groups{0, 0, 0};
+                depth = 0;
+              }
             } else {
               emit(64, RTX_TX_BVH_QUAD_LEAF);
               n_nodes++;
@@ -1710,36 +1855,71 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
         emit(64, RTX_TX_BVH_INTERNAL_NODE);
         n_nodes++;
         const bool top = (flags & kFlTop) != 0;
-        const int ex = (int)(int8_t)byte_of(nd, 18);
-        const int ey = (int)(int8_t)byte_of(nd, 19);
-        const int ez = (int)(int8_t)byte_of(nd, 20);
+        const F3 sc = child_scales((int)(int8_t)byte_of(nd, 18), (int)(int8_t)byte_of(nd, 19), (int)(int8_t)byte_of(nd, 20));
         const F3 o = top ? ro : cur.o;
         const F3 idir = top ? ridir : cur.idir;
-        const float tmin = top ? rtmin : cur.tmin;
-        const float tmax = top ? rtmax : cur.tmax;
-        const float cull = top ? min_thit : min_thit * cur.tmult;
-        const bool fast = (top ? ray_ok : cur_ok) && !__builtin_isnan(f_of(nd, 0) + f_of(nd, 1) + f_of(nd, 2));
-        bool h = false;
-        if (j < 6u && (byte_at(nd, 22, j) & 3u) != 0u) {
-          const F3 sc = child_scales(ex, ey, ez);
-          const float ox = f_of(nd, 0), oy = f_of(nd, 1), oz = f_of(nd, 2);
+        const float tscale = top ? 1.0f : cur.tmult;
+        const float tmin = rtmin * tscale, tmax = rtmax * tscale, cull = min_thit * tscale;
+        const uint32_t info = __builtin_amdgcn_perm(nd.w[6], nd.w[5], sel_hi) & 0x3fu;  // size and type of child j
+        const float ox = f_of(nd, 0), oy = f_of(nd, 1), oz = f_of(nd, 2);
+        float th;
+        bool h;
+        if (__ballot(!((top ? ray_ok : cur_ok) && p.ordered_boxes)) == 0) {
+          // a bound is a byte q times the scale: q as the low byte of a half is q *
+          // 2^-24 exactly, and the FMA takes halves (see trace_kernel)
+          auto bound = [](uint32_t q, float scale, float origin) -> float {
+            return __builtin_fmaf((float)__builtin_bit_cast(_Float16, (uint16_t)q), scale * 0x1p24f, origin);
+          };
           F3 lo, hi;
-          lo.x = __builtin_fmaf((float)byte_at(nd, 28, j), sc.x, ox);
-          lo.y = __builtin_fmaf((float)byte_at(nd, 40, j), sc.y, oy);
-          lo.z = __builtin_fmaf((float)byte_at(nd, 52, j), sc.z, oz);
-          hi.x = __builtin_fmaf((float)byte_at(nd, 34, j), sc.x, ox);
-          hi.y = __builtin_fmaf((float)byte_at(nd, 46, j), sc.y, oy);
-          hi.z = __builtin_fmaf((float)byte_at(nd, 58, j), sc.z, oz);
-          float th;
-          h = fast ? ray_box_fast(lo, hi, idir, o, tmin, tmax, th) : ray_box(lo, hi, idir, o, tmin, tmax, th);
-          if (h && th >= cull) h = false;
+          lo.x = bound(__builtin_amdgcn_perm(nd.w[8], nd.w[7], sel_lo), sc.x, ox);
+          lo.y = bound(__builtin_amdgcn_perm(nd.w[11], nd.w[10], sel_lo), sc.y, oy);
+          lo.z = bound(__builtin_amdgcn_perm(nd.w[14], nd.w[13], sel_lo), sc.z, oz);
+          hi.x = bound(__builtin_amdgcn_perm(nd.w[9], nd.w[8], sel_hi), sc.x, ox);
+          hi.y = bound(__builtin_amdgcn_perm(nd.w[12], nd.w[11], sel_hi), sc.y, oy);
+          hi.z = bound(__builtin_amdgcn_perm(nd.w[15], nd.w[14], sel_hi), sc.z, oz);
+          h = ray_box_fast(lo, hi, idir, o, tmin, tmax, th);
+        } else {
+          F3 lo, hi;
+          lo.x = __builtin_fmaf((float)byte_at(nd, 28, jj), sc.x, ox);
+          lo.y = __builtin_fmaf((float)byte_at(nd, 40, jj), sc.y, oy);
+          lo.z = __builtin_fmaf((float)byte_at(nd, 52, jj), sc.z, oz);
+          hi.x = __builtin_fmaf((float)byte_at(nd, 34, jj), sc.x, ox);
+          hi.y = __builtin_fmaf((float)byte_at(nd, 46, jj), sc.y, oy);
+          hi.z = __builtin_fmaf((float)byte_at(nd, 58, jj), sc.z, oz);
+          h = ray_box(lo, hi, idir, o, tmin, tmax, th);
         }
+        h = h && !(th >= cull) && j < 6u && (info & 3u) != 0u;
         const uint32_t hitmask = (uint32_t)(__ballot(h) >> gbase) & 0x3fu;
         if (hitmask) {
           const uint32_t lvl = level + 1;
           if (lvl > max_level) max_level = lvl;
           const uint32_t inst = top ? 0u : e_inst_rel(e);
           const uint32_t base_flags = top ? kFlTop : 0u;
+          if (MODE == 0 && p.regular_nodes) {
+            // the hit children as one group, the first internal one the next entry
+            const uint32_t n_push = (uint32_t)__popc(hitmask);
+            if (depth + n_push > cap) {
+              err |= kErrStack;
+            } else {
+              const uint32_t leaves = (uint32_t)(__ballot(j < 6u && (info >> 2) != 0u) >> gbase) & 0x3fu;
+              const uint32_t word = group_word(base_flags, lvl, leaves, 0u);
+              const uint32_t first = slot + nd.w[3];
+              const uint32_t im = hitmask & ~leaves;
+              const uint32_t rest = hitmask & ~(im & (0u - im));
+              depth += n_push;
+              if (rest) {
+                save_group();
+                gs.base = first;
+                gs.word = word | (rest << 16);
+              }
+              if (im) {
+                e = group_entry(first, word, (uint32_t)__builtin_ctz(im));
+                has_e = true;
+                depth--;
+                if (n_rec > kMaxStepsPerRay) err |= kErrSteps;
+              }
+            }
+          } else {
           // Lane j pushes hit child j itself, at the position the per-lane
           // kernel's push sequence gives it: hit children in slot order (in
           // plain order the first internal one last), a list's pushes failing
@@ -1748,7 +1928,7 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
 #pragma unroll
           for (int i = 0; i < 5; ++i)
             if ((uint32_t)i < j) c += (uint64_t)(byte_of(nd, 22 + i) & 3u) * 64;
-          const uint32_t ctype = j < 6u ? (byte_at(nd, 22, j) & 0x3fu) >> 2 : 0u;
+          const uint32_t ctype = j < 6u ? info >> 2 : 0u;
           const bool leaf = ctype != 0;
           const bool mine = j < 6u && ((hitmask >> j) & 1u);
           const bool pushed = mine && !(c & 63) && c + 64 <= bytes;
@@ -1763,8 +1943,17 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
             const uint32_t n = (uint32_t)__popc(m_push);
             const uint32_t d = m_int ? (uint32_t)__builtin_ctz(m_int) : 8u;  // deferred child, 8 = none
             const uint32_t rest = m_push & ~(d < 8u ? 1u << d : 0u);
-            pos = j == d ? da + n - 1u : da + (uint32_t)__popc(rest & below);
-            da = min(cap, da + n);
+            // groups of one child, the newest group among the older ones first
+            save_group();
+            gs.word = 0;
+            pos = j == d ? n - 1u : (uint32_t)__popc(rest & below);
+            const uint32_t fit = min(n, cap - depth);
+            if (pushed && pos < fit)
+              sta[da + pos] = (uint64_t)(uint32_t)(c >> 6) |
+                              ((uint64_t)group_word(base_flags, lvl, leaf ? 1u : 0u, 1u) << 32);
+            da += fit;
+            depth += fit;
+            if (fit < n) err |= kErrStack;
           } else {
             const uint32_t m_a = (uint32_t)(__ballot(pushed && to_a) >> gbase) & 0x3fu;
             const uint32_t m_b = m_push & ~m_a;
@@ -1772,11 +1961,12 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
             da = min(cap, da + (uint32_t)__popc(m_a));
             db = min(cap, db + (uint32_t)__popc(m_b));
           }
-          const bool fits = pos < cap;
-          if (pushed && fits)
+          const bool fits = MODE == 0 || pos < cap;
+          if (MODE == 1 && pushed && fits)
             *(to_a ? sta + pos : stb + pos) =
                 make_entry((uint32_t)(c >> 6), base_flags | (leaf ? kFlLeaf : 0u), lvl, inst);
           if ((__ballot(pushed && !fits) >> gbase) & 0x3fu) err |= kErrStack;
+          }
         }
       }
     }
