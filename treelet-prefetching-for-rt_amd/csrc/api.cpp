@@ -691,7 +691,8 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
   grid = std::max(grid, 1u);
   const uint32_t spill_cap = 128;
   const uint32_t ns = opts->mode == RTX_MODE_TREELET ? 2 : 1;
-  rtx_status st = ensure_spill(c, (size_t)grid * bs * spill_cap * ns);
+  // staged treelet order keeps fewer entries in LDS (trace_kernel's R)
+  rtx_status st = ensure_spill(c, (size_t)grid * bs * (spill_cap + (stage ? lds_stack : 0)) * ns);
   if (st != RTX_OK) return st;
 
   TraceParams p{};

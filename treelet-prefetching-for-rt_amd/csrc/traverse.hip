@@ -19,12 +19,12 @@
 //    address (:1752), so every later child goes to "other".  Which children
 //    the first treelet owns is precomputed with the partition, one byte per
 //    node slot, so a node costs one extra byte load, not one per child.
-//    Entries carry the instance leaf that opened them; the object-space ray
-//    is recomputed from that leaf when it differs from the cached one (same
-//    inputs, same floats).
+//    Entries carry the instance leaf that opened them (groups pushed after the
+//    switch need none, see Groups); the object-space ray is recomputed from
+//    that leaf when it differs from the cached one (same inputs, same floats).
 //
-// Stacks: a ring of K entries (plain order: K groups) per lane in LDS, spilling
-// the oldest to a per-lane region in global memory (exact LIFO order).
+// Stacks: a ring of K groups or entries per lane and list in LDS, spilling the
+// oldest to a per-lane region in global memory (exact LIFO order).
 //
 // One wave iteration runs three passes, each only for the lanes that need it:
 // instance leaves, triangle leaves, then internal nodes.  A lane that finishes
@@ -65,7 +65,7 @@ constexpr uint32_t kFlTop = 1u, kFlLeaf = 2u;
 constexpr uint32_t kNoSlot = 0xffffffffu;
 constexpr uint32_t kNone = 0xffffffffu;
 
-// A stack entry: node slot (32 bits), flags (2), tree level (8) and the
+// An entry: node slot (32 bits), flags (2), tree level (8) and the
 // instance leaf that opened the entry (22 bits, treelet order only).  The
 // instance is stored as its slot's distance from the TLAS header slot, a
 // signed 22-bit value, so instance leaves may lie anywhere within 128 MiB of
@@ -90,111 +90,90 @@ __device__ __forceinline__ bool inst_rel_of(uint32_t inst, uint32_t tlas_slot, u
   return d >= -kInstRelMax && d < kInstRelMax;
 }
 
-struct Stack {
-  uint32_t bot, cnt, g;
-};
-
 // LDS and global stack words are reached through pointers typed by address
 // space, so a pop compiles to ds_read or global_load and never to a flat load
 // (which would also wait for every outstanding store of the lane).
 typedef __attribute__((address_space(3))) uint64_t lds_u64;
 typedef __attribute__((address_space(1))) uint64_t glb_u64;
 
-template <int K, uint32_t BS>
-__device__ __forceinline__ bool st_push(Stack& s, uint64_t e, lds_u64* lds, glb_u64* g, uint32_t gcap) {
-  if (s.cnt == (uint32_t)K) {
-    if (s.g >= gcap) return false;
-    g[s.g++] = lds[s.bot * BS];
-    s.bot = (s.bot + 1) & (K - 1);
-    s.cnt--;
-  }
-  lds[((s.bot + s.cnt) & (K - 1)) * BS] = e;
-  s.cnt++;
-  return true;
-}
-
-template <int K, uint32_t BS>
-__device__ __forceinline__ uint64_t st_pop(Stack& s, lds_u64* lds, glb_u64* g) {
-  if (s.cnt == 0) return g[--s.g];
-  s.cnt--;
-  return lds[((s.bot + s.cnt) & (K - 1)) * BS];
-}
-
-__device__ __forceinline__ bool st_empty(const Stack& s) { return s.cnt == 0 && s.g == 0; }
-
-// ---- plain order: stack of child groups ---------------------------------------
+// ---- stacks of child groups ------------------------------------------------------
 // A node's hit children left for later are one group: the slot of its first
 // child and a word with the children still to visit (bits 16-21), which children
-// are leaves (10-15), the tree level (2-9) and whether it is a TLAS node (0).
+// are leaves (10-15), the tree level (2-9) and whether it is a TLAS node (1).
 // The children are visited highest slot first, which is the order of popping
-// them after pushing each in slot order; the first internal child, which is
-// pushed last, goes on as the lane's next entry.  The newest group stays in
-// registers, older ones are a ring of K per lane in LDS whose oldest groups
-// spill to global memory.  `depth` counts the children outstanding, one entry
-// each, and the ray reports a stack overflow at K + spill_cap of them.
+// them after pushing each in slot order.  The child visited next goes on as the
+// lane's next entry: in plain order the first internal one, which is pushed last
+// there, in treelet order the highest.  The newest group stays in registers,
+// older ones are a ring of K per lane in LDS whose oldest spill to global memory.
+// The depth counts the children outstanding, one each, and the ray reports a
+// stack overflow at K + spill_cap of them.
 // A group needs a regular node: children packed from slot 0 on, an instance leaf
 // two slots and any other child one.  The scene walk checks that once for all
-// nodes; other scenes push every child as a group of its own.
+// nodes; other scenes push every child on its own.
 // A push of up to six entries, each placed and stored under its own branch, was
 // a third of the vector instructions of an internal node; a group takes 45
-// instead of 155 and at most one LDS store, and the next internal child reaches
-// the next iteration without LDS.  With the slab test on halves below, 1.34M
-// camera and bounce rays on the 1M-triangle scene take 263 -> 228 M vector
-// instructions and 594 -> 558 us; the registers it frees keep five waves.
+// instead of 155 and at most one LDS store, and the next child reaches the next
+// iteration without LDS.  With the slab test on halves below, 1.34M camera and
+// bounce rays on the 1M-triangle scene take 263 -> 228 M vector instructions and
+// 594 -> 558 us in plain order; the registers it frees keep five waves there.  In
+// treelet order 2.6M rays on the 21M-triangle scene take 2.33 -> 2.21 ms, and the
+// diffuse batch with whole treelets staged 1.66 -> 1.44 ms.
+//
+// Treelet order has two lists.  The register group belongs to the list the next
+// pop takes (the current one, and the other one after the switch); before the
+// switch the other list is only pushed to.  An entry of a BLAS also names its
+// instance, for which a group has no room: after the switch the lists are one
+// stack, so whenever a group pushed since comes up, the ray's instance is again
+// the one it was pushed in.  Before the switch, children in a BLAS are pushed
+// one by one as entries (make_entry), told apart by bit 0 with bits 10 and up.
 struct Groups {
   uint32_t base, word;  // the newest group; word < kGroupFirst: none left in it
-  // older groups (bits 0-7; position p of them is in LDS unless p < bits 8-15),
-  // depth (16-23, at most 144) and the ray's opaque and terminate flags (24, 25)
+  // its list: items in the ring and spilled (bits 0-7; position p of them is in
+  // LDS unless p < bits 8-15), depth (16-23, at most 144); and the ray's opaque
+  // and terminate flags (24, 25)
   uint32_t state;
 };
-constexpr uint32_t kGroupDepth = 1u << 16, kGroupDepthMask = 0xff0000u, kGroupOpaque = 1u << 24, kGroupTerminate = 1u << 25;
-constexpr uint32_t kGroupFirst = 1u << 16, kGroupLeaf = 10;
-__device__ __forceinline__ uint32_t group_word(uint32_t flags, uint32_t level, uint32_t leaves, uint32_t mask) {
-  return (flags & kFlTop) | ((level > 255u ? 255u : level) << 2) | (leaves << kGroupLeaf) | (mask << 16);
+constexpr uint32_t kGroupFirst = 1u << 16, kGroupLeaf = 10, kGroupTag = 1u, kGroupTop = 2u;
+constexpr uint32_t kListItems = 0xffu, kListDepth = 1u << 16, kListDepthMask = 0xff0000u;
+constexpr uint32_t kRayOpaque = 1u << 24, kRayTerminate = 1u << 25;
+__device__ __forceinline__ uint32_t group_word(bool top, uint32_t level, uint32_t leaves, uint32_t mask) {
+  return kGroupTag | (top ? kGroupTop : 0u) | ((level > 255u ? 255u : level) << 2) | (leaves << kGroupLeaf) | (mask << 16);
+}
+__device__ __forceinline__ bool is_group(uint64_t v) {
+  const uint32_t w = (uint32_t)(v >> 32);
+  return (w & kGroupTag) && (w >> kGroupLeaf);
 }
 
-// the slot of child i of a group and its entry's upper word (flags and level)
+// child i of a group as an entry (make_entry) without its instance
 __device__ __forceinline__ uint64_t group_entry(uint32_t base, uint32_t word, uint32_t i) {
   const uint32_t leaves = __builtin_amdgcn_ubfe(word, kGroupLeaf, i);  // the leaves below child i
-  const uint32_t two = (uint32_t)__builtin_amdgcn_sbfe((int)word, 0, 1) & leaves;
+  const uint32_t two = (uint32_t)__builtin_amdgcn_sbfe((int)word, 1, 1) & leaves;
   const uint32_t leaf = (word >> (kGroupLeaf + i)) & 1u;
-  return (uint64_t)(base + i + (uint32_t)__popc(two)) | ((uint64_t)((word & 0x3fdu) | (leaf << 1)) << 32);
+  return (uint64_t)(base + i + (uint32_t)__popc(two)) |
+         ((uint64_t)((word & 0x3fcu) | __builtin_amdgcn_ubfe(word, 1, 1) | (leaf << 1)) << 32);
 }
 
-template <int K, uint32_t BS, typename Spill>
-__device__ __forceinline__ void groups_save(Groups& q, lds_u64* lds, Spill&& spill) {
-  if (q.word < kGroupFirst) return;
-  const uint32_t cnt = q.state & 0xffu, out = (q.state >> 8) & 0xffu;
-  if (cnt - out == (uint32_t)K) {
-    spill()[out] = lds[(out & (K - 1)) * BS];
-    q.state += 0x100u;
+// One list's ring: `state` as in Groups, R its length, `lds` and spill() the
+// lane's words.
+template <int R, uint32_t BS, typename Spill>
+__device__ __forceinline__ void ring_put(uint32_t& state, uint64_t v, lds_u64* lds, Spill&& spill) {
+  const uint32_t cnt = state & kListItems, out = (state >> 8) & 0xffu;
+  if (cnt - out == (uint32_t)R) {
+    spill()[out] = lds[(out & (R - 1)) * BS];
+    state += 0x100u;
   }
-  lds[(cnt & (K - 1)) * BS] = (uint64_t)q.base | ((uint64_t)q.word << 32);
-  q.state++;
+  lds[(cnt & (R - 1)) * BS] = v;
+  state++;
 }
-
-// the next entry; false when nothing is left
-template <int K, uint32_t BS, typename Spill>
-__device__ __forceinline__ bool groups_pop(Groups& q, uint64_t& e, lds_u64* lds, Spill&& spill) {
-  if (q.word < kGroupFirst) {
-    const uint32_t cnt = q.state & 0xffu;
-    if (cnt == 0) return false;
-    q.state--;
-    uint64_t v;
-    if (cnt <= ((q.state >> 8) & 0xffu)) {
-      v = spill()[cnt - 1];
-      q.state -= 0x100u;
-    } else {
-      v = lds[((cnt - 1) & (K - 1)) * BS];
-    }
-    q.base = (uint32_t)v;
-    q.word = (uint32_t)(v >> 32);
+template <int R, uint32_t BS, typename Spill>
+__device__ __forceinline__ uint64_t ring_get(uint32_t& state, lds_u64* lds, Spill&& spill) {
+  const uint32_t cnt = state & kListItems;
+  state--;
+  if (cnt <= ((state >> 8) & 0xffu)) {
+    state -= 0x100u;
+    return spill()[cnt - 1];
   }
-  const uint32_t i = 15u - (uint32_t)__builtin_clz(q.word);
-  e = group_entry(q.base, q.word, i);
-  q.word ^= kGroupFirst << i;
-  q.state -= kGroupDepth;
-  return true;
+  return lds[((cnt - 1) & (R - 1)) * BS];
 }
 
 // Masks of a node's six children from its size/type bytes (22-27), one bit a
@@ -259,9 +238,12 @@ void trace_kernel(TraceParams p) {
   static_assert(!LM || (!REC && STAGE == 0 && !MULTI), "the level pass writes max_level only");
   constexpr uint32_t BS = STAGE ? 64u : 256u;
   constexpr int NS = MODE == 1 ? 2 : 1;
+  // ring length per list: staged treelet order keeps four groups, so that two
+  // more waves fit beside a CU's staging areas
+  constexpr int R = STAGE && MODE == 1 ? 4 : K;
   constexpr uint32_t UNITS = STAGE / 64;
   constexpr uint32_t HSIZE = STAGE ? 2 * UNITS : 1;
-  __shared__ uint64_t lds_stack[NS * K * BS];
+  __shared__ uint64_t lds_stack[NS * R * BS];
   __shared__ uint4 stage_img[STAGE ? STAGE / 16 : 1];
   __shared__ uint32_t hkey[HSIZE];
   __shared__ uint16_t hpos[HSIZE];
@@ -294,17 +276,21 @@ void trace_kernel(TraceParams p) {
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & 63u;
   lds_u64* ldsA = (lds_u64*)(lds_stack + tid);
-  lds_u64* ldsB = (lds_u64*)(lds_stack + (NS - 1) * K * BS + tid);
   lds_u64* ring = (lds_u64*)(rec_ring + (REC == kRecSlab ? tid : 0u));
   const uint64_t lane_slot = (uint64_t)blockIdx.x * BS + tid;
-  // The lane's spill area, formed where it is used (rarely) instead of held in
-  // two registers for the whole launch.
-  auto spill_a = [&]() -> glb_u64* {
+  bool phase2 = false;  // treelet order: the current treelet was left (the lists are one stack from then on)
+  // The lane's words of list l (0: the current one before the switch, 1: the
+  // other), and of the list that the register group belongs to.  The spill area
+  // is formed where it is used (rarely) instead of held in two registers.
+  auto lds_of = [&](bool l) -> lds_u64* { return ldsA + (MODE == 1 && l ? (uint32_t)R * BS : 0u); };
+  auto spill_of = [&](bool l) -> glb_u64* {
     uint32_t t = threadIdx.x;
     asm volatile("" : "+v"(t));
-    return (glb_u64*)(p.spill + ((uint64_t)blockIdx.x * BS + t) * (uint64_t)p.spill_cap * NS);
+    const uint32_t per = p.spill_cap + (uint32_t)(K - R);
+    return (glb_u64*)(p.spill + (((uint64_t)blockIdx.x * BS + t) * NS + (MODE == 1 && l ? 1u : 0u)) * per);
   };
-  auto spill_b = [&]() -> glb_u64* { return spill_a() + (NS - 1) * (uint64_t)p.spill_cap; };
+  auto spill_cur = [&]() -> glb_u64* { return spill_of(phase2); };
+  auto spill_other = [&]() -> glb_u64* { return spill_of(true); };
   // Scene of the lane's current ray (a batch kernel switches it per ray).
   const uint8_t* __restrict__ A = p.arena;
   uint64_t bytes = p.arena_bytes;
@@ -320,15 +306,14 @@ void trace_kernel(TraceParams p) {
     __syncthreads();
   }
 
-  Stack sa{0, 0, 0}, sb{0, 0, 0};  // treelet order
-  Groups gs{0, 0, 0};              // plain order
+  Groups gs{0, 0, 0};
+  uint32_t other = 0;  // treelet order before the switch: state of the other list
   bool active = false, exhausted = false;
   bool pending = false;  // the lane's completed ray still has to write its hit record
   uint32_t err = 0;
 
   F3 ro{}, rd{}, ridir{};
   float rtmin = 0.f, rtmax = 0.f;
-  uint32_t rflags = 0;  // treelet order (plain order keeps them in gs.state)
   float min_thit = 0.f, min_thit_obj = 0.f;
   uint32_t closest_leaf = kNoSlot, closest_inst = kNoSlot;
   ObjRay cur{};
@@ -338,7 +323,6 @@ void trace_kernel(TraceParams p) {
   uint32_t n_rec = 0, n_nodes = 0, fetch_bytes = 0, n_any = 0, max_level = 0;
   uint64_t rec_base = 0;
   uint32_t rec_flushed = 0;  // slab records: entries of the ray already in its slab
-  bool phase2 = false;
 
   // The entry a lane popped this iteration and processes below.
   bool has_e = false;
@@ -433,25 +417,43 @@ void trace_kernel(TraceParams p) {
     }
   };
 
-  auto push_entry = [&](uint64_t e, bool to_a) {
-    if constexpr (MODE == 0) {
-      // a group of one child
-      if ((gs.state & kGroupDepthMask) >= ((uint32_t)K + p.spill_cap) * kGroupDepth) {
+  const uint32_t depth_limit = ((uint32_t)K + p.spill_cap) * kListDepth;
+  auto save_group = [&]() {
+    if (gs.word >= kGroupFirst)
+      ring_put<R, BS>(gs.state, (uint64_t)gs.base | ((uint64_t)gs.word << 32), lds_of(phase2), spill_cur);
+  };
+  // Push one child, to the current list or the other one (after the switch
+  // both are the list of the register group).
+  auto push_entry = [&](uint64_t v, bool to_a) {
+    if (MODE == 0 || to_a || phase2) {
+      if ((gs.state & kListDepthMask) >= depth_limit) {
         err |= kErrStack;
         return;
       }
-      groups_save<K, BS>(gs, ldsA, spill_a);
-      gs.base = e_slot(e);
-      gs.word = group_word(e_flags(e), e_level(e), (e_flags(e) >> 1) & 1u, 1u);
-      gs.state += kGroupDepth;
-      return;
+      save_group();
+      gs.state += kListDepth;
+      if constexpr (MODE == 0) {
+        gs.base = e_slot(v);
+        gs.word = group_word(e_flags(v) & kFlTop, e_level(v), (e_flags(v) >> 1) & 1u, 1u);
+      } else {
+        gs.word = 0;
+        ring_put<R, BS>(gs.state, v, lds_of(phase2), spill_cur);
+      }
+    } else {
+      if ((other & kListDepthMask) >= depth_limit) {
+        err |= kErrStack;
+        return;
+      }
+      other += kListDepth;
+      ring_put<R, BS>(other, v, lds_of(true), spill_other);
     }
-    bool ok;
-    if (to_a)
-      ok = st_push<K, BS>(sa, e, ldsA, spill_a(), p.spill_cap);
-    else
-      ok = st_push<K, BS>(sb, e, ldsB, spill_b(), p.spill_cap);
-    if (!ok) err |= kErrStack;
+  };
+  auto list_empty = [&]() -> bool { return gs.word < kGroupFirst && (gs.state & kListItems) == 0; };
+  // current_treelet_root := host address of the moved node (:1748-1754)
+  auto leave_treelet = [&]() {
+    phase2 = true;
+    gs.state |= other;  // the current list is empty: only the ray's flags are set
+    other = 0;
   };
 
   // ---- the level pass's per-lane tree_level_map: open addressing over
@@ -689,18 +691,30 @@ void trace_kernel(TraceParams p) {
     return false;
   };
 
-  // Pop the lane's next entry into `e`; false when its stacks are empty.
+  // Pop the lane's next entry into `e`; false when its lists are empty.
   auto pop_next = [&]() -> bool {
-    if constexpr (MODE == 0) {
-      if (!groups_pop<K, BS>(gs, e, ldsA, spill_a)) return false;
-    } else if (st_empty(sa) && st_empty(sb)) {
-      return false;
-    } else if (!st_empty(sa)) {
-      e = st_pop<K, BS>(sa, ldsA, spill_a());
-    } else {
-      phase2 = true;  // current_treelet_root := host address of the moved node (:1748-1754)
-      e = st_pop<K, BS>(sb, ldsB, spill_b());
+    bool whole = false;
+    if (gs.word < kGroupFirst) {
+      if ((gs.state & kListItems) == 0) {
+        if (MODE == 0 || (other & kListItems) == 0) return false;
+        leave_treelet();
+      }
+      const uint64_t v = ring_get<R, BS>(gs.state, lds_of(phase2), spill_cur);
+      if (MODE == 1 && !is_group(v)) {
+        e = v;
+        whole = true;
+      } else {
+        gs.base = (uint32_t)v;
+        gs.word = (uint32_t)(v >> 32);
+      }
     }
+    if (!whole) {
+      const uint32_t i = 15u - (uint32_t)__builtin_clz(gs.word);
+      e = group_entry(gs.base, gs.word, i);
+      if (MODE == 1 && !(gs.word & kGroupTop)) e |= (uint64_t)((cur_inst - (uint32_t)(tlas >> 6)) << 10) << 32;
+      gs.word ^= kGroupFirst << i;
+    }
+    gs.state -= kListDepth;
     // every processed entry emits at least one record
     if (n_rec > kMaxStepsPerRay) err |= kErrSteps;
     return true;
@@ -827,7 +841,6 @@ void trace_kernel(TraceParams p) {
           rtmin = __uint_as_float(r0.w);
           rd = mk3(__uint_as_float(r1.x), __uint_as_float(r1.y), __uint_as_float(r1.z));
           rtmax = __uint_as_float(r1.w);
-          rflags = r2.x;
           ridir = calc_idir(rd);
           ray_ok = slab_inputs_ok(ro, rd, ridir, rtmin, rtmax);
           octant = (rd.x < 0.f ? 1u : 0u) | (rd.y < 0.f ? 2u : 0u) | (rd.z < 0.f ? 4u : 0u);
@@ -840,10 +853,9 @@ void trace_kernel(TraceParams p) {
           rec_flushed = 0;
           max_level = 1;  // tree_level_map[topRootAddr] = 1
           if constexpr (REC == kRecCsr) rec_base = p.record_offsets[r];
-          sa = Stack{0, 0, 0};
-          sb = Stack{0, 0, 0};
-          gs = Groups{0, 0, ((r2.x & RTX_RAY_FLAG_OPAQUE) ? kGroupOpaque : 0u) |
-                                ((r2.x & RTX_RAY_FLAG_TERMINATE_ON_FIRST_HIT) ? kGroupTerminate : 0u)};
+          gs = Groups{0, 0, ((r2.x & RTX_RAY_FLAG_OPAQUE) ? kRayOpaque : 0u) |
+                                ((r2.x & RTX_RAY_FLAG_TERMINATE_ON_FIRST_HIT) ? kRayTerminate : 0u)};
+          other = 0;
           phase2 = false;
           err = 0;
           // TLAS header record and bounds test (vulkan_ray_tracing.cc:2444-2484)
@@ -1044,8 +1056,8 @@ void trace_kernel(TraceParams p) {
               // when it joins the current list, or the other list while the
               // current one is empty (that pop starts phase 2).  Such a root is
               // tested in this iteration's internal-node pass instead.
-              if (err == 0 && (MODE == 0 || to_a || st_empty(sa))) {
-                if (MODE == 1 && !to_a) phase2 = true;  // current_treelet_root := host address (:1748-1754)
+              if (err == 0 && (MODE == 0 || to_a || phase2 || list_empty())) {
+                if (MODE == 1 && !to_a && !phase2) leave_treelet();
                 e = make_entry(rs, 0u, level, irel);
                 inner = true;
               } else {
@@ -1072,7 +1084,7 @@ void trace_kernel(TraceParams p) {
             bool accept;
             if (MODE == 0) {
               accept = h && rtmin <= wt && wt <= rtmax;
-              if (accept && (gs.state & kGroupOpaque) && wt < min_thit) min_thit = th / cur.tmult;
+              if (accept && (gs.state & kRayOpaque) && wt < min_thit) min_thit = th / cur.tmult;
             } else {
               accept = h && rtmin <= wt && wt <= rtmax && wt < min_thit;
               if (accept) min_thit = th / cur.tmult;
@@ -1083,11 +1095,10 @@ void trace_kernel(TraceParams p) {
               closest_inst = cur_inst;
               emit(off, 64, RTX_TX_BVH_QUAD_LEAF_HIT, level);
               n_nodes++;
-              if (MODE == 0 && !(gs.state & kGroupOpaque)) n_any++;
-              if (MODE == 0 ? (gs.state & kGroupTerminate) : (rflags & RTX_RAY_FLAG_TERMINATE_ON_FIRST_HIT)) {
-                sa = Stack{0, 0, 0};
-                sb = Stack{0, 0, 0};
-                gs = Groups{0, 0, gs.state & (kGroupOpaque | kGroupTerminate)};
+              if (MODE == 0 && !(gs.state & kRayOpaque)) n_any++;
+              if (gs.state & kRayTerminate) {
+                gs = Groups{0, 0, gs.state & (kRayOpaque | kRayTerminate)};
+                other = 0;
               }
             } else {
               emit(off, 64, RTX_TX_BVH_QUAD_LEAF, level);
@@ -1245,86 +1256,57 @@ void trace_kernel(TraceParams p) {
               const uint32_t inst = top ? 0u : e_inst_rel(e);
               const uint32_t base_flags = top ? kFlTop : 0u;
               bool pushed = false;
-              if constexpr (MODE == 0 && !LM) {
-                // Plain order in a scene of regular nodes: the hit children are
-                // one group, without the first internal one, which is the
-                // lane's next entry.  No child needs a check here: the scene
-                // walk placed all of them in the arena.
+              if constexpr (!LM) {
+                // A scene of regular nodes: the hit children of a list are one
+                // group, without the one that its next pop would take.  No child
+                // needs a check here: the scene walk placed all of them in the
+                // arena.
                 if (p.regular_nodes) {
                   pushed = true;
-                  const uint32_t n_push = (uint32_t)__popc(hitmask);
-                  if ((gs.state & kGroupDepthMask) + n_push * kGroupDepth > ((uint32_t)K + p.spill_cap) * kGroupDepth) {
+                  const uint32_t mine = MODE == 0 || phase2 ? hitmask : hitmask & fbits;  // to the register group's list
+                  const uint32_t theirs = hitmask & ~mine;
+                  const uint32_t d_mine = (uint32_t)__popc(mine) * kListDepth, d_theirs = (uint32_t)__popc(theirs) * kListDepth;
+                  if ((gs.state & kListDepthMask) + d_mine > depth_limit ||
+                      (MODE == 1 && (other & kListDepthMask) + d_theirs > depth_limit)) {
                     err |= kErrStack;
                   } else {
                     const uint32_t leaves = kids_leaves(kids);
-                    const uint32_t word = group_word(base_flags, lvl, leaves, 0u);
+                    const uint32_t word = group_word(top, lvl, leaves, 0u);
                     const uint32_t first = slot + nd.w[3];
-                    const uint32_t im = hitmask & ~leaves;
-                    const uint32_t rest = hitmask & ~(im & (0u - im));
-                    gs.state += n_push * kGroupDepth;
-                    if (rest) {
-                      groups_save<K, BS>(gs, ldsA, spill_a);
-                      gs.base = first;
-                      gs.word = word | (rest << 16);
+                    uint32_t next;  // one bit
+                    if (MODE == 0) {
+                      const uint32_t im = mine & ~leaves;
+                      next = im & (0u - im);
+                    } else {
+                      next = mine ? 0x80000000u >> __builtin_clz(mine) : 0u;
                     }
-                    if (im) {
-                      e = group_entry(first, word, (uint32_t)__builtin_ctz(im));
+                    if (MODE == 0 || phase2 || top) {
+                      const uint32_t rest = mine & ~next;
+                      if (rest) {
+                        save_group();
+                        gs.base = first;
+                        gs.word = word | (rest << 16);
+                      }
+                      gs.state += d_mine;
+                      if (MODE == 1 && theirs) {
+                        ring_put<R, BS>(other, (uint64_t)first | ((uint64_t)(word | (theirs << 16)) << 32), lds_of(true),
+                                        spill_other);
+                        other += d_theirs;
+                      }
+                    } else {
+                      for (uint32_t m = hitmask & ~next; m; m &= m - 1) {
+                        const uint32_t i = (uint32_t)__builtin_ctz(m);
+                        push_entry(group_entry(first, word, i) | ((uint64_t)inst << 42), (mine >> i) & 1u);
+                      }
+                      gs.state += next ? kListDepth : 0u;
+                    }
+                    if (next) {
+                      e = group_entry(first, word, (uint32_t)__builtin_ctz(next)) | ((uint64_t)inst << 42);
                       has_e = true;
-                      gs.state -= kGroupDepth;
+                      gs.state -= kListDepth;
                       if (n_rec > kMaxStepsPerRay) err |= kErrSteps;
                     }
                   }
-                }
-              } else if constexpr (MODE == 1 && !LM) {
-                // Treelet order, same conditions: the children go in slot
-                // order, a child owned by the first treelet to the current
-                // list (A), the others to list B.  Each list first spills its
-                // ring's oldest entries, as many as pushing one by one would
-                // (at most K new entries per list, so new ones never spill
-                // each other), then stores each child at its place.
-                const uint32_t iw0 = __builtin_amdgcn_alignbyte(nd.w[6], nd.w[5], 2);
-                const uint32_t iw1 = nd.w[6] >> 16;
-                uint32_t pre[6], tot = 0, leafm = 0;
-#pragma unroll
-                for (int i = 0; i < 6; ++i) {
-                  const uint32_t info = (i < 4 ? iw0 >> (8 * i) : iw1 >> (8 * (i - 4))) & 0x3fu;
-                  pre[i] = tot;
-                  tot += info & 3u;
-                  leafm |= (info >> 2) != 0u ? 1u << i : 0u;
-                }
-                const uint32_t pmA = hitmask & fbits, pmB = hitmask & ~fbits;
-                const uint32_t nA = (uint32_t)__builtin_popcount(pmA), nB = (uint32_t)__builtin_popcount(pmB);
-                const uint32_t spA = sa.cnt + nA > (uint32_t)K ? sa.cnt + nA - (uint32_t)K : 0u;
-                const uint32_t spB = sb.cnt + nB > (uint32_t)K ? sb.cnt + nB - (uint32_t)K : 0u;
-                const bool ok = first_child < bytes && first_child + (uint64_t)tot * 64 <= bytes &&
-                                !(top && ((iw0 & 0x38383838u) | (iw1 & 0x3838u)) != 0u) && nA <= (uint32_t)K &&
-                                nB <= (uint32_t)K && sa.g + spA <= p.spill_cap && sb.g + spB <= p.spill_cap;
-                if (ok) {
-                  pushed = true;
-                  const uint32_t first_slot = (uint32_t)(first_child >> 6);
-                  const uint32_t hi = base_flags | ((lvl > 255u ? 255u : lvl) << 2) | ((inst & 0x3fffffu) << 10);
-                  auto spill_list = [&](Stack& st, lds_u64* lds, glb_u64* g, uint32_t sp) {
-                    for (uint32_t j = 0; j < sp; ++j) {
-                      g[st.g++] = lds[st.bot * BS];
-                      st.bot = (st.bot + 1) & (K - 1);
-                      st.cnt--;
-                    }
-                  };
-                  if (spA) spill_list(sa, ldsA, spill_a(), spA);
-                  if (spB) spill_list(sb, ldsB, spill_b(), spB);
-                  // one store per hit child, into the list it goes to
-                  const uint32_t topA = sa.bot + sa.cnt, topB = sb.bot + sb.cnt;
-#pragma unroll
-                  for (int i = 0; i < 6; ++i) {
-                    if ((hitmask >> i) & 1u) {
-                      const bool a = (fbits >> i) & 1u;
-                      const uint32_t r = (uint32_t)__builtin_popcount((a ? pmA : pmB) & ((1u << i) - 1u));
-                      (a ? ldsA : ldsB)[(((a ? topA : topB) + r) & (K - 1)) * BS] =
-                          (uint64_t)(first_slot + pre[i]) | ((uint64_t)(hi | (((leafm >> i) & 1u) ? kFlLeaf : 0u)) << 32);
-                    }
-                  }
-                  sa.cnt += nA;
-                  sb.cnt += nB;
                 }
               }
               int deferred = -1;
@@ -1543,7 +1525,7 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
       }
       save_group();
       gs.base = e_slot(v);
-      gs.word = group_word(e_flags(v), e_level(v), (e_flags(v) >> 1) & 1u, 1u);
+      gs.word = group_word(e_flags(v) & kFlTop, e_level(v), (e_flags(v) >> 1) & 1u, 1u);
       depth++;
       return;
     }
@@ -1902,7 +1884,7 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
               err |= kErrStack;
             } else {
               const uint32_t leaves = (uint32_t)(__ballot(j < 6u && (info >> 2) != 0u) >> gbase) & 0x3fu;
-              const uint32_t word = group_word(base_flags, lvl, leaves, 0u);
+              const uint32_t word = group_word(top, lvl, leaves, 0u);
               const uint32_t first = slot + nd.w[3];
               const uint32_t im = hitmask & ~leaves;
               const uint32_t rest = hitmask & ~(im & (0u - im));
@@ -1950,7 +1932,7 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
             const uint32_t fit = min(n, cap - depth);
             if (pushed && pos < fit)
               sta[da + pos] = (uint64_t)(uint32_t)(c >> 6) |
-                              ((uint64_t)group_word(base_flags, lvl, leaf ? 1u : 0u, 1u) << 32);
+                              ((uint64_t)group_word(top, lvl, leaf ? 1u : 0u, 1u) << 32);
             da += fit;
             depth += fit;
             if (fit < n) err |= kErrStack;
