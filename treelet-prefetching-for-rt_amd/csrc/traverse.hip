@@ -803,7 +803,7 @@ void trace_kernel(TraceParams p) {
       const uint32_t leader = (uint32_t)__ffsll((long long)idle) - 1u;
       uint32_t base = 0;
       if (lane == leader) base = atomicAdd(p.ray_counter, nidle);
-      base = __shfl(base, (int)leader, 64);
+      base = (uint32_t)__builtin_amdgcn_readlane((int)base, (int)leader);
       if ((uint64_t)base + nidle >= p.n) exhausted = true;
       if (!active) {
         const uint32_t k = base + lanes_below(idle);
@@ -931,15 +931,16 @@ void trace_kernel(TraceParams p) {
           // treelet of every lane's next node is counted, and the most
           // popular one wins, ties going to the lowest root offset (the
           // ordered map's first maximum; dense treelet indices follow root
-          // offsets).  Each round takes one distinct treelet, so the loop
-          // ends after at most 64 rounds.
+          // offsets).  Each round takes one distinct treelet, and the loop ends
+          // when fewer lanes remain than the best count.  The candidate is read
+          // by lane number (one v_readlane; a shuffle goes through LDS).
           const uint32_t own = (want && off + 64 <= bytes) ? owner[slot] : kNone;
           uint64_t rem = __ballot(own != kNone);
           const uint32_t voters = (uint32_t)__popcll(rem);
           uint32_t best = kNone, bestc = 0;
-          while (rem) {
+          while (rem && (uint32_t)__popcll(rem) >= bestc) {
             const uint32_t lead = (uint32_t)__ffsll((long long)rem) - 1u;
-            const uint32_t cand = __shfl(own, (int)lead, 64);
+            const uint32_t cand = (uint32_t)__builtin_amdgcn_readlane((int)own, (int)lead);
             const uint64_t m = __ballot(own == cand);
             const uint32_t cnt = (uint32_t)__popcll(m);
             if (cnt > bestc || (cnt == bestc && cand < best)) {
@@ -981,7 +982,7 @@ void trace_kernel(TraceParams p) {
               const uint64_t has = __ballot(mine != 0);
               if (has == 0) break;
               const uint32_t lead = (uint32_t)__ffsll((long long)has) - 1u;
-              const uint32_t cand = __shfl(mine, (int)lead, 64) & 0xffffffu;
+              const uint32_t cand = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)lead) & 0xffffffu;
               float sc = 0.f;
               for (int k = 0; k < 4; ++k)
                 if (ent[k] != 0 && (ent[k] & 0xffffffu) == cand) {
