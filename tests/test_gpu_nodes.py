@@ -69,3 +69,47 @@ def test_unusual_nodes_match_the_oracle(gpu, oracle, instanced, mode, change):
         assert_records_equal(o, r, o_ref, r_ref, f"stack {stack}")
     for lanes in (1, 8):
         assert_hits_equal(gpu.trace(rays, mode=mode, lanes_per_ray=lanes), h_ref, f"{lanes} lanes")
+
+
+def _corner_rays(arena, nodes, rays, rng, far):
+    """Rays through corners of child boxes, where entry and exit distances meet: world-space
+    aims at TLAS children and at points of BLAS boxes, from near and from far away."""
+    f32 = np.float32
+    out = rays[rng.integers(0, len(rays), 4096)].copy()
+    for k in range(len(out)):
+        off = nodes[rng.integers(0, len(nodes))] if k % 2 else nodes[0]
+        origin = arena[off:off + 12].view(f32)
+        i = rng.integers(0, 6)
+        corner = [origin[a] + f32(np.ldexp(float(arena[off + 28 + 12 * a + 6 * rng.integers(0, 2) + i]),
+                                           int(arena[off + 18 + a:off + 19 + a].view(np.int8)[0]) - 8)) for a in range(3)]
+        corner = np.array(corner, f32)
+        d = rng.normal(size=3)
+        kind = k % 7
+        if kind < 2:  # parallel to an axis, or nearly so
+            d[rng.permutation(3)[:2]] *= 0.0 if kind else 1e-6
+        d = (d / np.linalg.norm(d)).astype(f32)
+        o = (corner - d * f32(far * rng.uniform(0.5, 2.0))).astype(f32)
+        if kind == 2:  # start on the plane
+            o = corner.copy()
+        out[k]["org"] = o
+        out[k]["dir"] = d
+        out[k]["tmin"] = 0.0
+        out[k]["tmax"] = [np.inf, 4.0 * far, np.nan, -np.inf, far, 1e30, 0.0][kind]
+    return out
+
+
+@pytest.mark.parametrize("far", [1e-3, 1.0, 50.0, 1e5, 1e12, 1e30])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_rays_through_box_corners_match_the_oracle(gpu, oracle, instanced, mode, far):
+    scene, rays = instanced
+    arena = scene.arena
+    nodes = _internal_nodes(arena, scene.tlas_offset)
+    rays = _corner_rays(arena, nodes, rays, np.random.default_rng(9), far)
+    part = oracle.Partition(arena, scene.tlas_offset, 1024)
+    h_ref, o_ref, r_ref = oracle.trace(arena, scene.tlas_offset, rays, mode=mode, partition=part)
+    gpu.set_scene(arena, scene.tlas_offset)
+    gpu.build_treelets(1024)
+    h, o, r = gpu.trace(rays, mode=mode, records=True)
+    assert_hits_equal(h, h_ref, "records")
+    assert_records_equal(o, r, o_ref, r_ref, "records")
+    assert_hits_equal(gpu.trace(rays, mode=mode, lanes_per_ray=1), h_ref, "hits")
