@@ -190,9 +190,10 @@ typedef struct rtx_trace_options {
                              (vulkan_ray_tracing.cc:2446-2450, 2509-2512); RTX_NO_NODE for a node
                              placed nowhere.  Needs the layout (else RTX_ERR_NO_PARTITION) */
   uint32_t record_slab;  /* records, one traversal: each ray's first record_slab records (at most
-                            1024; 0 = 256) go to a per-ray slab in library memory and are compacted
-                            into the caller's CSR buffer; only rays with more records are traced a
-                            second time.  The slabs (8 bytes per record) take at most 16 GiB: a
+                            1024; 0 = 512 in 4-byte entries, 256 where the scene needs 8-byte ones)
+                            go to a per-ray slab in library memory and are expanded into the
+                            caller's CSR buffer; only rays with more records are traced a second
+                            time.  The slabs take at most 2^31 entries (16 GiB of 8 bytes): a
                             batch that needs more is traced in consecutive ray ranges that fit; with
                             a claim_order or staging it takes a counting pass and a writing pass
                             instead */

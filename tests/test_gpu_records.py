@@ -1,0 +1,67 @@
+"""Records out of their slabs: row lengths around the two arrays of a slab, batch
+sizes around the one-launch limit, short rays (many per chunk of records), and
+scenes with 4-byte and with 8-byte slab entries.  Exact by contract, so equal to
+the oracle's bit for bit."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+from conftest import assert_hits_equal, assert_records_equal
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden"))
+import tiny_scene  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+def _rays(rtx, rays, n, short, seed):
+    """n of the rays in a random order; `short` of them turned away (one record each) in runs."""
+    rng = np.random.default_rng(seed)
+    out = rays[rng.integers(0, len(rays), n)].copy()
+    away = np.zeros(n, bool)
+    for at in rng.integers(0, n, max(1, int(short * n) // 200)) if short else []:
+        away[at:at + 200] = True
+    out["org"][away] = 1e6
+    out["dir"][away] = (0.0, 0.0, 1.0)
+    return out
+
+
+def _two_depth_rays(rtx, n, seed):
+    rng = np.random.default_rng(seed)
+    r = np.zeros(n, dtype=rtx.RAY_DTYPE)
+    r["org"][:, :2] = rng.uniform(-1.2, 3.2, (n, 2))
+    r["dir"] = (0.0, 0.0, 1.0)
+    r["tmax"] = rng.choice([100.0, 4.5, 2.5], n)
+    r["cull_mask"] = 0xFF
+    return r
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("n,short,slab", [(1, 0, 0), (255, 0.5, 31), (256, 0, 32), (257, 0, 33), (8192, 0.5, 40),
+                                          (8193, 0.5, 0), (9217, 0.9, 8), (12000, 1.0, 100)])
+def test_records_at_slab_and_batch_edges(gpu, rtx, oracle, instanced, mode, n, short, slab):
+    scene, rays = instanced
+    rays = _rays(rtx, rays, n, short, n)
+    part = oracle.Partition(scene.arena, scene.tlas_offset, 1024)
+    h_ref, o_ref, r_ref = oracle.trace(scene.arena, scene.tlas_offset, rays, mode=mode, partition=part)
+    gpu.set_scene(scene.arena, scene.tlas_offset)
+    gpu.build_treelets(1024)
+    h, o, r = gpu.trace(rays, mode=mode, records=True, record_slab=slab)
+    assert_hits_equal(h, h_ref, "hits")
+    assert_records_equal(o, r, o_ref, r_ref, "records")
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("n,slab", [(100, 0), (8192, 5), (8193, 0), (20000, 9)])
+def test_records_of_a_scene_with_two_levels_per_node(gpu, rtx, oracle, mode, n, slab):
+    arena = tiny_scene.tiny_two_depth_arena()
+    rays = _two_depth_rays(rtx, n, n)
+    part = oracle.Partition(arena, 0, 8192)
+    h_ref, o_ref, r_ref = oracle.trace(arena, 0, rays, mode=mode, partition=part)
+    gpu.set_scene(arena, 0)
+    gpu.build_treelets(8192)
+    h, o, r = gpu.trace(rays, mode=mode, records=True, record_slab=slab)
+    assert_hits_equal(h, h_ref, "hits")
+    assert_records_equal(o, r, o_ref, r_ref, "records")

@@ -24,10 +24,10 @@ using namespace rtxk;
 // bytes of the control block cleared before and read after a traversal
 static constexpr uint32_t kSlots = 64;
 // words of the mapped host block (err_host, 16 words): word 0 is the ray-error
-// flag, words kReportWord.. receive launch_report_words
+// flag, words kReportWord.. the records' total and the overflowed rays
 static constexpr uint32_t kReportWord = 8;
-// most device memory the per-ray record slabs (8 bytes per record) may take
-static constexpr uint64_t kSlabBytesMax = 16ull << 30;
+// most entries the per-ray record slabs may take (16 GiB of 8-byte entries)
+static constexpr uint64_t kSlabEntriesMax = 2ull << 30;
 
 // most coherence scratch a context keeps (ten million rays)
 static constexpr size_t kCoherenceKept = 256ull << 20;
@@ -51,6 +51,8 @@ struct rtx_ctx {
   // every reachable node has one tree level (scene_check); otherwise hits take
   // their max_level from the level pass
   bool levels_consistent = false;
+  // slab records: slot bits of the 4-byte entries, 0 when the scene needs 8-byte ones
+  uint32_t rec_level_shift = 0;
   // partition
   Partition part;
   // scratch
@@ -170,6 +172,17 @@ void free_scene(rtx_ctx* c) {
   c->ordered = false;
   c->regular = false;
   c->levels_consistent = false;
+  c->rec_level_shift = 0;
+}
+
+// Slot bits of a scene's 4-byte slab entries: levels known beforehand, and slots
+// and levels in 29 bits together; else 0 (8-byte entries).
+uint32_t slab4_shift(const SceneCheck& ck, uint64_t bytes) {
+  if (!ck.valid || !ck.level_consistent || ck.max_level > 255) return 0;
+  uint32_t slot_bits = 1, level_bits = 1;
+  while (slot_bits < 32 && (bytes / 64 - 1) >> slot_bits) slot_bits++;
+  while (ck.max_level >> level_bits) level_bits++;
+  return slot_bits + level_bits <= kSlab4TypeShift ? slot_bits : 0;
 }
 
 rtx_status ensure_spill(rtx_ctx* c, size_t entries) {
@@ -511,6 +524,7 @@ rtx_status rtx_set_scene(rtx_ctx* c, const void* host, size_t bytes, uint64_t tl
   c->ordered = ck.valid && ck.ordered;
   c->regular = ck.valid && ck.regular;
   c->levels_consistent = ck.valid && ck.level_consistent;
+  c->rec_level_shift = slab4_shift(ck, bytes);
   return RTX_OK;
 }
 
@@ -531,6 +545,7 @@ rtx_status rtx_set_scene_device(rtx_ctx* c, const void* dev, size_t bytes, uint6
   c->ordered = ck.valid && ck.ordered;
   c->regular = ck.valid && ck.regular;
   c->levels_consistent = ck.valid && ck.level_consistent;
+  c->rec_level_shift = slab4_shift(ck, bytes);
   return RTX_OK;
 }
 
@@ -662,19 +677,24 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
   if (opts->lanes_per_ray != 0 && opts->lanes_per_ray != 1 && opts->lanes_per_ray != kWideRayLanes)
     return RTX_ERR_INVALID_ARGUMENT;
   const bool wide_ok = !opts->emit_records && stage == 0;
-  // records in one traversal: per-ray slabs of `slab` records (default 256: a
-  // 1M-triangle diffuse batch has at most about 210 per ray), compacted into the
-  // caller's CSR buffer; only rays with more records are traced again.  The
-  // slabs take at most 16 GiB: a larger batch is traced in consecutive ray
+  // records in one traversal: per-ray slabs of `slab` records, compacted into the
+  // caller's CSR buffer; only rays with more records are traced again, which
+  // costs such a ray's whole latency (a 1M-triangle diffuse batch has some of 300
+  // records: 250 us).  Default 512 in 4-byte entries (scenes whose slots and levels
+  // fit them, see slab4_shift), 256 in 8-byte ones and for batches that only fit
+  // so.  The slabs take at most 2^31 entries: a larger batch is traced in consecutive ray
   // ranges that fit, each compacted before the next reuses the slabs.  With a
   // claim order or staging such a batch takes a counting pass and a writing
   // pass instead.
-  const uint32_t slab = opts->record_slab ? opts->record_slab : 256;
-  const uint64_t chunk_rays = std::max<uint64_t>(1, kSlabBytesMax / ((uint64_t)slab_stride(slab) * sizeof(uint64_t)));
+  const bool long_rows = c->rec_level_shift != 0 && stage == 0 && (uint64_t)n * 512 <= kSlabEntriesMax;
+  const uint32_t slab = opts->record_slab ? opts->record_slab : long_rows ? 512 : 256;
+  const uint64_t chunk_rays = std::max<uint64_t>(1, kSlabEntriesMax / slab_stride(slab));
   const bool use_slab = opts->emit_records && ((uint64_t)n <= chunk_rays || (!opts->claim_order && stage == 0));
   const uint32_t per_chunk = (uint32_t)std::min<uint64_t>(n, chunk_rays);
   const uint32_t n_chunks = use_slab ? (n + per_chunk - 1) / per_chunk : 1;
-  const int main_rec = !opts->emit_records ? kRecNone : use_slab ? kRecSlab : kRecNone;
+  // (staged kernels write 8-byte entries)
+  const uint32_t shift4 = use_slab && stage == 0 ? c->rec_level_shift : 0;
+  const int main_rec = !use_slab ? kRecNone : shift4 ? kRecSlab4 : kRecSlab;
   if (opts->lanes_per_ray == kWideRayLanes && !wide_ok) return RTX_ERR_INVALID_ARGUMENT;
   const bool wide = wide_ok && (opts->lanes_per_ray == kWideRayLanes ||
                                 (opts->lanes_per_ray == 0 &&
@@ -691,8 +711,8 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
   grid = std::max(grid, 1u);
   const uint32_t spill_cap = 128;
   const uint32_t ns = opts->mode == RTX_MODE_TREELET ? 2 : 1;
-  // staged treelet order keeps fewer entries in LDS (trace_kernel's R)
-  rtx_status st = ensure_spill(c, (size_t)grid * bs * (spill_cap + (stage ? lds_stack : 0)) * ns);
+  // treelet order with staging or records keeps fewer entries in LDS (trace_kernel's R)
+  rtx_status st = ensure_spill(c, (size_t)grid * bs * (spill_cap + (stage || use_slab ? lds_stack : 0)) * ns);
   if (st != RTX_OK) return st;
 
   TraceParams p{};
@@ -766,23 +786,24 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
   };
   c->kernel_timed = false;
   if (use_slab) {
-    st = ensure_buffer(c->slabs, c->slab_entries, (size_t)per_chunk * slab_stride(slab));
+    st = ensure_buffer(c->slabs, c->slab_entries, (size_t)per_chunk * slab_stride(slab) / (shift4 ? 2 : 1));
     if (st != RTX_OK) return st;
     st = ensure_buffer(c->rec_counts, c->rec_count_entries, (size_t)n);
     if (st != RTX_OK) return st;
     st = ensure_buffer(c->overflow_list, c->overflow_entries, (size_t)n);
     if (st != RTX_OK) return st;
     p.slabs = c->slabs;
+    p.slabs_rest = c->slabs + (size_t)per_chunk * slab_front(slab) / (shift4 ? 2 : 1);
     p.record_slab = slab;
+    p.rec_level_shift = shift4;
     p.rec_counts = c->rec_counts;
   }
-  // scan tiles of the largest scanned range, and one word for a range's base offset
+  // scan tiles of the largest scanned range
   const uint32_t scan_n = use_slab ? per_chunk : n;
   if (opts->emit_records) {
-    st = ensure_scan_tmp(c, (size_t)(scan_n + 1023) / 1024 + 2);
+    st = ensure_scan_tmp(c, (size_t)(scan_n + 1023) / 1024 + 1);
     if (st != RTX_OK) return st;
   }
-  uint64_t* const base_word = opts->emit_records ? c->scan_tmp + (scan_n + 1023) / 1024 + 1 : nullptr;
   st = use_slot();
   if (st != RTX_OK) return st;
   uint32_t* main_slot = p.ray_counter;
@@ -801,17 +822,27 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
     q.rec_counts = c->rec_counts + b;
     if (b > 0) HIP_TRY(launch_fill_zero(main_slot, 1, c->stream));
     const uint32_t gq = std::max(1u, (uint32_t)std::min<uint64_t>(grid, ((uint64_t)(e - b) + bs - 1) / bs));
-    HIP_TRY(launch_trace(q, opts->mode, kRecSlab, lds_stack, stage, gq, c->stream));
+    HIP_TRY(launch_trace(q, opts->mode, main_rec, lds_stack, stage, gq, c->stream));
     if (last) HIP_TRY(hipEventRecord(c->evk1, c->stream));
-    if (b == 0)
-      HIP_TRY(launch_fill_zero(reinterpret_cast<uint32_t*>(base_word), 2, c->stream));
-    else
-      HIP_TRY(hipMemcpyAsync(base_word, offsets + b, sizeof(uint64_t), hipMemcpyDeviceToDevice, c->stream));
-    HIP_TRY(launch_scan_records(nullptr, c->rec_counts + b, e - b, offsets + b, c->scan_tmp, c->stream));
-    if (b > 0) HIP_TRY(launch_add_offset(offsets + b, (uint64_t)(e - b) + 1, base_word, c->stream));
-    // the kernel copies nothing when the running total exceeds the capacity
-    HIP_TRY(launch_compact_records(c->rec_counts + b, e - b, c->slabs, slab, p.owner, p.layout_remap, offsets + b,
-                                   records, records ? capacity : 0, b, c->overflow_list, main_slot + 2, c->stream));
+    FinishParams f{};
+    f.counts = c->rec_counts + b;
+    f.n = e - b;
+    f.slab = slab;
+    f.slabs = p.slabs;
+    f.slabs_rest = p.slabs_rest;
+    f.shift = shift4;
+    f.add_base = b > 0;
+    f.owner = p.owner;
+    f.layout_remap = p.layout_remap;
+    f.slots = c->arena_bytes / 64;
+    f.offsets = offsets + b;
+    f.records = records;
+    f.capacity = records ? capacity : 0;
+    f.ray_base = b;
+    f.overflow_list = c->overflow_list;
+    f.overflow_count = main_slot + 2;
+    f.host = last ? c->err_host_dev + kReportWord : nullptr;
+    HIP_TRY(launch_finish_records(f, c->scan_tmp, c->stream));
     return RTX_OK;
   };
   // the timed span: the traversal launch (from the first range's to the end of the last range's)
@@ -833,11 +864,12 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
   unsigned long long stats[11] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   if (stage) HIP_TRY(hipMemcpyAsync(stats, p.stats, sizeof(stats), hipMemcpyDeviceToHost, c->stream));
   if (opts->emit_records) {
-    if (!use_slab) HIP_TRY(launch_scan_records(hits, nullptr, n, offsets, c->scan_tmp, c->stream));
     // the rays the writing pass traces (slab overflows) and the records'
-    // total, through mapped host words
-    HIP_TRY(launch_report_words(use_slab ? main_slot + 2 : nullptr, offsets + n, c->err_host_dev + kReportWord,
-                                c->stream));
+    // total come through mapped host words
+    if (!use_slab) {
+      HIP_TRY(launch_scan_records(hits, n, offsets, c->scan_tmp, c->stream));
+      HIP_TRY(launch_report_total(offsets + n, c->err_host_dev + kReportWord, c->stream));
+    }
     HIP_TRY(hipStreamSynchronize(c->stream));
     st = launch_error();
     if (st != RTX_OK) return st;

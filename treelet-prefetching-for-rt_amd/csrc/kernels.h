@@ -23,7 +23,8 @@ enum : uint32_t {
 enum : int {
   kRecNone = 0,  // hits only
   kRecCsr = 1,   // records at record_offsets[ray]
-  kRecSlab = 2   // a ray's first record_slab records at ray * slab_stride(record_slab)
+  kRecSlab = 2,   // a ray's first record_slab records as slab entries
+  kRecSlab4 = 3   // the same in 4-byte entries
 };
 
 constexpr uint32_t kBlock = 256;        // threads per block (4 waves of 64)
@@ -56,10 +57,12 @@ struct TraceParams {
   rtx_record* records;
   uint64_t record_capacity;
   const uint64_t* record_offsets;
-  // slab records: ray r's first record_slab records as 8-byte slab entries at
-  // slabs[r * slab_stride(record_slab)] (`records` unused)
+  // slab records: ray r's first record_slab records as slab entries of 8 bytes (4
+  // with kRecSlab4), at slab_place() of the two arrays (`records` unused)
   uint64_t* slabs;
+  uint64_t* slabs_rest;
   uint32_t record_slab;
+  uint32_t rec_level_shift;  // kRecSlab4: the entries' slot bits
   uint32_t* rec_counts;    // slab records: ray r's record count at rec_counts[r]
   // level pass: per lane a tree_level_map of lm_cap u64 entries (zero between
   // rays) at lm_table + lane * lm_cap, and lm_cap / 2 positions at lm_list
@@ -142,13 +145,11 @@ constexpr uint64_t level_pass_lane_bytes(uint32_t lm_cap) { return (uint64_t)lm_
 constexpr uint32_t kLevelMapCap = 4096;  // map entries per lane: at most 2,048 nodes assigned per ray
 // Clears `words` 32-bit words with a kernel (usable inside graph capture).
 hipError_t launch_fill_zero(uint32_t* dst, uint32_t words, hipStream_t s);
-// host[0] = *word, host[2..3] = *dword (host: mapped host memory), so that the
-// caller reads both after a stream synchronisation without a copy each.
-hipError_t launch_report_words(const uint32_t* word, const uint64_t* dword, uint32_t* host, hipStream_t s);
-// CSR offsets[0..n] of the rays' record counts: hits[i].n_records, or
-// counts[i] when `counts` is given.
-hipError_t launch_scan_records(const rtx_hit* hits, const uint32_t* counts, uint32_t n, uint64_t* offsets,
-                               uint64_t* block_tmp, hipStream_t s);
+// host[2..3] = *total (host: mapped host memory), so that the caller reads it
+// after a stream synchronisation without a copy.
+hipError_t launch_report_total(const uint64_t* total, uint32_t* host, hipStream_t s);
+// CSR offsets[0..n] of the rays' record counts (hits[i].n_records).
+hipError_t launch_scan_records(const rtx_hit* hits, uint32_t n, uint64_t* offsets, uint64_t* block_tmp, hipStream_t s);
 // Statistics of a traced batch: acc[0..6] records per type, [7] hits, [8] any
 // hits, [9] nodes, [10] max nodes, [11] max level, [12] fetch bytes, [13]
 // accessed bytes (acc must start at 0; records may be null).
@@ -159,27 +160,71 @@ hipError_t launch_trace_stats(const rtx_hit* hits, uint32_t n, const rtx_record*
 size_t coherence_scratch_bytes(uint32_t n);
 hipError_t coherence_order(const rtx_ray* rays, uint32_t n, const rtx_coherence_config& cfg, const float wmin[3],
                            const float wmax[3], uint32_t* order, uint32_t* hashes_out, void* scratch, hipStream_t s);
-// Slab records: each lane holds its last kRecRing entries in LDS and writes
-// them to the slab in aligned groups of four (32 bytes), so slab rows are
-// padded to a multiple of four entries.
-constexpr uint32_t kRecRing = 8;
-__host__ __device__ inline uint32_t slab_stride(uint32_t record_slab) { return (record_slab + 3u) & ~3u; }
+// Slab records: each lane holds its last 64 bytes of entries in LDS and writes
+// them to the slab in aligned groups of 32 bytes (four entries, eight of four
+// bytes), so slab rows are padded to a multiple of eight entries.
+__host__ __device__ inline uint32_t slab_stride(uint32_t record_slab) { return (record_slab + 7u) & ~7u; }
+// A row's first entries lie in one array and the rest in another, so that the
+// entries of most rays (21 of them on average in the 1M-triangle diffuse batch)
+// are dense in memory: rows of 512 entries would spread 110 MB of them over 2.7 GB.
+constexpr uint32_t kSlabFront = 32;
+__host__ __device__ inline uint32_t slab_front(uint32_t record_slab) {
+  const uint32_t stride = slab_stride(record_slab);
+  return stride < kSlabFront ? stride : kSlabFront;
+}
+// entry k of ray r's row, k a multiple of 4 (k < slab_stride)
+template <typename E>
+__host__ __device__ inline E* slab_place(uint64_t* slabs, uint64_t* rest, uint32_t record_slab, uint64_t r, uint32_t k) {
+  const uint32_t front = slab_front(record_slab);
+  return k < front ? reinterpret_cast<E*>(slabs) + r * front + k
+                   : reinterpret_cast<E*>(rest) + r * (slab_stride(record_slab) - front) + (k - front);
+}
 // A slab entry: the node's arena slot (offset / 64) in the low word, the
 // record type and level in the high word.  The size follows from the type;
 // the treelet and the layout offset are looked up when the entry is expanded.
 __host__ __device__ inline uint64_t slab_entry(uint32_t slot, uint32_t type, uint32_t level) {
   return (uint64_t)slot | ((uint64_t)(type | ((level > 255u ? 255u : level) << 8)) << 32);
 }
-// Expand each ray's slab entries (at most `slab`) into rtx_records at its CSR
-// position (owner and layout_remap nullable, as in TraceParams); rays with
-// more than `slab` records are appended to overflow_list as ray_base + their
-// index (count in overflow_count, which must start at 0).  Nothing is copied
-// when the total (offsets[n]) exceeds `capacity`.
-hipError_t launch_compact_records(const uint32_t* counts, uint32_t n, const uint64_t* slabs, uint32_t slab,
-                                  const uint32_t* owner, const uint64_t* layout_remap, const uint64_t* offsets,
-                                  rtx_record* records, uint64_t capacity, uint32_t ray_base, uint32_t* overflow_list,
-                                  uint32_t* overflow_count, hipStream_t s);
-// v[0..count) += *addend (a device word).
-hipError_t launch_add_offset(uint64_t* v, uint64_t count, const uint64_t* addend, hipStream_t s);
+// The 4-byte form: the slot in the low `shift` bits, the level above them, the
+// type in the top three.  For scenes whose slots and levels fit 29 bits together
+// (every node at one tree level, so the level is known beforehand to be at most
+// the scene walk's).
+constexpr uint32_t kSlab4TypeShift = 29;
+__host__ __device__ inline uint32_t slab_entry4(uint32_t slot, uint32_t type, uint32_t level, uint32_t shift) {
+  return slot | (level << shift) | (type << kSlab4TypeShift);
+}
+// The records of n rays out of their slabs: offsets[0..n] of the counts, each row's
+// first `slab` entries as rtx_records at its offset (owner and layout_remap
+// nullable, as in TraceParams), rays with more than `slab` records appended to
+// overflow_list as ray_base + their index (count in overflow_count, which must
+// start at 0).  With add_base the offsets go on from offsets[0].  No record is
+// written when the total exceeds `capacity`.  host (nullable, mapped host memory):
+// host[0] = *overflow_count, host[2..3] = offsets[n].
+struct FinishParams {
+  const uint32_t* counts;
+  uint32_t n;
+  uint32_t slab;
+  uint64_t* slabs;
+  uint64_t* slabs_rest;
+  uint32_t shift;  // the 4-byte entries' rec_level_shift, 0 for 8-byte entries
+  uint32_t add_base;
+  const uint32_t* owner;
+  const uint64_t* layout_remap;
+  uint64_t slots;  // of the arena (owner and layout_remap entries)
+  uint64_t* offsets;
+  rtx_record* records;
+  uint64_t capacity;
+  uint32_t ray_base;
+  uint32_t n_tiles;
+  uint32_t* overflow_list;
+  uint32_t* overflow_count;
+  uint32_t* host;
+  const uint64_t* tile_sums;  // set by launch_finish_records
+};
+// Batches of at most this many rays sum their counts in every workgroup (64 KiB
+// of counts from L2) instead of in a launch of its own.
+constexpr uint32_t kFinishAlone = 8192;
+// tile_sums: n / 1024 + 1 words
+hipError_t launch_finish_records(FinishParams p, uint64_t* tile_sums, hipStream_t s);
 
 }  // namespace rtxk

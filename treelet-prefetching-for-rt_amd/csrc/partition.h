@@ -54,6 +54,7 @@ struct SceneCheck {
                                   // a NaN origin or a scale above 2^103
   bool level_consistent = false;  // every reachable node has one tree level (every path agrees)
   bool cyclic = false;            // some node reaches itself
+  uint32_t max_level = 0;         // the deepest tree level (each node at the first level it was reached at)
 };
 SceneCheck scene_check(const uint8_t* arena, uint64_t bytes, uint64_t tlas, hipStream_t s);
 // remapBVHToTreeletLayout of the partition with -treelet_remap_stride `stride`

@@ -1033,6 +1033,7 @@ rtx_status run_validate(const uint8_t* A, uint64_t bytes, uint64_t tlas, hipStre
     check->ordered = c[3] == 0;
     check->regular = c[6] == 0;
     check->level_consistent = c[4] == 0;
+    check->max_level = round + 1;  // the last walked nodes are at level `round`, their leaves one below
     check->cyclic = false;
     // A cycle reaches a node at two levels, so only inconsistent scenes are peeled.
     if (!check->level_consistent) {

@@ -323,9 +323,11 @@ void trace_kernel(TraceParams p) {
   static_assert(!LM || (!REC && STAGE == 0 && !MULTI), "the level pass writes max_level only");
   constexpr uint32_t BS = STAGE ? 64u : 256u;
   constexpr int NS = MODE == 1 ? 2 : 1;
-  // ring length per list: staged treelet order keeps four groups, so that two
-  // more waves fit beside a CU's staging areas
-  constexpr int R = STAGE && MODE == 1 ? 4 : K;
+  constexpr bool kSlab = REC == kRecSlab || REC == kRecSlab4;
+  // ring length per list: treelet order keeps four groups where other LDS bounds
+  // the waves on a CU (staging areas: two more waves; record rings: four blocks
+  // instead of three, diffuse batch 1001 -> 946 us)
+  constexpr int R = (STAGE || kSlab) && MODE == 1 ? 4 : K;
   constexpr uint32_t UNITS = STAGE / 64;
   constexpr uint32_t HSIZE = STAGE ? 2 * UNITS : 1;
   __shared__ uint64_t lds_stack[NS * R * BS];
@@ -343,9 +345,11 @@ void trace_kernel(TraceParams p) {
   // direct-mapped table (a collision forgets the older slot)
   constexpr uint32_t EV = STAGE ? 128 : 1;
   __shared__ uint32_t ev_key[EV], dm_key[EV];
-  // slab records: each lane's last kRecRing slab entries (entry k at ring
-  // position k % kRecRing), written to the slab four at a time
-  __shared__ uint64_t rec_ring[REC == kRecSlab ? kRecRing * BS : 1];
+  // slab records: each lane's last RR slab entries (entry k at ring position
+  // k % RR), written to the slab RG at a time
+  typedef std::conditional_t<REC == kRecSlab4, uint32_t, uint64_t> rec_t;
+  constexpr uint32_t RR = 64 / sizeof(rec_t), RG = 32 / sizeof(rec_t);
+  __shared__ rec_t rec_ring[kSlab ? RR * BS : 1];
 
   // Staging-only parameters are read from the kernel-argument segment where
   // they are used (a scalar load each time; the empty asm keeps the compiler
@@ -361,7 +365,8 @@ void trace_kernel(TraceParams p) {
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & 63u;
   lds_u64* ldsA = (lds_u64*)(lds_stack + tid);
-  lds_u64* ring = (lds_u64*)(rec_ring + (REC == kRecSlab ? tid : 0u));
+  typedef __attribute__((address_space(3))) rec_t lds_rec;
+  lds_rec* ring = (lds_rec*)(rec_ring + (kSlab ? tid : 0u));
   const uint64_t lane_slot = (uint64_t)blockIdx.x * BS + tid;
   bool phase2 = false;  // treelet order: the current treelet was left (the lists are one stack from then on)
   // The lane's words of list l (0: the current one before the switch, 1: the
@@ -405,7 +410,7 @@ void trace_kernel(TraceParams p) {
   uint32_t cur_inst = kNoSlot;
   uint32_t n_rec = 0, n_nodes = 0, fetch_bytes = 0, n_any = 0, max_level = 0;
   uint64_t rec_base = 0;
-  uint32_t rec_flushed = 0;  // slab records: entries of the ray already in its slab
+  uint32_t rec_flushed = 0;  // slab records: entries of the ray taken out of the ring
 
   // The entry a lane popped this iteration and processes below.
   bool has_e = false;
@@ -440,13 +445,17 @@ void trace_kernel(TraceParams p) {
 
   auto emit = [&](uint64_t off, uint32_t size, uint32_t type, uint32_t lvl) {
     if (type != RTX_TX_BVH_PRIMITIVE_LEAF_DESCRIPTOR) fetch_bytes += size;
-    if constexpr (REC == kRecSlab) {
+    if constexpr (kSlab) {
       // a slab keeps the ray's first record_slab records, the rest are written
       // by a second pass over the rays that had more.  The entry holds what
       // the traversal knows; the owner and layout lookups wait for the
       // compaction, off the traversal's dependent chain.  It goes to the
       // lane's LDS ring first (flush_slab_group writes it out).
-      if (n_rec < p.record_slab) ring[(n_rec & (kRecRing - 1)) * BS] = slab_entry((uint32_t)(off >> 6), type, lvl);
+      const uint32_t slot = (uint32_t)(off >> 6);
+      if constexpr (REC == kRecSlab4)
+        ring[(n_rec & (RR - 1)) * BS] = slab_entry4(slot, type, lvl, p.rec_level_shift);
+      else
+        ring[(n_rec & (RR - 1)) * BS] = slab_entry(slot, type, lvl);
     } else if constexpr (REC == kRecCsr) {
       const uint64_t idx = rec_base + n_rec;
       if (idx < p.record_capacity) {
@@ -465,38 +474,54 @@ void trace_kernel(TraceParams p) {
     n_rec++;
   };
 
-  // Slab records: entries [rec_flushed, rec_flushed + 4) of the lane's ray go
-  // from the LDS ring to the slab once all four exist, as two 16-byte stores
-  // that fill one aligned 32-byte sector (8-byte stores scattered over the
-  // slabs cost partial-sector writes and fills).  Called at the top of every
-  // iteration, which adds at most three entries, so at most six are ever
-  // waiting and the ring of eight never overwrites one.
+  // Slab records: one group of the lane's ring, from entry rec_flushed on, to the
+  // slab as two 16-byte stores that fill one aligned 32-byte sector (stores of
+  // single entries scattered over the slabs cost partial-sector writes and fills).
+  auto store_group = [&]() {
+    if constexpr (kSlab) {
+      uint4* dst = reinterpret_cast<uint4*>(slab_place<rec_t>(p.slabs, p.slabs_rest, p.record_slab, local_id, rec_flushed));
+      uint4 v[2];
+#pragma unroll
+      for (uint32_t h = 0; h < 2; ++h) {
+        uint32_t w[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 16 / sizeof(rec_t); ++k) {
+          const rec_t x = ring[((rec_flushed & (RR - 1)) + h * (16 / sizeof(rec_t)) + k) * BS];
+          if constexpr (sizeof(rec_t) == 4) {
+            w[k] = (uint32_t)x;
+          } else {
+            w[2 * k] = (uint32_t)x;
+            w[2 * k + 1] = (uint32_t)((uint64_t)x >> 32);
+          }
+        }
+        v[h] = make_uint4(w[0], w[1], w[2], w[3]);
+      }
+      dst[0] = v[0];
+      dst[1] = v[1];
+    }
+  };
+  // At the top of every iteration, which adds at most four entries (a refilled
+  // ray's header and a visit's three): once some lane has no room for four
+  // more, every lane with a whole group writes it.  Waiting for such a lane
+  // keeps this out of most iterations.
   auto flush_slab_group = [&]() {
-    if constexpr (REC == kRecSlab) {
-      if (rec_flushed + 4u <= min(n_rec, p.record_slab)) {
-        const uint32_t q = rec_flushed & (kRecRing - 1);
-        const uint64_t a0 = ring[q * BS], a1 = ring[(q + 1) * BS], a2 = ring[(q + 2) * BS], a3 = ring[(q + 3) * BS];
-        uint4* dst = reinterpret_cast<uint4*>(p.slabs + (uint64_t)local_id * slab_stride(p.record_slab) + rec_flushed);
-        dst[0] = make_uint4((uint32_t)a0, (uint32_t)(a0 >> 32), (uint32_t)a1, (uint32_t)(a1 >> 32));
-        dst[1] = make_uint4((uint32_t)a2, (uint32_t)(a2 >> 32), (uint32_t)a3, (uint32_t)(a3 >> 32));
-        rec_flushed += 4u;
+    if constexpr (kSlab) {
+      if (__ballot(n_rec - rec_flushed > RR - 4u) == 0) return;
+      if (n_rec - rec_flushed >= RG) {
+        // entries past the slab are only counted
+        if (rec_flushed < p.record_slab) store_group();
+        rec_flushed += RG;
       }
     }
   };
   // The entries still in the ring when the ray's hit is written, as whole
-  // groups too: the row is padded to a multiple of four entries, and the
-  // entries past the ray's count (stale ring words) are never read.
+  // groups too: the row is padded to whole groups, and the entries past the
+  // ray's count (stale ring words) are never read.
   auto flush_slab_rest = [&]() {
-    if constexpr (REC == kRecSlab) {
+    if constexpr (kSlab) {
       const uint32_t end = min(n_rec, p.record_slab);
-      uint4* row = reinterpret_cast<uint4*>(p.slabs + (uint64_t)local_id * slab_stride(p.record_slab));
-      for (; rec_flushed < end; rec_flushed += 4u) {
-        const uint32_t q = rec_flushed & (kRecRing - 1);
-        const uint64_t a0 = ring[q * BS], a1 = ring[(q + 1) * BS], a2 = ring[(q + 2) * BS], a3 = ring[(q + 3) * BS];
-        row[rec_flushed / 2] = make_uint4((uint32_t)a0, (uint32_t)(a0 >> 32), (uint32_t)a1, (uint32_t)(a1 >> 32));
-        row[rec_flushed / 2 + 1] = make_uint4((uint32_t)a2, (uint32_t)(a2 >> 32), (uint32_t)a3, (uint32_t)(a3 >> 32));
-      }
-      rec_flushed = end;
+      for (; rec_flushed < end; rec_flushed += RG) store_group();
+      rec_flushed = n_rec;
     }
   };
 
@@ -858,7 +883,7 @@ void trace_kernel(TraceParams p) {
     hq[2] = o2;
     hq[3] = make_uint4(n_nodes, fetch_bytes, n_any, max_level);
     hq[4] = o4;
-    if constexpr (REC == kRecSlab) p.rec_counts[local_id] = n_rec;
+    if constexpr (kSlab) p.rec_counts[local_id] = n_rec;
     if (err) {
       atomicOr(p.error, err);
       if (p.host_err) *reinterpret_cast<volatile uint32_t*>(p.host_err) = 1u;
@@ -1401,25 +1426,16 @@ __device__ __forceinline__ uint64_t block_exclusive_scan(uint64_t v, uint64_t* s
   return wsum + x - v;
 }
 
-__global__ __launch_bounds__(kScanBlock) void scan_tiles(const rtx_hit* hits, const uint32_t* counts, uint32_t n,
-                                                         uint64_t* out, uint64_t* tile_sums) {
+__global__ __launch_bounds__(kScanBlock) void scan_tiles(const rtx_hit* hits, uint32_t n, uint64_t* out,
+                                                         uint64_t* tile_sums) {
   __shared__ uint64_t smem[4];
   const uint64_t base = (uint64_t)blockIdx.x * kScanTile + threadIdx.x * kScanItems;
   uint64_t v[kScanItems];
   uint64_t s = 0;
-  if (counts && base + kScanItems <= n) {
-    const uint4 c = *reinterpret_cast<const uint4*>(counts + base);  // base is a multiple of 4
-    v[0] = c.x;
-    v[1] = c.y;
-    v[2] = c.z;
-    v[3] = c.w;
-    s = v[0] + v[1] + v[2] + v[3];
-  } else {
 #pragma unroll
-    for (uint32_t k = 0; k < kScanItems; ++k) {
-      v[k] = base + k < n ? (counts ? counts[base + k] : hits[base + k].n_records) : 0;
-      s += v[k];
-    }
+  for (uint32_t k = 0; k < kScanItems; ++k) {
+    v[k] = base + k < n ? hits[base + k].n_records : 0;
+    s += v[k];
   }
   uint64_t total;
   uint64_t ex = block_exclusive_scan(s, smem, total);
@@ -1980,13 +1996,17 @@ TraceFn pick_k(uint32_t lds_stack, uint32_t stage) {
       default: return nullptr;
     }
   }
-  switch (stage) {
-    case 4096: return trace_kernel<MODE, REC, 8, 4096>;
-    case 8192: return trace_kernel<MODE, REC, 8, 8192>;
-    case 16384: return trace_kernel<MODE, REC, 8, 16384>;
-    case 32768: return trace_kernel<MODE, REC, 8, 32768>;
-    case 65536: return trace_kernel<MODE, REC, 8, 65536>;
-    default: return nullptr;
+  if constexpr (REC == kRecSlab4) {  // staged kernels use 8-byte entries
+    return nullptr;
+  } else {
+    switch (stage) {
+      case 4096: return trace_kernel<MODE, REC, 8, 4096>;
+      case 8192: return trace_kernel<MODE, REC, 8, 8192>;
+      case 16384: return trace_kernel<MODE, REC, 8, 16384>;
+      case 32768: return trace_kernel<MODE, REC, 8, 32768>;
+      case 65536: return trace_kernel<MODE, REC, 8, 65536>;
+      default: return nullptr;
+    }
   }
 }
 
@@ -1996,6 +2016,7 @@ TraceFn pick_rec(int records, uint32_t lds_stack, uint32_t stage) {
     case kRecNone: return pick_k<MODE, kRecNone>(lds_stack, stage);
     case kRecCsr: return pick_k<MODE, kRecCsr>(lds_stack, stage);
     case kRecSlab: return pick_k<MODE, kRecSlab>(lds_stack, stage);
+    case kRecSlab4: return pick_k<MODE, kRecSlab4>(lds_stack, stage);
     default: return nullptr;
   }
 }
@@ -2004,95 +2025,250 @@ TraceFn pick_trace(uint32_t mode, int records, uint32_t lds_stack, uint32_t stag
   return mode == RTX_MODE_PLAIN ? pick_rec<0>(records, lds_stack, stage) : pick_rec<1>(records, lds_stack, stage);
 }
 
-// ---- slab records -> CSR ----------------------------------------------------
-// A wave takes 64 consecutive rays, whose records fill one contiguous CSR
-// range: lane i holds ray i's record count and the inclusive prefix of the
-// counts, and output position f of the range (f = lane, lane + 64, ...)
-// belongs to the ray whose prefix first exceeds f (a binary search over the
-// wave's prefixes with shuffles).  Loads and stores are 16 bytes, the stores
-// contiguous, and each lane has four loads in flight.  Records past a ray's
-// slab are left to the second pass, which lists the ray.
-__global__ void report_words_kernel(const uint32_t* word, const uint64_t* dword, uint32_t* host) {
+__global__ void report_total_kernel(const uint64_t* total, uint32_t* host) {
   if (threadIdx.x == 0) {
     volatile uint32_t* h = host;
-    const uint64_t d = *dword;
-    h[0] = word ? *word : 0u;
+    const uint64_t d = *total;
     h[2] = (uint32_t)d;
     h[3] = (uint32_t)(d >> 32);
   }
 }
 
-__global__ __launch_bounds__(256) void compact_records(const uint32_t* counts, uint32_t n, const uint64_t* slabs,
-                                                       uint32_t slab, const uint32_t* owner,
-                                                       const uint64_t* layout_remap, const uint64_t* offsets,
-                                                       uint4* records, uint64_t capacity, uint32_t ray_base,
-                                                       uint32_t* overflow_list, uint32_t* overflow_count) {
-  if (offsets[n] > capacity) return;  // the caller reports RTX_ERR_TRACE_OVERFLOW
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t wave = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const uint32_t waves = gridDim.x * 4;
+// ---- slab records -> CSR ----------------------------------------------------
+// Three launches: record sums of tiles of kScanTile rays (with the list of rays whose
+// records overflowed their slab), the rays' offsets (each workgroup summing the
+// tiles before its own), and the expansion.  A batch of at most kFinishAlone rays
+// takes one launch, whose workgroups sum the counts themselves and expand their
+// own 256 rays: six launches and 12 us less than scans, clear, compaction and
+// report had for a 32-ray batch (122 -> 110 us).
+//
+// The expansion reads 128 MB and writes 468 MB for the 28M records of 1.34M rays
+// (100 us at this card's rates) but is bound by the address units: each record
+// costs a slab load, an owner gather and a 16-byte store whatever the lanes in
+// use.  With one output record per lane all lanes are in use: 174 us; eight lanes
+// per ray take 240 us, a search for each record's ray among 64 counts took 202 us
+// and the separate scans 28 us more.
+__global__ __launch_bounds__(kScanBlock) void sum_record_tiles(const uint32_t* counts, uint32_t n, uint32_t slab,
+                                                               uint64_t* tile_sums, uint32_t ray_base,
+                                                               uint32_t* overflow_list, uint32_t* overflow_count) {
+  __shared__ uint64_t smem[4];
+  uint64_t sum = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < kScanItems; ++k) {
+    const uint64_t r = (uint64_t)blockIdx.x * kScanTile + k * kScanBlock + threadIdx.x;
+    const uint32_t c = r < n ? counts[r] : 0u;
+    if (c > slab) overflow_list[atomicAdd(overflow_count, 1u)] = ray_base + (uint32_t)r;
+    sum += c;
+  }
+  uint64_t total;
+  block_exclusive_scan(sum, smem, total);
+  if (threadIdx.x == 0) tile_sums[blockIdx.x] = total;
+}
+
+__device__ __forceinline__ void report_records(const FinishParams& p, uint32_t overflowed, uint64_t total) {
+  if (!p.host) return;
+  volatile uint32_t* h = p.host;
+  h[0] = overflowed;
+  h[2] = (uint32_t)total;
+  h[3] = (uint32_t)(total >> 32);
+}
+
+// The rtx_record of a slab entry.
+template <typename E>
+__device__ __forceinline__ uint4 record_of(E v, uint32_t shift, uint64_t offset, uint32_t treelet) {
+  const uint32_t lo = (uint32_t)v, hw = (uint32_t)((uint64_t)v >> 32);
+  const uint32_t type = sizeof(E) == 4 ? lo >> kSlab4TypeShift : hw & 0xffu;
+  const uint32_t level = sizeof(E) == 4 ? (lo & ((1u << kSlab4TypeShift) - 1u)) >> shift : hw >> 8;
+  const uint32_t size = type == RTX_TX_BVH_INSTANCE_LEAF ? 128u : type == RTX_TX_BVH_PRIMITIVE_LEAF_DESCRIPTOR ? 8u : 64u;
+  return make_uint4((uint32_t)offset, (uint32_t)(offset >> 32), treelet, size | (type << 16) | (level << 24));
+}
+
+// The first c records of a ray to `out`, by the eight lanes j = 0 .. 7.
+template <typename E>
+__device__ __forceinline__ void expand_row(const FinishParams& p, uint64_t ray, uint4* out, uint32_t c, uint32_t j) {
   constexpr uint32_t kUnroll = 4;
-  for (uint32_t base = wave * 64; base < n; base += waves * 64) {
-    const uint32_t r = base + lane;
-    uint32_t cnt = 0;
-    if (r < n) {
-      cnt = counts[r];
-      if (cnt > slab) overflow_list[atomicAdd(overflow_count, 1u)] = ray_base + r;
+  static_assert(kSlabFront == 8 * kUnroll, "a pass reads from one of the two arrays");
+  for (uint32_t pass = 0; pass < c; pass += kSlabFront) {
+    const E* row = slab_place<E>(p.slabs, p.slabs_rest, p.slab, ray, pass) + j;
+    E v[kUnroll];
+    uint32_t slot[kUnroll], tl[kUnroll];
+    uint64_t roff[kUnroll];
+#pragma unroll
+    for (uint32_t u = 0; u < kUnroll; ++u) v[u] = pass + 8 * u + j < c ? row[8 * u] : (E)0;
+#pragma unroll
+    for (uint32_t u = 0; u < kUnroll; ++u) {
+      slot[u] = sizeof(E) == 4 ? (uint32_t)v[u] & ((1u << p.shift) - 1u) : (uint32_t)v[u];
+      // (a ray that no claim listed keeps an older row: never looked up out of range)
+      const bool ok = pass + 8 * u + j < c && slot[u] < p.slots;
+      tl[u] = p.owner && ok ? p.owner[slot[u]] : RTX_NO_TREELET;
+      roff[u] = p.layout_remap && ok ? p.layout_remap[slot[u]] : (uint64_t)slot[u] << 6;
     }
-    uint32_t incl = cnt;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const uint32_t y = __shfl_up(incl, d, 64);
-      if (lane >= (uint32_t)d) incl += y;
+    for (uint32_t u = 0; u < kUnroll; ++u) {
+      const uint32_t k = pass + 8 * u + j;
+      if (k >= c) continue;
+      out[k] = record_of(v[u], p.shift, roff[u], tl[u]);
     }
-    const uint32_t total = __shfl(incl, 63, 64);
-    const uint64_t out = offsets[base];
-    // wave-uniform loop: every lane takes part in the shuffles.  The kUnroll
-    // searches run interleaved and every load is issued unconditionally (an
-    // index past the end reads entry 0 and is not stored), so the slab loads
-    // and then the owner loads of a pass are in flight together.
-    const uint32_t stride = slab_stride(slab);
-    for (uint32_t f0 = 0; f0 < total; f0 += 64 * kUnroll) {
-      uint32_t lo[kUnroll];
+  }
+}
+
+// Offsets of a tile's rays.
+__global__ __launch_bounds__(kScanBlock) void place_records(FinishParams p) {
+  __shared__ uint64_t smem[4];
+  const uint32_t tid = threadIdx.x;
+  uint64_t all = 0, before = 0;
+  for (uint32_t i = tid; i < p.n_tiles; i += kScanBlock) {
+    const uint64_t v = p.tile_sums[i];
+    all += v;
+    before += i < blockIdx.x ? v : 0u;
+  }
+  uint64_t n_all, n_before, n_mine;
+  block_exclusive_scan(all, smem, n_all);
+  block_exclusive_scan(before, smem, n_before);
+  const uint64_t base = p.add_base ? p.offsets[0] : 0;
+  const uint64_t r = (uint64_t)blockIdx.x * kScanTile + tid * kScanItems;
+  uint32_t c[kScanItems], sum = 0;
 #pragma unroll
-      for (uint32_t u = 0; u < kUnroll; ++u) lo[u] = 0;
-      // first ray i with prefix(i) > f
+  for (uint32_t k = 0; k < kScanItems; ++k) {
+    c[k] = r + k < p.n ? p.counts[r + k] : 0u;
+    sum += c[k];
+  }
+  uint64_t at = base + n_before + block_exclusive_scan(sum, smem, n_mine);
 #pragma unroll
-      for (uint32_t step = 32; step > 0; step >>= 1) {
+  for (uint32_t k = 0; k < kScanItems; ++k) {
+    if (r + k < p.n && (r + k > 0 || !p.add_base)) p.offsets[r + k] = at;
+    at += c[k];
+  }
+  if (blockIdx.x == 0 && tid == 0) {
+    p.offsets[p.n] = base + n_all;
+    report_records(p, *p.overflow_count, base + n_all);
+  }
+}
+
+// A small batch at once: offsets and records of 256 rays, the workgroups all
+// summing the batch's counts.
+template <typename E>
+__global__ __launch_bounds__(kScanBlock) void finish_records(FinishParams p) {
+  __shared__ uint64_t smem[4];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t first = blockIdx.x * kScanBlock;  // the workgroup's first ray
+  // records of all rays, and of those before the workgroup's
+  uint64_t all = 0, before = 0;
+  uint32_t over = 0;
+#pragma unroll 4
+  for (uint32_t i = tid; i < p.n; i += kScanBlock) {
+    const uint32_t v = p.counts[i];
+    all += v;
+    before += i < first ? v : 0u;
+    over += v > p.slab ? 1u : 0u;
+  }
+  uint64_t n_all, n_before, n_over = 0, n_mine;
+  block_exclusive_scan(all, smem, n_all);
+  block_exclusive_scan(before, smem, n_before);
+  block_exclusive_scan(over, smem, n_over);
+  const uint64_t base = p.add_base ? p.offsets[0] : 0;
+  const uint32_t r = first + tid;
+  const uint32_t cnt = r < p.n ? p.counts[r] : 0u;
+  if (cnt > p.slab) p.overflow_list[atomicAdd(p.overflow_count, 1u)] = p.ray_base + r;
+  const uint64_t at = base + n_before + block_exclusive_scan(cnt, smem, n_mine);
+  if (r < p.n && (r > 0 || !p.add_base)) p.offsets[r] = at;
+  if (blockIdx.x == 0 && tid == 0) {
+    p.offsets[p.n] = base + n_all;
+    report_records(p, (uint32_t)n_over, base + n_all);
+  }
+  if (base + n_all > p.capacity) return;  // the caller reports RTX_ERR_TRACE_OVERFLOW
+  for (uint32_t i = lane >> 3; i < 64; i += 8) {  // lanes 8g .. 8g + 7: rays g, g + 8, ... of the wave
+    const uint32_t c = min((uint32_t)__shfl(cnt, (int)i, 64), p.slab);
+    const uint64_t o = (uint64_t)__shfl((uint32_t)at, (int)i, 64) | ((uint64_t)__shfl((uint32_t)(at >> 32), (int)i, 64) << 32);
+    expand_row<E>(p, first + (tid & ~63u) + i, reinterpret_cast<uint4*>(p.records) + o, c, lane & 7u);
+  }
+}
+
+// Waves take chunks of kExpandChunk consecutive records, and find their first ray
+// by a 64-way search of the offsets.  Lane f takes record f of a window of 64: its
+// ray is the last one that starts at or before f, counted in a bitmap of the rays'
+// starts.
+constexpr uint32_t kExpandChunk = 1024;
+template <typename E>
+__global__ __launch_bounds__(kScanBlock) void expand_records(FinishParams p) {
+  __shared__ uint64_t starts_of[kScanBlock / 64][kExpandChunk / 64];
+  __shared__ int2 row_of[kScanBlock / 64][64];  // a batch's rays in the chunk: first record, ray
+  const uint32_t lane = threadIdx.x & 63u, wave = blockIdx.x * (kScanBlock / 64) + (threadIdx.x >> 6);
+  uint64_t* starts = starts_of[threadIdx.x >> 6];
+  int2* rows = row_of[threadIdx.x >> 6];
+  auto wave_sync = []() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  const uint64_t begin = p.offsets[0], end = p.offsets[p.n];
+  if (end > p.capacity) return;  // the caller reports RTX_ERR_TRACE_OVERFLOW
+  const uint32_t front = slab_front(p.slab), rest = slab_stride(p.slab) - front;
+  const uint64_t stride = (uint64_t)gridDim.x * (kScanBlock / 64) * kExpandChunk;
+  for (uint64_t f0 = begin + (uint64_t)wave * kExpandChunk; f0 < end; f0 += stride) {
+    const uint32_t size = (uint32_t)min((uint64_t)kExpandChunk, end - f0);
+    // the last ray whose offset is at most f0, among lo .. lo + len - 1
+    uint32_t lo = 0, len = p.n;
+    while (len > 1) {
+      const uint32_t step = (len + 63) / 64, at = lane * step;
+      const bool below = at < len && p.offsets[lo + at] <= f0;
+      const uint32_t k = (uint32_t)__popcll(__ballot(below)) - 1u;  // (lane 0 always is)
+      lo += k * step;
+      len = min(step, len - k * step);
+    }
+    for (uint32_t r0 = lo; r0 < p.n; r0 += 64) {
+      const uint32_t r = min(r0 + lane, p.n - 1);
+      const int64_t off = (int64_t)(p.offsets[r] - f0), next = (int64_t)(p.offsets[r + 1] - f0);
+      const bool mine = r0 + lane < p.n && off < (int64_t)size;
+      const bool some = mine && next > 0 && next > off;  // has records in the chunk
+      // (a ray of the chunk starts at most a slab's rows and 2^24 steps before it)
+      const uint32_t s = (uint32_t)max(off, (int64_t)0);
+      const uint64_t have = __ballot(some);
+      if (lane < kExpandChunk / 64) starts[lane] = 0;
+      wave_sync();
+      if (some) {
+        atomicOr(reinterpret_cast<unsigned long long*>(&starts[s >> 6]), 1ull << (s & 63u));
+        rows[lanes_below(have)] = make_int2((int)off, (int)(r0 + lane));
+      }
+      wave_sync();
+      if (have) {
+        const int first = (int)__builtin_ctzll(have), last = 63 - (int)__builtin_clzll(have);
+        const uint32_t b0 = (uint32_t)__builtin_amdgcn_readlane((int)s, first);
+        const uint32_t b1 = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)min(next, (int64_t)size), last);
+        uint32_t before = 0;  // starts in the words before w
+        constexpr uint32_t kUnroll = 4;
+        for (uint32_t w = b0 >> 6; w * 64 < b1; w += kUnroll) {
+          E v[kUnroll];
+          uint32_t slot[kUnroll], tl[kUnroll];
+          uint64_t roff[kUnroll];
+          bool ok[kUnroll];
 #pragma unroll
-        for (uint32_t u = 0; u < kUnroll; ++u) {
-          const uint32_t pre = __shfl(incl, (int)(lo[u] + step - 1), 64);
-          if (pre <= f0 + u * 64 + lane) lo[u] += step;
+          for (uint32_t u = 0; u < kUnroll; ++u) {
+            const uint64_t m = starts[min(w + u, kExpandChunk / 64 - 1)];
+            const uint32_t f = (w + u) * 64 + lane;
+            const uint32_t k = before + lanes_below(m) + (uint32_t)((m >> lane) & 1u);
+            const int2 row = rows[k ? min(k, 64u) - 1u : 0u];
+            const uint32_t j = f - (uint32_t)row.x;
+            ok[u] = f >= b0 && f < b1 && j < p.slab;
+            const E* q = j < front ? reinterpret_cast<const E*>(p.slabs) + (uint64_t)(uint32_t)row.y * front + j
+                                   : reinterpret_cast<const E*>(p.slabs_rest) + (uint64_t)(uint32_t)row.y * rest + (j - front);
+            v[u] = ok[u] ? *q : (E)0;
+            before += (uint32_t)__popcll(m);
+          }
+#pragma unroll
+          for (uint32_t u = 0; u < kUnroll; ++u) {
+            slot[u] = sizeof(E) == 4 ? (uint32_t)v[u] & ((1u << p.shift) - 1u) : (uint32_t)v[u];
+            const bool in = ok[u] && slot[u] < p.slots;  // (see expand_row)
+            tl[u] = p.owner && in ? p.owner[slot[u]] : RTX_NO_TREELET;
+            roff[u] = p.layout_remap && in ? p.layout_remap[slot[u]] : (uint64_t)slot[u] << 6;
+          }
+#pragma unroll
+          for (uint32_t u = 0; u < kUnroll; ++u)
+            if (ok[u])
+              reinterpret_cast<uint4*>(p.records)[f0 + (w + u) * 64 + lane] = record_of(v[u], p.shift, roff[u], tl[u]);
         }
       }
-      uint64_t v[kUnroll];
-      bool ok[kUnroll];
-#pragma unroll
-      for (uint32_t u = 0; u < kUnroll; ++u) {
-        const uint32_t f = f0 + u * 64 + lane;
-        const uint32_t before = __shfl(incl, (int)(lo[u] ? lo[u] - 1 : 0), 64);
-        const uint32_t k = f - (lo[u] ? before : 0u);
-        ok[u] = f < total && k < slab;
-        v[u] = slabs[ok[u] ? (uint64_t)(base + lo[u]) * stride + k : 0u];
-      }
-      uint32_t tl[kUnroll];
-      uint64_t roff[kUnroll];
-#pragma unroll
-      for (uint32_t u = 0; u < kUnroll; ++u) {
-        const uint32_t slot = ok[u] ? (uint32_t)v[u] : 0u;
-        tl[u] = owner ? owner[slot] : RTX_NO_TREELET;
-        roff[u] = layout_remap ? layout_remap[slot] : (uint64_t)slot << 6;
-      }
-#pragma unroll
-      for (uint32_t u = 0; u < kUnroll; ++u) {
-        if (!ok[u]) continue;
-        const uint32_t hw = (uint32_t)(v[u] >> 32);
-        const uint32_t type = hw & 0xffu;
-        const uint32_t size = type == RTX_TX_BVH_INSTANCE_LEAF ? 128u
-                              : type == RTX_TX_BVH_PRIMITIVE_LEAF_DESCRIPTOR ? 8u : 64u;
-        records[out + f0 + u * 64 + lane] = make_uint4((uint32_t)roff[u], (uint32_t)(roff[u] >> 32), tl[u],
-                                                       size | (type << 16) | ((hw >> 8) << 24));
-      }
+      if (__ballot(mine) != ~0ull) break;
     }
   }
 }
@@ -2122,12 +2298,6 @@ uint32_t blocks_per_cu(TraceFn f, uint32_t bs) {
   return nb > 0 ? (uint32_t)nb : 0u;
 }
 
-__global__ void add_offset_kernel(uint64_t* v, uint64_t count, const uint64_t* addend) {
-  const uint64_t a = *addend;
-  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < count; i += (uint64_t)gridDim.x * blockDim.x)
-    v[i] += a;
-}
-
 __global__ void fill_zero_kernel(uint32_t* dst, uint32_t words) {
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x) dst[i] = 0u;
 }
@@ -2144,8 +2314,8 @@ uint32_t trace_batch_blocks_per_cu(uint32_t mode, uint32_t lds_stack) {
   return blocks_per_cu(pick_batch(mode, lds_stack), 256);
 }
 
-hipError_t launch_report_words(const uint32_t* word, const uint64_t* dword, uint32_t* host, hipStream_t s) {
-  hipLaunchKernelGGL(report_words_kernel, dim3(1), dim3(64), 0, s, word, dword, host);
+hipError_t launch_report_total(const uint64_t* total, uint32_t* host, hipStream_t s) {
+  hipLaunchKernelGGL(report_total_kernel, dim3(1), dim3(64), 0, s, total, host);
   return hipGetLastError();
 }
 
@@ -2226,21 +2396,26 @@ hipError_t launch_trace_stats(const rtx_hit* hits, uint32_t n, const rtx_record*
   return hipGetLastError();
 }
 
-hipError_t launch_compact_records(const uint32_t* counts, uint32_t n, const uint64_t* slabs, uint32_t slab,
-                                  const uint32_t* owner, const uint64_t* layout_remap, const uint64_t* offsets,
-                                  rtx_record* records, uint64_t capacity, uint32_t ray_base, uint32_t* overflow_list,
-                                  uint32_t* overflow_count, hipStream_t s) {
-  if (n == 0 || slab == 0) return hipSuccess;
-  const uint32_t grid = std::max(1u, std::min<uint32_t>(4096, (n + 255) / 256));
-  hipLaunchKernelGGL(compact_records, dim3(grid), dim3(256), 0, s, counts, n, slabs, slab, owner, layout_remap, offsets,
-                     reinterpret_cast<uint4*>(records), capacity, ray_base, overflow_list, overflow_count);
-  return hipGetLastError();
-}
-
-hipError_t launch_add_offset(uint64_t* v, uint64_t count, const uint64_t* addend, hipStream_t s) {
-  if (count == 0) return hipSuccess;
-  const uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(4096, (count + 255) / 256));
-  hipLaunchKernelGGL(add_offset_kernel, dim3(grid), dim3(256), 0, s, v, count, addend);
+hipError_t launch_finish_records(FinishParams p, uint64_t* tile_sums, hipStream_t s) {
+  if (p.n == 0 || p.slab == 0) return hipSuccess;
+  const uint32_t grid = (p.n + kScanBlock - 1) / kScanBlock;
+  if (p.n <= kFinishAlone) {
+    if (p.shift)
+      hipLaunchKernelGGL(finish_records<uint32_t>, dim3(grid), dim3(kScanBlock), 0, s, p);
+    else
+      hipLaunchKernelGGL(finish_records<uint64_t>, dim3(grid), dim3(kScanBlock), 0, s, p);
+    return hipGetLastError();
+  }
+  p.n_tiles = (p.n + kScanTile - 1) / kScanTile;
+  p.tile_sums = tile_sums;
+  hipLaunchKernelGGL(sum_record_tiles, dim3(p.n_tiles), dim3(kScanBlock), 0, s, p.counts, p.n, p.slab, tile_sums,
+                     p.ray_base, p.overflow_list, p.overflow_count);
+  hipLaunchKernelGGL(place_records, dim3(p.n_tiles), dim3(kScanBlock), 0, s, p);
+  const uint32_t chunks = std::min<uint32_t>(2048, grid);
+  if (p.shift)
+    hipLaunchKernelGGL(expand_records<uint32_t>, dim3(chunks), dim3(kScanBlock), 0, s, p);
+  else
+    hipLaunchKernelGGL(expand_records<uint64_t>, dim3(chunks), dim3(kScanBlock), 0, s, p);
   return hipGetLastError();
 }
 
@@ -2277,12 +2452,10 @@ uint32_t trace_blocks_per_cu(uint32_t mode, int records, uint32_t lds_stack, uin
   return blocks_per_cu(pick_trace(mode, records, lds_stack, stage_bytes), trace_block_size(stage_bytes));
 }
 
-hipError_t launch_scan_records(const rtx_hit* hits, const uint32_t* counts, uint32_t n, uint64_t* offsets,
-                               uint64_t* tile_sums, hipStream_t s) {
-  static_assert(kScanItems == 4, "scan_tiles reads four counts as one uint4");
+hipError_t launch_scan_records(const rtx_hit* hits, uint32_t n, uint64_t* offsets, uint64_t* tile_sums, hipStream_t s) {
   const uint32_t tiles = (n + kScanTile - 1) / kScanTile;
   if (tiles > 0) {
-    hipLaunchKernelGGL(scan_tiles, dim3(tiles), dim3(kScanBlock), 0, s, hits, counts, n, offsets, tile_sums);
+    hipLaunchKernelGGL(scan_tiles, dim3(tiles), dim3(kScanBlock), 0, s, hits, n, offsets, tile_sums);
   }
   hipLaunchKernelGGL(scan_sums, dim3(1), dim3(kScanBlock), 0, s, tile_sums, tiles, offsets, n);
   if (tiles > 0) {
