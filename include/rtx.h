@@ -175,9 +175,9 @@ typedef struct rtx_trace_options {
                             (0 = default 0.25; 1 = the whole image) */
   uint32_t lanes_per_ray; /* 1: one lane per ray; 8: eight lanes per ray, testing a node's six
                              children at once (either order, no records or staging), for batches
-                             too small to fill the GPU; 0 = 8 when those hold and the batch has
-                             at most 128 rays per CU (PLAIN) or 256 (TREELET), else 1.  Results
-                             are identical.
+                             too small to fill the GPU; 0 = 8 without staging when the batch has
+                             at most 128 rays per CU (64 for TREELET with records), else 1.
+                             Results are identical.
                              rtx_trace only; batches ignore it. */
   uint32_t claim_start;  /* persistent waves claim rays starting at this index and wrap around to 0
                             (outputs stay at input indices).  A batch that holds camera rays followed

@@ -65,3 +65,27 @@ def test_records_of_a_scene_with_two_levels_per_node(gpu, rtx, oracle, mode, n, 
     h, o, r = gpu.trace(rays, mode=mode, records=True, record_slab=slab)
     assert_hits_equal(h, h_ref, "hits")
     assert_records_equal(o, r, o_ref, r_ref, "records")
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("n", [1, 33, 1023, 1025, 9000])
+@pytest.mark.parametrize("waves_per_cu", [0, 1])
+def test_small_batches_by_place_and_by_counter(gpu, rtx, oracle, instanced, mode, n, waves_per_cu):
+    """Waves with one ray and with eight at a time, rays taken by the wave's place (all
+    resident) and from the counter (one workgroup per CU holds 8,192 of 256 CUs)."""
+    scene, rays = instanced
+    rays = _rays(rtx, rays, n, 0, n + 1)
+    part = oracle.Partition(scene.arena, scene.tlas_offset, 1024)
+    h_ref, o_ref, r_ref = oracle.trace(scene.arena, scene.tlas_offset, rays, mode=mode, partition=part)
+    gpu.set_scene(scene.arena, scene.tlas_offset)
+    gpu.build_treelets(1024)
+    for order in (None, np.random.default_rng(n).permutation(n).astype(np.uint32)):
+        claim = dict(claim_order=gpu.to_device(order)) if order is not None else {}
+        rb, hb = gpu.to_device(rays), gpu.buffer(n * rtx.HIT_DTYPE.itemsize)
+        assert gpu.trace_device(rb, n, hb, mode=mode, lanes_per_ray=8, waves_per_cu=waves_per_cu, **claim) == 0
+        assert_hits_equal(hb.download(rtx.HIT_DTYPE, n), h_ref, "hits")
+        ob, recb = gpu.buffer((n + 1) * 8), gpu.buffer(int(o_ref[-1]) * rtx.RECORD_DTYPE.itemsize)
+        assert gpu.trace_device(rb, n, hb, mode=mode, records_buf=recb, record_capacity=int(o_ref[-1]), offsets_buf=ob,
+                                waves_per_cu=waves_per_cu, **claim) == 0
+        assert_hits_equal(hb.download(rtx.HIT_DTYPE, n), h_ref, "hits with records")
+        assert_records_equal(ob.download(np.uint64, n + 1), recb.download(rtx.RECORD_DTYPE, int(o_ref[-1])), o_ref, r_ref, "records")

@@ -225,7 +225,7 @@ uint32_t cached_blocks_per_cu(rtx_ctx* c, uint32_t mode, uint32_t lds_stack, uin
   const uint64_t key = ((uint64_t)mode << 48) | ((uint64_t)records << 40) | ((uint64_t)lds_stack << 32) | stage;
   auto it = c->occupancy.find(key);
   if (it != c->occupancy.end()) return it->second;
-  const uint32_t b = mode >= kWideOccupancyKey ? trace_wide_blocks_per_cu(mode - kWideOccupancyKey)
+  const uint32_t b = mode >= kWideOccupancyKey ? trace_wide_blocks_per_cu(mode - kWideOccupancyKey, records != kRecNone)
                                                : trace_blocks_per_cu(mode, records, lds_stack, stage);
   c->occupancy[key] = b;
   return b;
@@ -357,7 +357,7 @@ rtx_status rtx_create(int device, rtx_ctx** out) {
   const uint32_t ks[3] = {4, 8, 16};
   for (uint32_t m = 0; m < 2; ++m) {
     for (int k = 0; k < 3; ++k) c->static_occ[m][k] = trace_blocks_per_cu(m, kRecNone, ks[k], 0);
-    c->static_wide_occ[m] = trace_wide_blocks_per_cu(m);
+    c->static_wide_occ[m] = trace_wide_blocks_per_cu(m, false);
   }
   *out = c;
   return RTX_OK;
@@ -669,21 +669,18 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
     if (!(opts->pred_fraction >= 0.f && opts->pred_fraction <= 1.f)) return RTX_ERR_INVALID_ARGUMENT;
     lds_stack = 8;
   }
-  // Eight lanes per ray (no records or staging) for batches that leave most of
-  // the GPU idle, at most 128 rays per CU in plain order and 256 in treelet
-  // order (where the two kernels meet on the 1M-triangle scene): their time is
-  // the step latency of the longest rays, and a group tests a node's six
-  // children at once.
+  // Eight lanes per ray for batches that leave most of the GPU idle (see
+  // wide_rays_per_cu; on request only without records and staging).
   if (opts->lanes_per_ray != 0 && opts->lanes_per_ray != 1 && opts->lanes_per_ray != kWideRayLanes)
     return RTX_ERR_INVALID_ARGUMENT;
   const bool wide_ok = !opts->emit_records && stage == 0;
-  // records in one traversal: per-ray slabs of `slab` records, compacted into the
+  // records in one traversal: per-ray slabs of `slab` records, expanded into the
   // caller's CSR buffer; only rays with more records are traced again, which
   // costs such a ray's whole latency (a 1M-triangle diffuse batch has some of 300
   // records: 250 us).  Default 512 in 4-byte entries (scenes whose slots and levels
   // fit them, see slab4_shift), 256 in 8-byte ones and for batches that only fit
-  // so.  The slabs take at most 2^31 entries: a larger batch is traced in consecutive ray
-  // ranges that fit, each compacted before the next reuses the slabs.  With a
+  // so.  The slabs take at most 2^31 entries: a larger batch is traced in
+  // consecutive ray ranges that fit, each expanded before the next reuses the slabs.  With a
   // claim order or staging such a batch takes a counting pass and a writing
   // pass instead.
   const bool long_rows = c->rec_level_shift != 0 && stage == 0 && (uint64_t)n * 512 <= kSlabEntriesMax;
@@ -696,23 +693,26 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
   const uint32_t shift4 = use_slab && stage == 0 ? c->rec_level_shift : 0;
   const int main_rec = !use_slab ? kRecNone : shift4 ? kRecSlab4 : kRecSlab;
   if (opts->lanes_per_ray == kWideRayLanes && !wide_ok) return RTX_ERR_INVALID_ARGUMENT;
-  const bool wide = wide_ok && (opts->lanes_per_ray == kWideRayLanes ||
-                                (opts->lanes_per_ray == 0 &&
-                                 (uint64_t)n <= (opts->mode == RTX_MODE_PLAIN ? 128ull : 256ull) * c->n_cus));
+  const bool wide = opts->lanes_per_ray == kWideRayLanes ||
+                    (opts->lanes_per_ray == 0 && stage == 0 && (!opts->emit_records || use_slab) &&
+                     (uint64_t)n <= (uint64_t)wide_rays_per_cu(opts->mode, opts->emit_records) * c->n_cus);
   const uint32_t bs = trace_block_size(stage);
   // persistent blocks: by default as many as fit on a CU at once
   uint32_t blocks_per_cu = opts->waves_per_cu ? std::max(1u, opts->waves_per_cu * 64 / bs)
-                           : wide             ? cached_blocks_per_cu(c, kWideOccupancyKey + opts->mode, 0, 0)
+                           : wide             ? cached_blocks_per_cu(c, kWideOccupancyKey + opts->mode, 0, 0, main_rec)
                                               : cached_blocks_per_cu(c, opts->mode, lds_stack, stage, main_rec);
   if (blocks_per_cu == 0) blocks_per_cu = 16 * 64 / bs;
   uint32_t grid = (uint32_t)c->n_cus * blocks_per_cu;
-  const uint64_t lanes = (uint64_t)n * (wide ? kWideRayLanes : 1u);
+  const uint32_t groups = wide ? wide_groups(n, (uint32_t)c->n_cus) : 1u;
+  const uint64_t lanes = (uint64_t)n * (wide ? 64u / groups : 1u);
   grid = (uint32_t)std::min<uint64_t>(grid, (lanes + bs - 1) / bs);
   grid = std::max(grid, 1u);
   const uint32_t spill_cap = 128;
   const uint32_t ns = opts->mode == RTX_MODE_TREELET ? 2 : 1;
   // treelet order with staging or records keeps fewer entries in LDS (trace_kernel's R)
-  rtx_status st = ensure_spill(c, (size_t)grid * bs * (spill_cap + (stage || use_slab ? lds_stack : 0)) * ns);
+  // (the eight-lanes kernel spills nothing; a second pass of its rays may)
+  const uint32_t spill_grid = wide ? (n + bs - 1) / bs : grid;
+  rtx_status st = ensure_spill(c, (size_t)spill_grid * bs * (spill_cap + (stage || use_slab ? lds_stack : 0)) * ns);
   if (st != RTX_OK) return st;
 
   TraceParams p{};
@@ -822,7 +822,10 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
     q.rec_counts = c->rec_counts + b;
     if (b > 0) HIP_TRY(launch_fill_zero(main_slot, 1, c->stream));
     const uint32_t gq = std::max(1u, (uint32_t)std::min<uint64_t>(grid, ((uint64_t)(e - b) + bs - 1) / bs));
-    HIP_TRY(launch_trace(q, opts->mode, main_rec, lds_stack, stage, gq, c->stream));
+    if (wide)  // (one range: such batches are small)
+      HIP_TRY(launch_trace_wide(q, opts->mode, true, lds_stack + spill_cap, grid, groups, c->stream));
+    else
+      HIP_TRY(launch_trace(q, opts->mode, main_rec, lds_stack, stage, gq, c->stream));
     if (last) HIP_TRY(hipEventRecord(c->evk1, c->stream));
     FinishParams f{};
     f.counts = c->rec_counts + b;
@@ -847,8 +850,8 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
   };
   // the timed span: the traversal launch (from the first range's to the end of the last range's)
   HIP_TRY(hipEventRecord(c->evk0, c->stream));
-  if (wide) {
-    HIP_TRY(launch_trace_wide(p, opts->mode, lds_stack + spill_cap, grid, c->stream));
+  if (wide && !use_slab) {
+    HIP_TRY(launch_trace_wide(p, opts->mode, false, lds_stack + spill_cap, grid, groups, c->stream));
     HIP_TRY(hipEventRecord(c->evk1, c->stream));
   } else if (use_slab) {
     for (uint32_t k = 0; k < n_chunks; ++k) {
@@ -992,13 +995,14 @@ rtx_status rtx_trace_static(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const r
   if (n == 0) return RTX_OK;
   const bool wide = opts->lanes_per_ray == kWideRayLanes ||
                     (opts->lanes_per_ray == 0 &&
-                     (uint64_t)n <= (opts->mode == RTX_MODE_PLAIN ? 128ull : 256ull) * c->n_cus);
+                     (uint64_t)n <= (uint64_t)wide_rays_per_cu(opts->mode, false) * c->n_cus);
   const uint32_t bs = 256;
   uint32_t per_cu = opts->waves_per_cu ? std::max(1u, opts->waves_per_cu * 64 / bs)
                     : wide             ? c->static_wide_occ[opts->mode]
                                        : c->static_occ[opts->mode][ki];
   if (per_cu == 0) per_cu = 4;
-  const uint64_t lanes = (uint64_t)n * (wide ? kWideRayLanes : 1u);
+  const uint32_t groups = wide ? wide_groups(n, (uint32_t)c->n_cus) : 1u;
+  const uint64_t lanes = (uint64_t)n * (wide ? 64u / groups : 1u);
   uint32_t grid = (uint32_t)std::min<uint64_t>((uint64_t)c->n_cus * per_cu, (lanes + bs - 1) / bs);
   grid = std::max(grid, 1u);
   // The spill area is what the scratch holds beyond its control words, split
@@ -1040,7 +1044,7 @@ rtx_status rtx_trace_static(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const r
   HIP_TRY(launch_fill_zero(control, 2, c->stream));
   HIP_TRY(hipEventRecord(c->evk0, c->stream));
   if (wide)
-    HIP_TRY(launch_trace_wide(p, opts->mode, lds_stack + 128, grid, c->stream));
+    HIP_TRY(launch_trace_wide(p, opts->mode, false, lds_stack + 128, grid, groups, c->stream));
   else
     HIP_TRY(launch_trace(p, opts->mode, kRecNone, lds_stack, 0, grid, c->stream));
   HIP_TRY(hipEventRecord(c->evk1, c->stream));

@@ -129,12 +129,33 @@ hipError_t launch_trace_batch(const TraceParams& p, uint32_t mode, uint32_t lds_
 // 0 when the configuration has no kernel.
 uint32_t trace_blocks_per_cu(uint32_t mode, int records, uint32_t lds_stack, uint32_t stage_bytes);
 uint32_t trace_batch_blocks_per_cu(uint32_t mode, uint32_t lds_stack);
-// Cooperative kernel for small batches (eight lanes per ray, no records or
-// staging), plain or treelet order: `cap` entries per list and ray (at most
-// 144), 256-lane blocks.
+// Cooperative kernel for small batches (eight lanes per ray, no staging), plain or
+// treelet order, with slab records or hits only: `cap` entries per list and ray
+// (at most 144), 256-lane blocks, `groups` rays at a time in a wave (at most 8).
 constexpr uint32_t kWideRayLanes = 8;
-hipError_t launch_trace_wide(const TraceParams& p, uint32_t mode, uint32_t cap, uint32_t grid, hipStream_t s);
-uint32_t trace_wide_blocks_per_cu(uint32_t mode);
+hipError_t launch_trace_wide(const TraceParams& p, uint32_t mode, bool records, uint32_t cap, uint32_t grid,
+                             uint32_t groups, hipStream_t s);
+uint32_t trace_wide_blocks_per_cu(uint32_t mode, bool records);
+// Batches that take that kernel by default, in rays per CU: a batch that leaves most
+// of the GPU idle is bound by the step latency of its longest rays, and a group
+// tests a node's six children at once.  Up to the lines every ray has a group of
+// its own, so waves claim without a counter (16,384 rays of the 1M-triangle scene
+// in plain order 149 -> 116 us); treelet order's two stacks let only half as many
+// be resident, and records make the second round cost more.  Eight lanes per ray
+// against one, camera rays of the 16,384-triangle sphere / the 1M-triangle scene, us:
+//   plain            32,768 rays 220 : 278 / 120 : 154, 40,960 rays 266 : 259 / 203 : 162
+//   plain, records   32,768 rays 326 : 345 / 183 : 204, 40,960 rays 362 : 328 / 267 : 216
+//   treelet          32,768 rays 235 : 253 / 212 : 217, 40,960 rays 189 : 186 / 226 : 217
+//   treelet, records 16,384 rays 260 : 293 / 214 : 251, 24,576 rays 238 : 227 / 277 : 270
+inline uint32_t wide_rays_per_cu(uint32_t mode, bool records) {
+  return mode == RTX_MODE_TREELET && records ? 64u : 128u;
+}
+// Rays at a time in a wave of that kernel: one while every ray can have a wave of
+// its own on one wave per SIMD, since the rays of a wave wait for each other's
+// passes (256 camera rays of the sphere in treelet order with records: one ray a
+// wave 122 us, two 132, four 143, eight 150; 2,048 rays take as long with one as
+// with eight)
+inline uint32_t wide_groups(uint64_t n, uint32_t n_cus) { return n <= 4ull * n_cus ? 1u : 8u; }
 // The level pass over p.n rays (p.ray_list / claim order as in launch_trace):
 // each hit's max_level becomes the maximum of the reference's final
 // tree_level_map.  p.lm_table must hold grid * 256 zeroed maps of p.lm_cap

@@ -34,9 +34,9 @@
 // keep their state until the wave's next refill, which writes their hit
 // records together.
 //
-// Small batches (at most 128 rays per CU in plain order, 256 in treelet
-// order) run trace_wide instead: eight lanes per ray, the six child boxes of
-// a node tested at once (see the section before its definition).
+// Small batches (wide_rays_per_cu) run trace_wide instead: eight lanes per ray,
+// the six child boxes of a node tested at once (see the section before its
+// definition).
 //
 // Treelet staging (STAGE > 0, one wave per workgroup): the wave keeps up to
 // stage/slot treelet images in LDS slots, copied from the treelet-contiguous
@@ -1477,7 +1477,10 @@ __global__ __launch_bounds__(kScanBlock) void scan_add(uint64_t* out, uint32_t n
 // are tested by lanes 0-5 of the group at once, so a traversal step issues a
 // fraction of the instructions of trace_kernel, whose lanes each test all six.
 // A batch too small to fill the GPU is bound by the step latency of its
-// longest rays, which this shortens.  The per-ray sequence of popped entries,
+// longest rays, which this shortens.  Slab records go to their row directly (one
+// store by the group's first lane): 256 rays of the 1M-triangle scene with records
+// take 127 -> 94 us in plain order and 179 -> 121 us in treelet order, the 32-ray
+// batch of the sphere 110 -> 79 us, of which the finishing launch is 10.  The per-ray sequence of popped entries,
 // and so every hit record and counter, is that of trace_kernel<MODE, false, K,
 // 0>: each list (one in plain order, two in treelet order) is an LDS array of
 // `cap` = K + spill_cap entries per ray, and a push fails exactly when the
@@ -1495,8 +1498,8 @@ __device__ __forceinline__ uint32_t byte_at(const Words16& n, int base, uint32_t
   return (w >> ((b & 3u) * 8u)) & 0xffu;
 }
 
-template <int MODE>
-__global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t cap) {
+template <int MODE, bool REC>
+__global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t cap, uint32_t groups) {
   constexpr uint32_t NS = MODE == 1 ? 2 : 1;
   __shared__ uint64_t stk[kWideBlock / kWideLanes][NS * kWideCap];
   const uint32_t tid = threadIdx.x;
@@ -1533,8 +1536,19 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
   bool has_e = false;
   uint64_t e = 0;
 
-  auto emit = [&](uint32_t size, uint32_t type) {
+  auto emit = [&](uint64_t off, uint32_t size, uint32_t type, uint32_t lvl) {
     if (type != RTX_TX_BVH_PRIMITIVE_LEAF_DESCRIPTOR) fetch_bytes += size;
+    if constexpr (REC) {
+      // straight to the ray's slab row
+      if (j == 0 && n_rec < p.record_slab) {
+        const uint32_t at = (uint32_t)(off >> 6), k = n_rec & ~7u;
+        if (p.rec_level_shift)
+          slab_place<uint32_t>(p.slabs, p.slabs_rest, p.record_slab, local_id, k)[n_rec & 7u] =
+              slab_entry4(at, type, lvl, p.rec_level_shift);
+        else
+          slab_place<uint64_t>(p.slabs, p.slabs_rest, p.record_slab, local_id, k)[n_rec & 7u] = slab_entry(at, type, lvl);
+      }
+    }
     n_rec++;
   };
   // lane 0 of the group writes; the group's later pops read it back in order
@@ -1658,6 +1672,7 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
       hq[3] = make_uint4(n_nodes, fetch_bytes, n_any, max_level);
     else if (j == 4)
       hq[4] = o4;
+    if (REC && j == 0) p.rec_counts[local_id] = n_rec;
     if (err && j == 0) {
       atomicOr(p.error, err);
       if (p.host_err) *reinterpret_cast<volatile uint32_t*>(p.host_err) = 1u;
@@ -1670,22 +1685,26 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
     tl_h0 = hq[0];
     tl_h1 = hq[1];
   }
-  const uint32_t groups = 64u / kWideLanes;
   while (true) {
     // ---- refill idle groups from the global ray counter (wave converged) ----
-    const uint64_t idle = __ballot(j == 0 && !active);
+    const uint64_t idle = __ballot(j == 0 && !active && gbase < groups * kWideLanes);
     const uint32_t nidle = (uint32_t)__popcll(idle);
     if (!exhausted && nidle > 0 && (nidle == groups || nidle * kWideLanes >= p.refill)) {
       if (pending) {
         write_hit();
         pending = false;
       }
-      const uint32_t leader = (uint32_t)__ffsll((long long)idle) - 1u;
-      uint32_t base = 0;
-      if (lane == leader) base = atomicAdd(p.ray_counter, nidle);
-      base = __shfl(base, (int)leader, 64);
-      if ((uint64_t)base + nidle >= p.n) exhausted = true;
-      if (!active) {
+      // a launch with a place for every ray takes them by wave: no counter
+      uint32_t base = (blockIdx.x * (kWideBlock / 64) + (tid >> 6)) * groups;
+      if ((uint64_t)gridDim.x * (kWideBlock / 64) * groups >= p.n) {
+        exhausted = true;
+      } else {
+        const uint32_t leader = (uint32_t)__ffsll((long long)idle) - 1u;
+        if (lane == leader) base = atomicAdd(p.ray_counter, nidle);
+        base = (uint32_t)__builtin_amdgcn_readlane((int)base, (int)leader);
+        if ((uint64_t)base + nidle >= p.n) exhausted = true;
+      }
+      if (!active && gbase < groups * kWideLanes) {
         const uint32_t k = base + (uint32_t)__popcll(idle & ((1ull << gbase) - 1ull));
         const uint32_t r = k < p.n ? claimed_ray(p, k) : 0u;
         if (k < p.n && r >= p.n_rays) {
@@ -1721,7 +1740,7 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
           if (tlas + 64 > bytes) {
             err |= kErrRange;
           } else {
-            emit(64, RTX_TX_BVH_STRUCTURE);
+            emit(tlas, 64, RTX_TX_BVH_STRUCTURE, 0);
             const uint64_t root = tlas + ((uint64_t)tl_h0.x | ((uint64_t)tl_h0.y << 32));
             const F3 lo = mk3(__uint_as_float(tl_h0.z), __uint_as_float(tl_h0.w), __uint_as_float(tl_h1.x));
             const F3 hi = mk3(__uint_as_float(tl_h1.y), __uint_as_float(tl_h1.z), __uint_as_float(tl_h1.w));
@@ -1777,14 +1796,14 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
                                __uint_as_float(b.x), __uint_as_float(b.y), __uint_as_float(b.z), __uint_as_float(b.w),
                                __uint_as_float(c.x), __uint_as_float(c.y), __uint_as_float(c.z), __uint_as_float(c.w)};
           const uint64_t bvh = (uint64_t)d.x | ((uint64_t)d.y << 32);
-          emit(128, RTX_TX_BVH_INSTANCE_LEAF);
+          emit(off, 128, RTX_TX_BVH_INSTANCE_LEAF, level);
           n_nodes++;
           const uint64_t blas = off + bvh;
           if ((blas & 63) || blas + 64 > bytes) {
             err |= kErrRange;
           } else {
             const uint2 ro2 = *reinterpret_cast<const uint2*>(A + blas);
-            emit(64, RTX_TX_BVH_STRUCTURE);
+            emit(blas, 64, RTX_TX_BVH_STRUCTURE, level);
             cur = transform_ray(m, ro, rd, rtmin, rtmax);
             cur_ok = slab_inputs_ok(cur.o, cur.d, cur.idir, cur.tmin, cur.tmax);
             cur_inst = slot;
@@ -1813,7 +1832,7 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
         if (off + 64 > bytes) {
           err |= kErrRange;
         } else {
-          emit(8, RTX_TX_BVH_PRIMITIVE_LEAF_DESCRIPTOR);
+          emit(off, 8, RTX_TX_BVH_PRIMITIVE_LEAF_DESCRIPTOR, level);
           const Words16 q = load64B(A + off);
           if (((q.w[1] >> 29) & 1u) == 0u) {
             if ((q.w[3] & 0x1ffffu) != 0u) err |= kErrType;
@@ -1835,7 +1854,7 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
               min_thit_obj = th;
               closest_leaf = slot;
               closest_inst = cur_inst;
-              emit(64, RTX_TX_BVH_QUAD_LEAF_HIT);
+              emit(off, 64, RTX_TX_BVH_QUAD_LEAF_HIT, level);
               n_nodes++;
               if (MODE == 0 && !(rflags & RTX_RAY_FLAG_OPAQUE)) n_any++;
               if (rflags & RTX_RAY_FLAG_TERMINATE_ON_FIRST_HIT) {
@@ -1844,11 +1863,11 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
                 depth = 0;
               }
             } else {
-              emit(64, RTX_TX_BVH_QUAD_LEAF);
+              emit(off, 64, RTX_TX_BVH_QUAD_LEAF, level);
               n_nodes++;
             }
           } else {
-            emit(64, RTX_TX_BVH_PROCEDURAL_LEAF);
+            emit(off, 64, RTX_TX_BVH_PROCEDURAL_LEAF, level);
             n_nodes++;
           }
         }
@@ -1862,7 +1881,7 @@ __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t
         const Words16 nd = load64B(A + off);
         // treelet order before the first switch: which children the first treelet owns
         const uint32_t cur_bits = (MODE == 1 && !phase2) ? first_bits(slot) : 0u;
-        emit(64, RTX_TX_BVH_INTERNAL_NODE);
+        emit(off, 64, RTX_TX_BVH_INTERNAL_NODE, level);
         n_nodes++;
         const bool top = (flags & kFlTop) != 0;
         const F3 sc = child_scales((int)(int8_t)byte_of(nd, 18), (int)(int8_t)byte_of(nd, 19), (int)(int8_t)byte_of(nd, 20));
@@ -2426,20 +2445,26 @@ hipError_t launch_level_pass(const TraceParams& p, uint32_t mode, uint32_t grid,
   return launch_fn(f, p, grid, 256, s);
 }
 
-hipError_t launch_trace_wide(const TraceParams& p, uint32_t mode, uint32_t cap, uint32_t grid, hipStream_t s) {
-  if (cap > kWideCap) return hipErrorInvalidValue;
-  if (mode == RTX_MODE_PLAIN)
-    hipLaunchKernelGGL(trace_wide<0>, dim3(grid), dim3(kWideBlock), 0, s, p, cap);
-  else
-    hipLaunchKernelGGL(trace_wide<1>, dim3(grid), dim3(kWideBlock), 0, s, p, cap);
+namespace {
+typedef void (*WideFn)(TraceParams, uint32_t, uint32_t);
+WideFn pick_wide(uint32_t mode, bool records) {
+  if (mode == RTX_MODE_PLAIN) return records ? trace_wide<0, true> : trace_wide<0, false>;
+  return records ? trace_wide<1, true> : trace_wide<1, false>;
+}
+}  // namespace
+
+hipError_t launch_trace_wide(const TraceParams& p, uint32_t mode, bool records, uint32_t cap, uint32_t grid,
+                             uint32_t groups, hipStream_t s) {
+  if (cap > kWideCap || groups < 1 || groups > 64 / kWideLanes) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(pick_wide(mode, records), dim3(grid), dim3(kWideBlock), 0, s, p, cap, groups);
   return hipGetLastError();
 }
 
-uint32_t trace_wide_blocks_per_cu(uint32_t mode) {
+uint32_t trace_wide_blocks_per_cu(uint32_t mode, bool records) {
   int nb = 0;
-  const void* f = mode == RTX_MODE_PLAIN ? reinterpret_cast<const void*>(trace_wide<0>)
-                                         : reinterpret_cast<const void*>(trace_wide<1>);
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, (int)kWideBlock, 0) != hipSuccess) return 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void*>(pick_wide(mode, records)),
+                                                   (int)kWideBlock, 0) != hipSuccess)
+    return 0;
   return nb > 0 ? (uint32_t)nb : 0u;
 }
 
