@@ -185,8 +185,13 @@ uint32_t slab4_shift(const SceneCheck& ck, uint64_t bytes) {
   return slot_bits + level_bits <= kSlab4TypeShift ? slot_bits : 0;
 }
 
+// A launch that fills the GPU gets room for any such launch (treelet order, four
+// blocks on a CU, 544 MiB on 256 CUs), so that one with another option later does
+// not free and allocate again (0.6 ms).
 rtx_status ensure_spill(rtx_ctx* c, size_t entries) {
   if (entries <= c->spill_entries) return RTX_OK;
+  const size_t full = (size_t)c->n_cus * 1024 * (128 + 8) * 2;
+  if (entries > full / 4) entries = std::max(entries, full);
   if (c->spill) HIP_TRY(hipFree(c->spill));
   c->spill = nullptr;
   c->spill_entries = 0;
@@ -712,7 +717,7 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
   // treelet order with staging or records keeps fewer entries in LDS (trace_kernel's R)
   // (the eight-lanes kernel spills nothing; a second pass of its rays may)
   const uint32_t spill_grid = wide ? (n + bs - 1) / bs : grid;
-  rtx_status st = ensure_spill(c, (size_t)spill_grid * bs * (spill_cap + (stage || use_slab ? lds_stack : 0)) * ns);
+  rtx_status st = ensure_spill(c, (size_t)spill_grid * bs * (spill_cap + (ns == 2 && (stage || use_slab) ? lds_stack : 0)) * ns);
   if (st != RTX_OK) return st;
 
   TraceParams p{};
