@@ -187,3 +187,28 @@ def test_training_matches_oracle_steps(gpu, T, C, n, batch):
         assert np.linalg.norm(grads - g) <= 0.1 * np.linalg.norm(g)
     finally:
         mlp.close()
+
+
+@pytest.mark.parametrize("order", ["up", "down", "equal", "steps", "wide"])
+@pytest.mark.parametrize("T,C,n", [(9, 4, 3), (9, 127, 70), (9, 129, 64), (9, 700, 17), (9, 3001, 300)])
+def test_predict_of_ordered_classes(gpu, T, C, n, order):
+    """Logits that are the class biases alone (zero weights): every class better than all
+    before it, none after the first four, all equal, equal in runs, and a spread whose
+    exponentials over- and underflow.  Equal logits go to the lower class.  The logits
+    are exact, and a sum of at most 3,001 exponentials in FP32, each within 2^-22, in
+    chains of at most 400, is within 400 * 2^-24 + 2^-22 < 3e-5 of its value."""
+    c = np.arange(C, dtype=np.float32)
+    o = dict(up=c * 0.01, down=-c * 0.01, equal=0 * c + 0.25, steps=np.floor(c / 37) % 5, wide=((c * 89) % C) / C * 180 - 90)[order]
+    mlp = gpu.mlp(T, C, seed=1)
+    try:
+        p = np.zeros_like(mlp.params())
+        p[-C:] = o.astype(np.float32)
+        mlp.set_params(p)
+        top, prob = mlp.predict(_samples(np.random.default_rng(C), T, C, n))
+        o = p[-C:].astype(np.float64)
+        best = np.argsort(-o, kind="stable")[:4]
+        assert np.array_equal(top, np.tile(best.astype(np.uint32), (n, 1)))
+        e = np.exp(o - o.max())
+        assert np.allclose(prob, np.tile((e / e.sum())[best], (n, 1)), rtol=3e-5, atol=1e-30)
+    finally:
+        mlp.close()

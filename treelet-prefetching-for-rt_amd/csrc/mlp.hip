@@ -503,7 +503,7 @@ __global__ __launch_bounds__(256) void weight_grads(WeightGrad w1, WeightGrad w2
 // stage.  1,024 rows x 16,384 classes: statistics 28 -> 12 us, both gradients 54
 // -> 22 us.  Bound by VALU work on each logit, the exponential above all.
 constexpr int kCeChunk = 256;  // classes per ce_stats wave
-constexpr int kCeCls = 256;    // classes per LDS stage of logits_top4
+constexpr int kCeCls = 128;    // classes per LDS stage of logits_top4
 constexpr int kCeRange = 512;  // classes per ce_grad wave that sums dQ
 
 // Eight FP32 values rounded to BF16 (round to nearest even, as the MFMA operand
@@ -770,17 +770,19 @@ struct Top4 {
 };
 static_assert(sizeof(Top4) == 40, "partial results are stored as Top4");
 
+// x into the list, when it is greater than the last one; classes come in ascending
+// order, so an equal value stays behind.  No branches: 15 instructions.
 __device__ __forceinline__ void top4_insert(Top4& t, float x, int c) {
-  // x > t.v[3]; classes come in ascending order, so an equal value stays behind
-  const bool b0 = x > t.v[0], b1 = x > t.v[1], b2 = x > t.v[2];
-  t.v[3] = b2 ? t.v[2] : x;
-  t.c[3] = b2 ? t.c[2] : c;
-  t.v[2] = b2 ? (b1 ? t.v[1] : x) : t.v[2];
-  t.c[2] = b2 ? (b1 ? t.c[1] : c) : t.c[2];
-  t.v[1] = b1 ? (b0 ? t.v[0] : x) : t.v[1];
-  t.c[1] = b1 ? (b0 ? t.c[0] : c) : t.c[1];
+  const bool b0 = x > t.v[0], b1 = x > t.v[1], b2 = x > t.v[2], b3 = x > t.v[3];
+  auto pick = [](bool b, int a, int other) { return b ? a : other; };
+  t.c[3] = pick(b2, t.c[2], pick(b3, c, t.c[3]));
+  t.c[2] = pick(b1, t.c[1], pick(b2, c, t.c[2]));
+  t.c[1] = pick(b0, t.c[0], pick(b1, c, t.c[1]));
+  t.c[0] = pick(b0, c, t.c[0]);
+  t.v[3] = __builtin_amdgcn_fmed3f(t.v[2], t.v[3], x);
+  t.v[2] = __builtin_amdgcn_fmed3f(t.v[1], t.v[2], x);
+  t.v[1] = __builtin_amdgcn_fmed3f(t.v[0], t.v[1], x);
   t.v[0] = b0 ? x : t.v[0];
-  t.c[0] = b0 ? c : t.c[0];
 }
 
 __device__ __forceinline__ bool top4_before(float v, int c, float v2, int c2) {
@@ -826,9 +828,16 @@ __device__ __forceinline__ void top4_merge(Top4& t, const Top4& o) {
 // columns the wave's samples, so a lane keeps one sample's best four over a
 // quarter of the classes, in registers, and the logits are never stored: 20,011
 // samples x 16,384 classes wrote and read 1.3 GB of them twice (3.4 ms in five
-// products and five scans) and take 0.26 ms here.  Bound by the VALU work on each
-// logit: the insertions of a list's first few hundred classes, then its compare
-// and exponential.
+// products and five scans) and take 0.18 ms here.  Bound by the VALU work on each
+// logit: its compare and exponential, then the insertions.  Some lane of a wave
+// has a better logit in nearly every step, so the lanes only put theirs aside
+// (kAside of them, in LDS) and insert together once one lane's places run out;
+// inserting in each step took 0.26 ms.  A lane passes over what the same sample's
+// other three lanes already have four better ones of (equal ones stay: the lower
+// class wins, and only a lane's own classes come in order).  Each class split
+// starts with empty lists, so there are only as many as one round of workgroups
+// has room for (kPredBlocks): with two rounds, and stages of 256 classes, 0.23 ms.
+constexpr int kAside = 11;
 __global__ __launch_bounds__(256) void logits_top4(const float* __restrict__ Q, int n, const float* __restrict__ O,
                                                    const float* __restrict__ cb, int C, int cper, Top4* part) {
   __shared__ uint4 Os[kCeCls * 4];
@@ -836,6 +845,8 @@ __global__ __launch_bounds__(256) void logits_top4(const float* __restrict__ Q, 
   const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
   const int row = blockIdx.x * 64 + (threadIdx.x >> 6) * 16 + c16;
   const bf16x8 b = ld_row8(Q, n, row, 8 * g);
+  __shared__ float aside_v[kAside][256];
+  __shared__ int aside_c[kAside][256];
   Top4 t;
   for (int k = 0; k < 4; ++k) {
     t.v[k] = -INFINITY;
@@ -843,6 +854,26 @@ __global__ __launch_bounds__(256) void logits_top4(const float* __restrict__ Q, 
   }
   t.m = -INFINITY;
   t.s = 0.f;
+  int held = 0;  // logits put aside
+  float least = -INFINITY, most = -INFINITY;  // what a logit has to exceed; the greatest so far
+  // insert them, and refer the exp-sum to the greatest logit
+  auto insert_held = [&]() {
+    for (int k = 0; __ballot(k < held); ++k) {
+      const float v = aside_v[k][threadIdx.x];
+      const int c = aside_c[k][threadIdx.x];
+      top4_insert(t, k < held ? v : -INFINITY, c);
+    }
+    held = 0;
+    float other = fmaxf(__shfl_xor(t.v[3], 16, 64), __shfl_xor(t.v[3], 32, 64));
+    other = fmaxf(other, __shfl_xor(t.v[3], 48, 64));
+    const uint32_t u = __float_as_uint(other);  // the next float below it
+    const float below = __uint_as_float((int)u > 0 ? u - 1u : (u << 1) == 0u ? 0x80000001u : u + 1u);
+    least = other > -INFINITY ? fmaxf(t.v[3], below) : t.v[3];
+    if (most > t.m) {
+      t.s *= expf(t.m - most);
+      t.m = most;
+    }
+  };
   const int cbeg = blockIdx.y * cper, cend = min(C, cbeg + cper);
   for (int cc = cbeg; cc < cend; cc += kCeCls) {
     const int nc = min(kCeCls, cend - cc);
@@ -851,24 +882,43 @@ __global__ __launch_bounds__(256) void logits_top4(const float* __restrict__ Q, 
     // a class past the end has a logit of -inf
     for (int i = threadIdx.x; i < kCeCls; i += blockDim.x) cbs[i] = i < nc ? cb[cc + i] : -INFINITY;
     __syncthreads();
-    for (int ct = 0; ct < nc; ct += 16) {
-      const bf16x8 a = lds_row8(Os, ct + c16, g, ct + c16 < nc);
-      const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-      const float4 bias = *reinterpret_cast<const float4*>(cbs + ct + 4 * g);
-      const float x[4] = {acc[0] + bias.x, acc[1] + bias.y, acc[2] + bias.z, acc[3] + bias.w};
-      const float mx = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
-      if (mx > t.v[3]) {
+    for (int ct = 0; ct < nc; ct += 32) {  // two tiles at a time
+      float x[8];
+      f32x4 acc[2];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (x[i] > t.v[3]) top4_insert(t, x[i], cc + ct + 4 * g + i);
-        if (mx > t.m) {
-          t.s *= expf(t.m - mx);
-          t.m = mx;
-        }
+      for (int h = 0; h < 2; ++h)
+        acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lds_row8(Os, ct + 16 * h + c16, g, ct + 16 * h + c16 < nc), b,
+                                                         f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const float4 bias = *reinterpret_cast<const float4*>(cbs + ct + 16 * h + 4 * g);
+        x[4 * h] = acc[h][0] + bias.x;
+        x[4 * h + 1] = acc[h][1] + bias.y;
+        x[4 * h + 2] = acc[h][2] + bias.z;
+        x[4 * h + 3] = acc[h][3] + bias.w;
       }
-      if (t.m > -INFINITY) t.s += (exp_term(x[0] - t.m) + exp_term(x[1] - t.m)) + (exp_term(x[2] - t.m) + exp_term(x[3] - t.m));
+      const float mx = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
+      if (mx > least) {
+        most = fmaxf(most, mx);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (x[i] > least) {
+            aside_v[held][threadIdx.x] = x[i];
+            aside_c[held][threadIdx.x] = cc + ct + 16 * (i >> 2) + 4 * g + (i & 3);
+            held++;
+          }
+      }
+      // (the exponentials stay below 2^47 by the second)
+      if (__ballot(held > kAside - 8 || mx > t.m + 32.f)) {
+        most = fmaxf(most, mx);
+        insert_held();
+      }
+      if (t.m > -INFINITY)
+        t.s += ((exp_term(x[0] - t.m) + exp_term(x[1] - t.m)) + (exp_term(x[2] - t.m) + exp_term(x[3] - t.m))) +
+               ((exp_term(x[4] - t.m) + exp_term(x[5] - t.m)) + (exp_term(x[6] - t.m) + exp_term(x[7] - t.m)));
     }
   }
+  insert_held();
   // the four lane groups hold quarters of the same rows' classes
   for (int o = 16; o < 64; o <<= 1) {
     Top4 u;
@@ -1009,8 +1059,8 @@ hipError_t pack(rtx_mlp* m, bool train) {
 }
 
 // Prediction: rows per pass, (row, class split) results it keeps (at most
-// 10 MB), and the workgroups it aims at (eight per CU).
-constexpr uint32_t kPredRows = 65536, kPredParts = 4 * kPredRows, kPredBlocks = 2048;
+// 10 MB), and the most workgroups it aims at (the five that a CU holds).
+constexpr uint32_t kPredRows = 65536, kPredParts = 4 * kPredRows, kPredBlocks = 1280;
 
 // Batches of at most this many rows accumulate in 64-deep partial products.
 constexpr uint32_t kChunkedRows = 1984;
@@ -1231,7 +1281,7 @@ rtx_status rtx_mlp_predict(rtx_mlp* m, const rtx_mlp_sample* samples, uint32_t n
     const uint32_t b = std::min(kPredRows, n - b0);
     // class splits: enough workgroups for the chip, of whole LDS stages
     const uint32_t row_blocks = (b + 63) / 64;
-    uint32_t splits = std::max(1u, std::min((kPredBlocks + row_blocks - 1) / row_blocks, (m->C + kCeCls - 1) / kCeCls));
+    uint32_t splits = std::max(1u, std::min(kPredBlocks / row_blocks, (m->C + 2 * kCeCls - 1) / (2 * kCeCls)));
     splits = std::min(splits, std::max(1u, kPredParts / b));
     const uint32_t stages = ((m->C + kCeCls - 1) / kCeCls + splits - 1) / splits;
     const int cper = (int)(stages * kCeCls);
