@@ -114,10 +114,11 @@ struct rtx_ctx {
   std::vector<rtx_batch_graph*> graphs;
   // rtx_trace_static: this device's copy of the static scratch array (from
   // hipGetSymbolAddress) and the occupancy of the kernels it may launch,
-  // [mode][lds_stack 4/8/16] and the eight-lanes-per-ray kernels [mode]
+  // [mode][lds_stack 4/8/16] and the eight-lanes-per-ray kernels
+  // [mode][rays a wave 1/2/4/8]
   uint8_t* static_scratch = nullptr;
   uint32_t static_occ[2][3] = {{0, 0, 0}, {0, 0, 0}};
-  uint32_t static_wide_occ[2] = {0, 0};
+  uint32_t static_wide_occ[2][4] = {};
 };
 
 struct rtx_batch_graph {
@@ -230,7 +231,7 @@ uint32_t cached_blocks_per_cu(rtx_ctx* c, uint32_t mode, uint32_t lds_stack, uin
   const uint64_t key = ((uint64_t)mode << 48) | ((uint64_t)records << 40) | ((uint64_t)lds_stack << 32) | stage;
   auto it = c->occupancy.find(key);
   if (it != c->occupancy.end()) return it->second;
-  const uint32_t b = mode >= kWideOccupancyKey ? trace_wide_blocks_per_cu(mode - kWideOccupancyKey, records != kRecNone)
+  const uint32_t b = mode >= kWideOccupancyKey ? trace_wide_blocks_per_cu(mode - kWideOccupancyKey, records != kRecNone, lds_stack)
                                                : trace_blocks_per_cu(mode, records, lds_stack, stage);
   c->occupancy[key] = b;
   return b;
@@ -362,7 +363,7 @@ rtx_status rtx_create(int device, rtx_ctx** out) {
   const uint32_t ks[3] = {4, 8, 16};
   for (uint32_t m = 0; m < 2; ++m) {
     for (int k = 0; k < 3; ++k) c->static_occ[m][k] = trace_blocks_per_cu(m, kRecNone, ks[k], 0);
-    c->static_wide_occ[m] = trace_wide_blocks_per_cu(m, false);
+    for (uint32_t g = 0; g < 4; ++g) c->static_wide_occ[m][g] = trace_wide_blocks_per_cu(m, false, 1u << g);
   }
   *out = c;
   return RTX_OK;
@@ -702,13 +703,13 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
                     (opts->lanes_per_ray == 0 && stage == 0 && (!opts->emit_records || use_slab) &&
                      (uint64_t)n <= (uint64_t)wide_rays_per_cu(opts->mode, opts->emit_records) * c->n_cus);
   const uint32_t bs = trace_block_size(stage);
+  const uint32_t groups = wide ? wide_groups(n, (uint32_t)c->n_cus) : 1u;
   // persistent blocks: by default as many as fit on a CU at once
   uint32_t blocks_per_cu = opts->waves_per_cu ? std::max(1u, opts->waves_per_cu * 64 / bs)
-                           : wide             ? cached_blocks_per_cu(c, kWideOccupancyKey + opts->mode, 0, 0, main_rec)
+                           : wide             ? cached_blocks_per_cu(c, kWideOccupancyKey + opts->mode, groups, 0, main_rec)
                                               : cached_blocks_per_cu(c, opts->mode, lds_stack, stage, main_rec);
   if (blocks_per_cu == 0) blocks_per_cu = 16 * 64 / bs;
   uint32_t grid = (uint32_t)c->n_cus * blocks_per_cu;
-  const uint32_t groups = wide ? wide_groups(n, (uint32_t)c->n_cus) : 1u;
   const uint64_t lanes = (uint64_t)n * (wide ? 64u / groups : 1u);
   grid = (uint32_t)std::min<uint64_t>(grid, (lanes + bs - 1) / bs);
   grid = std::max(grid, 1u);
@@ -1001,12 +1002,12 @@ rtx_status rtx_trace_static(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const r
   const bool wide = opts->lanes_per_ray == kWideRayLanes ||
                     (opts->lanes_per_ray == 0 &&
                      (uint64_t)n <= (uint64_t)wide_rays_per_cu(opts->mode, false) * c->n_cus);
+  const uint32_t groups = wide ? wide_groups(n, (uint32_t)c->n_cus) : 1u;
   const uint32_t bs = 256;
   uint32_t per_cu = opts->waves_per_cu ? std::max(1u, opts->waves_per_cu * 64 / bs)
-                    : wide             ? c->static_wide_occ[opts->mode]
+                    : wide             ? c->static_wide_occ[opts->mode][__builtin_ctz(groups)]
                                        : c->static_occ[opts->mode][ki];
   if (per_cu == 0) per_cu = 4;
-  const uint32_t groups = wide ? wide_groups(n, (uint32_t)c->n_cus) : 1u;
   const uint64_t lanes = (uint64_t)n * (wide ? 64u / groups : 1u);
   uint32_t grid = (uint32_t)std::min<uint64_t>((uint64_t)c->n_cus * per_cu, (lanes + bs - 1) / bs);
   grid = std::max(grid, 1u);

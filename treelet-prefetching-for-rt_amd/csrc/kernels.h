@@ -135,7 +135,7 @@ uint32_t trace_batch_blocks_per_cu(uint32_t mode, uint32_t lds_stack);
 constexpr uint32_t kWideRayLanes = 8;
 hipError_t launch_trace_wide(const TraceParams& p, uint32_t mode, bool records, uint32_t cap, uint32_t grid,
                              uint32_t groups, hipStream_t s);
-uint32_t trace_wide_blocks_per_cu(uint32_t mode, bool records);
+uint32_t trace_wide_blocks_per_cu(uint32_t mode, bool records, uint32_t groups);
 // Batches that take that kernel by default, in rays per CU: a batch that leaves most
 // of the GPU idle is bound by the step latency of its longest rays, and a group
 // tests a node's six children at once.  Up to the lines every ray has a group of
@@ -150,12 +150,16 @@ uint32_t trace_wide_blocks_per_cu(uint32_t mode, bool records);
 inline uint32_t wide_rays_per_cu(uint32_t mode, bool records) {
   return mode == RTX_MODE_TREELET && records ? 64u : 128u;
 }
-// Rays at a time in a wave of that kernel: one while every ray can have a wave of
-// its own on one wave per SIMD, since the rays of a wave wait for each other's
-// passes (256 camera rays of the sphere in treelet order with records: one ray a
-// wave 122 us, two 132, four 143, eight 150; 2,048 rays take as long with one as
-// with eight)
-inline uint32_t wide_groups(uint64_t n, uint32_t n_cus) { return n <= 4ull * n_cus ? 1u : 8u; }
+// Rays at a time in a wave of that kernel: the fewest with which all are resident
+// (16 waves on a CU), since the rays of a wave wait for each other's passes.  Camera
+// rays of the 16,384-triangle sphere in plain order, one / two / four / eight a wave, us:
+//    4,096 rays 152 / 188 / 198 / 213,  8,192 rays 235 / 178 / 208 / 230,
+//   16,384 rays 345 / 273 / 210 / 223
+inline uint32_t wide_groups(uint64_t n, uint32_t n_cus) {
+  uint32_t groups = 1;
+  while (groups < 8 && n > 16ull * n_cus * groups) groups *= 2;
+  return groups;
+}
 // The level pass over p.n rays (p.ray_list / claim order as in launch_trace):
 // each hit's max_level becomes the maximum of the reference's final
 // tree_level_map.  p.lm_table must hold grid * 256 zeroed maps of p.lm_cap

@@ -1501,13 +1501,14 @@ __device__ __forceinline__ uint32_t byte_at(const Words16& n, int base, uint32_t
 template <int MODE, bool REC>
 __global__ __launch_bounds__(kWideBlock) void trace_wide(TraceParams p, uint32_t cap, uint32_t groups) {
   constexpr uint32_t NS = MODE == 1 ? 2 : 1;
-  __shared__ uint64_t stk[kWideBlock / kWideLanes][NS * kWideCap];
+  extern __shared__ uint64_t wide_stk[];  // NS * kWideCap entries per ray (wide_lds_bytes)
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & 63u;
   const uint32_t j = tid & (kWideLanes - 1);
   const uint32_t gbase = lane & ~(kWideLanes - 1);  // the group's first lane in the wave
-  lds_u64* sta = (lds_u64*)&stk[tid / kWideLanes][0];
-  lds_u64* stb = (lds_u64*)&stk[tid / kWideLanes][(NS - 1) * kWideCap];
+  // (groups past the launch's limit hold no ray)
+  lds_u64* sta = (lds_u64*)wide_stk + ((tid >> 6) * groups + min(gbase / kWideLanes, groups - 1u)) * (NS * kWideCap);
+  lds_u64* stb = sta + (NS - 1) * kWideCap;
   const uint8_t* __restrict__ A = p.arena;
   const uint64_t bytes = p.arena_bytes;
   const uint64_t tlas = p.tlas;
@@ -2451,19 +2452,23 @@ WideFn pick_wide(uint32_t mode, bool records) {
   if (mode == RTX_MODE_PLAIN) return records ? trace_wide<0, true> : trace_wide<0, false>;
   return records ? trace_wide<1, true> : trace_wide<1, false>;
 }
+uint32_t wide_lds_bytes(uint32_t mode, uint32_t groups) {
+  return kWideBlock / 64 * groups * (mode == RTX_MODE_PLAIN ? 1u : 2u) * kWideCap * (uint32_t)sizeof(uint64_t);
+}
 }  // namespace
 
 hipError_t launch_trace_wide(const TraceParams& p, uint32_t mode, bool records, uint32_t cap, uint32_t grid,
                              uint32_t groups, hipStream_t s) {
   if (cap > kWideCap || groups < 1 || groups > 64 / kWideLanes) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(pick_wide(mode, records), dim3(grid), dim3(kWideBlock), 0, s, p, cap, groups);
+  hipLaunchKernelGGL(pick_wide(mode, records), dim3(grid), dim3(kWideBlock), wide_lds_bytes(mode, groups), s, p, cap,
+                     groups);
   return hipGetLastError();
 }
 
-uint32_t trace_wide_blocks_per_cu(uint32_t mode, bool records) {
+uint32_t trace_wide_blocks_per_cu(uint32_t mode, bool records, uint32_t groups) {
   int nb = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void*>(pick_wide(mode, records)),
-                                                   (int)kWideBlock, 0) != hipSuccess)
+                                                   (int)kWideBlock, wide_lds_bytes(mode, groups)) != hipSuccess)
     return 0;
   return nb > 0 ? (uint32_t)nb : 0u;
 }
