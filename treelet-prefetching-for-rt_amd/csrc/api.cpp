@@ -186,6 +186,15 @@ uint32_t slab4_shift(const SceneCheck& ck, uint64_t bytes) {
   return slot_bits + level_bits <= kSlab4TypeShift ? slot_bits : 0;
 }
 
+// Idle lanes a wave refills at.  New rays mixed among old ones cost a wave its
+// coherence, waiting for more idle lanes costs occupied ones; rays of large scenes
+// take more steps and are incoherent anyway.  1.31M camera and bounce rays, 48 / 40 /
+// 28 lanes, us: plain order on 90 MB of nodes 510 / 533 / 617, on 360 MB 682 / 690 /
+// 709, on 528 MB 754 / 752 / 752, on 720 MB 847 / 848 / 829; treelet order on 90 MB
+// 626 / 631 / 674, on 360 MB 938 / 942 / 925, on 720 MB 1149 / 1159 / 1128; 2.6M rays
+// on 1.8 GB in plain order 1398 / 1384 / 1356.
+uint32_t default_refill(uint64_t arena_bytes) { return arena_bytes > (400ull << 20) ? 28u : 48u; }
+
 // A launch that fills the GPU gets room for any such launch (treelet order, four
 // blocks on a CU, 544 MiB on 256 CUs), so that one with another option later does
 // not free and allocate again (0.6 ms).
@@ -728,10 +737,7 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
   p.rays = rays;
   p.n = n;
   if (opts->refill > 64) return RTX_ERR_INVALID_ARGUMENT;
-  // default refill: 40 idle lanes (on the 1M-triangle diffuse batch 2.6 %
-  // faster than 32 and 0.5 % slower than 48; on the 21M-triangle scene 0.2 %
-  // faster than 32 and 1.2 % faster than 48)
-  p.refill = opts->refill ? opts->refill : 40;
+  p.refill = opts->refill ? opts->refill : default_refill(c->arena_bytes);
   p.ordered_boxes = c->ordered ? 1u : 0u;
   p.regular_nodes = c->regular ? 1u : 0u;
   p.hits = hits;
@@ -1030,7 +1036,7 @@ rtx_status rtx_trace_static(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const r
   p.tlas = c->tlas;
   p.rays = rays;
   p.n = n;
-  p.refill = opts->refill ? opts->refill : 40;
+  p.refill = opts->refill ? opts->refill : default_refill(c->arena_bytes);
   p.ordered_boxes = c->ordered ? 1u : 0u;
   p.regular_nodes = c->regular ? 1u : 0u;
   p.hits = hits;
