@@ -113,3 +113,30 @@ def test_rays_through_box_corners_match_the_oracle(gpu, oracle, instanced, mode,
     assert_hits_equal(h, h_ref, "records")
     assert_records_equal(o, r, o_ref, r_ref, "records")
     assert_hits_equal(gpu.trace(rays, mode=mode, lanes_per_ray=1), h_ref, "hits")
+
+
+def test_a_batch_reports_a_malformed_leaf_and_the_next_one_none(gpu, rtx, instanced):
+    """A leaf of an unknown kind under one scene of a batch: launched directly and from a
+    graph, the batch reports it each time, and a batch without that scene does not."""
+    scene, rays = instanced
+    bad = scene.arena.copy()
+    for off in _internal_nodes(bad, scene.tlas_offset)[1:]:
+        c = off + 64 * int(bad[off + 12:off + 16].view(np.int32)[0])
+        for i in range(6):
+            size, kind = int(bad[off + 22 + i]) & 3, (int(bad[off + 22 + i]) >> 2) & 15
+            if size == 1 and kind:
+                bad[c + 12] |= 1
+            c += 64 * size
+    n = len(rays)
+    jobs = []
+    for arena in (scene.arena, bad):
+        sid = gpu.add_scene(arena, scene.tlas_offset)
+        jobs.append((sid, gpu.to_device(rays), n, gpu.buffer(n * rtx.HIT_DTYPE.itemsize)))
+    good, mixed = gpu.batch_graph(jobs[:1]), gpu.batch_graph(jobs)
+    try:
+        for _ in range(2):
+            assert gpu.trace_batch(jobs[:1]) == 0 and good.launch()[0] == 0
+            assert gpu.trace_batch(jobs) == 2 and mixed.launch()[0] == 2 and mixed.launch(2)[0] == 2
+    finally:
+        good.close()
+        mixed.close()

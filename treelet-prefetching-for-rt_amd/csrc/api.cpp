@@ -1289,6 +1289,7 @@ TraceParams batch_params(rtx_ctx* c, const BatchJob* jobs_dev, uint32_t n_jobs, 
   p.spill_cap = kBatchSpillCap;
   p.ray_counter = counters;
   p.error = counters + 1;
+  p.host_err = c->err_host_dev;
   p.stats = c->stats;
   p.jobs = jobs_dev;
   p.n_jobs = n_jobs;
@@ -1312,6 +1313,15 @@ bool batch_needs_levels(const rtx_ctx* c, const rtx_batch_job* jobs, uint32_t n_
 // launch (capturable: the ray counter is cleared by a kernel, and the error
 // word, counters[1], collects the passes' errors with the batch's).  `spill`
 // holds kBatchSpillCap entries per list for min(n_cus, rays / 256) workgroups.
+// After a batch's launches have run: an error-free one needs no read-back (a ray
+// error also sets the mapped host word).
+rtx_status batch_error(rtx_ctx* c, const uint32_t* counters) {
+  if (*static_cast<volatile uint32_t*>(c->err_host) == 0) return RTX_OK;
+  uint32_t err = 0;
+  HIP_TRY(hipMemcpy(&err, counters + 1, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  return kernel_error_status(err);
+}
+
 hipError_t batch_level_passes(rtx_ctx* c, const std::vector<BatchJob>& hj, const rtx_batch_job* jobs,
                               uint32_t n_jobs, uint32_t mode, uint64_t* spill, uint32_t* counters, hipStream_t s) {
   for (uint32_t j = 0; j < n_jobs; ++j) {
@@ -1333,6 +1343,7 @@ hipError_t batch_level_passes(rtx_ctx* c, const std::vector<BatchJob>& hj, const
     p.spill_cap = kBatchSpillCap;
     p.ray_counter = counters;
     p.error = counters + 1;
+    p.host_err = c->err_host_dev;
     p.stats = c->stats;
     set_level_maps(p, c->lm_mem, (uint64_t)c->n_cus * kBlock);
     const uint32_t grid = std::max(1u, std::min<uint32_t>(c->n_cus, (hj[j].n + kBlock - 1) / kBlock));
@@ -1407,15 +1418,14 @@ rtx_status rtx_trace_batch(rtx_ctx* c, const rtx_batch_job* jobs, uint32_t n_job
   }
   TraceParams p = batch_params(c, c->jobs_dev, n_jobs, total, s, c->spill, c->counters);
   c->kernel_timed = false;
+  *static_cast<volatile uint32_t*>(c->err_host) = 0;
   HIP_TRY(hipEventRecord(c->evk0, c->stream));
   HIP_TRY(launch_trace_batch(p, o->mode, s.lds_stack, s.grid, c->stream));
   HIP_TRY(hipEventRecord(c->evk1, c->stream));
   c->kernel_timed = true;
   if (levels) HIP_TRY(batch_level_passes(c, hj, jobs, n_jobs, o->mode, c->spill, c->counters, c->stream));
-  uint32_t err = 0;
-  HIP_TRY(hipMemcpyAsync(&err, c->counters + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
-  return kernel_error_status(err);
+  return batch_error(c, c->counters);
 }
 
 rtx_status rtx_batch_graph_create(rtx_ctx* c, const rtx_batch_job* jobs, uint32_t n_jobs,
@@ -1476,14 +1486,13 @@ rtx_status rtx_batch_graph_launch(rtx_batch_graph* g, uint32_t replays, float* m
   for (const auto& d : g->deps)
     if (c->scenes[d.first].part_gen != d.second) return RTX_ERR_STALE;
   HIP_TRY(hipSetDevice(c->device));
+  *static_cast<volatile uint32_t*>(c->err_host) = 0;
   HIP_TRY(hipEventRecord(c->ev0, c->stream));
   for (uint32_t r = 0; r < replays; ++r) HIP_TRY(hipGraphLaunch(g->exec, c->stream));
   HIP_TRY(hipEventRecord(c->ev1, c->stream));
-  uint32_t err = 0;
-  HIP_TRY(hipMemcpyAsync(&err, g->counters + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   if (ms) HIP_TRY(hipEventElapsedTime(ms, c->ev0, c->ev1));
-  return kernel_error_status(err);
+  return batch_error(c, g->counters);
 }
 
 rtx_status rtx_batch_graph_destroy(rtx_batch_graph* g) {

@@ -80,8 +80,7 @@ struct TraceParams {
   uint32_t* ray_counter;
   uint32_t* error;
   unsigned long long* stats;  // rtx_prefetch_stats counters
-  // single-scene launches: a mapped host word set to 1 when any ray reports
-  // an error
+  // a mapped host word set to 1 when any ray reports an error
   uint32_t* host_err;
   // treelet staging
   uint32_t prefetch;                 // RTX_PREFETCH_*
