@@ -500,8 +500,8 @@ __global__ __launch_bounds__(256) void weight_grads(WeightGrad w1, WeightGrad w2
 // 16-byte load per lane from L2, used for two tiles: rows staged through LDS had
 // cost sixteen 2-byte LDS reads per lane and 32 classes for the transposed
 // operand, the FP32 conversions again in each workgroup and two barriers per
-// stage.  1,024 rows x 16,384 classes: statistics 28 -> 12 us, both gradients 54
-// -> 22 us.  Bound by VALU work on each logit, the exponential above all.
+// stage.  1,024 rows x 16,384 classes: statistics 28 -> 17 us, both gradients 54
+// -> 31 us.  Bound by VALU work on each logit, the exponential above all.
 constexpr int kCeChunk = 256;  // classes per ce_stats wave
 constexpr int kCeCls = 128;    // classes per LDS stage of logits_top4
 constexpr int kCeRange = 512;  // classes per ce_grad wave that sums dQ
@@ -537,11 +537,12 @@ __device__ __forceinline__ bf16x8 frag(const uint4* __restrict__ f, int at, int 
   return __builtin_bit_cast(bf16x8, f[(size_t)at * 64 + lane]);
 }
 
-// e^d for the terms of a softmax, d <= 0 up to rounding: one product and the
-// hardware's 2^x.  The product's rounding makes the relative error about
+// e^d for the terms of the prediction's softmax, d <= 0 up to rounding: one product
+// and the hardware's 2^x.  The product's rounding makes the relative error about
 // 1e-7 |d|, and a term weighs e^d, so a sum relative to its largest term is off by
 // at most 4e-8 per term, as with expf (whose range handling costs a dozen more
-// instructions per logit).
+// instructions per logit).  Training takes expf: there each term is a gradient of
+// its own, and errors of 1e-7 |d| turned roundings to BF16 (13 us of a step).
 __device__ __forceinline__ float exp_term(float d) { return __builtin_amdgcn_exp2f(d * 1.44269504088896340736f); }
 
 // (m, s) <- the log-sum-exp pair of the union of two sets: max and exp-sum relative to it.
@@ -578,7 +579,7 @@ __global__ __launch_bounds__(256) void ce_stats(const uint4* __restrict__ qa, in
         m[k] = mx;
       }
       // a group whose classes are all padding so far keeps its empty sum
-      if (m[k] > -INFINITY) s[k] += (exp_term(x0 - m[k]) + exp_term(x1 - m[k])) + (exp_term(x2 - m[k]) + exp_term(x3 - m[k]));
+      if (m[k] > -INFINITY) s[k] += (expf(x0 - m[k]) + expf(x1 - m[k])) + (expf(x2 - m[k]) + expf(x3 - m[k]));
     }
   }
   // the four lane groups hold quarters of the chunk's classes
@@ -639,7 +640,7 @@ __global__ __launch_bounds__(256) void ce_finish(const float* pm, const float* p
 
 // dL of one logit: (softmax - onehot) / n.
 __device__ __forceinline__ float ce_dl(float logit, float bias, float lse, bool hot, float inv_n) {
-  return (exp_term(logit + bias - lse) - (hot ? 1.f : 0.f)) * inv_n;
+  return (expf(logit + bias - lse) - (hot ? 1.f : 0.f)) * inv_n;
 }
 
 // Two kinds of workgroup in one launch, so that both fill the chip together.
