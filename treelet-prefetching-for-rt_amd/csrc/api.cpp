@@ -821,10 +821,10 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
   uint32_t* main_slot = p.ray_counter;
   const TraceParams scene_params = p;  // for the level pass
   // One ray range of a slab traversal (all of it when it fits): traced, its
-  // counts scanned into offsets[b..e] (plus the previous ranges' total), its
-  // slabs compacted.  The ranges share the control slot: its ray counter is
-  // cleared between them, its error word and word 2 (the rays whose records
-  // overflowed their slab) collect all of them.
+  // offsets[b..e] formed (going on from the previous range's) and its rows
+  // expanded.  The ranges share the control slot: its ray counter is cleared
+  // between them, its error word and word 2 (the rays whose records overflowed
+  // their slab) collect all of them.
   auto slab_range = [&](uint32_t b, uint32_t e, bool last) -> rtx_status {
     TraceParams q = p;
     q.rays = rays + b;

@@ -449,7 +449,7 @@ void trace_kernel(TraceParams p) {
       // a slab keeps the ray's first record_slab records, the rest are written
       // by a second pass over the rays that had more.  The entry holds what
       // the traversal knows; the owner and layout lookups wait for the
-      // compaction, off the traversal's dependent chain.  It goes to the
+      // expansion, off the traversal's dependent chain.  It goes to the
       // lane's LDS ring first (flush_slab_group writes it out).
       const uint32_t slot = (uint32_t)(off >> 6);
       if constexpr (REC == kRecSlab4)
