@@ -89,3 +89,35 @@ def test_small_batches_by_place_and_by_counter(gpu, rtx, oracle, instanced, mode
                                 waves_per_cu=waves_per_cu, **claim) == 0
         assert_hits_equal(hb.download(rtx.HIT_DTYPE, n), h_ref, "hits with records")
         assert_records_equal(ob.download(np.uint64, n + 1), recb.download(rtx.RECORD_DTYPE, int(o_ref[-1])), o_ref, r_ref, "records")
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_overflows_of_an_earlier_range_are_traced_again(gpu, rtx, oracle, mode):
+    """2^31 entries hold 2,097,152 rays of 1,024-entry rows: 100 rays more are a second
+    range of their own, small enough for the one-launch finish.  Rays with more records
+    than a row lie in both ranges; all of them are complete.  Nearly all other rays
+    miss the scene (one record each)."""
+    d = rtx.workload_desc(rtx.WORKLOAD_INSTANCED_SPHERES, n_instances=600, slices=8, stacks=4, shared_blas=0, width=8,
+                          height=8, seed=11, box_size=0.5)
+    scene = rtx.workload_scene(d)
+    long = rtx.primary_rays(d)
+    gpu.set_scene(scene.arena, scene.tlas_offset)
+    gpu.build_treelets(1024)
+    part = oracle.Partition(scene.arena, scene.tlas_offset, 1024)
+    h_ref, o_ref, r_ref = oracle.trace(scene.arena, scene.tlas_offset, long, mode=mode, partition=part)
+    counts = np.diff(o_ref).astype(np.int64)
+    over = np.flatnonzero(counts > 1024)
+    assert len(over) >= 8
+    n = (1 << 21) + 100
+    rays = np.repeat(long[:1], n)
+    rays["org"], rays["dir"] = 1e6, (0.0, 0.0, 1.0)
+    # the traced rays: those with long rows, in the first range but for the last three
+    at = np.concatenate([np.arange(len(over) - 3) * 7919 + 5, n - 1 - 30 * np.arange(3)[::-1]])
+    rays[at] = long[over]
+    h, o, r = gpu.trace(rays, mode=mode, records=True, record_slab=1024, records_per_ray=4)
+    want = np.ones(n, np.uint64)
+    want[at] = counts[over]
+    assert np.array_equal(o, np.concatenate([[np.uint64(0)], np.cumsum(want)]))
+    assert_hits_equal(h[at], h_ref[over], "hits")
+    for ray, k in zip(at, over):
+        assert np.array_equal(r[o[ray]:o[ray + 1]], r_ref[o_ref[k]:o_ref[k + 1]]), f"ray {ray}"

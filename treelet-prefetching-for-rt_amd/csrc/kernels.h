@@ -221,9 +221,10 @@ __host__ __device__ inline uint32_t slab_entry4(uint32_t slot, uint32_t type, ui
 // first `slab` entries as rtx_records at its offset (owner and layout_remap
 // nullable, as in TraceParams), rays with more than `slab` records appended to
 // overflow_list as ray_base + their index (count in overflow_count, which must
-// start at 0).  With add_base the offsets go on from offsets[0].  No record is
-// written when the total exceeds `capacity`.  host (nullable, mapped host memory):
-// host[0] = *overflow_count, host[2..3] = offsets[n].
+// start at 0 with a batch's first range).  With add_base the offsets go on from
+// offsets[0], and the list and its count from the batch's earlier ranges.  No
+// record is written when the total exceeds `capacity`.  host (nullable, mapped host
+// memory): host[0] = the batch's overflowed rays so far, host[2..3] = offsets[n].
 struct FinishParams {
   const uint32_t* counts;
   uint32_t n;
@@ -245,7 +246,7 @@ struct FinishParams {
   uint32_t* host;
   const uint64_t* tile_sums;  // set by launch_finish_records
 };
-// Batches of at most this many rays sum their counts in every workgroup (64 KiB
+// Batches of at most this many rays sum their counts in every workgroup (32 KiB
 // of counts from L2) instead of in a launch of its own.
 constexpr uint32_t kFinishAlone = 8192;
 // tile_sums: n / 1024 + 1 words

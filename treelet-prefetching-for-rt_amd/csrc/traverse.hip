@@ -2060,7 +2060,10 @@ __global__ void report_total_kernel(const uint64_t* total, uint32_t* host) {
 // tiles before its own), and the expansion.  A batch of at most kFinishAlone rays
 // takes one launch, whose workgroups sum the counts themselves and expand their
 // own 256 rays: six launches and 12 us less than scans, clear, compaction and
-// report had for a 32-ray batch (122 -> 110 us).
+// report had for a 32-ray batch (122 -> 110 us).  It reports the overflows it has
+// counted itself, for which its workgroups need not wait for each other; a later
+// range of a batch, whose report is of all ranges, takes the three launches
+// whatever its size.
 //
 // The expansion reads 128 MB and writes 468 MB for the 28M records of 1.34M rays
 // (100 us at this card's rates) but is bound by the address units: each record
@@ -2165,8 +2168,8 @@ __global__ __launch_bounds__(kScanBlock) void place_records(FinishParams p) {
   }
 }
 
-// A small batch at once: offsets and records of 256 rays, the workgroups all
-// summing the batch's counts.
+// A small batch of one range at once: offsets and records of 256 rays, the
+// workgroups all summing the batch's counts.
 template <typename E>
 __global__ __launch_bounds__(kScanBlock) void finish_records(FinishParams p) {
   __shared__ uint64_t smem[4];
@@ -2186,17 +2189,16 @@ __global__ __launch_bounds__(kScanBlock) void finish_records(FinishParams p) {
   block_exclusive_scan(all, smem, n_all);
   block_exclusive_scan(before, smem, n_before);
   block_exclusive_scan(over, smem, n_over);
-  const uint64_t base = p.add_base ? p.offsets[0] : 0;
   const uint32_t r = first + tid;
   const uint32_t cnt = r < p.n ? p.counts[r] : 0u;
   if (cnt > p.slab) p.overflow_list[atomicAdd(p.overflow_count, 1u)] = p.ray_base + r;
-  const uint64_t at = base + n_before + block_exclusive_scan(cnt, smem, n_mine);
-  if (r < p.n && (r > 0 || !p.add_base)) p.offsets[r] = at;
+  const uint64_t at = n_before + block_exclusive_scan(cnt, smem, n_mine);
+  if (r < p.n) p.offsets[r] = at;
   if (blockIdx.x == 0 && tid == 0) {
-    p.offsets[p.n] = base + n_all;
-    report_records(p, (uint32_t)n_over, base + n_all);
+    p.offsets[p.n] = n_all;
+    report_records(p, (uint32_t)n_over, n_all);
   }
-  if (base + n_all > p.capacity) return;  // the caller reports RTX_ERR_TRACE_OVERFLOW
+  if (n_all > p.capacity) return;  // the caller reports RTX_ERR_TRACE_OVERFLOW
   for (uint32_t i = lane >> 3; i < 64; i += 8) {  // lanes 8g .. 8g + 7: rays g, g + 8, ... of the wave
     const uint32_t c = min((uint32_t)__shfl(cnt, (int)i, 64), p.slab);
     const uint64_t o = (uint64_t)__shfl((uint32_t)at, (int)i, 64) | ((uint64_t)__shfl((uint32_t)(at >> 32), (int)i, 64) << 32);
@@ -2419,7 +2421,7 @@ hipError_t launch_trace_stats(const rtx_hit* hits, uint32_t n, const rtx_record*
 hipError_t launch_finish_records(FinishParams p, uint64_t* tile_sums, hipStream_t s) {
   if (p.n == 0 || p.slab == 0) return hipSuccess;
   const uint32_t grid = (p.n + kScanBlock - 1) / kScanBlock;
-  if (p.n <= kFinishAlone) {
+  if (p.n <= kFinishAlone && !p.add_base) {
     if (p.shift)
       hipLaunchKernelGGL(finish_records<uint32_t>, dim3(grid), dim3(kScanBlock), 0, s, p);
     else
