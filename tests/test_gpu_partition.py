@@ -45,3 +45,32 @@ def test_partition_matches_the_oracle(rtx, oracle, n_inst, slices, stacks, share
         staged = ctx.trace(rays, mode=rtx.MODE_TREELET, prefetch=rtx.PREFETCH_ALWAYS, stage_bytes=8192)
         assert ctx.prefetch_stats()["lds_hits"] > 0
         assert plain.tobytes() == staged.tobytes()
+
+
+def test_lists_past_their_room_are_reported(rtx, oracle):
+    """20,000 instances of 16 shared meshes: at 2 KiB the treelets' lists outgrow the room
+    for them in a round of the eight-lane kernel, in the middle of a batch of rounds (at
+    8 KiB in a round of the one-wave kernel).  The build reports it, and the next one, whose
+    lists fit, is the oracle's."""
+    rng = np.random.default_rng(5)
+    builder = rtx.SceneBuilder()
+    blas = [builder.add_blas(rtx.displaced_sphere(64, 32, 1.0, 0.05, seed=1 + i)) for i in range(16)]
+    for i in range(20000):
+        m = np.zeros((3, 4), np.float32)
+        m[:, :3] = np.eye(3) * 0.5
+        m[:, 3] = rng.uniform(0, 60, 3)
+        builder.add_instance(int(blas[i % 16]), m, instance_id=i)
+    scene = builder.finish()
+    with rtx.Context(0) as ctx:
+        ctx.set_scene(scene.arena, scene.tlas_offset)
+        for budget in (2048, 8192):
+            with pytest.raises(rtx.RtxError) as e:
+                ctx.build_treelets(budget)
+            assert e.value.status == 12  # out of memory
+        ctx.build_treelets(256)
+        part = oracle.Partition(scene.arena, scene.tlas_offset, 256)
+        t = ctx.get_treelets()
+        assert np.array_equal(t["roots"], part.roots)
+        assert np.array_equal(t["list_offsets"], part.list_offsets)
+        assert np.array_equal(t["list_nodes"], part.list_nodes)
+        assert np.array_equal(t["owner"], part.owner)

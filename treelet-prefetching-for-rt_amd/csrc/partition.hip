@@ -192,6 +192,7 @@ __global__ __launch_bounds__(256) void form_small(FormParams p) {
   __shared__ uint8_t qk[kSmallGroups * kSmallStride];
   __shared__ uint32_t g_list[kSmallGroups], g_pend[kSmallGroups], g_big[kSmallGroups];
   __shared__ unsigned long long list_base;
+  __shared__ bool listed;  // the workgroup's lists have their place
   const uint32_t lane = threadIdx.x & 63u, j = threadIdx.x & (kSmallLanes - 1), g = threadIdx.x / kSmallLanes;
   const uint32_t gsh = lane & ~(kSmallLanes - 1);  // the group's first lane in its wave
   uint32_t* Q = qs + g * kSmallStride;
@@ -292,7 +293,10 @@ __global__ __launch_bounds__(256) void form_small(FormParams p) {
     }
     __syncthreads();
     if (threadIdx.x < 64) {
-      // the first wave reserves the workgroup's places (exclusive prefixes per group)
+      // The first wave reserves the workgroup's places (exclusive prefixes per group).
+      // Roots are counted into the next frontier only once the lists have theirs: the
+      // host looks at the error word after a few rounds, and until then every counted
+      // frontier place has to hold an entry.
       const bool in = lane < kSmallGroups;
       const uint32_t nl = in ? g_list[lane] : 0u, np = in ? g_pend[lane] : 0u, nb = in ? g_big[lane] : 0u;
       const uint32_t li = wave_incl_scan<uint32_t>(nl, lane), pi = wave_incl_scan<uint32_t>(np, lane),
@@ -305,7 +309,9 @@ __global__ __launch_bounds__(256) void form_small(FormParams p) {
         list_base = lt ? atomicAdd(&p.tot->listed, (unsigned long long)lt) : 0ull;
         sum_nodes += lt;
         max_nodes = max(max_nodes, mx);
-        if (pt) po = atomicAdd(&p.cnt[p.round + 1], pt);
+        listed = lt == 0 || list_base + lt <= p.raw_cap;
+        if (!listed) atomicOr(&p.tot->error, kErrQueue);
+        if (pt && listed) po = atomicAdd(&p.cnt[p.round + 1], pt);
         if (bt) bo = atomicAdd(&p.nbig[p.round], bt);
       }
       po = __shfl(po, 0, 64);
@@ -318,24 +324,20 @@ __global__ __launch_bounds__(256) void form_small(FormParams p) {
     }
     __syncthreads();
     if (large && j == 0) p.big[g_big[g]] = idx;
-    if (done) {
+    if (done && listed) {
       const unsigned long long pos = list_base + g_list[g];
-      if (pos + head > p.raw_cap) {
-        if (j == 0) atomicOr(&p.tot->error, kErrQueue);
-      } else {
-        // Q[0, head) was overwritten by nothing: the roots moved to head and on
-        bool twice = false;
-        for (uint32_t k = j; k < head; k += kSmallLanes) {
-          const uint32_t s = Q[k];
-          p.raw_list[pos + k] = s;
-          p.kind[s] = slot_kind(K[k]);
-          twice |= atomicMax(&p.owner_root1[s], root_slot + 1) != 0u;
-        }
-        if (twice) atomicOr(&p.tot->shared, 1u);
-        if (j == 0) p.desc[base + idx] = make_uint4(root_slot, (uint32_t)pos, head, head * 64u);
-        for (uint32_t k = j; k < pend; k += kSmallLanes)
-          p.out[g_pend[g] + k] = qentry(Q[head + k], K[head + k]);
+      // Q[0, head) was overwritten by nothing: the roots moved to head and on
+      bool twice = false;
+      for (uint32_t k = j; k < head; k += kSmallLanes) {
+        const uint32_t s = Q[k];
+        p.raw_list[pos + k] = s;
+        p.kind[s] = slot_kind(K[k]);
+        twice |= atomicMax(&p.owner_root1[s], root_slot + 1) != 0u;
       }
+      if (twice) atomicOr(&p.tot->shared, 1u);
+      if (j == 0) p.desc[base + idx] = make_uint4(root_slot, (uint32_t)pos, head, head * 64u);
+      for (uint32_t k = j; k < pend; k += kSmallLanes)
+        p.out[g_pend[g] + k] = qentry(Q[head + k], K[head + k]);
     }
     __syncthreads();
   }
