@@ -1268,9 +1268,13 @@ rtx_status rtx_mlp_predict(rtx_mlp* m, const rtx_mlp_sample* samples, uint32_t n
   if (!m || !samples || !top4_dev || n == 0) return RTX_ERR_INVALID_ARGUMENT;
   MK(hipSetDevice(m->device));
   if (!m->pred_q) {
+    // both or neither
     if (hipMalloc(&m->pred_q, (size_t)kPredRows * kEmb * 4) != hipSuccess ||
         hipMalloc(&m->pred_part, (size_t)kPredParts * sizeof(Top4)) != hipSuccess) {
       (void)hipGetLastError();
+      if (m->pred_q) (void)hipFree(m->pred_q);
+      m->pred_q = nullptr;
+      m->pred_part = nullptr;
       return RTX_ERR_OUT_OF_MEMORY;
     }
   }
