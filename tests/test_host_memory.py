@@ -66,3 +66,30 @@ def test_prediction_after_a_failed_allocation(fake_hip):
         net2.predict(samples, n=50)
         assert fake.fake_live() - before > 16 * MIB
     """)
+
+
+TRACE = """
+scene = rtx.workload_scene(rtx.workload_desc(rtx.WORKLOAD_SPHERE_AND_QUAD, slices=16, stacks=8, width=8, height=8, seed=1))
+ctx.set_scene(scene.arena, scene.tlas_offset)
+owner = np.zeros(len(scene.arena) // 64, np.uint32)
+tlas = np.array([scene.tlas_offset], np.uint64)
+ctx.set_treelets(8192, tlas, np.array([0, 1], np.uint64), tlas, owner)
+dummy = rtx.DeviceBuffer(ctx, 64)  # (no kernel runs: rays and hits are never read)
+def trace(n, mode, **kw):
+    fake.fake_reset()
+    before = fake.fake_live()
+    status = ctx.trace_device(dummy, n, dummy, mode=mode, **kw)
+    return status, (fake.fake_peak() - before) / MIB
+"""
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_eight_lanes_per_ray_take_no_spill_area(fake_hip, mode):
+    """The eight-lanes kernel keeps its stacks in LDS: a call of any size that asks for it
+    allocates nothing for them."""
+    _run(fake_hip, TRACE + f"""
+status, mib = trace(50_000_000, {mode}, lanes_per_ray=8)
+assert status == 0 and mib < 1, (status, mib)
+status, mib = trace(1000, {mode})
+assert status == 0 and mib < 1, (status, mib)
+""")

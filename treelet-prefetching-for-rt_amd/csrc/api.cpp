@@ -725,8 +725,9 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
   const uint32_t spill_cap = 128;
   const uint32_t ns = opts->mode == RTX_MODE_TREELET ? 2 : 1;
   // treelet order with staging or records keeps fewer entries in LDS (trace_kernel's R)
-  // (the eight-lanes kernel spills nothing; a second pass of its rays may)
-  const uint32_t spill_grid = wide ? (n + bs - 1) / bs : grid;
+  // (The eight-lanes kernel spills nothing.  With records, which it takes only for small
+  // batches, a second pass of its rays may.)
+  const uint32_t spill_grid = !wide ? grid : use_slab ? (n + bs - 1) / bs : 0u;
   rtx_status st = ensure_spill(c, (size_t)spill_grid * bs * (spill_cap + (ns == 2 && (stage || use_slab) ? lds_stack : 0)) * ns);
   if (st != RTX_OK) return st;
 
