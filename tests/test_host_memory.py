@@ -93,3 +93,20 @@ assert status == 0 and mib < 1, (status, mib)
 status, mib = trace(1000, {mode})
 assert status == 0 and mib < 1, (status, mib)
 """)
+
+
+def test_a_spill_area_of_the_size_asked_for_is_enough(fake_hip):
+    """A launch that fills the GPU asks for more than its own spill area, so that one with
+    other options finds room; where that cannot be had, its own is enough."""
+    _run(fake_hip, TRACE + """
+fake.fake_limit(fake.fake_live() + 300 * MIB)
+status, mib = trace(2_000_000, 0)
+assert status == 0 and 0 < mib <= 300, (status, mib)
+status, mib = trace(2_000_000, 0)
+assert status == 0 and mib == 0, (status, mib)
+status, _ = trace(2_000_000, 1)  # 512 MiB of its own
+assert status == 7, status
+fake.fake_limit(2**63)
+status, mib = trace(2_000_000, 1)
+assert status == 0 and mib > 500, (status, mib)
+""")

@@ -197,14 +197,22 @@ uint32_t default_refill(uint64_t arena_bytes) { return arena_bytes > (400ull << 
 
 // A launch that fills the GPU gets room for any such launch (treelet order, four
 // blocks on a CU, 544 MiB on 256 CUs), so that one with another option later does
-// not free and allocate again (0.6 ms).
+// not free and allocate again (0.6 ms; a first allocation of 320 and of 544 MiB take
+// 25-90 us alike).  Where that cannot be had, its own room is enough.
 rtx_status ensure_spill(rtx_ctx* c, size_t entries) {
   if (entries <= c->spill_entries) return RTX_OK;
-  const size_t full = (size_t)c->n_cus * 1024 * (128 + 8) * 2;
-  if (entries > full / 4) entries = std::max(entries, full);
   if (c->spill) HIP_TRY(hipFree(c->spill));
   c->spill = nullptr;
   c->spill_entries = 0;
+  const size_t full = (size_t)c->n_cus * 1024 * (128 + 8) * 2;
+  if (entries > full / 4 && entries < full) {
+    if (hipMalloc(&c->spill, full * sizeof(uint64_t)) == hipSuccess) {
+      c->spill_entries = full;
+      return RTX_OK;
+    }
+    (void)hipGetLastError();
+    c->spill = nullptr;
+  }
   HIP_TRY(hipMalloc(&c->spill, entries * sizeof(uint64_t)));
   c->spill_entries = entries;
   return RTX_OK;
