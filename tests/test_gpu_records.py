@@ -92,11 +92,13 @@ def test_small_batches_by_place_and_by_counter(gpu, rtx, oracle, instanced, mode
 
 
 @pytest.mark.parametrize("mode", [0, 1])
-def test_overflows_of_an_earlier_range_are_traced_again(gpu, rtx, oracle, mode):
+@pytest.mark.parametrize("n,slab", [((1 << 21) + 100, 1024), (1 << 22, 0), ((1 << 22) + 1, 0), ((1 << 23) + 1000, 0)])
+def test_long_rays_in_large_batches(gpu, rtx, oracle, mode, n, slab):
     """2^31 entries hold 2,097,152 rays of 1,024-entry rows: 100 rays more are a second
     range of their own, small enough for the one-launch finish.  Rays with more records
-    than a row lie in both ranges; all of them are complete.  Nearly all other rays
-    miss the scene (one record each)."""
+    than a row lie in both ranges; all of them are complete.  Also one range of 4,096
+    tiles and one ray more, where the tiles' sums are scanned, and two ranges of default
+    rows.  Nearly all other rays miss the scene (one record each)."""
     d = rtx.workload_desc(rtx.WORKLOAD_INSTANCED_SPHERES, n_instances=600, slices=8, stacks=4, shared_blas=0, width=8,
                           height=8, seed=11, box_size=0.5)
     scene = rtx.workload_scene(d)
@@ -108,13 +110,12 @@ def test_overflows_of_an_earlier_range_are_traced_again(gpu, rtx, oracle, mode):
     counts = np.diff(o_ref).astype(np.int64)
     over = np.flatnonzero(counts > 1024)
     assert len(over) >= 8
-    n = (1 << 21) + 100
     rays = np.repeat(long[:1], n)
     rays["org"], rays["dir"] = 1e6, (0.0, 0.0, 1.0)
     # the traced rays: those with long rows, in the first range but for the last three
     at = np.concatenate([np.arange(len(over) - 3) * 7919 + 5, n - 1 - 30 * np.arange(3)[::-1]])
     rays[at] = long[over]
-    h, o, r = gpu.trace(rays, mode=mode, records=True, record_slab=1024, records_per_ray=4)
+    h, o, r = gpu.trace(rays, mode=mode, records=True, record_slab=slab, records_per_ray=2)
     want = np.ones(n, np.uint64)
     want[at] = counts[over]
     assert np.array_equal(o, np.concatenate([[np.uint64(0)], np.cumsum(want)]))

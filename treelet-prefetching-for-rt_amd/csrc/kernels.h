@@ -249,7 +249,12 @@ struct FinishParams {
 // Batches of at most this many rays sum their counts in every workgroup (32 KiB
 // of counts from L2) instead of in a launch of its own.
 constexpr uint32_t kFinishAlone = 8192;
-// tile_sums: n / 1024 + 1 words
+// Larger ones: up to this many tiles of 1,024 rays each workgroup sums them all, which
+// costs the square of their number; more (ranges of short rows have up to 262,144) are
+// scanned in a launch of their own.  1,024 / 4,096 / 8,192 / 32,768 tiles, us: summed
+// 8.5 / 26 / 62 / 589, scanned 11 / 30 / 54 / 198.
+constexpr uint32_t kTilesSummed = 4096;
+// tile_sums: a word for each 1,024 rays begun, and one more
 hipError_t launch_finish_records(FinishParams p, uint64_t* tile_sums, hipStream_t s);
 
 }  // namespace rtxk

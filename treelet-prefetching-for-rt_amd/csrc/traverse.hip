@@ -2057,7 +2057,7 @@ __global__ void report_total_kernel(const uint64_t* total, uint32_t* host) {
 // ---- slab records -> CSR ----------------------------------------------------
 // Three launches: record sums of tiles of kScanTile rays (with the list of rays whose
 // records overflowed their slab), the rays' offsets (each workgroup summing the
-// tiles before its own), and the expansion.  A batch of at most kFinishAlone rays
+// tiles before its own; a scan before it for many tiles), and the expansion.  A batch of at most kFinishAlone rays
 // takes one launch, whose workgroups sum the counts themselves and expand their
 // own 256 rays: six launches and 12 us less than scans, clear, compaction and
 // report had for a 32-ray batch (122 -> 110 us).  It reports the overflows it has
@@ -2135,19 +2135,26 @@ __device__ __forceinline__ void expand_row(const FinishParams& p, uint64_t ray, 
   }
 }
 
-// Offsets of a tile's rays.
+// Offsets of a tile's rays.  The workgroups of up to kTilesSummed tiles sum all tiles
+// each; more are scanned before (tile_sums then holds the sums before each tile, and
+// all tiles' sum behind them).
 __global__ __launch_bounds__(kScanBlock) void place_records(FinishParams p) {
   __shared__ uint64_t smem[4];
   const uint32_t tid = threadIdx.x;
-  uint64_t all = 0, before = 0;
-  for (uint32_t i = tid; i < p.n_tiles; i += kScanBlock) {
-    const uint64_t v = p.tile_sums[i];
-    all += v;
-    before += i < blockIdx.x ? v : 0u;
-  }
   uint64_t n_all, n_before, n_mine;
-  block_exclusive_scan(all, smem, n_all);
-  block_exclusive_scan(before, smem, n_before);
+  if (p.n_tiles > kTilesSummed) {
+    n_before = p.tile_sums[blockIdx.x];
+    n_all = p.tile_sums[p.n_tiles];
+  } else {
+    uint64_t all = 0, before = 0;
+    for (uint32_t i = tid; i < p.n_tiles; i += kScanBlock) {
+      const uint64_t v = p.tile_sums[i];
+      all += v;
+      before += i < blockIdx.x ? v : 0u;
+    }
+    block_exclusive_scan(all, smem, n_all);
+    block_exclusive_scan(before, smem, n_before);
+  }
   const uint64_t base = p.add_base ? p.offsets[0] : 0;
   const uint64_t r = (uint64_t)blockIdx.x * kScanTile + tid * kScanItems;
   uint32_t c[kScanItems], sum = 0;
@@ -2432,6 +2439,8 @@ hipError_t launch_finish_records(FinishParams p, uint64_t* tile_sums, hipStream_
   p.tile_sums = tile_sums;
   hipLaunchKernelGGL(sum_record_tiles, dim3(p.n_tiles), dim3(kScanBlock), 0, s, p.counts, p.n, p.slab, tile_sums,
                      p.ray_base, p.overflow_list, p.overflow_count);
+  if (p.n_tiles > kTilesSummed)
+    hipLaunchKernelGGL(scan_sums, dim3(1), dim3(kScanBlock), 0, s, tile_sums, p.n_tiles, tile_sums, p.n_tiles);
   hipLaunchKernelGGL(place_records, dim3(p.n_tiles), dim3(kScanBlock), 0, s, p);
   const uint32_t chunks = std::min<uint32_t>(2048, grid);
   if (p.shift)
