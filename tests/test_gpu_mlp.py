@@ -212,3 +212,36 @@ def test_predict_of_ordered_classes(gpu, T, C, n, order):
         assert np.allclose(prob, np.tile((e / e.sum())[best], (n, 1)), rtol=3e-5, atol=1e-30)
     finally:
         mlp.close()
+
+
+def _bias_network(gpu, T, o):
+    """A network whose logits are exactly the class biases o."""
+    mlp = gpu.mlp(T, len(o), seed=1)
+    p = np.zeros_like(mlp.params())
+    p[-len(o):] = o
+    mlp.set_params(p)
+    return mlp
+
+
+def test_probability_of_a_confident_class(gpu):
+    """One class far above those before it, which met a lower maximum: its exponential
+    dominates the sum.  To the top probability's relative error the hardware's 2^x and
+    the two expf that refer sums to another maximum add at most 2^-23 each, and seven
+    roundings (of the corrected exponential, the reference changes, three merges and the
+    division) 2^-24 each."""
+    C, T, tol = 160, 4, 13 * 2.0 ** -24
+    rng = np.random.default_rng(3)
+    s = _samples(np.random.default_rng(5), T, C, 33)
+    for d in np.linspace(0.5, 31.5, 125):
+        o = np.sort(rng.uniform(-0.4, 0.0, C).astype(np.float32))[::-1].copy()
+        at = int(rng.integers(64, C))
+        o[at] = np.float32(d) + np.float32(rng.uniform(0, 0.25))
+        mlp = _bias_network(gpu, T, o)
+        try:
+            top, prob = mlp.predict(s)
+        finally:
+            mlp.close()
+        e = np.exp(o.astype(np.float64) - float(o.max()))
+        want = 1.0 / e.sum()
+        assert np.all(top[:, 0] == at)
+        assert np.all(np.abs(prob[:, 0] - want) <= tol * want), (d, np.max(np.abs(prob[:, 0] / want - 1)))
