@@ -245,3 +245,22 @@ def test_probability_of_a_confident_class(gpu):
         want = 1.0 / e.sum()
         assert np.all(top[:, 0] == at)
         assert np.all(np.abs(prob[:, 0] - want) <= tol * want), (d, np.max(np.abs(prob[:, 0] / want - 1)))
+
+
+@pytest.mark.parametrize("C,nan", [(200, slice(0, 40)), (20, slice(4, 8)), (700, slice(0, 4)), (700, slice(690, 700))])
+def test_a_nan_logit_reaches_probabilities_and_loss(gpu, C, nan):
+    """A NaN among the logits makes the sum of exponentials NaN, wherever it stands: also in
+    the classes that a lane meets first, and beside the padding of a tile."""
+    T, n = 4, 40
+    o = np.random.default_rng(C).uniform(-1, 1, C).astype(np.float32)
+    o[nan] = np.nan
+    s = _samples(np.random.default_rng(6), T, C, n)
+    s["target"] = 10 if C != 200 else 100
+    mlp = _bias_network(gpu, T, o)
+    try:
+        top, prob = mlp.predict(s)
+        assert not np.isin(top, np.arange(C)[nan]).any()
+        assert np.isnan(prob).all()
+        assert np.isnan(mlp.loss_grad(s))
+    finally:
+        mlp.close()

@@ -556,9 +556,14 @@ __device__ __forceinline__ float exp_term(float d) {
 }
 
 // (m, s) <- the log-sum-exp pair of the union of two sets: max and exp-sum relative to it.
+// A set without a logit above -inf has an exp-sum of 0, or NaN when one of its logits is
+// NaN.
 __device__ __forceinline__ void lse_merge(float& m, float& s, float m2, float s2) {
   const float mx = fmaxf(m, m2);
-  if (mx == -INFINITY) return;
+  if (mx == -INFINITY) {
+    s += s2;
+    return;
+  }
   s = s * expf(m - mx) + s2 * expf(m2 - mx);
   m = mx;
 }
@@ -588,8 +593,11 @@ __global__ __launch_bounds__(256) void ce_stats(const uint4* __restrict__ qa, in
         s[k] *= expf(m[k] - mx);
         m[k] = mx;
       }
-      // a group whose classes are all padding so far keeps its empty sum
-      if (m[k] > -INFINITY) s[k] += (expf(x0 - m[k]) + expf(x1 - m[k])) + (expf(x2 - m[k]) + expf(x3 - m[k]));
+      // a group whose classes are all padding so far keeps its empty sum, unless one is NaN
+      if (m[k] > -INFINITY)
+        s[k] += (expf(x0 - m[k]) + expf(x1 - m[k])) + (expf(x2 - m[k]) + expf(x3 - m[k]));
+      else if (__builtin_isunordered(x0, x1) || __builtin_isunordered(x2, x3))
+        s[k] = __builtin_nanf("");
     }
   }
   // the four lane groups hold quarters of the chunk's classes
@@ -927,6 +935,10 @@ __global__ __launch_bounds__(256) void logits_top4(const float* __restrict__ Q, 
       if (t.m > -INFINITY)
         t.s += ((exp_term(x[0] - t.m) + exp_term(x[1] - t.m)) + (exp_term(x[2] - t.m) + exp_term(x[3] - t.m))) +
                ((exp_term(x[4] - t.m) + exp_term(x[5] - t.m)) + (exp_term(x[6] - t.m) + exp_term(x[7] - t.m)));
+      else
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (__builtin_isnan(x[i])) t.s = x[i];
     }
   }
   insert_held();
