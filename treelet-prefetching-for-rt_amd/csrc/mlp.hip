@@ -808,8 +808,8 @@ __device__ __forceinline__ bool top4_before(float v, int c, float v2, int c2) {
   return c >= 0 && (c2 < 0 || v > v2 || (v == v2 && c < c2));
 }
 
-// t <- the four best of both, and the exp-sum of the union
-__device__ __forceinline__ void top4_merge(Top4& t, const Top4& o) {
+// t <- the four best of both, and (top4_merge) the exp-sum of the union
+__device__ __forceinline__ void top4_merge_lists(Top4& t, const Top4& o) {
   // Both are sorted, so the four best of the union are the better of t[k] and
   // o[3 - k] for each k; two exchange steps order them.
   float v[4];
@@ -839,6 +839,10 @@ __device__ __forceinline__ void top4_merge(Top4& t, const Top4& o) {
     t.v[k] = v[k];
     t.c[k] = c[k];
   }
+}
+
+__device__ __forceinline__ void top4_merge(Top4& t, const Top4& o) {
+  top4_merge_lists(t, o);
   lse_merge(t.m, t.s, o.m, o.s);
 }
 
@@ -847,7 +851,7 @@ __device__ __forceinline__ void top4_merge(Top4& t, const Top4& o) {
 // columns the wave's samples, so a lane keeps one sample's best four over a
 // quarter of the classes, in registers, and the logits are never stored: 20,011
 // samples x 16,384 classes wrote and read 1.3 GB of them twice (3.4 ms in five
-// products and five scans) and take 0.18 ms here.  Bound by the VALU work on each
+// products and five scans) and take 0.21 ms here.  Bound by the VALU work on each
 // logit: its compare and exponential, then the insertions.  Some lane of a wave
 // has a better logit in nearly every step, so the lanes only put theirs aside
 // (kAside of them, in LDS) and insert together once one lane's places run out;
@@ -856,6 +860,8 @@ __device__ __forceinline__ void top4_merge(Top4& t, const Top4& o) {
 // class wins, and only a lane's own classes come in order).  Each class split
 // starts with empty lists, so there are only as many as one round of workgroups
 // has room for (kPredBlocks): with two rounds, and stages of 256 classes, 0.23 ms.
+// (The two alternatives were measured before exp_term was corrected, when this took
+// 0.18 ms.)
 constexpr int kAside = 11;
 __global__ __launch_bounds__(256) void logits_top4(const float* __restrict__ Q, int n, const float* __restrict__ O,
                                                    const float* __restrict__ cb, int C, int cper, Top4* part) {
@@ -956,12 +962,26 @@ __global__ __launch_bounds__(256) void logits_top4(const float* __restrict__ Q, 
   if (g == 0 && row < n) part[(size_t)blockIdx.y * n + row] = t;
 }
 
-// One thread per row: its class splits merged, then classes and probabilities.
+// One thread per row: its class splits merged, then classes and probabilities.  The
+// splits' exp-sums, of which a few rows have one per 256 classes, are referred to the
+// row's maximum once each and added in FP64: a chain of FP32 merges doubled the error of
+// 64 rows' probabilities over 16,384 classes (7e-8 -> 1.4e-7 for logits within 1).
 __global__ __launch_bounds__(64) void top4_finish(const Top4* part, int n, int splits, uint32_t* out, float* prob) {
   const int r = blockIdx.x * 64 + threadIdx.x;
   if (r >= n) return;
   Top4 t = part[r];
-  for (int k = 1; k < splits; ++k) top4_merge(t, part[(size_t)k * n + r]);
+  for (int k = 1; k < splits; ++k) {
+    const Top4 o = part[(size_t)k * n + r];
+    top4_merge_lists(t, o);
+    t.m = fmaxf(t.m, o.m);
+  }
+  double sum = 0.0;
+  for (int k = 0; k < splits; ++k) {
+    const Top4& o = part[(size_t)k * n + r];
+    // (a set of no logit above -inf has an exp-sum of 0 or NaN)
+    sum += o.m > -INFINITY ? (double)o.s * (double)expf(o.m - t.m) : (double)o.s;
+  }
+  t.s = (float)sum;
   for (int k = 0; k < 4; ++k) out[(size_t)r * 4 + k] = t.c[k] < 0 ? RTX_NO_TREELET : (uint32_t)t.c[k];
   if (prob)
     for (int k = 0; k < 4; ++k) prob[(size_t)r * 4 + k] = t.c[k] < 0 ? 0.f : expf(t.v[k] - t.m) / t.s;
