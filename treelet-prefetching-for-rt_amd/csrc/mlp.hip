@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <climits>
 #include <cmath>
 #include <cstring>
@@ -556,14 +557,11 @@ __device__ __forceinline__ float exp_term(float d) {
 }
 
 // (m, s) <- the log-sum-exp pair of the union of two sets: max and exp-sum relative to it.
-// A set without a logit above -inf has an exp-sum of 0, or NaN when one of its logits is
-// NaN.
+// The maximum of no logits is kLowest, which no finite one is below: terms of -inf (and
+// of padding) are 0 relative to it, and a NaN makes the sum NaN wherever it stands.
+constexpr float kLowest = -FLT_MAX;
 __device__ __forceinline__ void lse_merge(float& m, float& s, float m2, float s2) {
   const float mx = fmaxf(m, m2);
-  if (mx == -INFINITY) {
-    s += s2;
-    return;
-  }
   s = s * expf(m - mx) + s2 * expf(m2 - mx);
   m = mx;
 }
@@ -579,7 +577,7 @@ __global__ __launch_bounds__(256) void ce_stats(const uint4* __restrict__ qa, in
   const int chunk = blockIdx.y * 4 + (threadIdx.x >> 6);
   if (chunk >= nchunk) return;
   const bf16x8 b[2] = {frag(qa, 2 * blockIdx.x, lane), frag(qa, 2 * blockIdx.x + 1, lane)};
-  float m[2] = {-INFINITY, -INFINITY}, s[2] = {0.f, 0.f};
+  float m[2] = {kLowest, kLowest}, s[2] = {0.f, 0.f};
   const int t0 = chunk * (kCeChunk / 16), t1 = min(c_tiles, t0 + kCeChunk / 16);
   for (int ct = t0; ct < t1; ++ct) {
     const bf16x8 a = frag(oa, ct, lane);
@@ -593,11 +591,7 @@ __global__ __launch_bounds__(256) void ce_stats(const uint4* __restrict__ qa, in
         s[k] *= expf(m[k] - mx);
         m[k] = mx;
       }
-      // a group whose classes are all padding so far keeps its empty sum, unless one is NaN
-      if (m[k] > -INFINITY)
-        s[k] += (expf(x0 - m[k]) + expf(x1 - m[k])) + (expf(x2 - m[k]) + expf(x3 - m[k]));
-      else if (__builtin_isunordered(x0, x1) || __builtin_isunordered(x2, x3))
-        s[k] = __builtin_nanf("");
+      s[k] += (expf(x0 - m[k]) + expf(x1 - m[k])) + (expf(x2 - m[k]) + expf(x3 - m[k]));
     }
   }
   // the four lane groups hold quarters of the chunk's classes
@@ -628,7 +622,7 @@ __global__ __launch_bounds__(256) void ce_finish(const float* pm, const float* p
   const int r = blockIdx.x * 4 + w;
   float nll = 0.f;
   if (r < n) {
-    float m = -INFINITY, sm = 0.f;
+    float m = kLowest, sm = 0.f;
     for (int c = lane; c < nchunk; c += 64) lse_merge(m, sm, pm[(size_t)r * nchunk + c], ps[(size_t)r * nchunk + c]);
     for (int o = 32; o > 0; o >>= 1) {
       const float m2 = __shfl_xor(m, o, 64), s2 = __shfl_xor(sm, o, 64);
@@ -877,7 +871,7 @@ __global__ __launch_bounds__(256) void logits_top4(const float* __restrict__ Q, 
     t.v[k] = -INFINITY;
     t.c[k] = -1;
   }
-  t.m = -INFINITY;
+  t.m = kLowest;
   t.s = 0.f;
   int held = 0;  // logits put aside
   float least = -INFINITY, most = -INFINITY;  // what a logit has to exceed; the greatest so far
@@ -938,13 +932,8 @@ __global__ __launch_bounds__(256) void logits_top4(const float* __restrict__ Q, 
         most = fmaxf(most, mx);
         insert_held();
       }
-      if (t.m > -INFINITY)
-        t.s += ((exp_term(x[0] - t.m) + exp_term(x[1] - t.m)) + (exp_term(x[2] - t.m) + exp_term(x[3] - t.m))) +
-               ((exp_term(x[4] - t.m) + exp_term(x[5] - t.m)) + (exp_term(x[6] - t.m) + exp_term(x[7] - t.m)));
-      else
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if (__builtin_isnan(x[i])) t.s = x[i];
+      t.s += ((exp_term(x[0] - t.m) + exp_term(x[1] - t.m)) + (exp_term(x[2] - t.m) + exp_term(x[3] - t.m))) +
+             ((exp_term(x[4] - t.m) + exp_term(x[5] - t.m)) + (exp_term(x[6] - t.m) + exp_term(x[7] - t.m)));
     }
   }
   insert_held();
@@ -978,8 +967,7 @@ __global__ __launch_bounds__(64) void top4_finish(const Top4* part, int n, int s
   double sum = 0.0;
   for (int k = 0; k < splits; ++k) {
     const Top4& o = part[(size_t)k * n + r];
-    // (a set of no logit above -inf has an exp-sum of 0 or NaN)
-    sum += o.m > -INFINITY ? (double)o.s * (double)expf(o.m - t.m) : (double)o.s;
+    sum += (double)o.s * (double)expf(o.m - t.m);
   }
   t.s = (float)sum;
   for (int k = 0; k < 4; ++k) out[(size_t)r * 4 + k] = t.c[k] < 0 ? RTX_NO_TREELET : (uint32_t)t.c[k];
