@@ -174,10 +174,10 @@ typedef struct rtx_trace_options {
   float pred_fraction;   /* LEARNED: share of a predicted treelet's image staged, root first
                             (0 = default 0.25; 1 = the whole image) */
   uint32_t lanes_per_ray; /* 1: one lane per ray; 8: eight lanes per ray, testing a node's six
-                             children at once (either order, no records or staging), for batches
-                             too small to fill the GPU; 0 = 8 without staging when the batch has
-                             at most 128 rays per CU (64 for TREELET with records), else 1.
-                             Results are identical.
+                             children at once (either order), for batches too small to fill the
+                             GPU; 0 = 8 without staging when the batch has at most 128 rays per
+                             CU (64 for TREELET with records), else 1.  An explicit 8 with records
+                             or staging is RTX_ERR_INVALID_ARGUMENT.  Results are identical.
                              rtx_trace only; batches ignore it. */
   uint32_t claim_start;  /* persistent waves claim rays starting at this index and wrap around to 0
                             (outputs stay at input indices).  A batch that holds camera rays followed

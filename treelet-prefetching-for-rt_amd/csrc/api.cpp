@@ -693,7 +693,7 @@ rtx_status trace_impl(rtx_ctx* c, const rtx_ray* rays, uint32_t n, const rtx_tra
     lds_stack = 8;
   }
   // Eight lanes per ray for batches that leave most of the GPU idle (see
-  // wide_rays_per_cu; on request only without records and staging).
+  // wide_rays_per_cu).  Asked for, it is refused with records or staging.
   if (opts->lanes_per_ray != 0 && opts->lanes_per_ray != 1 && opts->lanes_per_ray != kWideRayLanes)
     return RTX_ERR_INVALID_ARGUMENT;
   const bool wide_ok = !opts->emit_records && stage == 0;
@@ -1318,10 +1318,6 @@ bool batch_needs_levels(const rtx_ctx* c, const rtx_batch_job* jobs, uint32_t n_
   return false;
 }
 
-// The level pass of every job whose scene needs it, queued after the batch
-// launch (capturable: the ray counter is cleared by a kernel, and the error
-// word, counters[1], collects the passes' errors with the batch's).  `spill`
-// holds kBatchSpillCap entries per list for min(n_cus, rays / 256) workgroups.
 // After a batch's launches have run: an error-free one needs no read-back (a ray
 // error also sets the mapped host word).
 rtx_status batch_error(rtx_ctx* c, const uint32_t* counters) {
@@ -1331,6 +1327,10 @@ rtx_status batch_error(rtx_ctx* c, const uint32_t* counters) {
   return kernel_error_status(err);
 }
 
+// The level pass of every job whose scene needs it, queued after the batch
+// launch (capturable: the ray counter is cleared by a kernel, and the error
+// word, counters[1], collects the passes' errors with the batch's).  `spill`
+// holds kBatchSpillCap entries per list for min(n_cus, rays / 256) workgroups.
 hipError_t batch_level_passes(rtx_ctx* c, const std::vector<BatchJob>& hj, const rtx_batch_job* jobs,
                               uint32_t n_jobs, uint32_t mode, uint64_t* spill, uint32_t* counters, hipStream_t s) {
   for (uint32_t j = 0; j < n_jobs; ++j) {

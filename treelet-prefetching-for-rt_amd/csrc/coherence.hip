@@ -21,7 +21,7 @@
 // set are sorted (12 for the grid hashes: two passes), the second sort takes
 // chunks, not rays (1.3M rays make some 25,000), and the scratch memory is the
 // context's.  1.29M rays: 1,040 us with two full-width sorts of all rays and
-// their allocations, 205 us now, most of it the latency of 26 launches.
+// their allocations, 205 us now, most of it the latency of 24 launches.
 #include <algorithm>
 #include <cmath>
 

@@ -501,7 +501,7 @@ __global__ __launch_bounds__(256) void weight_grads(WeightGrad w1, WeightGrad w2
 // 16-byte load per lane from L2, used for two tiles: rows staged through LDS had
 // cost sixteen 2-byte LDS reads per lane and 32 classes for the transposed
 // operand, the FP32 conversions again in each workgroup and two barriers per
-// stage.  1,024 rows x 16,384 classes: statistics 28 -> 17 us, both gradients 54
+// stage.  1,024 rows x 16,384 classes: statistics 28 -> 16 us, both gradients 54
 // -> 31 us.  Bound by VALU work on each logit, the exponential above all.
 constexpr int kCeChunk = 256;  // classes per ce_stats wave
 constexpr int kCeCls = 128;    // classes per LDS stage of logits_top4
@@ -545,7 +545,7 @@ __device__ __forceinline__ bf16x8 frag(const uint4* __restrict__ f, int at, int 
 // relative error is at most 1.4e-7, 3.6e-8 in the mean square (expf 8.3e-8 and 2.6e-8);
 // without r it was 1e-7 |d|, with d up to 32 (see logits_top4).  Probabilities against
 // 64 bits are as with expf (1e-7; a class 20 or 28 above the rest 8e-7, without r
-// 1.2e-6).  20,011 rows of 16,384 classes 257 us without r, 282 so, 326 with expf, whose
+// 1.2e-6).  20,011 rows of 16,384 classes 257 us without r, 279 so, 326 with expf, whose
 // range handling takes a dozen more instructions.  Training takes expf: there each term
 // is a gradient of its own.
 __device__ __forceinline__ float exp_term(float d) {
