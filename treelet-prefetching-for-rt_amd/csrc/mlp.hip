@@ -538,22 +538,24 @@ __device__ __forceinline__ bf16x8 frag(const uint4* __restrict__ f, int at, int 
   return __builtin_bit_cast(bf16x8, f[(size_t)at * 64 + lane]);
 }
 
-// e^d for the terms of the prediction's softmax: with h = d log2(e) rounded, e^d is
-// 2^h (1 + r) but for r^2, where r = d - h ln(2), the rounding's error, comes exactly
-// from two FMAs (ln(2) in two parts).  Where h overflows (d of -inf among them) r is no
-// number, and the median with -1 and 1 keeps the term at 0.  For d in [-80, 32] the
-// relative error is at most 1.4e-7, 3.6e-8 in the mean square (expf 8.3e-8 and 2.6e-8);
-// without r it was 1e-7 |d|, with d up to 32 (see logits_top4).  Probabilities against
-// 64 bits are as with expf (1e-7; a class 20 or 28 above the rest 8e-7, without r
-// 1.2e-6).  20,011 rows of 16,384 classes 257 us without r, 279 so, 326 with expf, whose
-// range handling takes a dozen more instructions.  Training takes expf: there each term
-// is a gradient of its own.
+// e^d for the terms of the prediction's softmax: for h near d log2(e), e^d is
+// 2^h (1 + r) but for r^2, where r = d - h ln(2) comes exactly from two FMAs (ln(2) in
+// two parts).  h is taken 8e-6 below the product, more than its rounding, so r lies in
+// [0, 2e-5] and the FMA's clamp to [0, 1], which costs nothing, only touches terms
+// below 1e-37 and those where h overflows (d of -inf among them): r is no number there,
+// and the clamp makes it 0.  For d in [-80, 32] the relative error is at most 1.4e-7,
+// 3.7e-8 in the mean square (expf 8.4e-8 and 2.7e-8); one product and 2^x alone had
+// 1e-7 |d|, with d up to 32 (see logits_top4).  Probabilities against 64 bits are as with
+// expf (1e-7; a class 20 or 28 above the rest 8e-7, with the product alone 1.2e-6).
+// 20,011 rows of 16,384 classes 253 us with the product alone, 268 so, 320 with expf,
+// whose range handling takes a dozen more instructions.  Training takes expf: there each
+// term is a gradient of its own.
 __device__ __forceinline__ float exp_term(float d) {
-  const float h = d * 1.44269504088896340736f;
+  const float h = __builtin_fmaf(d, 1.44269504088896340736f, -8e-6f);
   float r = __builtin_fmaf(h, -0x1.62e430p-1f, d);
   r = __builtin_fmaf(h, 0x1.05c610p-29f, r);
   const float e = __builtin_amdgcn_exp2f(h);
-  return __builtin_fmaf(e, __builtin_amdgcn_fmed3f(r, -1.f, 1.f), e);
+  return __builtin_fmaf(e, __builtin_amdgcn_fmed3f(r, 0.f, 1.f), e);
 }
 
 // (m, s) <- the log-sum-exp pair of the union of two sets: max and exp-sum relative to it.
@@ -845,7 +847,7 @@ __device__ __forceinline__ void top4_merge(Top4& t, const Top4& o) {
 // columns the wave's samples, so a lane keeps one sample's best four over a
 // quarter of the classes, in registers, and the logits are never stored: 20,011
 // samples x 16,384 classes wrote and read 1.3 GB of them twice (3.4 ms in five
-// products and five scans) and take 0.21 ms here.  Bound by the VALU work on each
+// products and five scans) and take 0.20 ms here.  Bound by the VALU work on each
 // logit: its compare and exponential, then the insertions.  Some lane of a wave
 // has a better logit in nearly every step, so the lanes only put theirs aside
 // (kAside of them, in LDS) and insert together once one lane's places run out;
