@@ -547,9 +547,9 @@ __device__ __forceinline__ bf16x8 frag(const uint4* __restrict__ f, int at, int 
 // 3.7e-8 in the mean square (expf 8.4e-8 and 2.7e-8); one product and 2^x alone had
 // 1e-7 |d|, with d up to 32 (see logits_top4).  Probabilities against 64 bits are as with
 // expf (1e-7; a class 20 or 28 above the rest 8e-7, with the product alone 1.2e-6).
-// 20,011 rows of 16,384 classes 253 us with the product alone, 268 so, 320 with expf,
-// whose range handling takes a dozen more instructions.  Training takes expf: there each
-// term is a gradient of its own.
+// 20,011 rows of 16,384 classes take 253 us with the product alone and 268 so; with expf,
+// whose range handling takes a dozen more instructions, 326 beside 257.  Training takes
+// expf: there each term is a gradient of its own.
 __device__ __forceinline__ float exp_term(float d) {
   const float h = __builtin_fmaf(d, 1.44269504088896340736f, -8e-6f);
   float r = __builtin_fmaf(h, -0x1.62e430p-1f, d);
